@@ -209,6 +209,77 @@ _RUN = {"linear": _run_linear, "step": _run_step, "prefill": _run_prefill, "moe"
 
 
 # --------------------------------------------------------------------------------------------------------------
+def _dense(w, rows=None):
+    """Rows of a packed matrix in float64, as the GGUF formats define them."""
+    bb = synth.BLOCK_BYTES[w.type]
+    b = w.data[: w.N * w.row_stride_bytes].view(w.N, w.row_stride_bytes)[:, : w.n_blocks * bb]
+    b = (b if rows is None else b[rows]).unflatten(1, (w.n_blocks, bb))
+
+    def f16(i):
+        return b[:, :, i:i + 2].contiguous().view(torch.float16).double()
+    if w.type == Q6_K:
+        ql, qh = b[:, :, :128].unflatten(2, (2, 2, 32)), b[:, :, 128:192].unflatten(2, (2, 32))
+        q = torch.stack([(ql[:, :, :, t & 1] >> (4 * (t >> 1)) & 15) | (qh >> (2 * t) & 3) << 4 for t in range(4)], 3)
+        sc = b[:, :, 192:208].contiguous().view(torch.int8).double().repeat_interleave(16, 2)
+        return (f16(208) * sc * (q.flatten(2).double() - 32)).flatten(1)
+    s = b[:, :, 4:16].to(torch.int32)
+    lo, mid, hi = s[:, :, :4], s[:, :, 4:8], s[:, :, 8:]
+    sc = torch.cat([lo & 63, hi & 15 | lo >> 6 << 4], 2).double().repeat_interleave(32, 2)
+    mn = torch.cat([mid & 63, hi >> 4 | mid >> 6 << 4], 2).double().repeat_interleave(32, 2)
+    qs = b[:, :, -128:].unflatten(2, (4, 32))
+    q = torch.stack([qs & 15, qs >> 4], 3).flatten(2)
+    if w.type == Q5_K:
+        q = q | torch.stack([b[:, :, 16:48] >> i & 1 for i in range(8)], 2).flatten(2) << 4
+    return (f16(0) * sc * q.double() - f16(2) * mn).flatten(1)
+
+
+def _product(x, w, step=16384):
+    return torch.cat([x @ _dense(w, slice(i, i + step)).T for i in range(0, w.N, step)], 1)
+
+
+def _norm(x, w):
+    return x * torch.rsqrt((x * x).mean(1, keepdim=True) + EPS) * w.double()
+
+
+def _silu_mul(gate_up):
+    gate, up = gate_up.chunk(2, 1)
+    return torch.nn.functional.silu(gate) * up
+
+
+def exact(case, seed):
+    """The outputs of a pass in float64; a prefill's activation rows are bf16, which prefill_rows_bf16 returns."""
+    s, kind = prepare(case, seed), case["kind"]
+    if kind == "embed":
+        return _dense(s["w"], s["rows"].long())
+    x = s["x"].double()
+    if kind == "linear":
+        y = _product(x, s["w"])
+        return y if s["bias"] is None else y + s["bias"].double()
+    if kind == "moe":
+        E, H, I = case["experts"], case["hidden"], case["inter"]
+        top, idx = torch.topk(x @ s["router"].double().T, case["top_k"], dim=1)
+        wt = torch.softmax(top, 1)
+        y = torch.zeros_like(x)
+        for e in range(E):
+            t, slot = (idx == e).nonzero(as_tuple=True)
+            if len(t):
+                xe = x[t]
+                act = _silu_mul(torch.cat([xe @ _dense(w, slice(e * I, e * I + I)).T for w in (s["gate"], s["up"])], 1))
+                y.index_add_(0, t, wt[t, slot, None] * (act @ _dense(s["down"], slice(e * H, e * H + H)).T))
+        return {"y": y, "experts": idx.int(), "weights": wt}
+    rows = (lambda v: v.bfloat16().double()) if kind == "prefill" else (lambda v: v)
+    out = []
+    for l in s["layers"]:
+        out.append(_product(rows(_norm(x, l["norm1"])), l["qkv"]))
+        x = x + _product(rows(l["attn"].double()), l["o"])
+        x = x + _product(rows(_silu_mul(_product(rows(_norm(x, l["norm2"])), l["gate_up"]))), l["down"])
+    if kind == "prefill":
+        return {"qkv": out, "x": x}
+    logits = _product(x, s["head"])
+    value, token = logits.max(1)
+    return {"qkv": out, "x": x, "logits": logits, "token": token.int(), "value": value}
+
+
 def work(case):
     kind = case["kind"]
     if kind == "linear":
