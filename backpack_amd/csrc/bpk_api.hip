@@ -23,6 +23,7 @@ constexpr size_t kPartialFloats = size_t(4) << 20;  // 16 MiB of split-K partial
 constexpr uint32_t kCounters = 1u << 16;
 // bf16 GEMM: two 256 x 256 fp32 slots per workgroup for the runs of cut tiles, a workgroup per CU
 constexpr size_t kGemmPartialFloats = size_t(2) * 256 * 65536;  // 128 MiB
+constexpr size_t kWideBytes = size_t(64) << 20;     // split activations of the many-token kernel: 1100 tokens at K = 14336
 constexpr size_t kMoeWords = size_t(4) << 20;       // 16 MiB of tile records for bpk_kq_moe_matmul
 static_assert(BPK_ARGMAX_STATIC_MAX_ROWS == kq::ARGMAX_MAX_ROWS, "the header's limit is the scratch array's");
 
@@ -81,6 +82,7 @@ struct DeviceState {
     bool ready = false;
     kq::SplitScratch split{};
     kq::SplitScratch gemm_split{};   // of the bf16 GEMM's cut tiles (its own, so that it can run beside a GEMV)
+    void* wide_x = nullptr;          // kWideBytes of split activations (used together with split)
     uint32_t* moe_tiles = nullptr;   // kMoeWords words
     uint32_t* argmax_scratch = nullptr;   // partial values | partial indices | tickets of bpk_argmax_rows
     float* route_logits = nullptr;   // ROUTE_SCRATCH_FLOATS router logits of a route call that does not return them
@@ -97,6 +99,7 @@ void free_device_buffers(DeviceState& st)
     (void)hipFree(st.split.partial);
     (void)hipFree(st.split.counters);
     (void)hipFree(st.gemm_split.partial);
+    (void)hipFree(st.wide_x);
     (void)hipFree(st.moe_tiles);
     (void)hipFree(st.route_logits);
     (void)hipFree(st.argmax_scratch);
@@ -121,6 +124,7 @@ int ensure_device(int device, DeviceState** out)
         if (e == hipSuccess) e = hipMalloc((void**)&st.split.counters, kCounters * sizeof(uint32_t));
         if (e == hipSuccess) e = hipMemset(st.split.counters, 0, kCounters * sizeof(uint32_t));
         if (e == hipSuccess) e = hipMalloc((void**)&st.gemm_split.partial, kGemmPartialFloats * sizeof(float));
+        if (e == hipSuccess) e = hipMalloc(&st.wide_x, kWideBytes);
         if (e == hipSuccess) e = hipMalloc((void**)&st.moe_tiles, kMoeWords * sizeof(uint32_t));
         constexpr size_t kArgmaxWords = (size_t)kq::ARGMAX_MAX_ROWS * (2u * kq::ARGMAX_PARTS + 1u);
         if (e == hipSuccess) e = hipMalloc((void**)&st.argmax_scratch, kArgmaxWords * sizeof(uint32_t));
@@ -185,7 +189,7 @@ const char* bpk_last_kernel(void) { return t_kernel; }
 
 int bpk_force_kernel(int family)
 {
-    if (family < 0 || family > 7) return fail(BPK_ERR_SHAPE, "kernel family %d unknown", family);
+    if (family < 0 || family > 8) return fail(BPK_ERR_SHAPE, "kernel family %d unknown", family);
     t_family = family;
     return BPK_OK;
 }
@@ -444,6 +448,15 @@ int bpk_weight_destroy(bpk_weight* w)
     return e == hipSuccess ? BPK_OK : hip_fail(e, "hipFree(weights)");
 }
 
+// More than 16 tokens, or any number by option.  Measured with the split of X included, us against the 16-token tile
+// kernel: at 17 .. 32 tokens Q4_K 6144x4096 16.7 against 26, 28672x4096 37 against 58, Q6_K 4096x14336 37 against 58,
+// 128256x4096 175 against 396; at 16 tokens 16.3 against 13.6, 30 against 30.6, 32 against 30 (128256 rows: 147
+// against 195, left for a rule of its own).  At 48: 19.6 / 39, 41 / 86, 41.5 / 86, 205 / 599.
+static bool takes_wide(const kq::MatmulArgs& a)
+{
+    return (t_family == 8 || (t_family == 0 && a.M > 16u)) && kq::wide_supported(a);
+}
+
 // fold: the greedy pick over the outputs, taken along by the launch where its kernel can (*folded says so)
 static int matmul_impl(int type, const float* X, const void* W, const float* bias, float* Y, uint32_t M, uint32_t N,
                        uint32_t K, uint32_t n_blocks, uint32_t row_stride_words, uint32_t y_offset, void* stream,
@@ -468,6 +481,12 @@ static int matmul_impl(int type, const float* X, const void* W, const float* bia
     const bool stream_ok = kq::gemv_stream_supported(a);
     const bool mtile_ok = kq::mtile_supported(a);
     if (t_family == 6 && !mtile_ok) return fail(BPK_ERR_SHAPE, "16x16 tile kernel cannot serve this call");
+    if (takes_wide(a)) {
+        t_kernel = "mtile";
+        e = kq::launch_wide(a, st->split, st->wide_x, kWideBytes, t_gemv.splits, s);
+        return e == hipSuccess ? BPK_OK : hip_fail(e, t_kernel);
+    }
+    if (t_family == 8) return fail(BPK_ERR_SHAPE, "many-token kernel cannot serve this call");
     // three and four tokens on the smaller matrices stay on the lanes-along-K kernel (four tokens share every
     // weight load and its unpack).  Measured at M = 4: Q4_K 4096x4096 8.5 against 10.6 us on the tile
     // kernel, 6144x4096 10.8 against 11.8, 28672x4096 32.6 against 19.2; Q6_K 4096x14336 23.2 against 27.0.
@@ -596,6 +615,15 @@ int bpk_kq_matmul_fused(int type, const float* X, const void* W, const float* bi
     if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15u))
         return fail(BPK_ERR_WORKSPACE, "this shape needs a 16-byte aligned workspace of %zu bytes (given %zu)", need,
                     workspace ? workspace_bytes : (size_t)0);
+    // many tokens: prologue, residual and epilogue inside the launches of the many-token kernel
+    if (!t_fused_separate && takes_wide(a)) {
+        t_kernel = "mtile";
+        a.pro = f->prologue; a.norm_w = f->norm_w; a.eps = f->eps; a.residual = f->residual; a.epi = f->epilogue;
+        if (kq::wide_supported(a)) {
+            const hipError_t e = kq::launch_wide(a, st->split, st->wide_x, kWideBytes, t_gemv.splits, s);
+            return e == hipSuccess ? BPK_OK : hip_fail(e, t_kernel);
+        }
+    }
     float* wx = (float*)workspace;
     float* wy = (float*)((uint8_t*)workspace + (need_x ? x_bytes : 0));
     if (need_x) {

@@ -139,6 +139,28 @@ bool mtile_grouped_dual_supported(const MatmulArgs& a);   // a.W2 honoured: Y = 
 hipError_t launch_mtile_grouped(const MatmulArgs& a, const uint32_t* tiles, const uint32_t* n_tiles,
                                 uint32_t tiles_bound, uint32_t cap, hipStream_t s);
 
+// fp32 X of more than 16 tokens (kq_wide.hip): X is split once into fp16 hi + lo operands in scratch, then up to 64
+// tokens share every weight byte.  Honours pro / norm_w / residual / epi, in two launches per x_bytes of split X.
+struct WideX {
+    uint8_t* xa;   // [row][superblock] 1024 bytes of operands
+    uint8_t* xv;   // [row][superblock] 32 bytes: sub-block sums (Q4_K, Q5_K)
+    float* xi;     // [row][superblock] 1 / scale
+};
+bool wide_supported(const MatmulArgs& a);
+// splits: workgroups along K, 0 = automatic
+hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scratch, size_t x_bytes, int splits, hipStream_t s);
+// xv and xi follow xa, or start at rest
+WideX wide_x_layout(void* xa, void* rest, uint32_t rows, uint32_t n_blocks);
+size_t wide_x_bytes(uint32_t rows, uint32_t n_blocks);
+size_t wide_x_rest_bytes(uint32_t rows, uint32_t n_blocks);
+// x.xa may be X (no prologue): every superblock is read before it is written
+hipError_t launch_wide_x(int type, const float* X, int pro, const float* norm_w, float eps, uint32_t rows,
+                         uint32_t n_blocks, const WideX& x, hipStream_t s);
+// grouped by expert: records of up to cap (16, 32, 48, 64) pairs, as launch_moe_group writes them with sets = cap / 2;
+// with a.W2, Y = silu(W x) * (W2 x)
+hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32_t* records, const uint32_t* n_records,
+                               uint32_t bound, uint32_t cap, hipStream_t s);
+
 // Row-per-lane matvec on the matrix cores, M <= 16 dense or grouped by expert.
 bool mrow_supported(const MatmulArgs& a);
 size_t mrow_scratch_floats(const MatmulArgs& a, const GemvTuning& t);

@@ -1,0 +1,611 @@
+// kq_wide.hip — fp32 activations of many tokens against k-quant weights on the matrix cores: up to 64 tokens share
+// every weight byte (decode steps of many sequences, short fp32 batches, mixture layers of a prompt).
+//
+// What bounds it.  The 16-token tile kernel (kq_mtile.hip) walks the weights once per 16 tokens and scales every
+// product of 32 elements on the vector units, once per token: its vector work grows with the tokens and the matrix
+// cores wait.  Here a weight is turned into (quant * sub-block scale) once for all tokens of the workgroup — an
+// integer of at most 63 * 31 (Q4_K, Q5_K), exact in fp16 — so a superblock's 256 elements accumulate in one chain of
+// matrix instructions and the vector units see one fused multiply-add per output and superblock.
+//
+// Activations.  A pass of its own (wide_x_kernel, with the call's prologue folded in) splits fp32 X once per call,
+// where the tile kernel did so in every workgroup: per (token, superblock) a power of two puts the largest magnitude
+// just below 2^15, x * s = hi + lo with both fp16 (22 bits), in operand order, 1 KB; beside it the eight sub-block
+// sums (hi and lo fp16, the factor of the Q4_K / Q5_K minima, one matrix instruction per superblock) and 1 / s.
+//
+// Q6_K.  scale * (q - 32) has up to 13 bits: it is Wh = fp16(product) and the exact rest Wl = fma(scale, q - 32, -Wh),
+// and the product takes three instructions, hi * Wh + lo * Wh + hi * Wl; the dropped lo * Wl is below 2^-22 of x * W.
+//
+// Operand order.  v_mfma_f32_16x16x32_f16 gives lane l eight of the 32 k of row l % 16, and any order of k will do as
+// long as both operands use it.  Lane group kq = l / 16 takes 64 consecutive weights' bytes of the superblock (Q4_K,
+// Q5_K: 32 bytes, sub-blocks 2kq and 2kq+1; Q6_K: 16 positions of a half, all four 32-element runs), so a lane reads
+// its bytes in 16-byte loads and needs two (four) scales per superblock.  Step j of eight multiplies
+//   Q4_K, Q5_K  elements 64 kq + 32 (j & 1) + 8 (j >> 1) ..+7        (low nibbles, then high ones)
+//   Q6_K        elements 128 (kq >> 1) + 32 (j >> 1) + 16 (kq & 1) + 8 (j & 1) ..+7
+// each group of eight in the order 0 2 1 3 4 6 5 7 (what masking dwords leaves).
+//
+// Work split.  Eight waves of two 16-row tiles each; the X of a superblock (TT tiles of 16 tokens, 16 KB each) is
+// staged in LDS (two buffers), shared by the waves.  K is cut over blockIdx.z when rows give too few
+// workgroups; the last one to arrive adds the partial tiles in split order.
+#include "kq_format.h"
+#include "kq_kernels.h"
+#include "kq_wave.h"
+
+namespace kq {
+
+typedef _Float16 w_half8 __attribute__((ext_vector_type(8)));
+typedef _Float16 w_half2 __attribute__((ext_vector_type(2)));
+typedef float w_f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t w_u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t w_u32x2 __attribute__((ext_vector_type(2)));
+
+constexpr int WIDE_WAVES = 8;
+constexpr uint32_t WIDE_XA = 1024, WIDE_XV = 32, WIDE_XI = 4;   // bytes per (token, superblock)
+
+WideX wide_x_layout(void* xa, void* rest, uint32_t rows, uint32_t n_blocks)
+{
+    const size_t n = (size_t)rows * n_blocks;
+    WideX x;
+    x.xa = (uint8_t*)xa;
+    x.xv = rest ? (uint8_t*)rest : (uint8_t*)xa + n * WIDE_XA;
+    x.xi = (float*)(x.xv + n * WIDE_XV);
+    return x;
+}
+size_t wide_x_bytes(uint32_t rows, uint32_t n_blocks) { return (size_t)rows * n_blocks * (WIDE_XA + WIDE_XV + WIDE_XI); }
+size_t wide_x_rest_bytes(uint32_t rows, uint32_t n_blocks) { return (size_t)rows * n_blocks * (WIDE_XV + WIDE_XI); }
+
+// ------------------------------------------------------------------------------------------------------------------
+// silu (2) or gelu_tanh (3)
+__device__ __forceinline__ float wide_act(int act, float g)
+{
+    return act == 2 ? g / (expf(-g) + 1.0f) : 0.5f * g * (1.0f + tanhf(0.7978845608f * (g + 0.044715f * g * g * g)));
+}
+
+// One workgroup: 16 superblocks of a row at a time, 32 threads each, 8 consecutive elements per thread.  pro as in
+// MatmulArgs (the stand-alone prologue kernels' formulas).  The norm needs the whole row first, so its workgroup
+// walks the row; the others spread it over blockIdx.y.  xa may be X itself: a superblock is read and written by the
+// same half wave, and its exponent needs every element of it before the first store.
+__global__ __launch_bounds__(512) void wide_x_kernel(const float* X, const float* norm_w, float eps, uint32_t n_blocks,
+                                                     int pro, int q6, uint8_t* xa, uint8_t* xv, float* xi)
+{
+    __shared__ float part[8];
+    const uint32_t tok = blockIdx.x, sub = threadIdx.x & 31u, at = threadIdx.x >> 5;
+    const uint32_t K = n_blocks * KQ_QK;
+    const float* row = X + (size_t)tok * (pro >= 2 ? 2u * (size_t)K : (size_t)K);
+    float rstd = 1.0f;
+    if (pro == 1) {
+        float ss = 0.0f;
+        for (uint32_t k = threadIdx.x * 4u; k < K; k += 2048u) {
+            const float4 v = *(const float4*)(row + k);
+            ss = fmaf(v.x, v.x, ss); ss = fmaf(v.y, v.y, ss); ss = fmaf(v.z, v.z, ss); ss = fmaf(v.w, v.w, ss);
+        }
+        ss = wave_total(ss);
+        if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = ss;
+        __syncthreads();
+        ss = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+        rstd = 1.0f / sqrtf(ss / (float)K + eps);
+    }
+    for (uint32_t b = blockIdx.y * 16u + at; b < n_blocks; b += 16u * gridDim.y) {
+        const uint32_t k = b * KQ_QK + sub * 8u;
+        float v[8];
+        *(float4*)v = *(const float4*)(row + k);
+        *(float4*)(v + 4) = *(const float4*)(row + k + 4);
+        if (pro == 1) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = v[i] * rstd * norm_w[k + i];
+        } else if (pro >= 2) {
+            float u[8];
+            *(float4*)u = *(const float4*)(row + K + k);
+            *(float4*)(u + 4) = *(const float4*)(row + K + k + 4);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float g = v[i];
+                v[i] = wide_act(pro, g) * u[i];
+            }
+        }
+        uint32_t amax = 0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) amax = max(amax, __builtin_bit_cast(uint32_t, v[i]) & 0x7FFFFFFFu);
+#pragma unroll
+        for (int o = 1; o < 32; o <<= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, o, 32));
+        uint32_t e = amax >> 23;
+        e = e < 15u ? 15u : (e > 253u ? 253u : e);
+        const float s = __builtin_bit_cast(float, (268u - e) << 23);     // 2^(141-e): amax * s in [2^14, 2^15)
+        const size_t cell = (size_t)tok * n_blocks + b;
+        if (sub == 0) xi[cell] = __builtin_bit_cast(float, (e - 14u) << 23);
+        _Float16 h[8], l[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const float a = v[i] * s;
+            h[i] = (_Float16)a;
+            l[i] = (_Float16)(a - (float)h[i]);
+        }
+        // the step and lane group that take this run of eight
+        const uint32_t j = q6 ? 2u * ((sub >> 2) & 3u) + (sub & 1u) : 2u * (sub & 3u) + ((sub >> 2) & 1u);
+        const uint32_t kq = q6 ? 2u * (sub >> 4) + ((sub >> 1) & 1u) : sub >> 3;
+        uint8_t* dst = xa + cell * WIDE_XA + j * 64u + kq * 16u;
+        *(w_half8*)dst = w_half8{h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
+        *(w_half8*)(dst + 512) = w_half8{l[0], l[2], l[1], l[3], l[4], l[6], l[5], l[7]};
+        if (!q6) {
+            float t = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+            t += group_partner<1>(t);
+            t += group_partner<2>(t);
+            if ((sub & 3u) == 0) {
+                const float a = t * (s * 0.03125f);   // 32 elements of at most 2^15 fit an fp16
+                const _Float16 th = (_Float16)a;
+                _Float16* o = (_Float16*)(xv + cell * WIDE_XV) + (sub >> 2);
+                o[0] = th;
+                o[8] = (_Float16)(a - (float)th);
+            }
+        }
+    }
+}
+
+hipError_t launch_wide_x(int type, const float* X, int pro, const float* norm_w, float eps, uint32_t rows,
+                         uint32_t n_blocks, const WideX& x, hipStream_t s)
+{
+    hipLaunchKernelGGL(wide_x_kernel, dim3(rows, pro == 1 ? 1u : (n_blocks + 15u) / 16u), dim3(512), 0, s, X, norm_w, eps,
+                       n_blocks, pro, type == KQ_TYPE_Q6_K ? 1 : 0, x.xa, x.xv, x.xi);
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------------------------------------------------------------
+struct WideParams {
+    WideX x;
+    const uint8_t* W;
+    const uint8_t* W2;       // act != 0: where the second tile's row 0 is (gate rows in W, up rows in W2)
+    const float* bias;       // [N] (act: [2N], the up half N on); nullptr for none
+    const float* residual;
+    float* Y;
+    uint32_t M, N;           // rows of x; outputs
+    uint32_t n_blocks, row_stride_bytes, y_offset, ldy;
+    uint32_t n_splits, blocks_per_split;
+    float* partial;          // [split][token group][workgroup][token][256 columns]
+    int act;                 // 0, or 2 / 3: Y = silu / gelu_tanh (W x) * (W2 x)
+    // grouped (records != nullptr): blockIdx.y walks records {expert, count, pair ids ...}, W and W2 advance by N rows
+    // per expert, a pair's X row is itself (x_per_slot) or pair / k_slots, its Y row the pair
+    const uint32_t* records;
+    const uint32_t* n_records;
+    uint32_t record_words, k_slots;
+    int x_per_slot;
+};
+
+// A row tile's bytes of one superblock, as this lane holds them.
+template <int TYPE> struct WideW;
+template <> struct WideW<KQ_TYPE_Q4_K> {
+    w_u32x4 hdr, q[2];
+    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t kq)
+    {
+        hdr = *(const w_u32x4*)blk;
+        q[0] = *(const w_u32x4*)(blk + 16 + 32 * kq);
+        q[1] = *(const w_u32x4*)(blk + 32 + 32 * kq);
+    }
+};
+template <> struct WideW<KQ_TYPE_Q5_K> {
+    w_u32x4 hdr, q[2], f[2];
+    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t kq)
+    {
+        hdr = *(const w_u32x4*)blk;
+        f[0] = *(const w_u32x4*)(blk + 16);
+        f[1] = *(const w_u32x4*)(blk + 32);
+        q[0] = *(const w_u32x4*)(blk + 48 + 32 * kq);
+        q[1] = *(const w_u32x4*)(blk + 64 + 32 * kq);
+    }
+};
+template <> struct WideW<KQ_TYPE_Q6_K> {
+    w_u32x4 ql[2], qh;   // (blocks are 210 bytes apart: 2-byte aligned loads)
+    w_u32x2 sc;
+    uint16_t d;
+    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t kq)
+    {
+        const uint32_t h = kq >> 1, lh = kq & 1u;
+        __builtin_memcpy(&ql[0], blk + 64 * h + 16 * lh, 16);
+        __builtin_memcpy(&ql[1], blk + 64 * h + 32 + 16 * lh, 16);
+        __builtin_memcpy(&qh, blk + 128 + 32 * h + 16 * lh, 16);
+        __builtin_memcpy(&sc, blk + 192 + 8 * h, 8);
+        __builtin_memcpy(&d, blk + 208, 2);
+    }
+};
+
+__device__ __forceinline__ uint32_t w_mul2(uint32_t a, w_half2 s)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(w_half2, a) * s);
+}
+
+// LDS writes of the workgroup are visible behind it; loads in flight stay in flight.
+__device__ __forceinline__ void wide_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+template <int TYPE, int TT>
+__global__ __launch_bounds__(512, 2) void wide_kernel(const WideParams p)
+{
+    constexpr bool Q6 = TYPE == KQ_TYPE_Q6_K, Q5 = TYPE == KQ_TYPE_Q5_K;
+    __shared__ __align__(16) uint8_t xs[2][TT * 16384];   // [tile of 16 tokens][hi, lo][step][lane] 16 B
+    __shared__ __align__(16) uint8_t vs[2][TT * 512];     // [tile][hi, lo][token] eight sub-block sums
+    __shared__ __align__(16) float is[2][TT * 16];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, kq = lane >> 4, r16 = lane & 15u;
+
+    const uint32_t* rec = nullptr;
+    uint32_t count, t0 = 0;
+    const uint8_t *W = p.W, *W2 = p.W2;
+    if (p.records) {
+        if (blockIdx.y >= *p.n_records) return;   // whole workgroup
+        rec = p.records + (size_t)blockIdx.y * p.record_words;
+        count = rec[1];
+        const size_t skip = (size_t)rec[0] * p.N * p.row_stride_bytes;
+        W += skip;
+        W2 += skip;
+        rec += 2;
+    } else {
+        t0 = blockIdx.y * (TT * 16u);
+        count = min(p.M - t0, TT * 16u);
+    }
+    // X row of slot i (slots beyond the count repeat the last: their outputs are dropped)
+    auto x_row = [&](uint32_t i) -> uint32_t {
+        i = min(i, count - 1u);
+        if (!rec) return t0 + i;
+        const uint32_t pr = rec[i];
+        return p.x_per_slot ? pr : pr / p.k_slots;
+    };
+    const uint8_t* xsrc[TT];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) xsrc[t] = p.x.xa + (size_t)x_row(16u * t + r16) * p.n_blocks * WIDE_XA + kq * 16u + wave * 64u;
+    const size_t vcell = (size_t)x_row(min(tid >> 1, TT * 16u - 1u)) * p.n_blocks;
+    const size_t icell = (size_t)x_row(min(tid, TT * 16u - 1u)) * p.n_blocks;
+
+    // this lane's row of the wave's two tiles
+    const uint32_t out0 = p.act ? (blockIdx.x * WIDE_WAVES + wave) * 16u : (blockIdx.x * WIDE_WAVES + wave) * 32u;
+    const uint8_t* wrow[2];
+    wrow[0] = W + (size_t)min(out0 + r16, p.N - 1u) * p.row_stride_bytes;
+    wrow[1] = p.act ? W2 + (size_t)min(out0 + r16, p.N - 1u) * p.row_stride_bytes
+                    : W + (size_t)min(out0 + 16u + r16, p.N - 1u) * p.row_stride_bytes;
+    constexpr uint32_t BB = TYPE == KQ_TYPE_Q4_K ? KQ_Q4K_BYTES : TYPE == KQ_TYPE_Q5_K ? KQ_Q5K_BYTES : KQ_Q6K_BYTES;
+
+    const uint32_t b0 = blockIdx.z * p.blocks_per_split, b1 = min(b0 + p.blocks_per_split, p.n_blocks);
+    // X of the next superblock travels through registers: requested ahead of this superblock's arithmetic, parked behind
+    // it.  (Written straight into LDS the compiler waits for the transfer ahead of every LDS read: it cannot tell the
+    // two buffers apart.)
+    w_u32x4 xreg[TT][2];
+    auto fetch_x = [&](uint32_t b) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int hl = 0; hl < 2; ++hl) xreg[t][hl] = *(const w_u32x4*)(xsrc[t] + (size_t)b * WIDE_XA + hl * 512);
+    };
+    auto park_x = [&](int buf) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int hl = 0; hl < 2; ++hl)
+                *(w_u32x4*)(&xs[buf][t * 16384 + hl * 8192 + wave * 1024u + lane * 16u]) = xreg[t][hl];
+    };
+    w_u32x4 vreg = {0, 0, 0, 0};
+    float ireg = 0.0f;
+    auto fetch_small = [&](uint32_t b) {
+        if (!Q6 && tid < TT * 32u) vreg = *(const w_u32x4*)(p.x.xv + (vcell + b) * WIDE_XV + (tid & 1u) * 16u);
+        if (tid < TT * 16u) ireg = p.x.xi[icell + b];
+    };
+    auto park_small = [&](int buf) {
+        if (!Q6 && tid < TT * 32u)
+            *(w_u32x4*)(&vs[buf][(tid >> 5) * 512u + (tid & 1u) * 256u + ((tid >> 1) & 15u) * 16u]) = vreg;
+        if (tid < TT * 16u) is[buf][tid] = ireg;
+    };
+
+    w_f32x4 tot[2][TT];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) tot[r][t] = w_f32x4{0, 0, 0, 0};
+
+    WideW<TYPE> w[2], wn[2];
+    fetch_x(b0);
+    fetch_small(b0);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) wn[r].load(wrow[r] + (size_t)b0 * BB, kq);
+    park_x(0);
+    park_small(0);
+    wide_barrier();
+
+    for (uint32_t b = b0; b < b1; ++b) {
+        const int buf = (int)((b - b0) & 1u);
+        const uint32_t bn = min(b + 1u, b1 - 1u);   // (the last step requests its own superblock again)
+        fetch_x(bn);
+        fetch_small(bn);
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            w[r] = wn[r];
+            wn[r].load(wrow[r] + (size_t)bn * BB, kq);
+        }
+        // per-lane scales, as pairs
+        w_half2 sc[2][Q6 ? 4 : 2];
+        w_u32x4 bmn[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            if constexpr (Q6) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const uint32_t word = t < 2 ? w[r].sc.x : w[r].sc.y;
+                    const int v = (int)(int8_t)(word >> (16 * (t & 1) + 8 * (kq & 1u)));
+                    const _Float16 h = (_Float16)(float)v;
+                    sc[r][t] = w_half2{h, h};
+                }
+            } else {
+                const w_u32x4 h = w[r].hdr;
+                const uint32_t scA = h.y & 0x3F3F3F3Fu, mnA = h.z & 0x3F3F3F3Fu;
+                const uint32_t scB = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
+                const uint32_t mnB = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
+                const uint32_t s2 = (kq < 2u ? scA : scB) >> (16u * (kq & 1u));
+                const _Float16 a = (_Float16)(float)(s2 & 255u), c = (_Float16)((float)((s2 >> 8) & 255u) * 0.0625f);
+                sc[r][0] = w_half2{a, a};
+                sc[r][1] = w_half2{c, c};   // (high nibbles sit four bits up)
+                // the eight minima as fp16 subnormals mn * 2^-24, against the hi sums (kq 0) and the lo sums (kq 1)
+                const uint32_t keep = kq < 2u ? 0xFFFFFFFFu : 0u;
+                bmn[r] = w_u32x4{__builtin_amdgcn_perm(0u, mnA, 0x0c010c00u) & keep, __builtin_amdgcn_perm(0u, mnA, 0x0c030c02u) & keep,
+                                 __builtin_amdgcn_perm(0u, mnB, 0x0c010c00u) & keep, __builtin_amdgcn_perm(0u, mnB, 0x0c030c02u) & keep};
+            }
+        }
+        w_f32x4 D[2][TT];
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int t = 0; t < TT; ++t) D[r][t] = w_f32x4{0, 0, 0, 0};
+        const uint8_t* xb = xs[buf] + lane * 16u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            w_half8 Bh[2], Bl[2];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                w_u32x4 o;
+                if constexpr (Q6) {
+                    const int t = j >> 1, u = j & 1;
+                    const uint32_t l0 = w[r].ql[t & 1][2 * u], l1 = w[r].ql[t & 1][2 * u + 1];
+                    const uint32_t h0 = w[r].qh[2 * u], h1 = w[r].qh[2 * u + 1];
+                    const uint32_t c0 = ((l0 >> (4 * (t >> 1))) & 0x0F0F0F0Fu) | (((h0 >> (2 * t)) & 0x03030303u) << 4);
+                    const uint32_t c1 = ((l1 >> (4 * (t >> 1))) & 0x0F0F0F0Fu) | (((h1 >> (2 * t)) & 0x03030303u) << 4);
+                    w_u32x4 lo;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const uint32_t c = i < 2 ? c0 : c1;
+                        const uint32_t oi = (((i & 1) ? c >> 8 : c) & 0x00FF00FFu) | 0x64006400u;   // 1024 + q
+                        const w_half2 q = __builtin_bit_cast(w_half2, oi) - w_half2{(_Float16)1056.0f, (_Float16)1056.0f};
+                        const w_half2 hi = q * sc[r][t];
+                        o[i] = __builtin_bit_cast(uint32_t, hi);
+                        lo[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(q, sc[r][t], -hi));
+                    }
+                    Bl[r] = __builtin_bit_cast(w_half8, lo);
+                } else {
+                    const int i = j >> 1;
+                    const uint32_t d0 = w[r].q[i >> 1][2 * (i & 1)], d1 = w[r].q[i >> 1][2 * (i & 1) + 1];
+                    const uint32_t e0 = d0 >> 8, e1 = d1 >> 8;
+                    const uint32_t m = (j & 1) ? 0x00F000F0u : 0x000F000Fu;
+                    o = w_u32x4{d0 & m, e0 & m, d1 & m, e1 & m};
+                    if constexpr (Q5) {
+                        // bit 2kq (2kq + 1) of a byte of fifth bits: bit 4 beside a low nibble, bit 8 beside a high one
+                        const uint32_t g0 = w[r].f[i >> 1][2 * (i & 1)] >> (2u * kq), g1 = w[r].f[i >> 1][2 * (i & 1) + 1] >> (2u * kq);
+                        if (j & 1) {
+                            o.x |= (g0 << 7) & 0x01000100u; o.y |= (g0 >> 1) & 0x01000100u;
+                            o.z |= (g1 << 7) & 0x01000100u; o.w |= (g1 >> 1) & 0x01000100u;
+                        } else {
+                            o.x |= (g0 << 4) & 0x00100010u; o.y |= (g0 >> 4) & 0x00100010u;
+                            o.z |= (g1 << 4) & 0x00100010u; o.w |= (g1 >> 4) & 0x00100010u;
+                        }
+                    }
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) o[n] = w_mul2(o[n], sc[r][j & 1]);
+                }
+                Bh[r] = __builtin_bit_cast(w_half8, o);
+            }
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const w_half8 ah = *(const w_half8*)(xb + t * 16384 + j * 1024);
+                const w_half8 al = *(const w_half8*)(xb + t * 16384 + 8192 + j * 1024);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    D[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, Bh[r], D[r][t], 0, 0, 0);
+                    D[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, Bh[r], D[r][t], 0, 0, 0);
+                    if constexpr (Q6) D[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, Bl[r], D[r][t], 0, 0, 0);
+                }
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+            const w_f32x4 inv = *(const w_f32x4*)(&is[buf][16 * t + 4u * kq]);
+            if constexpr (Q6) {
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    const float d = half_bits_to_float(w[r].d);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) tot[r][t][i] = fmaf(inv[i] * d, D[r][t][i], tot[r][t][i]);
+                }
+            } else {
+                const w_half8 av = *(const w_half8*)(&vs[buf][t * 512 + (lane & 31u) * 16u]);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) {
+                    w_f32x4 V = {0, 0, 0, 0};
+                    V = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, __builtin_bit_cast(w_half8, bmn[r]), V, 0, 0, 0);
+                    const float d24 = half_bits_to_float(w[r].hdr.x & 0xFFFFu) * 16777216.0f;
+                    const float m24 = half_bits_to_float(w[r].hdr.x >> 16) * (16777216.0f * 32.0f);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) tot[r][t][i] += inv[i] * fmaf(d24, D[r][t][i], -(m24 * V[i]));
+                }
+            }
+        }
+        park_x(buf ^ 1);
+        park_small(buf ^ 1);
+        wide_barrier();
+    }
+
+    // The outputs change hands through LDS (the X buffers are free: every wave is past the loop's last barrier) and
+    // leave in rolled loops of whole rows (from the accumulators they went as 64-byte pieces).
+    constexpr uint32_t OP = 260;   // floats between tokens: the four lane groups write to different banks
+    float* ot = (float*)&xs[0][0];
+    static_assert(TT * 16 * OP * 4 <= sizeof(xs), "the output tile fits the X buffers");
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ot[(16 * t + 4u * kq + i) * OP + wave * 32u + 16u * r + r16] = tot[r][t][i];
+    __syncthreads();
+    if (p.n_splits > 1) {   // (dense calls only) wide_sum_kernel adds the splits' tiles
+        float* tile = p.partial + (((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (TT * 16u * 256u);
+        for (uint32_t n = tid; n < TT * 1024u; n += 512u)
+            *(float4*)(tile + 4u * n) = *(const float4*)(ot + (n >> 6) * OP + 4u * (n & 63u));
+        return;
+    }
+    if (p.act) {
+        // columns: per wave 16 gate rows, then their 16 up rows
+        const uint32_t c = tid & 127u, n = blockIdx.x * 128u + c;
+        const float bg = p.bias && n < p.N ? p.bias[n] : 0.0f, bu = p.bias && n < p.N ? p.bias[p.N + n] : 0.0f;
+#pragma nounroll
+        for (uint32_t slot = tid >> 7; slot < count; slot += 4u) {
+            const float* o = ot + slot * OP + (c >> 4) * 32u + (c & 15u);
+            const float g = o[0] + bg, u = o[16] + bu;
+            const float a = wide_act(p.act, g);
+            if (n < p.N) p.Y[(size_t)(rec ? rec[slot] : t0 + slot) * p.ldy + p.y_offset + n] = a * u;
+        }
+    } else {
+        const uint32_t c = tid & 255u, n = blockIdx.x * 256u + c;
+        const float bv = p.bias && n < p.N ? p.bias[n] : 0.0f;
+#pragma unroll 4
+        for (uint32_t slot = tid >> 8; slot < count; slot += 2u) {
+            if (n >= p.N) break;
+            const size_t at = (size_t)(rec ? rec[slot] : t0 + slot) * p.ldy + p.y_offset + n;
+            float y = ot[slot * OP + c] + bv;
+            if (p.residual) y += p.residual[at];
+            p.Y[at] = y;
+        }
+    }
+}
+
+// Adds the splits' partial tiles in split order, with the call's epilogue.  Workgroup (x, y): 256 columns of four
+// tokens.  A launch of its own: added by the last workgroup of a tile to arrive, the splits were read one round
+// trip after the other by that one workgroup (19 us of a 64-token call with eight splits).
+__global__ __launch_bounds__(256) void wide_sum_kernel(const WideParams p, uint32_t tokens, uint32_t groups)
+{
+    const uint32_t slot = blockIdx.y * 4u + (threadIdx.x >> 6);          // token over all groups of `tokens`
+    const uint32_t c = (threadIdx.x & 63u) * 4u;
+    if (slot >= p.M) return;
+    const uint32_t group = slot / tokens;
+    const float* src = p.partial + (((size_t)group * gridDim.x + blockIdx.x) * tokens + slot % tokens) * 256u + c;
+    const size_t zs = (size_t)groups * gridDim.x * tokens * 256u;
+    float4 a = {0, 0, 0, 0};
+#pragma unroll 8
+    for (uint32_t z = 0; z < p.n_splits; ++z) {
+        const float4 v = *(const float4*)(src + z * zs);
+        a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w;
+    }
+    const size_t at = (size_t)slot * p.ldy + p.y_offset;
+    float y[4] = {a.x, a.y, a.z, a.w};
+    if (p.act) {
+        // 16 gate columns, then their 16 up columns: the up quad sits four lanes on
+        const uint32_t n = blockIdx.x * 128u + (c >> 5) * 16u + (c & 15u);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float u = __shfl_down(y[i], 4, 64);
+            if ((c & 16u) || n + i >= p.N) continue;
+            float g = y[i];
+            if (p.bias) { g += p.bias[n + i]; u += p.bias[p.N + n + i]; }
+            p.Y[at + n + i] = wide_act(p.act, g) * u;
+        }
+        return;
+    }
+    const uint32_t n = blockIdx.x * 256u + c;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (n + i >= p.N) continue;
+        float v = y[i];
+        if (p.bias) v += p.bias[n + i];
+        if (p.residual) v += p.residual[at + n + i];
+        p.Y[at + n + i] = v;
+    }
+}
+
+template <int TYPE>
+static void launch_wide_type(const WideParams& p, uint32_t tt, dim3 grid, hipStream_t s)
+{
+    if (tt == 1u) hipLaunchKernelGGL((wide_kernel<TYPE, 1>), grid, dim3(512), 0, s, p);
+    else if (tt == 2u) hipLaunchKernelGGL((wide_kernel<TYPE, 2>), grid, dim3(512), 0, s, p);
+    else if (tt == 3u) hipLaunchKernelGGL((wide_kernel<TYPE, 3>), grid, dim3(512), 0, s, p);
+    else hipLaunchKernelGGL((wide_kernel<TYPE, 4>), grid, dim3(512), 0, s, p);
+}
+
+static hipError_t launch_wide_any(int type, const WideParams& p, uint32_t tt, dim3 grid, hipStream_t s)
+{
+    if (type == KQ_TYPE_Q4_K) launch_wide_type<KQ_TYPE_Q4_K>(p, tt, grid, s);
+    else if (type == KQ_TYPE_Q5_K) launch_wide_type<KQ_TYPE_Q5_K>(p, tt, grid, s);
+    else launch_wide_type<KQ_TYPE_Q6_K>(p, tt, grid, s);
+    return hipGetLastError();
+}
+
+bool wide_supported(const MatmulArgs& a)
+{
+    // X in 16-byte loads; Q4_K and Q5_K blocks too (their 144 and 176 bytes keep a 16-byte aligned row aligned)
+    if (((uintptr_t)a.X | (uintptr_t)a.norm_w) & 15u) return false;
+    if (a.n_blocks * KQ_QK != a.K || a.N == 0) return false;
+    if (a.type == KQ_TYPE_Q6_K) return !((uintptr_t)a.W & 1u) && !((uintptr_t)a.W2 & 1u);
+    return !(((uintptr_t)a.W | (uintptr_t)a.W2) & 15u) && !(a.row_stride_bytes & 15u);
+}
+
+hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scratch, size_t x_bytes, int splits, hipStream_t s)
+{
+    const uint32_t outs = a.epi ? a.N / 2u : a.N;
+    const size_t per_row = wide_x_bytes(1, a.n_blocks);
+    size_t step = x_bytes / per_row;
+    if (step < a.M) step = step / 64u * 64u;
+    if (step == 0) return hipErrorInvalidValue;
+    const uint32_t x_row = a.pro >= 2 ? 2u * a.K : a.K;
+    for (uint32_t m0 = 0; m0 < a.M; m0 += (uint32_t)step) {
+        const uint32_t M = a.M - m0 < step ? a.M - m0 : (uint32_t)step;
+        WideParams p{};
+        p.x = wide_x_layout(x_scratch, nullptr, M, a.n_blocks);
+        if (hipError_t e = launch_wide_x(a.type, (const float*)a.X + (size_t)m0 * x_row, a.pro, a.norm_w, a.eps, M, a.n_blocks, p.x, s);
+            e != hipSuccess) return e;
+        p.W = a.W; p.W2 = a.W + (size_t)outs * a.row_stride_bytes;
+        p.bias = a.bias;
+        p.residual = a.residual ? a.residual + (size_t)m0 * a.ldy : nullptr;
+        p.Y = a.Y + (size_t)m0 * a.ldy;
+        p.M = M; p.N = outs; p.n_blocks = a.n_blocks; p.row_stride_bytes = a.row_stride_bytes;
+        p.y_offset = a.y_offset; p.ldy = a.ldy; p.act = a.epi;
+        const uint32_t gy = (M + 63u) / 64u, tiles = (M + 15u) / 16u, tt = (tiles + gy - 1u) / gy;
+        const uint32_t gy2 = (tiles + tt - 1u) / tt;
+        const uint32_t per_wg = a.epi ? WIDE_WAVES * 16u : WIDE_WAVES * 32u, gx = (outs + per_wg - 1u) / per_wg;
+        // K is cut where the rows alone leave CUs idle (one workgroup per CU).  Prices in us, measured: a superblock of a
+        // workgroup's walk 0.8 + 0.7 per tile of tokens (Q6_K 3 + 0.9), the launch that adds the splits 5, and its
+        // traffic, written and read once, at 4 TB/s
+        const double step_us = a.type == KQ_TYPE_Q6_K ? 3.0 + 0.9 * tt : 0.8 + 0.7 * tt;
+        const size_t tile_floats = (size_t)gy2 * tt * 16u * gx * (WIDE_WAVES * 32u);
+        uint32_t z = 1;
+        double best = 1e30;
+        for (uint32_t c = 1; c <= a.n_blocks && c <= 16u; ++c) {
+            if (c > 1u && c * tile_floats > sc.capacity_floats) break;
+            const uint32_t cus = device_cu_count(), rounds = (gx * gy2 * c + cus - 1u) / cus;
+            const double t = (double)rounds * ((a.n_blocks + c - 1u) / c) * step_us + (c > 1u ? 5.0 + 2e-6 * c * tile_floats : 0.0);
+            if (splits ? (uint32_t)splits >= c : t < best) { best = t; z = c; }
+        }
+        p.blocks_per_split = (a.n_blocks + z - 1u) / z;
+        p.n_splits = (a.n_blocks + p.blocks_per_split - 1u) / p.blocks_per_split;
+        p.partial = sc.partial;
+        if (hipError_t e = launch_wide_any(a.type, p, tt, dim3(gx, gy2, p.n_splits), s); e != hipSuccess) return e;
+        if (p.n_splits > 1u) {
+            hipLaunchKernelGGL(wide_sum_kernel, dim3(gx, (M + 3u) / 4u), dim3(256), 0, s, p, tt * 16u, gy2);
+            if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+        }
+    }
+    return hipSuccess;
+}
+
+hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32_t* records, const uint32_t* n_records,
+                               uint32_t bound, uint32_t cap, hipStream_t s)
+{
+    WideParams p{};
+    p.x = x;
+    p.W = a.W; p.W2 = a.W2 ? a.W2 : a.W;
+    p.Y = a.Y;
+    p.M = a.M; p.N = a.N; p.n_blocks = a.n_blocks; p.row_stride_bytes = a.row_stride_bytes; p.ldy = a.ldy;
+    p.n_splits = 1; p.blocks_per_split = a.n_blocks;
+    p.act = a.W2 ? 2 : 0;
+    p.records = records; p.n_records = n_records; p.record_words = 2u + cap; p.k_slots = a.k_slots; p.x_per_slot = a.x_per_slot;
+    const uint32_t per_wg = a.W2 ? WIDE_WAVES * 16u : WIDE_WAVES * 32u;
+    return launch_wide_any(a.type, p, cap / 16u, dim3((a.N + per_wg - 1u) / per_wg, bound, 1u), s);
+}
+
+}  // namespace kq

@@ -500,8 +500,9 @@ BPK_API const char *bpk_last_kernel(void);
  * 0 = automatic, 1 = generic, 2 = row-per-lane GEMV (M <= 4), 3 = row-per-lane
  * kernel on the 4x4x4 matrix-core op (M <= 16), 4 = matrix-core tiled GEMM
  * (bf16 X only), 5 = lanes-along-K GEMV (M = 1), 6 = 16-row x 16-token
- * matrix-core tiles (M <= 16), 7 = one token on the matrix cores (Q4_K rows of
- * up to 16 superblocks).  A forced family that cannot serve the call's
+ * matrix-core tiles (groups of 16 tokens), 7 = one token on the matrix cores
+ * (Q4_K rows of up to 16 superblocks), 8 = matrix-core tiles of up to 64 tokens
+ * (taken by itself from 17 tokens on; bpk_last_kernel says "mtile" for both).  A forced family that cannot serve the call's
  * shape fails with BPK_ERR_SHAPE instead of falling back. */
 BPK_API int bpk_force_kernel(int family);
 
