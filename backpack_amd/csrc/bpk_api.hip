@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -1093,6 +1094,42 @@ size_t bpk_kq_moe_ffn_scratch_bytes(uint32_t T, uint32_t k, uint32_t hidden, uin
     return (P * inter * 2 + P * hidden) * sizeof(float) + (P * 10 + 4) * sizeof(uint32_t);
 }
 
+// Pairs per record of the many-token kernel for an expert FFN's two launches, 0 where another kernel takes the call.
+// The records' words go behind the activations' sums and scales in U, the split X into D.
+static uint32_t moe_wide_cap(const kq::MatmulArgs& a, const kq::MatmulArgs& d, const uint8_t* up, uint32_t T, uint32_t n_experts)
+{
+    const uint32_t P = a.M;
+    kq::MatmulArgs g = a;
+    g.W2 = up;
+    if ((t_family != 0 && t_family != 8) || n_experts > 8192u || !kq::wide_supported(g) || !kq::wide_supported(d)) return 0;
+    // From 1.25 pairs per expert on, where the 16-token tile kernel's records took over from one matvec per pair; us
+    // against that kernel's: 128 experts x 8, 2048 / 768, 1.25 pairs per expert 113 / 153, 4: 145 / 166, 16: 195 / 265, 128: 785 /
+    // 1266; 32 x 4, 2048 / 512, 1.25: 51 / 58, 128: 184 / 288; 64 x 6, 1536 / 768 Q5_K, 1.5: 75 / 81, 192: 479 / 766.
+    if (t_family == 0 && 4ull * P < 5ull * n_experts) return 0;
+    const size_t u_bytes = (size_t)P * a.N * sizeof(float), u_used = kq::wide_x_rest_bytes(P, d.n_blocks);
+    if (kq::wide_x_bytes(T, a.n_blocks) > (size_t)P * d.N * sizeof(float) || u_used > u_bytes) return 0;   // (one slot per token)
+    // The price of a launch: rounds of its workgroups over the CUs, each of a superblock's 1 + 0.5 per tile of 16 pairs
+    // (Q6_K half as much again) per step and 3 us around the walk.  Measured on 128 experts x 8 slots, 2048 / 768, us at
+    // 16 / 32 / 48 / 64 pairs per record: 6 pairs per expert 148 / 175 / 200 / -, 16: 208 / 195 / 221 / 243, 32: 319 / 296 /
+    // 286 / 279, 128: 958 / 853 / 810 / 785; 8 experts x 2, 1024 / 512, 24 pairs per expert: 41 / 48 / 53 / 57.
+    const double cus = (double)kq::device_cu_count();
+    const auto launch_us = [&](double workgroups, const kq::MatmulArgs& m, uint32_t tiles) {
+        const double step = (1.0 + 0.5 * tiles) * (m.type == KQ_TYPE_Q6_K ? 1.5 : 1.0);
+        // (a tenth of a round is within the spread of the records' number)
+        return std::fmax(1.0, std::ceil(workgroups / cus - 0.1)) * (m.n_blocks * step + 3.0);
+    };
+    uint32_t best = 0;
+    double best_us = 1e30;
+    for (uint32_t cap = 16u; cap <= 64u; cap += 16u) {
+        const uint32_t bound = kq::moe_tiles_bound(P, n_experts, (int)(cap / 2u));
+        if (bound > 65535u || (kq::moe_tiles_words(P, n_experts, (int)(cap / 2u)) + 3u) * sizeof(uint32_t) > u_bytes - u_used) continue;
+        const double records = kq::moe_expected_records(P, n_experts, cap);
+        const double us = launch_us(records * ((a.N + 127u) / 128u), a, cap / 16u) + launch_us(records * ((d.N + 255u) / 256u), d, cap / 16u);
+        if (us < best_us) { best_us = us; best = cap; }
+    }
+    return best;
+}
+
 int bpk_kq_moe_ffn(int type_gu, int type_dn, const float* X, const void* gate, const void* up, const void* down,
                    const uint32_t* expert_idx, const float* expert_wt, float* out, uint32_t T, uint32_t k,
                    uint32_t n_experts, uint32_t hidden, uint32_t inter, void* scratch, size_t scratch_bytes,
@@ -1137,6 +1174,7 @@ int bpk_kq_moe_ffn(int type_gu, int type_dn, const float* X, const void* gate, c
                       kq::mrow_supported(d);
     hipError_t e = hipSuccess;
     const uint32_t bound8 = kq::moe_tiles_bound(P, n_experts, 4);
+    const uint32_t wide_cap = moe_wide_cap(a, d, (const uint8_t*)up, T, n_experts);
     // Pairs per expert from which the tile kernel's records (every touched expert's matrices read once per record
     // of pairs) beat one lanes-along-K matvec per pair.  Measured on 128 experts x 8 slots, 2048 / 768: 128 pairs 119
     // against 104 us, 160 pairs 142 against 150-159, 192 pairs 145 against 179.
@@ -1147,7 +1185,22 @@ int bpk_kq_moe_ffn(int type_gu, int type_dn, const float* X, const void* gate, c
                              kq::gemv_stream_supported(a) && kq::gemv_stream_supported(d);
     // (Q5_K has no matrix-core row kernel: its thinly spread pairs take the tile kernel too)
     const bool tile_path = tile_ok && !stream_path && (dense || !fast);
-    if (stream_path) {
+    if (wide_cap) {
+        // Every touched expert's matrices read once per record of up to wide_cap pairs.  X is split once (into D, not in
+        // use yet), gate and up share a launch that stores silu(gate x) * (up x), and those rows are split where they
+        // lie for down's launch.
+        t_kernel = "moe_ffn_mtile";
+        const int rsets = (int)(wide_cap / 2u);
+        const uint32_t rbound = kq::moe_tiles_bound(P, n_experts, rsets);
+        uint32_t* words = (uint32_t*)((uint8_t*)U + kq::wide_x_rest_bytes(P, nb_dn));
+        const kq::WideX x = kq::wide_x_layout(D, nullptr, T, nb_gu), act = kq::wide_x_layout(G, U, P, nb_dn);
+        a.W2 = (const uint8_t*)up;
+        e = kq::launch_moe_group(expert_idx, P, n_experts, rsets, words + 4, words, s);
+        if (e == hipSuccess) e = kq::launch_wide_x(type_gu, X, 0, nullptr, 0.0f, T, nb_gu, x, s);
+        if (e == hipSuccess) e = kq::launch_wide_grouped(a, x, words + 4, words, rbound, wide_cap, s);
+        if (e == hipSuccess) e = kq::launch_wide_x(type_dn, G, 0, nullptr, 0.0f, P, nb_dn, act, s);
+        if (e == hipSuccess) e = kq::launch_wide_grouped(d, act, words + 4, words, rbound, wide_cap, s);
+    } else if (stream_path) {
         // a handful of pairs (decode): one lanes-along-K matvec per pair, no grouping pass
         // gate and up in one launch (they read the same x), the activation folded into down's load of x
         t_kernel = "moe_ffn_stream";

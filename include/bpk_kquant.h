@@ -524,10 +524,10 @@ BPK_API int bpk_force_kernel(int family);
  * "moe_fold": 0 keeps the weighted sum over a token's slots behind the expert FFN
  * a launch of its own (default 1: inside the last matvec's launch where its
  * kernel can: a few pairs, Q6_K down projection, at most 8 slots per token),
- * and the batched tile path's gate and up two launches and an activation
- * kernel (default: one launch that stores silu(gate x) * (up x), where hidden
+ * and, where a batch of pairs goes to the 16-token tiles (family 6; one slot per
+ * token), gate and up two launches and an activation kernel (default: one launch that stores silu(gate x) * (up x), where hidden
  * spans more than four superblocks); "moe_tile_iters": tiles of 16 rows a wave
- * of the batched tile path walks with a record's activations staged once, where
+ * of that path walks with a record's activations staged once, where
  * K is at most four superblocks (1, 2, 4 or 8; 0 = chosen per call from the
  * expected number of records, so that the workgroups fill whole rounds);
  * "chain_spin_us": bound of a wait between the ops of a chain in microseconds

@@ -59,3 +59,37 @@ def test_many_tokens_fused_vs_separate(gpu, type_, M, N, K, pro, epi, res):  # n
     assert np.isfinite(a).all()
     # the same split products from x that differs by the rounding of its norm (a few 2^-24)
     assert float(np.abs(a - b).max()) <= 1e-5 * rms + 1e-5 * float(np.abs(b).max())
+
+
+# pairs per expert around the record sizes (16 .. 64), a skewed routing, one slot per token (whose split X does not fit
+# beside the records: the 16-token tile kernel), rows that are no multiple of a workgroup's 256
+@pytest.mark.parametrize("tgu,tdn,T,E,k,H,I,skew", [(Q4_K, Q6_K, 5, 8, 2, 256, 256, False), (Q4_K, Q6_K, 17, 2, 2, 512, 256, False),
+                                                    (Q5_K, Q5_K, 65, 4, 2, 768, 512, False), (Q6_K, Q4_K, 200, 8, 3, 512, 768, True),
+                                                    (Q4_K, Q4_K, 300, 4, 2, 256, 512, False), (Q4_K, Q6_K, 40, 4, 1, 512, 256, False)])
+def test_moe_ffn_many_pairs_vs_oracle(gpu, kqo, tgu, tdn, T, E, k, H, I, skew):  # noqa: F811
+    from backpack_amd import capi, kquant
+    print("wide moe", tgu, tdn, T, E, k, H, I, skew, flush=True)
+    _, gp, gw = gpu.make_weight(tgu, E * I, H, seed=81)
+    _, up, uw = gpu.make_weight(tgu, E * I, H, seed=82)
+    _, dp, dw = gpu.make_weight(tdn, E * H, I, seed=83)
+    rng = np.random.default_rng(T)
+    eidx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32)
+    if skew:   # every token's first slot is expert 3: one expert of many records beside experts of few
+        eidx[:, 1:][eidx[:, 1:] == 3] = 0
+        eidx[:, 0] = 3
+    ew = rng.random((T, k)).astype(np.float32)
+    X = (rng.standard_normal((T, H)) * 0.1).astype(np.float32)
+    args = (gpu.dev(X), gw, uw, dw, gpu.dev(eidx.view(np.int32)), gpu.dev(ew), E)
+    got = kquant.moe_ffn(*args).cpu().numpy()
+    assert capi.last_kernel() == "moe_ffn_mtile"
+    assert np.array_equal(got, kquant.moe_ffn(*args).cpu().numpy()), "a pair's result does not depend on its place"
+    capi.force_kernel(6)
+    try:
+        tile = kquant.moe_ffn(*args).cpu().numpy()
+    finally:
+        capi.force_kernel(0)
+    want = kqo.moe_ffn(tgu, tdn, X, gp, up, dp, eidx, ew, H, I)
+    rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    assert np.all(np.abs(got - want) <= 1e-3 * rms + 1e-3 * np.abs(want))
+    # both split x into 22 bits of its superblock's largest: the sums' order is what differs
+    assert np.abs(got - tile).max() <= 1e-4 * rms + 1e-4 * np.abs(want).max()
