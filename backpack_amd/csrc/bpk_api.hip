@@ -676,6 +676,14 @@ int bpk_kq_matmul_bf16(int type, const uint16_t* X, const void* W, const float* 
     if (!kq::gemm_bf16_supported(a))
         return fail(BPK_ERR_ALIGN, "bf16 GEMM needs 16-byte aligned X and (for Q4_K) 16-byte aligned W rows");
     t_kernel = "gemm_bf16";
+    // a short prompt on the kernel that cuts K over workgroups, where that is priced below the GEMM
+    if (t_gemm_tile == 0 && t_gemm_split == 0 && M <= kq::SHORT_MAX_M) {
+        const kq::ShortPlan plan = kq::plan_short(a, st->gemm_split.capacity_floats, kq::device_cu_count());
+        if (plan.us < plan.gemm_us) {
+            const hipError_t es = kq::launch_short(a, plan, st->gemm_split, (hipStream_t)stream);
+            return es == hipSuccess ? BPK_OK : hip_fail(es, t_kernel);
+        }
+    }
     hipError_t e = kq::launch_gemm_bf16(a, t_gemm_tile, t_gemm_split, st->gemm_split, (hipStream_t)stream);
     return e == hipSuccess ? BPK_OK : hip_fail(e, t_kernel);
 }

@@ -161,6 +161,17 @@ hipError_t launch_wide_x(int type, const float* X, int pro, const float* norm_w,
 hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32_t* records, const uint32_t* n_records,
                                uint32_t bound, uint32_t cap, hipStream_t s);
 
+// bf16 X of a short prompt (kq_wide.hip): groups of up to 128 tokens, K cut over workgroups.  Takes what
+// gemm_bf16_supported accepts.
+struct ShortPlan {
+    uint32_t tiles, groups;   // tiles of 16 tokens per workgroup, groups of that many
+    uint32_t splits, blocks_per_split;
+    double us, gemm_us;       // its price, and the GEMM's
+};
+constexpr uint32_t SHORT_MAX_M = 512;
+ShortPlan plan_short(const MatmulArgs& a, size_t capacity_floats, uint32_t cus);
+hipError_t launch_short(const MatmulArgs& a, const ShortPlan& plan, const SplitScratch& sc, hipStream_t s);
+
 // Row-per-lane matvec on the matrix cores, M <= 16 dense or grouped by expert.
 bool mrow_supported(const MatmulArgs& a);
 size_t mrow_scratch_floats(const MatmulArgs& a, const GemvTuning& t);

@@ -29,6 +29,7 @@
 #include "kq_format.h"
 #include "kq_kernels.h"
 #include "kq_wave.h"
+#include <cmath>
 
 namespace kq {
 
@@ -606,6 +607,230 @@ hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32
     p.records = records; p.n_records = n_records; p.record_words = 2u + cap; p.k_slots = a.k_slots; p.x_per_slot = a.x_per_slot;
     const uint32_t per_wg = a.W2 ? WIDE_WAVES * 16u : WIDE_WAVES * 32u;
     return launch_wide_any(a.type, p, cap / 16u, dim3((a.N + per_wg - 1u) / per_wg, bound, 1u), s);
+}
+
+// ------------------------------------------------------------------------------------------------------------------
+// bf16 rows of a short prompt (one launch serves up to 128 tokens per workgroup, K cut over workgroups).
+//
+// The GEMM's tiles of 128 and 256 tokens walk K in steps of 64 with one barrier each and mostly find one workgroup per
+// CU here: 1.4 us per step and CU, whatever the tokens.  This kernel walks whole superblocks: the X of TT tiles of 16
+// tokens is staged in LDS (two buffers), a wave turns its 32 rows' weights into bf16 in registers (the GEMM's formula and
+// its one rounding, so both compute the same products) and meets every token with them: no weight passes through LDS,
+// and a step is bounded by the matrix cores and the LDS reads about equally at 128 tokens.  Accumulation is in fp32
+// over the workgroup's whole range of K.
+//
+// LDS order of X: [tile][step][lane group kq][token] of 16 bytes; the token's place is turned by 2 * step + kq % 2, so that
+// the 16-byte pieces that a wave has read along K (whole lines) go to different banks.
+typedef __bf16 w_bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 w_bf16x2 __attribute__((ext_vector_type(2)));
+typedef float w_f32x2 __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ uint32_t w_pack_bf16(float lo, float hi)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector((w_f32x2{lo, hi}), w_bf16x2));
+}
+
+template <int TYPE, int TT>
+__global__ __launch_bounds__(512, 2) void short_kernel(const WideParams p)
+{
+    constexpr bool Q6 = TYPE == KQ_TYPE_Q6_K, Q5 = TYPE == KQ_TYPE_Q5_K;
+    constexpr uint32_t OP = 260;   // floats between tokens of the output tile, as in wide_kernel
+    constexpr uint32_t X_BYTES = TT * 8192u, O_BYTES = TT * 16u * OP * 4u;
+    __shared__ __align__(16) uint8_t xs[2u * X_BYTES > O_BYTES ? 2u * X_BYTES : O_BYTES];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, kq = lane >> 4, r16 = lane & 15u;
+    const uint32_t t0 = blockIdx.y * (TT * 16u), count = min(p.M - t0, TT * 16u);
+
+    // X: 32 threads copy a token's 512 bytes of a superblock; piece c (eight k) goes to step cj of lane group ck
+    const uint32_t c = tid & 31u, tok = tid >> 5;
+    const uint32_t cj = Q6 ? 2u * ((c >> 2) & 3u) + (c & 1u) : 2u * (c & 3u) + ((c >> 2) & 1u);
+    const uint32_t ck = Q6 ? 2u * (c >> 4) + ((c >> 1) & 1u) : c >> 3;
+    const uint32_t xdst = cj * 1024u + ck * 256u + ((tok + 2u * cj + (ck & 1u)) & 15u) * 16u;
+    const size_t x_row = (size_t)p.n_blocks * 512u;
+    const uint8_t* xsrc[TT];   // tokens beyond the count repeat the last: their outputs are dropped
+#pragma unroll
+    for (int t = 0; t < TT; ++t) xsrc[t] = p.x.xa + (size_t)(t0 + min(16u * t + tok, count - 1u)) * x_row + c * 16u;
+
+    const uint32_t out0 = (blockIdx.x * WIDE_WAVES + wave) * 32u;
+    const uint8_t* wrow[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) wrow[r] = p.W + (size_t)min(out0 + 16u * r + r16, p.N - 1u) * p.row_stride_bytes;
+    constexpr uint32_t BB = TYPE == KQ_TYPE_Q4_K ? KQ_Q4K_BYTES : TYPE == KQ_TYPE_Q5_K ? KQ_Q5K_BYTES : KQ_Q6K_BYTES;
+    const uint32_t b0 = blockIdx.z * p.blocks_per_split, b1 = min(b0 + p.blocks_per_split, p.n_blocks);
+
+    w_u32x4 xreg[TT];
+    auto fetch_x = [&](uint32_t b) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t) xreg[t] = *(const w_u32x4*)(xsrc[t] + (size_t)b * 512u);
+    };
+    auto park_x = [&](uint32_t buf) {
+#pragma unroll
+        for (int t = 0; t < TT; ++t) *(w_u32x4*)(&xs[buf * X_BYTES + t * 8192u + xdst]) = xreg[t];
+    };
+    w_f32x4 acc[2][TT];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) acc[r][t] = w_f32x4{0, 0, 0, 0};
+
+    WideW<TYPE> w[2], wn[2];
+    fetch_x(b0);
+#pragma unroll
+    for (int r = 0; r < 2; ++r) wn[r].load(wrow[r] + (size_t)b0 * BB, kq);
+    park_x(0);
+    wide_barrier();
+    for (uint32_t b = b0; b < b1; ++b) {
+        const uint32_t buf = (b - b0) & 1u;
+        const uint32_t bn = min(b + 1u, b1 - 1u);   // (the last step requests its own superblock again)
+        fetch_x(bn);
+        float sa[2][Q6 ? 4 : 2], sb[2][Q6 ? 4 : 2];   // a weight is q * sa + sb
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            w[r] = wn[r];
+            wn[r].load(wrow[r] + (size_t)bn * BB, kq);
+            if constexpr (Q6) {
+                const float d = half_bits_to_float(w[r].d);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const uint32_t word = t < 2 ? w[r].sc.x : w[r].sc.y;
+                    sa[r][t] = d * (float)(int)(int8_t)(word >> (16 * (t & 1) + 8 * (kq & 1u)));
+                    sb[r][t] = -32.0f * sa[r][t];   // exact: the sum rounds once, as s * (q - 32) does
+                }
+            } else {
+                const w_u32x4 h = w[r].hdr;
+                const float d = half_bits_to_float(h.x & 0xFFFFu), dmin = half_bits_to_float(h.x >> 16);
+                const uint32_t sc = kq < 2u ? h.y & 0x3F3F3F3Fu : (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
+                const uint32_t mn = kq < 2u ? h.z & 0x3F3F3F3Fu : ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
+                const uint32_t s2 = sc >> (16u * (kq & 1u)), m2 = mn >> (16u * (kq & 1u));
+                sa[r][0] = d * (float)(s2 & 255u);
+                sa[r][1] = d * (float)((s2 >> 8) & 255u);
+                sb[r][0] = -(dmin * (float)(m2 & 255u));
+                sb[r][1] = -(dmin * (float)((m2 >> 8) & 255u));
+            }
+        }
+        const uint8_t* xb = xs + buf * X_BYTES + kq * 256u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            w_bf16x8 B[2];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                uint32_t q[2];
+                if constexpr (Q6) {
+                    const int t = j >> 1, u = j & 1;
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        q[i] = ((w[r].ql[t & 1][2 * u + i] >> (4 * (t >> 1))) & 0x0F0F0F0Fu) |
+                               (((w[r].qh[2 * u + i] >> (2 * t)) & 0x03030303u) << 4);
+                } else {
+                    const int i8 = j >> 1;
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        q[i] = (w[r].q[i8 >> 1][2 * (i8 & 1) + i] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
+                        if constexpr (Q5) q[i] |= ((w[r].f[i8 >> 1][2 * (i8 & 1) + i] >> (2u * kq + (j & 1))) & 0x01010101u) << 4;
+                    }
+                }
+                const float a = sa[r][Q6 ? j >> 1 : j & 1], nb = sb[r][Q6 ? j >> 1 : j & 1];
+                w_u32x4 o;
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    o[2 * i] = w_pack_bf16(fmaf(a, (float)(q[i] & 255u), nb), fmaf(a, (float)((q[i] >> 8) & 255u), nb));
+                    o[2 * i + 1] = w_pack_bf16(fmaf(a, (float)((q[i] >> 16) & 255u), nb), fmaf(a, (float)(q[i] >> 24), nb));
+                }
+                B[r] = __builtin_bit_cast(w_bf16x8, o);
+            }
+            const uint8_t* xj = xb + j * 1024 + ((r16 + 2u * j + (kq & 1u)) & 15u) * 16u;
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+                const w_bf16x8 A = *(const w_bf16x8*)(xj + t * 8192);
+#pragma unroll
+                for (int r = 0; r < 2; ++r) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[r], acc[r][t], 0, 0, 0);
+            }
+        }
+        park_x(buf ^ 1u);
+        wide_barrier();
+    }
+
+    // outputs through LDS, as in wide_kernel
+    float* ot = (float*)xs;
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ot[(16 * t + 4u * kq + i) * OP + wave * 32u + 16u * r + r16] = acc[r][t][i];
+    __syncthreads();
+    if (p.n_splits > 1) {   // wide_sum_kernel adds the splits' tiles
+        float* tile = p.partial + (((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (TT * 16u * 256u);
+        for (uint32_t n = tid; n < TT * 1024u; n += 512u)
+            *(float4*)(tile + 4u * n) = *(const float4*)(ot + (n >> 6) * OP + 4u * (n & 63u));
+        return;
+    }
+    const uint32_t col = tid & 255u, n = blockIdx.x * 256u + col;
+    if (n >= p.N) return;
+    const float bv = p.bias ? p.bias[n] : 0.0f;
+#pragma unroll 4
+    for (uint32_t slot = tid >> 8; slot < count; slot += 2u) p.Y[(size_t)(t0 + slot) * p.ldy + n] = ot[slot * OP + col] + bv;
+}
+
+template <int TYPE>
+static void launch_short_type(const WideParams& p, uint32_t tt, dim3 grid, hipStream_t s)
+{
+    switch (tt) {
+    case 1: case 2: hipLaunchKernelGGL((short_kernel<TYPE, 2>), grid, dim3(512), 0, s, p); break;
+    case 3: hipLaunchKernelGGL((short_kernel<TYPE, 3>), grid, dim3(512), 0, s, p); break;
+    case 4: hipLaunchKernelGGL((short_kernel<TYPE, 4>), grid, dim3(512), 0, s, p); break;
+    case 5: hipLaunchKernelGGL((short_kernel<TYPE, 5>), grid, dim3(512), 0, s, p); break;
+    case 6: hipLaunchKernelGGL((short_kernel<TYPE, 6>), grid, dim3(512), 0, s, p); break;
+    case 7: hipLaunchKernelGGL((short_kernel<TYPE, 7>), grid, dim3(512), 0, s, p); break;
+    default: hipLaunchKernelGGL((short_kernel<TYPE, 8>), grid, dim3(512), 0, s, p); break;
+    }
+}
+
+// How a call of M bf16 tokens is cut, its price in us and what the GEMM takes.  A superblock of a workgroup's walk costs
+// 1.35 + 0.41 per tile of tokens (Q5_K 1.6 + 0.41, Q6_K 3.5 + 0.27), a round over the CUs 5, the launch that adds the splits
+// 3 and 1.2 per 10^6 floats.  Measured against the GEMM, us, at 100 / 128 / 256 tokens: Q4_K 4096x4096 20 / 22 / 28 against
+// 37 / 37 / 39, 6144x4096 23 / 25 / 36 against 38, 28672x4096 55 / 62 / 89 against 65 / 62 / 66 (32 tokens 30 against 61),
+// Q6_K 4096x14336 40 / 43 / 61 against 61 / 61 / 63, 7168x1024 21 / 21 / 27 against 22 / 20 / 20; at 384 tokens 4096x4096 36
+// against 51, 28672x4096 163 against 108.
+ShortPlan plan_short(const MatmulArgs& a, size_t capacity_floats, uint32_t cus)
+{
+    ShortPlan best{0, 0, 0, 0, 1e30, 0.0};
+    const uint32_t tiles = (a.M + 15u) / 16u, gy0 = (tiles + 7u) / 8u;
+    uint32_t tt = (tiles + gy0 - 1u) / gy0;
+    if (tt < 2u) tt = 2u;
+    const uint32_t gy = (tiles + tt - 1u) / tt, gx = (a.N + 255u) / 256u;
+    const double step_us = a.type == KQ_TYPE_Q4_K ? 1.35 + 0.41 * tt : a.type == KQ_TYPE_Q5_K ? 1.6 + 0.41 * tt : 3.5 + 0.27 * tt;
+    const size_t tile_floats = (size_t)gy * tt * 16u * gx * 256u;
+    for (uint32_t c = 1; c <= a.n_blocks && c <= 16u; ++c) {
+        const uint32_t per = (a.n_blocks + c - 1u) / c, z = (a.n_blocks + per - 1u) / per;
+        if (z > 1u && z * tile_floats > capacity_floats) break;
+        const double rounds = (double)(((uint64_t)gx * gy * z + cus - 1u) / cus);
+        const double us = 2.0 + rounds * (per * step_us + 5.0) + (z > 1u ? 3.0 + 1.2e-6 * (double)z * (double)tile_floats : 0.0);
+        if (us < best.us) best = ShortPlan{tt, gy, z, per, us, 0.0};
+    }
+    // The GEMM up to 256 tokens: 14 + 5.7 per 1024 of K while its tiles leave CUs idle (60 at most: it cuts K too), from
+    // there on 16 + 1.5 per 1000 rows of 4096; up to 512 tokens 1.4 times the former (measured at K from 4096 on only)
+    const double few = std::fmin(60.0, 14.0 + 5.7 * a.K / 1024.0), many = 16.0 + 1.5e-3 * a.N * (a.K / 4096.0);
+    if (a.M <= 256u) best.gemm_us = std::fmax(few, many);
+    else if (a.K >= 4096u) best.gemm_us = 1.4 * few;
+    return best;
+}
+
+hipError_t launch_short(const MatmulArgs& a, const ShortPlan& plan, const SplitScratch& sc, hipStream_t s)
+{
+    WideParams p{};
+    p.x.xa = (uint8_t*)const_cast<void*>((const void*)a.X);
+    p.W = a.W; p.bias = a.bias; p.Y = a.Y;
+    p.M = a.M; p.N = a.N; p.n_blocks = a.n_blocks; p.row_stride_bytes = a.row_stride_bytes; p.ldy = a.ldy;
+    p.blocks_per_split = plan.blocks_per_split;
+    p.n_splits = plan.splits;
+    p.partial = sc.partial;
+    const dim3 grid((a.N + 255u) / 256u, plan.groups, plan.splits);
+    if (a.type == KQ_TYPE_Q4_K) launch_short_type<KQ_TYPE_Q4_K>(p, plan.tiles, grid, s);
+    else if (a.type == KQ_TYPE_Q5_K) launch_short_type<KQ_TYPE_Q5_K>(p, plan.tiles, grid, s);
+    else launch_short_type<KQ_TYPE_Q6_K>(p, plan.tiles, grid, s);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess || plan.splits <= 1u) return e;
+    hipLaunchKernelGGL(wide_sum_kernel, dim3(grid.x, (a.M + 3u) / 4u), dim3(256), 0, s, p, plan.tiles * 16u, plan.groups);
+    return hipGetLastError();
 }
 
 }  // namespace kq

@@ -547,7 +547,9 @@ BPK_API int bpk_set_option(const char *name, int value);
  * walk over the 256-tiles' k steps cut into equal shares (*share k steps each);
  * 3 = tiles of 256 tokens x 128 weight rows; 4 = the full rounds of 256-tiles
  * over the first *rows_first weight rows, then the rest as in 3; 5 = tiles of
- * 256 tokens x 192 weight rows. */
+ * 256 tokens x 192 weight rows.  Short prompts (up to 512 tokens, where it is
+ * priced lower) go to a kernel with K cut over workgroups instead, unless
+ * "gemm_tile" or "gemm_split" is set. */
 BPK_API int bpk_gemm_plan(int type, uint32_t M, uint32_t N, uint32_t K, uint32_t compute_units,
                           int *form, uint32_t *share, uint32_t *rows_first);
 

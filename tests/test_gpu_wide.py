@@ -93,3 +93,29 @@ def test_moe_ffn_many_pairs_vs_oracle(gpu, kqo, tgu, tdn, T, E, k, H, I, skew): 
     assert np.all(np.abs(got - want) <= 1e-3 * rms + 1e-3 * np.abs(want))
     # both split x into 22 bits of its superblock's largest: the sums' order is what differs
     assert np.abs(got - tile).max() <= 1e-4 * rms + 1e-4 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("type_", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 256), (17, 255, 512), (33, 257, 2816), (100, 520, 4096), (128, 256, 256), (129, 300, 1024)])
+def test_short_prompt_vs_oracle(gpu, kqo, type_, M, N, K):  # noqa: F811
+    """bf16 rows of a short prompt: tokens around the groups of 16 and 128, rows around 256, K cut over workgroups and
+    not, with a bias; against the oracle on the same bf16 rows and against the GEMM's 128-tile (the same products)."""
+    import torch
+    from backpack_amd import capi, kquant
+    print("short", type_, M, N, K, flush=True)
+    raw, packed, w = gpu.make_weight(type_, N, K, seed=M + N)
+    rng = np.random.default_rng(K + M)
+    X = gpu.dev(rng.standard_normal((M, K)).astype(np.float32)).bfloat16()
+    bias = gpu.dev(rng.standard_normal(N).astype(np.float32))
+    got = kquant.matmul(X, w, bias=bias).cpu().numpy()
+    capi.set_option("gemm_tile", 128)
+    try:
+        gemm = kquant.matmul(X, w, bias=bias).cpu().numpy()
+    finally:
+        capi.set_option("gemm_tile", 0)
+    want = kqo.matmul(type_, X.float().cpu().numpy(), packed, N, K) + bias.cpu().numpy()
+    rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    # weights rounded to bf16: 2^-9 per product, K independent ones
+    assert np.sqrt(np.mean((got - want) ** 2.0)) <= 2.0 ** -8 * rms
+    # the same products in another order: fp32 sums of K of them
+    assert np.abs(got - gemm).max() <= 2.0 ** -23 * K ** 0.5 * 8 * max(rms, float(np.abs(want).max()))
