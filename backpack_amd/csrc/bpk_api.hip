@@ -451,11 +451,15 @@ int bpk_weight_destroy(bpk_weight* w)
 
 // More than 16 tokens, or any number by option.  Measured with the split of X included, us against the 16-token tile
 // kernel: at 17 .. 32 tokens Q4_K 6144x4096 16.7 against 26, 28672x4096 37 against 58, Q6_K 4096x14336 37 against 58,
-// 128256x4096 175 against 396; at 16 tokens 16.3 against 13.6, 30 against 30.6, 32 against 30 (128256 rows: 147
-// against 195, left for a rule of its own).  At 48: 19.6 / 39, 41 / 86, 41.5 / 86, 205 / 599.
+// 128256x4096 175 against 396; at 48: 19.6 / 39, 41 / 86, 41.5 / 86, 205 / 599.
+// 9 .. 16 tokens too where the rows alone give (nearly) every CU a workgroup of 256: at 9 / 16 tokens Q4_K 128256x4096 72 /
+// 78 against 98 / 113, Q6_K 142 / 145 against 176 / 183, 64000x4096 77 / 78 against 89 / 93.  On fewer rows the tile kernel
+// stays ahead (28672x4096 at 16: Q6_K 46 against 48, Q5_K 34 against 36; Q6_K 32000x2048 28 against 30), and up to 8
+// tokens the two are level (Q6_K 128256x4096 at 8: 147 against 142, 64000x4096 75 against 77).
 static bool takes_wide(const kq::MatmulArgs& a)
 {
-    return (t_family == 8 || (t_family == 0 && a.M > 16u)) && kq::wide_supported(a);
+    const bool rows_fill = a.M > 8u && 16ull * ((a.N + 255u) / 256u) >= 15ull * kq::device_cu_count();
+    return (t_family == 8 || (t_family == 0 && (a.M > 16u || rows_fill))) && kq::wide_supported(a);
 }
 
 // fold: the greedy pick over the outputs, taken along by the launch where its kernel can (*folded says so)

@@ -13,7 +13,7 @@ Q4_K, Q5_K, Q6_K = 12, 13, 14
 
 @pytest.mark.parametrize("type_", [Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("M,N,K", [(17, 1, 256), (32, 255, 512), (33, 257, 2816), (64, 300, 1024), (65, 256, 256),
-                                   (129, 520, 4096)])
+                                   (129, 520, 4096), (9, 61500, 256), (16, 65537, 256)])
 def test_many_tokens_vs_oracle(gpu, kqo, type_, M, N, K):  # noqa: F811
     from backpack_amd import capi, kquant
     print("wide", type_, M, N, K, flush=True)
