@@ -25,7 +25,10 @@
 //
 // Work split.  Eight waves of two 16-row tiles each; the X of a superblock (TT tiles of 16 tokens, 16 KB each) is
 // staged in LDS (two buffers), shared by the waves.  K is cut over blockIdx.z when rows give too few
-// workgroups; the last one to arrive adds the partial tiles in split order.
+// workgroups; a second launch adds the partial tiles in split order.
+//
+// Mixture layers (records of pairs of one expert): 128 experts x 8 slots, 2048 / 768, 2048 tokens 1266 us on the
+// 16-token tiles, 739 here; 24 tokens 153 and 128.
 #include "kq_format.h"
 #include "kq_kernels.h"
 #include "kq_wave.h"

@@ -502,7 +502,8 @@ BPK_API const char *bpk_last_kernel(void);
  * (bf16 X only), 5 = lanes-along-K GEMV (M = 1), 6 = 16-row x 16-token
  * matrix-core tiles (groups of 16 tokens), 7 = one token on the matrix cores
  * (Q4_K rows of up to 16 superblocks), 8 = matrix-core tiles of up to 64 tokens
- * (taken by itself from 17 tokens on; bpk_last_kernel says "mtile" for both).  A forced family that cannot serve the call's
+ * (taken by itself from 17 tokens on, from 9 on
+ * matrices whose rows fill the part; bpk_last_kernel says "mtile" for both).  A forced family that cannot serve the call's
  * shape fails with BPK_ERR_SHAPE instead of falling back. */
 BPK_API int bpk_force_kernel(int family);
 
