@@ -15,6 +15,9 @@
  * wrapper that wants that behaviour prints bpk_last_error() and returns.
  *
  * One host thread per stream, as in the reference (runtime/model_runner.h:27-30).
+ * Matmuls that cut K over workgroups, and fp32 ones of more than eight tokens, use
+ * scratch memory of the device: on one device their calls go to one stream, or
+ * are ordered by the caller, so that they do not overlap.
  */
 #ifndef BPK_KQUANT_H
 #define BPK_KQUANT_H
