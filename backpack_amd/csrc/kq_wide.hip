@@ -24,11 +24,21 @@
 // each group of eight in the order 0 2 1 3 4 6 5 7 (what masking dwords leaves).
 //
 // Work split.  Eight waves of two 16-row tiles each; the X of a superblock (TT tiles of 16 tokens, 16 KB each) is
-// staged in LDS (two buffers), shared by the waves.  K is cut over blockIdx.z when rows give too few
-// workgroups; a second launch adds the partial tiles in split order.
+// staged in LDS, shared by the waves.  K is cut over blockIdx.z when rows give too few workgroups; a second launch
+// adds the partial tiles in split order.
 //
-// Mixture layers (records of pairs of one expert): 128 experts x 8 slots, 2048 / 768, us with the router, against the
-// 16-token tiles: 2048 tokens 733-775 / 1264, 256 tokens 190-195 / 267, 24 tokens 118-129 / 153 (several boxes).
+// The walk.  X (halves of a superblock, a ring of three) and W (each wave its own rows) go from memory to LDS without
+// registers, requested a superblock ahead and spread over its eight steps; a step's LDS reads and its expansion of weights
+// stand between the matrix instructions of the step before (sched_group_barrier), and the two meetings per superblock lie
+// ahead of a step whose operands are already in registers.  What that replaced: every lane fetched its 16-byte pieces
+// of W and X itself (52 cache accesses per load instruction, 20 now) and the compiler read operands right ahead of their
+// use.  A workgroup's walk still takes 1.4 times its matrix instructions' time: a matrix instruction holds the issue for 8
+// cycles and a vector one for 4, so beside two vector instructions each they no longer overlap.
+//
+// Mixture layers (records of pairs of one expert): consecutive workgroups go to the same XCD, so a record's row groups
+// and an expert's records meet their X and W in that L2 (128 experts x 8 slots, 2048 / 768, 2048 tokens: 750 -> 703 us).
+// us with the router, now / with the walk before / on the 16-token tiles: 2048 tokens 645 / 777 / 1264, 256 tokens
+// 190 / 196 / 267, 24 tokens 125 / 125 / 153 (one box).
 #include "kq_format.h"
 #include "kq_kernels.h"
 #include "kq_wave.h"
@@ -165,11 +175,11 @@ struct WideParams {
     uint32_t n_splits, blocks_per_split;
     float* partial;          // [split][token group][workgroup][token][256 columns]
     int act;                 // 0, or 2 / 3: Y = silu / gelu_tanh (W x) * (W2 x)
-    // grouped (records != nullptr): blockIdx.y walks records {expert, count, pair ids ...}, W and W2 advance by N rows
-    // per expert, a pair's X row is itself (x_per_slot) or pair / k_slots, its Y row the pair
+    // grouped (records != nullptr): the workgroups walk records {expert, count, pair ids ...}, row_groups of them each; W and
+    // W2 advance by N rows per expert, a pair's X row is itself (x_per_slot) or pair / k_slots, its Y row the pair
     const uint32_t* records;
     const uint32_t* n_records;
-    uint32_t record_words, k_slots;
+    uint32_t record_words, k_slots, row_groups;
     int x_per_slot;
 };
 
@@ -183,6 +193,8 @@ template <> struct WideW<KQ_TYPE_Q4_K> {
         q[0] = *(const w_u32x4*)(blk + 16 + 32 * kq);
         q[1] = *(const w_u32x4*)(blk + 32 + 32 * kq);
     }
+    __device__ __forceinline__ void load_lds(const uint8_t* blk, const uint8_t*, uint32_t kq) { load(blk, kq); }
+    __device__ __forceinline__ void arrived() const { asm volatile("" ::"v"(hdr), "v"(q[0]), "v"(q[1]) : "memory"); }
 };
 template <> struct WideW<KQ_TYPE_Q5_K> {
     w_u32x4 hdr, q[2], f[2];
@@ -194,6 +206,8 @@ template <> struct WideW<KQ_TYPE_Q5_K> {
         q[0] = *(const w_u32x4*)(blk + 48 + 32 * kq);
         q[1] = *(const w_u32x4*)(blk + 64 + 32 * kq);
     }
+    __device__ __forceinline__ void load_lds(const uint8_t* blk, const uint8_t*, uint32_t kq) { load(blk, kq); }
+    __device__ __forceinline__ void arrived() const { asm volatile("" ::"v"(hdr), "v"(f[0]), "v"(f[1]), "v"(q[0]), "v"(q[1]) : "memory"); }
 };
 template <> struct WideW<KQ_TYPE_Q6_K> {
     w_u32x4 ql[2], qh;   // (blocks are 210 bytes apart: 2-byte aligned loads)
@@ -208,6 +222,17 @@ template <> struct WideW<KQ_TYPE_Q6_K> {
         __builtin_memcpy(&sc, blk + 192 + 8 * h, 8);
         __builtin_memcpy(&d, blk + 208, 2);
     }
+    // the block's 208 bytes ahead of d on a 16-byte boundary, d in the upper half of a word of its own
+    __device__ __forceinline__ void load_lds(const uint8_t* blk, const uint8_t* dw, uint32_t kq)
+    {
+        const uint32_t h = kq >> 1, lh = kq & 1u;
+        ql[0] = *(const w_u32x4*)(blk + 64 * h + 16 * lh);
+        ql[1] = *(const w_u32x4*)(blk + 64 * h + 32 + 16 * lh);
+        qh = *(const w_u32x4*)(blk + 128 + 32 * h + 16 * lh);
+        sc = *(const w_u32x2*)(blk + 192 + 8 * h);
+        d = (uint16_t)(*(const uint32_t*)dw >> 16);
+    }
+    __device__ __forceinline__ void arrived() const { asm volatile("" ::"v"(ql[0]), "v"(ql[1]), "v"(qh), "v"(sc), "v"((uint32_t)d) : "memory"); }
 };
 
 __device__ __forceinline__ uint32_t w_mul2(uint32_t a, w_half2 s)
@@ -218,21 +243,76 @@ __device__ __forceinline__ uint32_t w_mul2(uint32_t a, w_half2 s)
 // LDS writes of the workgroup are visible behind it; loads in flight stay in flight.
 __device__ __forceinline__ void wide_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-template <int TYPE, int TT>
-__global__ __launch_bounds__(512, 2) void wide_kernel(const WideParams p)
+// Memory -> LDS without registers: lane l's 16 (4) bytes land at m0 + 16 l (4 l).  Inline asm, because the compiler
+// would wait for such a load ahead of every LDS read that it cannot tell apart from its target; the waits are the
+// kernel's own (wide_meet).  No register is written, so none can be reused while a load is in flight.  The compiler does not
+// see into these statements, so the wait states between a vector instruction that writes a scalar register (a spill read
+// back, a readfirstlane) and a load that uses it (5), and ahead of a load that uses m0 (1), stand in them.
+__device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* src)
 {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+__device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* base, uint32_t off)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+}
+// ... with the lanes of `lanes` only (none: it moves nothing, but keeps its place in the count of loads in flight).  Called
+// with every lane active; no branch, so the steps of the walk stay one basic block.
+__device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* src, int lanes)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(src), "s"(lanes) : "memory");
+}
+__device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* base, uint32_t off, uint64_t lanes)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\ts_nop 2\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(off), "s"(base), "s"(lanes) : "memory");
+}
+__device__ __forceinline__ void lds_dma4(uint32_t lds, const uint8_t* base, uint32_t off, uint64_t lanes)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\ts_nop 2\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(off), "s"(base), "s"(lanes) : "memory");
+}
+__device__ __forceinline__ void lds_dma4(uint32_t lds, const void* src, int lanes)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\tglobal_load_lds_dword %1, off\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(src), "s"(lanes) : "memory");
+}
+// At most N of this wave's loads are still in flight, its LDS reads have returned, and so have the other waves'.
+template <int N>
+__device__ __forceinline__ void wide_meet() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
+
+// The kernel's LDS, in bytes.  X: a ring of three halves of a superblock, [token][hi, lo][16 pieces of 16 bytes], a piece's
+// place exchanged by its token (^ token % 16) so that the 16 tokens that a wave reads a piece of lie in different banks.
+// W: per wave its two row tiles' blocks as they are in memory (9, 11 or 13 units of 16 bytes per row: odd, so 16 rows start
+// in different banks), Q6_K's d behind them.  S: two buffers of the sums and the scales of X.
+template <int TYPE, int TT> struct WideLds {
+    static constexpr bool Q6 = TYPE == KQ_TYPE_Q6_K;
+    static constexpr uint32_t UNITS = TYPE == KQ_TYPE_Q4_K ? 9u : TYPE == KQ_TYPE_Q5_K ? 11u : 13u;   // per row and superblock
+    static constexpr uint32_t W_INSTR = (16u * UNITS + 63u) / 64u, W_LAST = 16u * UNITS - 64u * (W_INSTR - 1u);   // per tile
+    static constexpr uint32_t W_TILE = 256u * UNITS, W_WAVE = 2u * W_TILE + (Q6 ? 128u : 0u);
+    static constexpr uint32_t X_HALF = TT * 8192u, V_BUF = Q6 ? 0u : (TT > 2 ? 2048u : 1024u), I_BUF = 256u;
+    static constexpr uint32_t W_AT = 3u * X_HALF, V_AT = W_AT + 8u * W_WAVE, I_AT = V_AT + 2u * V_BUF, R_AT = I_AT + 2u * I_BUF, BYTES = R_AT + TT * 1024u;
+    static constexpr int N_W = 2 * (int)W_INSTR + (Q6 ? 2 : 0);   // a wave's loads for its weights of a superblock
+};
+
+template <int TYPE, int TT>
+__global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WideParams p)
+{
+    using L = WideLds<TYPE, TT>;
     constexpr bool Q6 = TYPE == KQ_TYPE_Q6_K, Q5 = TYPE == KQ_TYPE_Q5_K;
-    __shared__ __align__(16) uint8_t xs[2][TT * 16384];   // [tile of 16 tokens][hi, lo][step][lane] 16 B
-    __shared__ __align__(16) uint8_t vs[2][TT * 512];     // [tile][hi, lo][token] eight sub-block sums
-    __shared__ __align__(16) float is[2][TT * 16];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, kq = lane >> 4, r16 = lane & 15u;
+    constexpr uint32_t OP = 260;   // output tile: floats between tokens (the four lane groups write to different banks)
+    __shared__ __align__(16) uint8_t lds[L::BYTES];
+    static_assert(TT * 16 * OP * 4 <= L::R_AT, "the output tile fits");
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, kq = lane >> 4, r16 = lane & 15u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
     const uint32_t* rec = nullptr;
-    uint32_t count, t0 = 0;
+    uint32_t count, t0 = 0, bx = blockIdx.x;
     const uint8_t *W = p.W, *W2 = p.W2;
     if (p.records) {
-        if (blockIdx.y >= *p.n_records) return;   // whole workgroup
-        rec = p.records + (size_t)blockIdx.y * p.record_words;
+        const uint32_t all = *p.n_records * p.row_groups, share = (all + 7u) >> 3, at = (bx & 7u) * share + (bx >> 3);
+        if ((bx >> 3) >= share || at >= all) return;   // whole workgroup
+        const uint32_t record = at / p.row_groups;
+        bx = at - record * p.row_groups;
+        rec = p.records + (size_t)record * p.record_words;
         count = rec[1];
         const size_t skip = (size_t)rec[0] * p.N * p.row_stride_bytes;
         W += skip;
@@ -242,85 +322,119 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideParams p)
         t0 = blockIdx.y * (TT * 16u);
         count = min(p.M - t0, TT * 16u);
     }
-    // X row of slot i (slots beyond the count repeat the last: their outputs are dropped)
-    auto x_row = [&](uint32_t i) -> uint32_t {
-        i = min(i, count - 1u);
-        if (!rec) return t0 + i;
-        const uint32_t pr = rec[i];
-        return p.x_per_slot ? pr : pr / p.k_slots;
-    };
-    const uint8_t* xsrc[TT];
-#pragma unroll
-    for (int t = 0; t < TT; ++t) xsrc[t] = p.x.xa + (size_t)x_row(16u * t + r16) * p.n_blocks * WIDE_XA + kq * 16u + wave * 64u;
-    const size_t vcell = (size_t)x_row(min(tid >> 1, TT * 16u - 1u)) * p.n_blocks;
-    const size_t icell = (size_t)x_row(min(tid, TT * 16u - 1u)) * p.n_blocks;
-
-    // this lane's row of the wave's two tiles
-    const uint32_t out0 = p.act ? (blockIdx.x * WIDE_WAVES + wave) * 16u : (blockIdx.x * WIDE_WAVES + wave) * 32u;
-    const uint8_t* wrow[2];
-    wrow[0] = W + (size_t)min(out0 + r16, p.N - 1u) * p.row_stride_bytes;
-    wrow[1] = p.act ? W2 + (size_t)min(out0 + r16, p.N - 1u) * p.row_stride_bytes
-                    : W + (size_t)min(out0 + 16u + r16, p.N - 1u) * p.row_stride_bytes;
     constexpr uint32_t BB = TYPE == KQ_TYPE_Q4_K ? KQ_Q4K_BYTES : TYPE == KQ_TYPE_Q5_K ? KQ_Q5K_BYTES : KQ_Q6K_BYTES;
-
     const uint32_t b0 = blockIdx.z * p.blocks_per_split, b1 = min(b0 + p.blocks_per_split, p.n_blocks);
-    // X of the next superblock travels through registers: requested ahead of this superblock's arithmetic, parked behind
-    // it.  (Written straight into LDS the compiler waits for the transfer ahead of every LDS read: it cannot tell the
-    // two buffers apart.)
-    w_u32x4 xreg[TT][2];
-    auto fetch_x = [&](uint32_t b) {
+    // The slots' rows of Y and X, a copy per wave (no meeting).  A record's go straight into LDS: the first weights are requested
+    // behind them and are under way while the rows are turned into addresses.  Slots beyond the count repeat the last: their
+    // outputs are dropped.
+    uint32_t* const out_rows = (uint32_t*)(lds + L::R_AT + wave * (TT * 128u));
+    uint32_t* const x_rows = out_rows + TT * 16u;
+    const uint32_t slot0 = min(lane, min(count, TT * 16u) - 1u);
+    if (rec) lds_dma4(lds0 + L::R_AT + wave * (TT * 128u), (const uint8_t*)rec, slot0 * 4u, TT == 4 ? ~0ull : (1ull << (TT * 16u % 64u)) - 1ull);
+
+    // W: the wave's two tiles of 16 rows, unit after unit
+    const uint32_t out0 = p.act ? (bx * WIDE_WAVES + wave) * 16u : (bx * WIDE_WAVES + wave) * 32u;
+    const uint32_t row_last = p.N - 1u;
+    const uint32_t first[2] = {min(out0, row_last), min(p.act ? out0 : out0 + 16u, row_last)};
+    const uint8_t* wbase[2];
+    wbase[0] = W + (size_t)first[0] * p.row_stride_bytes + (size_t)b0 * BB;
+    wbase[1] = (p.act ? W2 : W) + (size_t)first[1] * p.row_stride_bytes + (size_t)b0 * BB;
+    uint32_t woff[2][L::W_INSTR], doff[2];
 #pragma unroll
-        for (int t = 0; t < TT; ++t)
+    for (int r = 0; r < 2; ++r) {
 #pragma unroll
-            for (int hl = 0; hl < 2; ++hl) xreg[t][hl] = *(const w_u32x4*)(xsrc[t] + (size_t)b * WIDE_XA + hl * 512);
+        for (uint32_t i = 0; i < L::W_INSTR; ++i) {
+            const uint32_t n = i * 64u + lane, row = n / L::UNITS, u = n % L::UNITS;
+            woff[r][i] = (min(first[r] + row, row_last) - first[r]) * p.row_stride_bytes + u * 16u;
+        }
+        doff[r] = (min(first[r] + r16, row_last) - first[r]) * p.row_stride_bytes + 206u;   // (d in the upper half; ends with the block)
+    }
+    const uint32_t w_lds = lds0 + L::W_AT + wave * L::W_WAVE;
+    // piece k of a superblock's weights: whole loads first, then each tile's last lanes (and d)
+    auto request_w = [&](int k) {
+        constexpr int WHOLE = 2 * ((int)L::W_INSTR - 1);
+        if (k < WHOLE) {
+            const uint32_t r = (uint32_t)k & 1u, i = (uint32_t)k >> 1;
+            lds_dma16(w_lds + r * L::W_TILE + i * 1024u, wbase[r], woff[r][i]);
+        } else if (k < WHOLE + 2) {
+            const uint32_t r = (uint32_t)k & 1u;
+            lds_dma16(w_lds + r * L::W_TILE + (L::W_INSTR - 1u) * 1024u, wbase[r], woff[r][L::W_INSTR - 1u], (1ull << L::W_LAST) - 1ull);
+        } else {
+            const uint32_t r = (uint32_t)k & 1u;
+            lds_dma4(w_lds + 2u * L::W_TILE + r * 64u, wbase[r], doff[r], 0xFFFFull);
+        }
     };
-    auto park_x = [&](int buf) {
+    auto next_w = [&](bool more) {
 #pragma unroll
-        for (int t = 0; t < TT; ++t)
+        for (int r = 0; r < 2; ++r) wbase[r] += more ? BB : 0u;
+    };
+    // Half h of the walk is superblock b0 + h / 2.  Requested ahead: X by two halves, W by one superblock (into the place it
+    // was read from), S half a superblock less; past the end the last is requested again.
+    constexpr int WAS = (TT + L::N_W + 3) / 4, XBS = (TT + 3) / 4;   // requests per step
+    const uint32_t n_sb = b1 - b0;
+    auto more = [&](uint32_t sb) { return sb + 1u < n_sb; };   // is there a superblock behind sb?
 #pragma unroll
-            for (int hl = 0; hl < 2; ++hl)
-                *(w_u32x4*)(&xs[buf][t * 16384 + hl * 8192 + wave * 1024u + lane * 16u]) = xreg[t][hl];
+    for (int k = 0; k < L::N_W; ++k) request_w(k);
+    next_w(more(0));
+
+    if (rec) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L::N_W) : "memory");   // the record's words
+        if (lane < TT * 16u) x_rows[lane] = p.x_per_slot ? out_rows[lane] : out_rows[lane] / p.k_slots;
+    } else if (lane < TT * 16u) {
+        out_rows[lane] = x_rows[lane] = t0 + slot0;
+    }
+    // X: load i of the wave takes half a superblock of two tokens
+    const uint8_t* xp[TT];
+#pragma unroll
+    for (int i = 0; i < TT; ++i) {
+        const uint32_t tok = 2u * (wave * TT + i) + (lane >> 5);
+        xp[i] = p.x.xa + ((size_t)x_rows[tok] * p.n_blocks + b0) * WIDE_XA + ((lane >> 4) & 1u) * 512u + ((lane ^ tok) & 15u) * 16u;
+    }
+    // its sums (waves 0, 1) and scales (the last wave)
+    const uint32_t vn = (wave & 1u) * 64u + lane;
+    const uint8_t* vp = p.x.xv + ((size_t)x_rows[min((vn >> 5) * 16u + (vn & 15u), TT * 16u - 1u)] * p.n_blocks + b0) * WIDE_XV + ((vn >> 4) & 1u) * 16u;
+    const float* ip = p.x.xi + (size_t)x_rows[min(lane, TT * 16u - 1u)] * p.n_blocks + b0;
+    int s_lanes = wave < (TT > 2 ? 2u : 1u) ? -1 : 0, i_lanes = wave == WIDE_WAVES - 1u ? -1 : 0;   // all or none
+    // (a scalar register each: the compiler would keep such a choice in a vector register)
+    asm("s_nop 1\n\tv_readfirstlane_b32 %0, %1" : "=s"(s_lanes) : "v"(s_lanes));
+    asm("s_nop 1\n\tv_readfirstlane_b32 %0, %1" : "=s"(i_lanes) : "v"(i_lanes));
+    auto request_x = [&](uint32_t ring, int i, int step) {   // piece i, which moves on by `step` bytes
+        lds_dma16(lds0 + ring * L::X_HALF + (wave * TT + i) * 1024u, xp[i]);
+        xp[i] += step;
     };
-    w_u32x4 vreg = {0, 0, 0, 0};
-    float ireg = 0.0f;
-    auto fetch_small = [&](uint32_t b) {
-        if (!Q6 && tid < TT * 32u) vreg = *(const w_u32x4*)(p.x.xv + (vcell + b) * WIDE_XV + (tid & 1u) * 16u);
-        if (tid < TT * 16u) ireg = p.x.xi[icell + b];
-    };
-    auto park_small = [&](int buf) {
-        if (!Q6 && tid < TT * 32u)
-            *(w_u32x4*)(&vs[buf][(tid >> 5) * 512u + (tid & 1u) * 256u + ((tid >> 1) & 15u) * 16u]) = vreg;
-        if (tid < TT * 16u) is[buf][tid] = ireg;
+    auto request_s = [&](uint32_t buf, uint32_t step) {   // step: superblocks
+        if constexpr (!Q6) lds_dma16(lds0 + L::V_AT + buf * L::V_BUF + (wave & 1u) * 1024u, vp, s_lanes);
+        lds_dma4(lds0 + L::I_AT + buf * L::I_BUF, (const void*)ip, i_lanes);
+        vp += step * WIDE_XV;
+        ip += step;
     };
 
-    w_f32x4 tot[2][TT];
+    // operands of X for step j: four places of the exchanged pieces
+    uint32_t a_lane[4];
 #pragma unroll
-    for (int r = 0; r < 2; ++r)
+    for (int jj = 0; jj < 4; ++jj) a_lane[jj] = r16 * 512u + (((4u * jj + kq) ^ r16) & 15u) * 16u;
+    w_half8 A[2][2][TT];   // [step % 2][hi, lo][tile]
+    auto read_a = [&](uint32_t ring, int j) {
+        const uint8_t* x = lds + ring * L::X_HALF + a_lane[j & 3];
 #pragma unroll
-        for (int t = 0; t < TT; ++t) tot[r][t] = w_f32x4{0, 0, 0, 0};
+        for (int hl = 0; hl < 2; ++hl)
+#pragma unroll
+            for (int t = 0; t < TT; ++t) A[j & 1][hl][t] = *(const w_half8*)(x + t * 8192 + hl * 256);
+    };
 
-    WideW<TYPE> w[2], wn[2];
-    fetch_x(b0);
-    fetch_small(b0);
-#pragma unroll
-    for (int r = 0; r < 2; ++r) wn[r].load(wrow[r] + (size_t)b0 * BB, kq);
-    park_x(0);
-    park_small(0);
-    wide_barrier();
-
-    for (uint32_t b = b0; b < b1; ++b) {
-        const int buf = (int)((b - b0) & 1u);
-        const uint32_t bn = min(b + 1u, b1 - 1u);   // (the last step requests its own superblock again)
-        fetch_x(bn);
-        fetch_small(bn);
+    WideW<TYPE> w[2];
+    auto read_w = [&]() {
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
-            w[r] = wn[r];
-            wn[r].load(wrow[r] + (size_t)bn * BB, kq);
+            const uint8_t* row = lds + L::W_AT + wave * L::W_WAVE + r * L::W_TILE + r16 * (L::UNITS * 16u);
+            w[r].load_lds(row, lds + L::W_AT + wave * L::W_WAVE + 2u * L::W_TILE + r * 64u + r16 * 4u, kq);
         }
-        // per-lane scales, as pairs
-        w_half2 sc[2][Q6 ? 4 : 2];
-        w_u32x4 bmn[2];
+    };
+    // what a superblock needs of its headers: per-lane scales as pairs, minima operands, super-scales
+    w_half2 sc[2][Q6 ? 4 : 2];
+    w_u32x4 bmn[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+    float d24[2] = {0.0f, 0.0f}, m24[2] = {0.0f, 0.0f};
+    auto headers = [&]() {
 #pragma unroll
         for (int r = 0; r < 2; ++r) {
             if constexpr (Q6) {
@@ -333,115 +447,201 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideParams p)
                 }
             } else {
                 const w_u32x4 h = w[r].hdr;
-                const uint32_t scA = h.y & 0x3F3F3F3Fu, mnA = h.z & 0x3F3F3F3Fu;
+                const uint32_t scA = h.y & 0x3F3F3F3Fu;
                 const uint32_t scB = (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
-                const uint32_t mnB = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
                 const uint32_t s2 = (kq < 2u ? scA : scB) >> (16u * (kq & 1u));
                 const _Float16 a = (_Float16)(float)(s2 & 255u), c = (_Float16)((float)((s2 >> 8) & 255u) * 0.0625f);
                 sc[r][0] = w_half2{a, a};
                 sc[r][1] = w_half2{c, c};   // (high nibbles sit four bits up)
+            }
+        }
+    };
+    auto headers2 = [&]() {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            if constexpr (Q6) {
+                d24[r] = half_bits_to_float(w[r].d);
+            } else {
+                const w_u32x4 h = w[r].hdr;
+                const uint32_t mnA = h.z & 0x3F3F3F3Fu, mnB = ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
                 // the eight minima as fp16 subnormals mn * 2^-24, against the hi sums (kq 0) and the lo sums (kq 1)
                 const uint32_t keep = kq < 2u ? 0xFFFFFFFFu : 0u;
                 bmn[r] = w_u32x4{__builtin_amdgcn_perm(0u, mnA, 0x0c010c00u) & keep, __builtin_amdgcn_perm(0u, mnA, 0x0c030c02u) & keep,
                                  __builtin_amdgcn_perm(0u, mnB, 0x0c010c00u) & keep, __builtin_amdgcn_perm(0u, mnB, 0x0c030c02u) & keep};
+                d24[r] = half_bits_to_float(h.x & 0xFFFFu) * 16777216.0f;
+                m24[r] = half_bits_to_float(h.x >> 16) * (16777216.0f * 32.0f);
             }
         }
-        w_f32x4 D[2][TT];
+    };
+    w_half8 Bh[2][2], Bl[2][2];   // [step % 2][tile]
+    auto expand = [&](int j) {
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
+        for (int r = 0; r < 2; ++r) {
+            w_u32x4 o;
+            if constexpr (Q6) {
+                const int t = j >> 1, u = j & 1;
+                const uint32_t l0 = w[r].ql[t & 1][2 * u], l1 = w[r].ql[t & 1][2 * u + 1];
+                const uint32_t h0 = w[r].qh[2 * u], h1 = w[r].qh[2 * u + 1];
+                const uint32_t c0 = ((l0 >> (4 * (t >> 1))) & 0x0F0F0F0Fu) | (((h0 >> (2 * t)) & 0x03030303u) << 4);
+                const uint32_t c1 = ((l1 >> (4 * (t >> 1))) & 0x0F0F0F0Fu) | (((h1 >> (2 * t)) & 0x03030303u) << 4);
+                w_u32x4 lo;
 #pragma unroll
-            for (int t = 0; t < TT; ++t) D[r][t] = w_f32x4{0, 0, 0, 0};
-        const uint8_t* xb = xs[buf] + lane * 16u;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            w_half8 Bh[2], Bl[2];
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                w_u32x4 o;
-                if constexpr (Q6) {
-                    const int t = j >> 1, u = j & 1;
-                    const uint32_t l0 = w[r].ql[t & 1][2 * u], l1 = w[r].ql[t & 1][2 * u + 1];
-                    const uint32_t h0 = w[r].qh[2 * u], h1 = w[r].qh[2 * u + 1];
-                    const uint32_t c0 = ((l0 >> (4 * (t >> 1))) & 0x0F0F0F0Fu) | (((h0 >> (2 * t)) & 0x03030303u) << 4);
-                    const uint32_t c1 = ((l1 >> (4 * (t >> 1))) & 0x0F0F0F0Fu) | (((h1 >> (2 * t)) & 0x03030303u) << 4);
-                    w_u32x4 lo;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const uint32_t c = i < 2 ? c0 : c1;
-                        const uint32_t oi = (((i & 1) ? c >> 8 : c) & 0x00FF00FFu) | 0x64006400u;   // 1024 + q
-                        const w_half2 q = __builtin_bit_cast(w_half2, oi) - w_half2{(_Float16)1056.0f, (_Float16)1056.0f};
-                        const w_half2 hi = q * sc[r][t];
-                        o[i] = __builtin_bit_cast(uint32_t, hi);
-                        lo[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(q, sc[r][t], -hi));
-                    }
-                    Bl[r] = __builtin_bit_cast(w_half8, lo);
-                } else {
-                    const int i = j >> 1;
-                    const uint32_t d0 = w[r].q[i >> 1][2 * (i & 1)], d1 = w[r].q[i >> 1][2 * (i & 1) + 1];
-                    const uint32_t e0 = d0 >> 8, e1 = d1 >> 8;
-                    const uint32_t m = (j & 1) ? 0x00F000F0u : 0x000F000Fu;
-                    o = w_u32x4{d0 & m, e0 & m, d1 & m, e1 & m};
-                    if constexpr (Q5) {
-                        // bit 2kq (2kq + 1) of a byte of fifth bits: bit 4 beside a low nibble, bit 8 beside a high one
-                        const uint32_t g0 = w[r].f[i >> 1][2 * (i & 1)] >> (2u * kq), g1 = w[r].f[i >> 1][2 * (i & 1) + 1] >> (2u * kq);
-                        if (j & 1) {
-                            o.x |= (g0 << 7) & 0x01000100u; o.y |= (g0 >> 1) & 0x01000100u;
-                            o.z |= (g1 << 7) & 0x01000100u; o.w |= (g1 >> 1) & 0x01000100u;
-                        } else {
-                            o.x |= (g0 << 4) & 0x00100010u; o.y |= (g0 >> 4) & 0x00100010u;
-                            o.z |= (g1 << 4) & 0x00100010u; o.w |= (g1 >> 4) & 0x00100010u;
-                        }
-                    }
-#pragma unroll
-                    for (int n = 0; n < 4; ++n) o[n] = w_mul2(o[n], sc[r][j & 1]);
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t c = i < 2 ? c0 : c1;
+                    const uint32_t oi = (((i & 1) ? c >> 8 : c) & 0x00FF00FFu) | 0x64006400u;   // 1024 + q
+                    const w_half2 q = __builtin_bit_cast(w_half2, oi) - w_half2{(_Float16)1056.0f, (_Float16)1056.0f};
+                    const w_half2 hi = q * sc[r][t];
+                    o[i] = __builtin_bit_cast(uint32_t, hi);
+                    lo[i] = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(q, sc[r][t], -hi));
                 }
-                Bh[r] = __builtin_bit_cast(w_half8, o);
-            }
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                const w_half8 ah = *(const w_half8*)(xb + t * 16384 + j * 1024);
-                const w_half8 al = *(const w_half8*)(xb + t * 16384 + 8192 + j * 1024);
-#pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    D[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, Bh[r], D[r][t], 0, 0, 0);
-                    D[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al, Bh[r], D[r][t], 0, 0, 0);
-                    if constexpr (Q6) D[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah, Bl[r], D[r][t], 0, 0, 0);
+                Bl[j & 1][r] = __builtin_bit_cast(w_half8, lo);
+            } else {
+                const int i = j >> 1;
+                const uint32_t d0 = w[r].q[i >> 1][2 * (i & 1)], d1 = w[r].q[i >> 1][2 * (i & 1) + 1];
+                const uint32_t e0 = d0 >> 8, e1 = d1 >> 8;
+                const uint32_t m = (j & 1) ? 0x00F000F0u : 0x000F000Fu;
+                o = w_u32x4{d0 & m, e0 & m, d1 & m, e1 & m};
+                if constexpr (Q5) {
+                    // bit 2kq (2kq + 1) of a byte of fifth bits: bit 4 beside a low nibble, bit 8 beside a high one
+                    const uint32_t g0 = w[r].f[i >> 1][2 * (i & 1)] >> (2u * kq), g1 = w[r].f[i >> 1][2 * (i & 1) + 1] >> (2u * kq);
+                    if (j & 1) {
+                        o.x |= (g0 << 7) & 0x01000100u; o.y |= (g0 >> 1) & 0x01000100u;
+                        o.z |= (g1 << 7) & 0x01000100u; o.w |= (g1 >> 1) & 0x01000100u;
+                    } else {
+                        o.x |= (g0 << 4) & 0x00100010u; o.y |= (g0 >> 4) & 0x00100010u;
+                        o.z |= (g1 << 4) & 0x00100010u; o.w |= (g1 >> 4) & 0x00100010u;
+                    }
                 }
+#pragma unroll
+                for (int n = 0; n < 4; ++n) o[n] = w_mul2(o[n], sc[r][j & 1]);
             }
+            Bh[j & 1][r] = __builtin_bit_cast(w_half8, o);
         }
+    };
+    w_f32x4 D[2][TT], tot[2][TT];
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int t = 0; t < TT; ++t) { D[r][t] = w_f32x4{0, 0, 0, 0}; tot[r][t] = w_f32x4{0, 0, 0, 0}; }
+    auto multiply = [&](int j) {
+        const int s = j & 1;
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+                D[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[s][0][t], Bh[s][r], j == 0 ? w_f32x4{0, 0, 0, 0} : D[r][t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int r = 0; r < 2; ++r) D[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[s][1][t], Bh[s][r], D[r][t], 0, 0, 0);
+        if constexpr (Q6) {
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int r = 0; r < 2; ++r) D[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[s][0][t], Bl[s][r], D[r][t], 0, 0, 0);
+        }
+    };
+
+    auto add_up = [&](uint32_t sbuf) {   // a finished superblock's products, scaled
 #pragma unroll
         for (int t = 0; t < TT; ++t) {
-            const w_f32x4 inv = *(const w_f32x4*)(&is[buf][16 * t + 4u * kq]);
+            const w_f32x4 inv = *(const w_f32x4*)(lds + L::I_AT + sbuf * L::I_BUF + (16 * t + 4u * kq) * 4u);
             if constexpr (Q6) {
 #pragma unroll
-                for (int r = 0; r < 2; ++r) {
-                    const float d = half_bits_to_float(w[r].d);
+                for (int r = 0; r < 2; ++r)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) tot[r][t][i] = fmaf(inv[i] * d, D[r][t][i], tot[r][t][i]);
-                }
+                    for (int i = 0; i < 4; ++i) tot[r][t][i] = fmaf(inv[i] * d24[r], D[r][t][i], tot[r][t][i]);
             } else {
-                const w_half8 av = *(const w_half8*)(&vs[buf][t * 512 + (lane & 31u) * 16u]);
+                const w_half8 av = *(const w_half8*)(lds + L::V_AT + sbuf * L::V_BUF + t * 512 + (lane & 31u) * 16u);
 #pragma unroll
                 for (int r = 0; r < 2; ++r) {
                     w_f32x4 V = {0, 0, 0, 0};
                     V = __builtin_amdgcn_mfma_f32_16x16x32_f16(av, __builtin_bit_cast(w_half8, bmn[r]), V, 0, 0, 0);
-                    const float d24 = half_bits_to_float(w[r].hdr.x & 0xFFFFu) * 16777216.0f;
-                    const float m24 = half_bits_to_float(w[r].hdr.x >> 16) * (16777216.0f * 32.0f);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) tot[r][t][i] += inv[i] * fmaf(d24, D[r][t][i], -(m24 * V[i]));
+                    for (int i = 0; i < 4; ++i) tot[r][t][i] += inv[i] * fmaf(d24[r], D[r][t][i], -(m24[r] * V[i]));
                 }
             }
         }
-        park_x(buf ^ 1);
-        park_small(buf ^ 1);
-        wide_barrier();
-    }
+    };
 
-    // The outputs change hands through LDS (the X buffers are free: every wave is past the loop's last barrier) and
-    // leave in rolled loops of whole rows (from the accumulators they went as 64-byte pieces).
-    constexpr uint32_t OP = 260;   // floats between tokens: the four lane groups write to different banks
-    float* ot = (float*)&xs[0][0];
-    static_assert(TT * 16 * OP * 4 <= sizeof(xs), "the output tile fits the X buffers");
+    // A step's matrix instructions with the next step's LDS reads and vector work between them
+    auto schedule = [&]() {
+        constexpr int NM = (Q6 ? 6 : 4) * TT, NV = Q6 ? 4 : Q5 ? 4 : 2;
+#pragma unroll
+        for (int i = 0; i < NM; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (i < 2 * TT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, NV, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    request_s(0, more(0) ? 1u : 0u);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < TT; ++i) request_x(h, i, h == 0 ? 256 : more(0) ? 768 : -256);
+    wide_meet<TT>();
+    read_w();
+    w[0].arrived(); w[1].arrived();
+#pragma unroll
+    for (int k = 0; k < WAS; ++k) request_w(k);
+    headers();
+    read_a(0, 0);
+    expand(0);
+
+    // The requests are spread over the steps: all of them behind the meetings, they found the memory path's queue full and
+    // the waves stood in front of it (6900 of a superblock's 19000 cycles).
+    uint32_t ring = 0;   // where the superblock's first half lies
+    for (uint32_t sb = 0; sb < n_sb; ++sb) {
+        const uint32_t ring1 = ring + 1u == 3u ? 0u : ring + 1u, ring2 = ring == 0u ? 2u : ring - 1u;
+        add_up(sb == 0u ? 0u : (sb - 1u) & 1u);   // of the superblock before
+        headers2();
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (j == 3) {
+                // every wave has read the first half; the second has arrived
+                wide_meet<TT + L::N_W>();
+                request_s((sb + 1u) & 1u, more(sb + 1u) ? 1u : 0u);
+                read_a(ring1, 4);
+                expand(4);
+            } else if (j == 7) {
+                wide_meet<TT>();
+                read_w();
+                read_a(ring2, 0);
+                w[0].arrived(); w[1].arrived();
+#pragma unroll
+                for (int k = 0; k < WAS; ++k) request_w(k);
+                headers();
+                expand(0);
+            } else {
+                read_a(j < 3 ? ring : ring1, j + 1);
+                expand(j + 1);
+                if (j < 3) {
+#pragma unroll
+                    for (int k = (j + 1) * WAS; k < (j + 2) * WAS && k < TT + L::N_W; ++k) {
+                        if (k < L::N_W) request_w(k);
+                        else request_x(ring2, k - L::N_W, 256);
+                    }
+                    if (j == 2) next_w(more(sb + 1u));
+                }
+            }
+            if (j >= 3 && j < 7) {
+#pragma unroll
+                for (int i = (j - 3) * XBS; i < (j - 2) * XBS && i < TT; ++i) request_x(ring, i, more(sb + 1u) ? 768 : -256);
+            }
+            multiply(j);
+            schedule();
+        }
+        ring = ring2;
+    }
+    add_up((n_sb - 1u) & 1u);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last requests have landed
+    __syncthreads();
+
+    // The outputs change hands through LDS and leave in rolled loops of whole rows (from the accumulators they went as
+    // 64-byte pieces).
+    float* ot = (float*)lds;
 #pragma unroll
     for (int r = 0; r < 2; ++r)
 #pragma unroll
@@ -457,22 +657,22 @@ __global__ __launch_bounds__(512, 2) void wide_kernel(const WideParams p)
     }
     if (p.act) {
         // columns: per wave 16 gate rows, then their 16 up rows
-        const uint32_t c = tid & 127u, n = blockIdx.x * 128u + c;
+        const uint32_t c = tid & 127u, n = bx * 128u + c;
         const float bg = p.bias && n < p.N ? p.bias[n] : 0.0f, bu = p.bias && n < p.N ? p.bias[p.N + n] : 0.0f;
-#pragma nounroll
+#pragma unroll 4
         for (uint32_t slot = tid >> 7; slot < count; slot += 4u) {
             const float* o = ot + slot * OP + (c >> 4) * 32u + (c & 15u);
             const float g = o[0] + bg, u = o[16] + bu;
             const float a = wide_act(p.act, g);
-            if (n < p.N) p.Y[(size_t)(rec ? rec[slot] : t0 + slot) * p.ldy + p.y_offset + n] = a * u;
+            if (n < p.N) p.Y[(size_t)out_rows[slot] * p.ldy + p.y_offset + n] = a * u;
         }
     } else {
-        const uint32_t c = tid & 255u, n = blockIdx.x * 256u + c;
+        const uint32_t c = tid & 255u, n = bx * 256u + c;
         const float bv = p.bias && n < p.N ? p.bias[n] : 0.0f;
 #pragma unroll 4
         for (uint32_t slot = tid >> 8; slot < count; slot += 2u) {
             if (n >= p.N) break;
-            const size_t at = (size_t)(rec ? rec[slot] : t0 + slot) * p.ldy + p.y_offset + n;
+            const size_t at = (size_t)out_rows[slot] * p.ldy + p.y_offset + n;
             float y = ot[slot * OP + c] + bv;
             if (p.residual) y += p.residual[at];
             p.Y[at] = y;
@@ -609,7 +809,8 @@ hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32
     p.act = a.W2 ? 2 : 0;
     p.records = records; p.n_records = n_records; p.record_words = 2u + cap; p.k_slots = a.k_slots; p.x_per_slot = a.x_per_slot;
     const uint32_t per_wg = a.W2 ? WIDE_WAVES * 16u : WIDE_WAVES * 32u;
-    return launch_wide_any(a.type, p, cap / 16u, dim3((a.N + per_wg - 1u) / per_wg, bound, 1u), s);
+    p.row_groups = (a.N + per_wg - 1u) / per_wg;
+    return launch_wide_any(a.type, p, cap / 16u, dim3((p.row_groups * bound + 7u) / 8u * 8u), s);
 }
 
 // ------------------------------------------------------------------------------------------------------------------

@@ -40,6 +40,25 @@ def test_many_tokens_vs_oracle(gpu, kqo, type_, M, N, K):  # noqa: F811
     assert float(np.abs(one[0] - got[0]).max()) <= 2e-6 * rms + 2e-6 * float(np.abs(got[0]).max())
 
 
+@pytest.mark.parametrize("type_", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("M", [17, 48, 64])
+@pytest.mark.parametrize("blocks", [1, 2, 3, 4, 5, 7])
+def test_walks_of_few_superblocks(gpu, kqo, type_, M, blocks):  # noqa: F811
+    """Every place in the ring of half superblocks as the last one, one workgroup's rows and a ragged second."""
+    from backpack_amd import capi, kquant
+    N, K = 270, 256 * blocks
+    raw, packed, w = gpu.make_weight(type_, N, K, seed=blocks)
+    X = np.random.default_rng(M).standard_normal((M, K)).astype(np.float32)
+    capi.force_kernel(8)
+    capi.set_option("gemv_splits", 1)
+    try:
+        got = kquant.matmul(gpu.dev(X), w).cpu().numpy()
+    finally:
+        capi.force_kernel(0)
+        capi.set_option("gemv_splits", 0)
+    gpu.check_matmul(kqo, type_, got, X, packed, N, K, label="walk", slack=1e-5)
+
+
 @pytest.mark.parametrize("type_,M,N,K,pro,epi,res", [(Q4_K, 48, 272, 512, 1, 2, False), (Q5_K, 17, 136, 4096, 1, 3, False),
                                                      (Q6_K, 70, 257, 1024, 2, 0, True), (Q4_K, 21, 96, 256, 3, 0, True)])
 def test_many_tokens_fused_vs_separate(gpu, type_, M, N, K, pro, epi, res):  # noqa: F811
