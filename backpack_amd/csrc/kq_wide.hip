@@ -35,10 +35,14 @@
 // use.  A workgroup's walk still takes 1.4 times its matrix instructions' time: a matrix instruction holds the issue for 8
 // cycles and a vector one for 4, so beside two vector instructions each they no longer overlap.
 //
+// A workgroup may walk several groups of 256 rows against the same tokens as one sequence of superblocks (groups_per_wg): its
+// start (records, addresses, the first loads' way: 8 us of 25 .. 40) is paid once and a group's stores go under the next
+// group's walk.
+//
 // Mixture layers (records of pairs of one expert): consecutive workgroups go to the same XCD, so a record's row groups
 // and an expert's records meet their X and W in that L2 (128 experts x 8 slots, 2048 / 768, 2048 tokens: 750 -> 703 us).
-// us with the router, now / with the walk before / on the 16-token tiles: 2048 tokens 645 / 777 / 1264, 256 tokens
-// 190 / 196 / 267, 24 tokens 125 / 125 / 153 (one box).
+// us with the router, now / with the walk before / on the 16-token tiles: 2048 tokens 592 / 734 / 1264, 256 tokens
+// 164 / 191 / 267, 24 tokens 125 / 128 / 153.
 #include "kq_format.h"
 #include "kq_kernels.h"
 #include "kq_wave.h"
@@ -173,13 +177,13 @@ struct WideParams {
     uint32_t M, N;           // rows of x; outputs
     uint32_t n_blocks, row_stride_bytes, y_offset, ldy;
     uint32_t n_splits, blocks_per_split;
-    float* partial;          // [split][token group][workgroup][token][256 columns]
+    float* partial;          // [split][token group][row group][token][256 columns]
+    uint32_t row_groups, per_wg, wgs;   // groups of 256 rows (act: 128 gate and their up rows); how many a workgroup walks; workgroups
     int act;                 // 0, or 2 / 3: Y = silu / gelu_tanh (W x) * (W2 x)
-    // grouped (records != nullptr): the workgroups walk records {expert, count, pair ids ...}, row_groups of them each; W and
-    // W2 advance by N rows per expert, a pair's X row is itself (x_per_slot) or pair / k_slots, its Y row the pair
+    // grouped (records != nullptr): `wgs` workgroups to a record {expert, count, pair ids ...}; W and W2 advance by N rows per expert, a pair's X row is itself (x_per_slot) or pair / k_slots, its Y row the pair
     const uint32_t* records;
     const uint32_t* n_records;
-    uint32_t record_words, k_slots, row_groups;
+    uint32_t record_words, k_slots;
     int x_per_slot;
 };
 
@@ -297,9 +301,7 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
 {
     using L = WideLds<TYPE, TT>;
     constexpr bool Q6 = TYPE == KQ_TYPE_Q6_K, Q5 = TYPE == KQ_TYPE_Q5_K;
-    constexpr uint32_t OP = 260;   // output tile: floats between tokens (the four lane groups write to different banks)
     __shared__ __align__(16) uint8_t lds[L::BYTES];
-    static_assert(TT * 16 * OP * 4 <= L::R_AT, "the output tile fits");
     const uint32_t tid = threadIdx.x, lane = tid & 63u, kq = lane >> 4, r16 = lane & 15u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
@@ -308,10 +310,10 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     uint32_t count, t0 = 0, bx = blockIdx.x;
     const uint8_t *W = p.W, *W2 = p.W2;
     if (p.records) {
-        const uint32_t all = *p.n_records * p.row_groups, share = (all + 7u) >> 3, at = (bx & 7u) * share + (bx >> 3);
+        const uint32_t all = *p.n_records * p.wgs, share = (all + 7u) >> 3, at = (bx & 7u) * share + (bx >> 3);
         if ((bx >> 3) >= share || at >= all) return;   // whole workgroup
-        const uint32_t record = at / p.row_groups;
-        bx = at - record * p.row_groups;
+        const uint32_t record = at / p.wgs;
+        bx = at - record * p.wgs;
         rec = p.records + (size_t)record * p.record_words;
         count = rec[1];
         const size_t skip = (size_t)rec[0] * p.N * p.row_stride_bytes;
@@ -332,50 +334,59 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     const uint32_t slot0 = min(lane, min(count, TT * 16u) - 1u);
     if (rec) lds_dma4(lds0 + L::R_AT + wave * (TT * 128u), (const uint8_t*)rec, slot0 * 4u, TT == 4 ? ~0ull : (1ull << (TT * 16u % 64u)) - 1ull);
 
-    // W: the wave's two tiles of 16 rows, unit after unit
-    const uint32_t out0 = p.act ? (bx * WIDE_WAVES + wave) * 16u : (bx * WIDE_WAVES + wave) * 32u;
-    const uint32_t row_last = p.N - 1u;
-    const uint32_t first[2] = {min(out0, row_last), min(p.act ? out0 : out0 + 16u, row_last)};
-    const uint8_t* wbase[2];
-    wbase[0] = W + (size_t)first[0] * p.row_stride_bytes + (size_t)b0 * BB;
-    wbase[1] = (p.act ? W2 : W) + (size_t)first[1] * p.row_stride_bytes + (size_t)b0 * BB;
-    uint32_t woff[2][L::W_INSTR], doff[2];
+    // W: the wave's two tiles of 16 rows, unit after unit.  The last rows of a matrix that does not fill its tiles are read from
+    // N - 16 on (what a tile has of an earlier one is not stored), so a lane's offsets are the same for every tile.
+    const uint32_t rows = min(p.N, 16u);
+    uint32_t woff[L::W_INSTR];
 #pragma unroll
-    for (int r = 0; r < 2; ++r) {
-#pragma unroll
-        for (uint32_t i = 0; i < L::W_INSTR; ++i) {
-            const uint32_t n = i * 64u + lane, row = n / L::UNITS, u = n % L::UNITS;
-            woff[r][i] = (min(first[r] + row, row_last) - first[r]) * p.row_stride_bytes + u * 16u;
-        }
-        doff[r] = (min(first[r] + r16, row_last) - first[r]) * p.row_stride_bytes + 206u;   // (d in the upper half; ends with the block)
+    for (uint32_t i = 0; i < L::W_INSTR; ++i) {
+        const uint32_t n = i * 64u + lane, row = n / L::UNITS, u = n % L::UNITS;
+        woff[i] = min(row, rows - 1u) * p.row_stride_bytes + u * 16u;
     }
+    const uint32_t doff = min(r16, rows - 1u) * p.row_stride_bytes + 206u;   // (d in the upper half; ends with the block)
+    auto tile_row = [&](uint32_t group, int r) { return (group * WIDE_WAVES + wave) * (p.act ? 16u : 32u) + (p.act ? 0u : 16u * r); };
+    const uint8_t* wbase[2];
+    auto set_w = [&](uint32_t group, uint32_t sb) {   // (no branch: the steps of the walk stay one basic block)
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+            wbase[r] = (r && p.act ? W2 : W) + (size_t)min(tile_row(group, r), p.N - rows) * p.row_stride_bytes + (size_t)((b0 + sb) * BB);
+    };
+    const uint32_t group0 = bx * p.per_wg, n_groups = min(p.per_wg, p.row_groups - group0);
+    set_w(group0, 0);
     const uint32_t w_lds = lds0 + L::W_AT + wave * L::W_WAVE;
     // piece k of a superblock's weights: whole loads first, then each tile's last lanes (and d)
     auto request_w = [&](int k) {
         constexpr int WHOLE = 2 * ((int)L::W_INSTR - 1);
         if (k < WHOLE) {
             const uint32_t r = (uint32_t)k & 1u, i = (uint32_t)k >> 1;
-            lds_dma16(w_lds + r * L::W_TILE + i * 1024u, wbase[r], woff[r][i]);
+            lds_dma16(w_lds + r * L::W_TILE + i * 1024u, wbase[r], woff[i]);
         } else if (k < WHOLE + 2) {
             const uint32_t r = (uint32_t)k & 1u;
-            lds_dma16(w_lds + r * L::W_TILE + (L::W_INSTR - 1u) * 1024u, wbase[r], woff[r][L::W_INSTR - 1u], (1ull << L::W_LAST) - 1ull);
+            lds_dma16(w_lds + r * L::W_TILE + (L::W_INSTR - 1u) * 1024u, wbase[r], woff[L::W_INSTR - 1u], (1ull << L::W_LAST) - 1ull);
         } else {
             const uint32_t r = (uint32_t)k & 1u;
-            lds_dma4(w_lds + 2u * L::W_TILE + r * 64u, wbase[r], doff[r], 0xFFFFull);
+            lds_dma4(w_lds + 2u * L::W_TILE + r * 64u, wbase[r], doff, 0xFFFFull);
         }
     };
-    auto next_w = [&](bool more) {
-#pragma unroll
-        for (int r = 0; r < 2; ++r) wbase[r] += more ? BB : 0u;
-    };
-    // Half h of the walk is superblock b0 + h / 2.  Requested ahead: X by two halves, W by one superblock (into the place it
-    // was read from), S half a superblock less; past the end the last is requested again.
+    // The walk: n_groups groups of rows against the same tokens, n_sb superblocks each, as one sequence of `all` superblocks:
+    // W and X of the next group are under way while a group's outputs leave.  Half h of it is superblock h / 2.  Requested
+    // ahead: X by two halves, W by one superblock (into the place it was read from), S half a superblock less; past the
+    // end the last is requested again.
     constexpr int WAS = (TT + L::N_W + 3) / 4, XBS = (TT + 3) / 4;   // requests per step
-    const uint32_t n_sb = b1 - b0;
-    auto more = [&](uint32_t sb) { return sb + 1u < n_sb; };   // is there a superblock behind sb?
+    const uint32_t n_sb = b1 - b0, all = n_groups * n_sb;
+    auto wrap = [&](uint32_t sb) { return sb + 1u == n_sb ? 0u : sb + 1u; };
+    uint32_t w_group = group0;   // the group whose W is requested
+    auto next_w = [&](uint32_t at, uint32_t sb) {   // from superblock `at`, number sb of its group, to the one behind it
+        const uint32_t go = at + 1u < all ? 1u : 0u, to = wrap(sb);
+        w_group += to == 0u ? go : 0u;
+        set_w(w_group, go ? to : sb);
+    };
+    // the way of X from the second half of superblock `at`, number sb of its group; of S from the superblock
+    auto x_step = [&](uint32_t at, uint32_t sb) -> int { return at + 1u >= all ? -256 : wrap(sb) ? 768 : -(int)(sb * WIDE_XA) - 256; };
+    auto s_step = [&](uint32_t at, uint32_t sb) -> int { return at + 1u >= all ? 0 : wrap(sb) ? 1 : -(int)sb; };
 #pragma unroll
     for (int k = 0; k < L::N_W; ++k) request_w(k);
-    next_w(more(0));
+    next_w(0, 0);
 
     if (rec) {
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L::N_W) : "memory");   // the record's words
@@ -402,10 +413,10 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
         lds_dma16(lds0 + ring * L::X_HALF + (wave * TT + i) * 1024u, xp[i]);
         xp[i] += step;
     };
-    auto request_s = [&](uint32_t buf, uint32_t step) {   // step: superblocks
+    auto request_s = [&](uint32_t buf, int step) {   // step: superblocks
         if constexpr (!Q6) lds_dma16(lds0 + L::V_AT + buf * L::V_BUF + (wave & 1u) * 1024u, vp, s_lanes);
         lds_dma4(lds0 + L::I_AT + buf * L::I_BUF, (const void*)ip, i_lanes);
-        vp += step * WIDE_XV;
+        vp += step * (int)WIDE_XV;
         ip += step;
     };
 
@@ -576,11 +587,11 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    request_s(0, more(0) ? 1u : 0u);
+    request_s(0, s_step(0, 0));
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < TT; ++i) request_x(h, i, h == 0 ? 256 : more(0) ? 768 : -256);
+        for (int i = 0; i < TT; ++i) request_x(h, i, h == 0 ? 256 : x_step(0, 0));
     wide_meet<TT>();
     read_w();
     w[0].arrived(); w[1].arrived();
@@ -590,19 +601,62 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     read_a(0, 0);
     expand(0);
 
+    // The group's outputs, from the accumulators: 64 bytes of a token's row per tile (128 for both; an activation's in one).
+    auto store = [&](uint32_t group) {
+        uint32_t n[2];
+        bool mine[2];
+        float bias[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const uint32_t from = tile_row(group, r);
+            n[r] = min(min(from, p.N - rows) + r16, p.N - 1u);
+            mine[r] = n[r] >= from && r16 < rows;
+            bias[r] = p.bias ? p.bias[n[r] + (p.act && r ? p.N : 0u)] : 0.0f;
+        }
+#pragma unroll
+        for (int t = 0; t < TT; ++t) {
+            __builtin_amdgcn_sched_barrier(0);   // (a tile's addresses at a time: registers)
+            const w_u32x4 row = *(const w_u32x4*)(out_rows + 16 * t + 4u * kq);
+            if (p.act) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float y = wide_act(p.act, tot[0][t][i] + bias[0]) * (tot[1][t][i] + bias[1]);
+                    if (16u * t + 4u * kq + i < count && mine[0]) p.Y[(size_t)row[i] * p.ldy + p.y_offset + n[0]] = y;
+                }
+            } else {
+                float y[2][4];
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        y[r][i] = tot[r][t][i] + bias[r];
+                        // (slots beyond the count, rows beyond the last: a value that is not stored)
+                        if (p.residual) y[r][i] += p.residual[(size_t)row[i] * p.ldy + p.y_offset + n[r]];
+                    }
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (16u * t + 4u * kq + i < count && mine[r]) p.Y[(size_t)row[i] * p.ldy + p.y_offset + n[r]] = y[r][i];
+            }
+        }
+    };
+
     // The requests are spread over the steps: all of them behind the meetings, they found the memory path's queue full and
     // the waves stood in front of it (6900 of a superblock's 19000 cycles).
     uint32_t ring = 0;   // where the superblock's first half lies
-    for (uint32_t sb = 0; sb < n_sb; ++sb) {
+    uint32_t sb = 0, group = group0;
+    for (uint32_t at = 0; at < all; ++at) {
         const uint32_t ring1 = ring + 1u == 3u ? 0u : ring + 1u, ring2 = ring == 0u ? 2u : ring - 1u;
-        add_up(sb == 0u ? 0u : (sb - 1u) & 1u);   // of the superblock before
+        const uint32_t sb1 = wrap(sb);   // number of the superblock behind this one in its group
+        add_up(at == 0u ? 0u : (at - 1u) & 1u);   // of the superblock before (a group's last is done: nothing)
         headers2();
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             if (j == 3) {
                 // every wave has read the first half; the second has arrived
                 wide_meet<TT + L::N_W>();
-                request_s((sb + 1u) & 1u, more(sb + 1u) ? 1u : 0u);
+                request_s((at + 1u) & 1u, s_step(at + 1u, sb1));
                 read_a(ring1, 4);
                 expand(4);
             } else if (j == 7) {
@@ -623,61 +677,55 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
                         if (k < L::N_W) request_w(k);
                         else request_x(ring2, k - L::N_W, 256);
                     }
-                    if (j == 2) next_w(more(sb + 1u));
                 }
             }
             if (j >= 3 && j < 7) {
 #pragma unroll
-                for (int i = (j - 3) * XBS; i < (j - 2) * XBS && i < TT; ++i) request_x(ring, i, more(sb + 1u) ? 768 : -256);
+                for (int i = (j - 3) * XBS; i < (j - 2) * XBS && i < TT; ++i) request_x(ring, i, x_step(at + 1u, sb1));
             }
             multiply(j);
-            schedule();
+            if (j == 0) __builtin_amdgcn_sched_barrier(0);   // (with the scaling of the superblock before: the compiler's own order)
+            else schedule();
+            if (j == 2) next_w(at + 1u, sb1);
         }
+        if (sb1 == 0u && p.n_splits == 1u) {   // the group's last
+            __builtin_amdgcn_sched_barrier(0);
+            add_up(at & 1u);
+            store(group++);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                d24[r] = m24[r] = 0.0f;
+                bmn[r] = w_u32x4{0, 0, 0, 0};
+#pragma unroll
+                for (int t = 0; t < TT; ++t) D[r][t] = tot[r][t] = w_f32x4{0, 0, 0, 0};
+            }
+        }
+        sb = sb1;
         ring = ring2;
     }
-    add_up((n_sb - 1u) & 1u);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // the last requests have landed
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in LDS that is no longer this workgroup's
+    if (p.n_splits == 1u) return;
+    // A share of K (dense calls, one group): wide_sum_kernel adds the shares' tiles.  They change hands through LDS and leave in
+    // whole rows (from the accumulators, in 64-byte pieces, a 28672 x 4096 call of 48 tokens took 1.5 us more).
+    add_up((all - 1u) & 1u);
     __syncthreads();
-
-    // The outputs change hands through LDS and leave in rolled loops of whole rows (from the accumulators they went as
-    // 64-byte pieces).
+    constexpr uint32_t OP = 260;   // floats between tokens: the four lane groups write to different banks
+    static_assert(TT * 16 * OP * 4 <= L::R_AT, "the output tile fits");
     float* ot = (float*)lds;
 #pragma unroll
-    for (int r = 0; r < 2; ++r)
+    for (int r = 0; r < 2; ++r) {
+        const uint32_t from = tile_row(group0, r), col = wave * 32u + 16u * r + min(from, p.N - rows) + r16 - from;
 #pragma unroll
         for (int t = 0; t < TT; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) ot[(16 * t + 4u * kq + i) * OP + wave * 32u + 16u * r + r16] = tot[r][t][i];
+            for (int i = 0; i < 4; ++i)
+                if (col >= wave * 32u + 16u * r && col < wave * 32u + 16u * r + 16u) ot[(16u * t + 4u * kq + i) * OP + col] = tot[r][t][i];
+    }
     __syncthreads();
-    if (p.n_splits > 1) {   // (dense calls only) wide_sum_kernel adds the splits' tiles
-        float* tile = p.partial + (((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (TT * 16u * 256u);
-        for (uint32_t n = tid; n < TT * 1024u; n += 512u)
-            *(float4*)(tile + 4u * n) = *(const float4*)(ot + (n >> 6) * OP + 4u * (n & 63u));
-        return;
-    }
-    if (p.act) {
-        // columns: per wave 16 gate rows, then their 16 up rows
-        const uint32_t c = tid & 127u, n = bx * 128u + c;
-        const float bg = p.bias && n < p.N ? p.bias[n] : 0.0f, bu = p.bias && n < p.N ? p.bias[p.N + n] : 0.0f;
-#pragma unroll 4
-        for (uint32_t slot = tid >> 7; slot < count; slot += 4u) {
-            const float* o = ot + slot * OP + (c >> 4) * 32u + (c & 15u);
-            const float g = o[0] + bg, u = o[16] + bu;
-            const float a = wide_act(p.act, g);
-            if (n < p.N) p.Y[(size_t)out_rows[slot] * p.ldy + p.y_offset + n] = a * u;
-        }
-    } else {
-        const uint32_t c = tid & 255u, n = bx * 256u + c;
-        const float bv = p.bias && n < p.N ? p.bias[n] : 0.0f;
-#pragma unroll 4
-        for (uint32_t slot = tid >> 8; slot < count; slot += 2u) {
-            if (n >= p.N) break;
-            const size_t at = (size_t)out_rows[slot] * p.ldy + p.y_offset + n;
-            float y = ot[slot * OP + c] + bv;
-            if (p.residual) y += p.residual[at];
-            p.Y[at] = y;
-        }
-    }
+    float* tile = p.partial + (((size_t)blockIdx.z * gridDim.y + blockIdx.y) * p.row_groups + group0) * (TT * 16u * 256u);
+    for (uint32_t n = tid; n < TT * 1024u; n += 512u)
+        *(float4*)(tile + 4u * n) = *(const float4*)(ot + (n >> 6) * OP + 4u * (n & 63u));
 }
 
 // Adds the splits' partial tiles in split order, with the call's epilogue.  Workgroup (x, y): 256 columns of four
@@ -749,6 +797,27 @@ bool wide_supported(const MatmulArgs& a)
     return !(((uintptr_t)a.W | (uintptr_t)a.W2) & 15u) && !(a.row_stride_bytes & 15u);
 }
 
+// Groups of rows that a workgroup walks one after the other: what leaves the fewest us over the CUs, at `step` us per
+// superblock and `start` beside a workgroup's walks.  At 16 tokens two workgroups share a CU (a step of one takes half the
+// two's, and its start goes under the other's walk); alone on it a workgroup is little faster than as one of two.
+// Measured, us, with one group / with those chosen: 128 experts x 8, 2048 / 768, gate and up, then down: 256 tokens (3, 4) 77 / 73
+// and 80 / 68, 2048 tokens (2, 2) 295 / 285 and 255 / 233, 24 tokens (1, 2) 52 / 52 (two groups 61, three 56) and 51.5 / 49.
+static uint32_t groups_per_wg(uint32_t row_groups, double others, int type, uint32_t tt, uint32_t blocks)
+{
+    const bool q6 = type == KQ_TYPE_Q6_K, two = tt == 1u;
+    const double cus = (double)device_cu_count();
+    const double step = two ? (q6 ? 3.0 : type == KQ_TYPE_Q5_K ? 2.1 : 1.75) : q6 ? 2.4 + 0.9 * tt : 0.8 + 0.8 * tt;
+    uint32_t best = 1;
+    double best_us = 1e30;
+    for (uint32_t c = 1; c <= row_groups && c <= 64u; ++c) {
+        const double per_cu = (double)((row_groups + c - 1u) / c) * others / cus;
+        const bool shared = two && per_cu > 1.0;
+        const double us = std::fmax(1.0, std::ceil(per_cu - 0.05)) * (c * (blocks * step) * (two && !shared ? 1.15 : 1.0) + (shared ? 4.0 : 9.0));
+        if (us < best_us) { best_us = us; best = c; }
+    }
+    return best;
+}
+
 hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scratch, size_t x_bytes, int splits, hipStream_t s)
 {
     const uint32_t outs = a.epi ? a.N / 2u : a.N;
@@ -788,7 +857,10 @@ hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scra
         p.blocks_per_split = (a.n_blocks + z - 1u) / z;
         p.n_splits = (a.n_blocks + p.blocks_per_split - 1u) / p.blocks_per_split;
         p.partial = sc.partial;
-        if (hipError_t e = launch_wide_any(a.type, p, tt, dim3(gx, gy2, p.n_splits), s); e != hipSuccess) return e;
+        p.row_groups = gx;
+        p.per_wg = p.n_splits > 1u ? 1u : groups_per_wg(gx, (double)gy2, a.type, tt, a.n_blocks);
+        p.wgs = (gx + p.per_wg - 1u) / p.per_wg;
+        if (hipError_t e = launch_wide_any(a.type, p, tt, dim3(p.wgs, gy2, p.n_splits), s); e != hipSuccess) return e;
         if (p.n_splits > 1u) {
             hipLaunchKernelGGL(wide_sum_kernel, dim3(gx, (M + 3u) / 4u), dim3(256), 0, s, p, tt * 16u, gy2);
             if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
@@ -798,7 +870,7 @@ hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scra
 }
 
 hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32_t* records, const uint32_t* n_records,
-                               uint32_t bound, uint32_t cap, hipStream_t s)
+                               uint32_t bound, uint32_t cap, double records_expected, hipStream_t s)
 {
     WideParams p{};
     p.x = x;
@@ -810,7 +882,10 @@ hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32
     p.records = records; p.n_records = n_records; p.record_words = 2u + cap; p.k_slots = a.k_slots; p.x_per_slot = a.x_per_slot;
     const uint32_t per_wg = a.W2 ? WIDE_WAVES * 16u : WIDE_WAVES * 32u;
     p.row_groups = (a.N + per_wg - 1u) / per_wg;
-    return launch_wide_any(a.type, p, cap / 16u, dim3((p.row_groups * bound + 7u) / 8u * 8u), s);
+    const uint32_t tt = cap / 16u;
+    p.per_wg = groups_per_wg(p.row_groups, records_expected, a.type, tt, a.n_blocks);
+    p.wgs = (p.row_groups + p.per_wg - 1u) / p.per_wg;
+    return launch_wide_any(a.type, p, tt, dim3((p.wgs * bound + 7u) / 8u * 8u), s);
 }
 
 // ------------------------------------------------------------------------------------------------------------------

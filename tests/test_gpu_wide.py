@@ -59,6 +59,63 @@ def test_walks_of_few_superblocks(gpu, kqo, type_, M, blocks):  # noqa: F811
     gpu.check_matmul(kqo, type_, got, X, packed, N, K, label="walk", slack=1e-5)
 
 
+@pytest.mark.parametrize("type_", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("M,blocks", [(17, 1), (48, 2), (64, 3)])
+def test_several_row_groups_per_workgroup(gpu, kqo, type_, M, blocks):  # noqa: F811
+    """More groups of 256 rows than CUs: a workgroup walks two, the last of them ragged.  Windows of rows at both
+    ends and in the middle, with a bias and, in place, a residual."""
+    from backpack_amd import capi, kquant, synth
+    N, K = 256 * 299 + 7, 256 * blocks
+    print("groups", type_, M, N, K, flush=True)
+    raw, packed, w = gpu.make_weight(type_, N, K, seed=blocks)
+    rng = np.random.default_rng(M)
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    bias, res = rng.standard_normal(N).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    got = kquant.matmul(gpu.dev(X), w, bias=gpu.dev(bias)).cpu().numpy()
+    assert capi.last_form() == "many_token"
+    y = gpu.dev(res)
+    kquant.matmul_fused(gpu.dev(X), w, residual=y, out=y)
+    y = y.cpu().numpy()
+    words = synth.row_stride_words(type_, K)
+    for a, b in ((0, 300), (256 * 149 - 20, 256 * 150 + 20), (N - 530, N)):
+        rows = packed[a * words:b * words]
+        gpu.check_matmul(kqo, type_, np.ascontiguousarray(got[:, a:b]), X, rows, b - a, K, bias=bias[a:b], label="groups", slack=1e-5)
+        # the residual is added to the same product, one rounding each
+        plain = got[:, a:b].astype(np.float64) - bias[a:b]
+        tol = 4e-7 * (np.abs(got[:, a:b]) + np.abs(bias[a:b]) + np.abs(res[:, a:b]) + np.abs(plain))
+        assert np.all(np.abs(y[:, a:b] - (plain + res[:, a:b])) <= tol)
+
+
+@pytest.mark.parametrize("tgu,tdn", [(Q4_K, Q6_K), (Q5_K, Q4_K), (Q6_K, Q5_K)])
+@pytest.mark.parametrize("T,H,I", [(80, 256, 1792), (80, 3328, 256), (320, 512, 2304), (320, 3328, 512)])
+def test_moe_several_row_groups_per_workgroup(gpu, kqo, tgu, tdn, T, H, I):  # noqa: F811
+    """64 experts of 5 or 20 pairs and 13 to 18 groups of rows: a workgroup walks several of a record's, the last one
+    fewer.  A few tokens against the oracle, all against the 16-token tile kernel."""
+    from backpack_amd import capi, kquant
+    print("moe groups", tgu, tdn, T, H, I, flush=True)
+    E, k = 64, 4
+    _, gp, gw = gpu.make_weight(tgu, E * I, H, seed=31)
+    _, up, uw = gpu.make_weight(tgu, E * I, H, seed=32)
+    _, dp, dw = gpu.make_weight(tdn, E * H, I, seed=33)
+    rng = np.random.default_rng(T + H)
+    eidx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32)
+    ew = rng.random((T, k)).astype(np.float32)
+    X = (rng.standard_normal((T, H)) * 0.1).astype(np.float32)
+    args = (gpu.dev(X), gw, uw, dw, gpu.dev(eidx.view(np.int32)), gpu.dev(ew), E)
+    capi.force_kernel(8)
+    try:
+        got = kquant.moe_ffn(*args).cpu().numpy()
+        capi.force_kernel(6)
+        tile = kquant.moe_ffn(*args).cpu().numpy()
+    finally:
+        capi.force_kernel(0)
+    sel = rng.choice(T, 4, replace=False)
+    want = kqo.moe_ffn(tgu, tdn, X[sel], gp, up, dp, eidx[sel], ew[sel], H, I)
+    rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    assert np.all(np.abs(got[sel] - want) <= 1e-3 * rms + 1e-3 * np.abs(want))
+    assert np.abs(got - tile).max() <= 1e-4 * rms + 1e-4 * np.abs(tile).max()
+
+
 @pytest.mark.parametrize("type_,M,N,K,pro,epi,res", [(Q4_K, 48, 272, 512, 1, 2, False), (Q5_K, 17, 136, 4096, 1, 3, False),
                                                      (Q6_K, 70, 257, 1024, 2, 0, True), (Q4_K, 21, 96, 256, 3, 0, True)])
 def test_many_tokens_fused_vs_separate(gpu, type_, M, N, K, pro, epi, res):  # noqa: F811
