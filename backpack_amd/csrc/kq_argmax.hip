@@ -35,25 +35,42 @@ __global__ __launch_bounds__(256) void argmax_rows_kernel(const float* logits, u
     __shared__ bool last;
     const uint32_t row = blockIdx.y, parts = gridDim.x;
     const float* x = logits + (size_t)row * ld;
-    const uint32_t chunk = (N + parts - 1u) / parts;
-    const uint32_t begin = blockIdx.x * chunk, end = min(begin + chunk, N);
+    const uint32_t chunk = ((N + parts - 1u) / parts + 3u) & ~3u;
+    const uint32_t begin = min(blockIdx.x * chunk, N), end = min(begin + chunk, N);
     float v = -1e30f;
     uint32_t i = 0xFFFFFFFFu;   // "none yet": any real index is lower
-    for (uint32_t k = begin + threadIdx.x; k < end; k += 256u) {
-        const float t = x[k];
-        if (t > v) { v = t; i = k; }   // ascending k per lane: the first of equals stays
+    // four logits per lane and load (a row may start at any float), four loads in flight
+    const uint32_t whole = begin + ((end - begin) & ~3u);
+    for (uint32_t k0 = begin + 4u * threadIdx.x; k0 < whole; k0 += 4096u) {
+        float t[4][4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) __builtin_memcpy(t[u], x + min(k0 + 1024u * u, whole - 4u), 16);
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u)
+#pragma unroll
+            for (uint32_t e = 0; e < 4u; ++e)
+                // ascending k per lane: the first of equals stays (a piece past the end is the last one again, seen by the lane
+                // that owns it or lost to it: equal values, and best_of takes the lower index)
+                if (t[u][e] > v) { v = t[u][e]; i = min(k0 + 1024u * u, whole - 4u) + e; }
+    }
+    if (threadIdx.x < end - whole) {
+        const float t = x[whole + threadIdx.x];
+        if (t > v) { v = t; i = whole + threadIdx.x; }
     }
     argmax_block(v, i, sv, si);
     if (threadIdx.x == 0) {
         const size_t cell = (size_t)row * parts + blockIdx.x;
         __hip_atomic_store(&part_val[cell], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(&part_idx[cell], i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // release: the partial is visible to whoever sees the ticket; acquire: the last one sees them all
-        const uint32_t t = __hip_atomic_fetch_add(&tickets[row], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+        // Write-through stores acknowledged before the ticket, agent-scope loads by the last to arrive.  (An acquire / release
+        // ticket wrote back and invalidated the XCD's L2 once per workgroup: 48 rows of 128256 logits 39 us.)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const uint32_t t = __hip_atomic_fetch_add(&tickets[row], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         last = t == parts - 1u;
     }
     __syncthreads();
     if (!last) return;
+    asm volatile("" ::: "memory");
     v = -1e30f;
     i = 0xFFFFFFFFu;
     for (uint32_t q = threadIdx.x; q < parts; q += 256u) {

@@ -111,3 +111,21 @@ def test_lm_head_pick_inside_the_matvec_launch(gpu, kqo):
         capi.force_kernel(0)
     assert np.array_equal(i2.cpu().numpy(), kqo.argmax_rows(l2.cpu().numpy()))
     assert np.array_equal(v2.cpu().numpy(), l2.cpu().numpy().max(axis=1))
+
+
+@pytest.mark.parametrize("M,N,ld", [(48, 8197, 8197), (5, 4099, 4101), (3, 7, 9), (2, 3, 3), (9, 128255, 128259), (64, 4096, 4097)])
+def test_argmax_pieces_of_four(gpu, kqo, M, N, ld):
+    """Rows that start at any float and lengths that leave one to three logits over; the largest value at every place of the
+    first and last pieces, and NaNs beside it."""
+    import torch
+    from backpack_amd import kquant
+    rng = np.random.default_rng(N)
+    buf = rng.standard_normal((M, ld)).astype(np.float32)
+    for m in range(M):
+        buf[m, (m if m % 2 else N - 1 - m) % N] = 9.0
+        if N > 8 and not buf[m, (m + 5) % N] == 9.0:
+            buf[m, (m + 5) % N] = np.nan
+        buf[m, N:] = 100.0   # not of the row
+    got, val = kquant.argmax_rows(torch.from_numpy(buf).cuda()[:, :N])
+    assert np.array_equal(got.cpu().numpy(), kqo.argmax_rows(np.ascontiguousarray(buf[:, :N])))
+    assert np.array_equal(val.cpu().numpy(), np.nanmax(buf[:, :N], axis=1))
