@@ -37,6 +37,48 @@ __global__ __launch_bounds__(256) void rms_norm_rows_kernel(const float* X, cons
     for (uint32_t k = threadIdx.x; k < K; k += 256u) put_out(out, o + k, x[k] * rstd * w[k]);
 }
 
+// Rows in pieces of four (K a multiple of four, pointers on 16 bytes: what every k-quant row has; the scalar forms above and
+// below serve the rest).  One pass over memory: a lane's pieces of X and w stay in registers across the row's sum.
+__device__ __forceinline__ void put_four(float* out, size_t at, float4 v) { *(float4*)(out + at) = v; }
+__device__ __forceinline__ void put_four(uint16_t* out, size_t at, float4 v)
+{
+    typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+    *(bf16x4*)(out + at) = bf16x4{(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
+}
+
+// Up to 8192 elements, 512 lanes.  2048 rows of 4096 17 -> 10 us, 100 rows 10 -> 6 (bf16 out; one dependent pass less, and 16
+// bytes a load).
+template <typename OUT>
+__global__ __launch_bounds__(512) void rms_norm_rows4_kernel(const float* X, const float* w, float eps, uint32_t K, OUT* out)
+{
+    __shared__ float part[8];
+    const uint32_t k4 = K / 4u;
+    const float4* x = (const float4*)(X + (size_t)blockIdx.x * K);
+    float4 v[4], g[4];
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) {
+        const uint32_t k = threadIdx.x + 512u * i;
+        v[i] = k < k4 ? x[k] : float4{0, 0, 0, 0};
+        g[i] = k < k4 ? ((const float4*)w)[k] : float4{0, 0, 0, 0};
+    }
+    float ss = 0.0f;
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) {
+        ss = fmaf(v[i].x, v[i].x, ss); ss = fmaf(v[i].y, v[i].y, ss); ss = fmaf(v[i].z, v[i].z, ss); ss = fmaf(v[i].w, v[i].w, ss);
+    }
+    ss = wave_total(ss);
+    if ((threadIdx.x & 63u) == 0) part[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    ss = ((part[0] + part[1]) + (part[2] + part[3])) + ((part[4] + part[5]) + (part[6] + part[7]));
+    const float rstd = 1.0f / sqrtf(ss / (float)K + eps);
+    const size_t o = (size_t)blockIdx.x * K;
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) {
+        const uint32_t k = threadIdx.x + 512u * i;
+        if (k < k4) put_four(out, o + 4u * k, float4{v[i].x * rstd * g[i].x, v[i].y * rstd * g[i].y, v[i].z * rstd * g[i].z, v[i].w * rstd * g[i].w});
+    }
+}
+
 // out[m, k] = X[m, k] converted (blockIdx.y = row)
 __global__ __launch_bounds__(256) void cast_rows_bf16_kernel(const float* X, uint32_t K, uint16_t* out)
 {
@@ -46,6 +88,44 @@ __global__ __launch_bounds__(256) void cast_rows_bf16_kernel(const float* X, uin
     put_out(out, at, X[at]);
 }
 
+__global__ __launch_bounds__(256) void cast_rows4_bf16_kernel(const float* X, uint32_t n4, uint16_t* out)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i < n4) put_four(out, 4u * (size_t)i, ((const float4*)X)[i]);
+}
+
+template <bool GELU>
+__device__ __forceinline__ float act_of(float gv)
+{
+    if (GELU) {
+        const float inner = 0.7978845608f * (gv + 0.044715f * gv * gv * gv);
+        return 0.5f * gv * (1.0f + tanhf(inner));
+    }
+    return gv / (expf(-gv) + 1.0f);
+}
+
+// GU rows are gate | up (2K floats); out rows are K floats.  Two pieces of four per lane, all four loads in flight: 2048 rows of
+// 14336 (294 MB) 75 -> 55 us.
+template <bool GELU, typename OUT>
+__global__ __launch_bounds__(256) void act_mul_rows4_kernel(const float* GU, uint32_t K, OUT* out)
+{
+    const float* row = GU + (size_t)blockIdx.y * 2u * K;
+    float4 g[2], u[2];
+    uint32_t k[2];
+#pragma unroll
+    for (uint32_t i = 0; i < 2u; ++i) {
+        k[i] = 4u * (blockIdx.x * 512u + i * 256u + threadIdx.x);
+        const uint32_t at = min(k[i], K - 4u);
+        g[i] = *(const float4*)(row + at);
+        u[i] = *(const float4*)(row + K + at);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 2u; ++i)
+        if (k[i] < K)
+            put_four(out, (size_t)blockIdx.y * K + k[i], float4{act_of<GELU>(g[i].x) * u[i].x, act_of<GELU>(g[i].y) * u[i].y,
+                                                               act_of<GELU>(g[i].z) * u[i].z, act_of<GELU>(g[i].w) * u[i].w});
+}
+
 // GU rows are gate | up (2K floats); out rows are K floats.
 template <bool GELU, typename OUT>
 __global__ __launch_bounds__(256) void act_mul_rows_kernel(const float* GU, uint32_t K, OUT* out)
@@ -53,15 +133,7 @@ __global__ __launch_bounds__(256) void act_mul_rows_kernel(const float* GU, uint
     const float* g = GU + (size_t)blockIdx.y * 2u * K;
     const uint32_t k = blockIdx.x * 256u + threadIdx.x;
     if (k >= K) return;
-    const float gv = g[k], uv = g[K + k];
-    float a;
-    if (GELU) {
-        const float inner = 0.7978845608f * (gv + 0.044715f * gv * gv * gv);
-        a = 0.5f * gv * (1.0f + tanhf(inner));
-    } else {
-        a = gv / (expf(-gv) + 1.0f);
-    }
-    put_out(out, (size_t)blockIdx.y * K + k, a * uv);
+    put_out(out, (size_t)blockIdx.y * K + k, act_of<GELU>(g[k]) * g[K + k]);
 }
 
 // Y[m, y_offset + n] = T[m, n] + R[m, y_offset + n]   (R may be Y)
@@ -78,7 +150,13 @@ template <typename OUT>
 static hipError_t launch_prologue_rows_as(int pro, const float* X, const float* norm_w, float eps, uint32_t M, uint32_t K,
                                           OUT* out, hipStream_t s)
 {
-    if (pro == 1) hipLaunchKernelGGL(rms_norm_rows_kernel<OUT>, dim3(M), dim3(256), 0, s, X, norm_w, eps, K, out);
+    const bool fours = K >= 4u && K % 4u == 0 && !(((uintptr_t)X | (uintptr_t)out | (pro == 1 ? (uintptr_t)norm_w : 0u)) & 15u);
+    if (fours && pro != 1) {
+        const dim3 grid((K / 4u + 511u) / 512u, M);
+        if (pro == 2) hipLaunchKernelGGL((act_mul_rows4_kernel<false, OUT>), grid, dim3(256), 0, s, X, K, out);
+        else hipLaunchKernelGGL((act_mul_rows4_kernel<true, OUT>), grid, dim3(256), 0, s, X, K, out);
+    } else if (fours && K <= 8192u) hipLaunchKernelGGL(rms_norm_rows4_kernel<OUT>, dim3(M), dim3(512), 0, s, X, norm_w, eps, K, out);
+    else if (pro == 1) hipLaunchKernelGGL(rms_norm_rows_kernel<OUT>, dim3(M), dim3(256), 0, s, X, norm_w, eps, K, out);
     else if (pro == 2) hipLaunchKernelGGL((act_mul_rows_kernel<false, OUT>), dim3((K + 255u) / 256u, M), dim3(256), 0, s, X, K, out);
     else hipLaunchKernelGGL((act_mul_rows_kernel<true, OUT>), dim3((K + 255u) / 256u, M), dim3(256), 0, s, X, K, out);
     return hipGetLastError();
@@ -95,6 +173,11 @@ hipError_t launch_prologue_rows_bf16(int pro, const float* X, const float* norm_
                                      uint16_t* out, hipStream_t s)
 {
     if (pro != 0) return launch_prologue_rows_as(pro, X, norm_w, eps, M, K, out, s);
+    const uint64_t n = (uint64_t)M * K;
+    if (n % 4u == 0 && n / 4u < 0xFFFFFF00ull && !(((uintptr_t)X | (uintptr_t)out) & 15u)) {
+        hipLaunchKernelGGL(cast_rows4_bf16_kernel, dim3((uint32_t)((n / 4u + 255u) / 256u)), dim3(256), 0, s, X, (uint32_t)(n / 4u), out);
+        return hipGetLastError();
+    }
     hipLaunchKernelGGL(cast_rows_bf16_kernel, dim3((K + 255u) / 256u, M), dim3(256), 0, s, X, K, out);
     return hipGetLastError();
 }

@@ -318,3 +318,27 @@ def test_prefill_rows_bf16_feeds_the_gemm_and_checks_arguments(gpu, kqo):
     assert L.bpk_prefill_rows_bf16(NONE, None, None, 0.0, M, K, xb.data_ptr(), None) == -3
     assert L.bpk_prefill_rows_bf16(NONE, x.data_ptr(), None, 0.0, M, 0, xb.data_ptr(), None) == -2
     assert L.bpk_prefill_rows_bf16(NONE, x.data_ptr(), None, 0.0, 0, K, xb.data_ptr(), None) == 0
+
+
+@pytest.mark.parametrize("M,K", [(3, 256), (2, 8192), (2, 8448), (5, 2816), (1, 512)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_prefill_rows_in_pieces_of_four(gpu, M, K, offset):
+    """Rows on a 16-byte boundary (pieces of four; up to 8192 elements under a norm) and one float past it (the scalar
+    forms): the same function.  bf16 keeps 8 bits (steps of 2^(e - 7) from 2^e on): rounding moves a value by at most 2^(e - 8),
+    2^-8 of itself, plus fp32 noise."""
+    import torch
+    from backpack_amd import capi, kquant
+    rng = np.random.default_rng(M * K + offset)
+    for pro, n in ((capi.PRO_NONE, K), (capi.PRO_RMS_NORM, K), (capi.PRO_SILU_MUL, 2 * K), (capi.PRO_GELU_MUL, 2 * K)):
+        buf = gpu.dev(rng.standard_normal(M * n + 4).astype(np.float32))
+        x = buf[offset:offset + M * n].view(M, n)
+        nw = gpu.dev((1 + 0.1 * rng.standard_normal(K)).astype(np.float32))
+        got = kquant.prefill_rows_bf16(x, K, prologue=pro, norm_w=nw if pro == capi.PRO_RMS_NORM else None, eps=1e-5).double()
+        v = x.double()
+        if pro == capi.PRO_RMS_NORM:
+            v = v * torch.rsqrt((v * v).mean(1, keepdim=True) + 1e-5) * nw.double()
+        elif pro != capi.PRO_NONE:
+            g, u = v[:, :K], v[:, K:]
+            v = u * (torch.nn.functional.silu(g) if pro == capi.PRO_SILU_MUL else torch.nn.functional.gelu(g, approximate="tanh"))
+        outside = int(((got - v).abs() > (2.0 ** -8 + 1e-5) * v.abs() + 1e-6).sum())
+        assert outside == 0, (pro, offset)
