@@ -219,6 +219,81 @@ __global__ __launch_bounds__(256) void route_logits_tiled_kernel(const float* X,
     }
 }
 
+// Many tokens: 16 tokens x 64 experts per workgroup on the fp32 matrix instructions, the four waves a quarter of hidden each.
+// A wave's 32 elements of its 80 rows go through LDS of its own (whole 128-byte lines in, operands out; no meeting in the
+// loop) while the next 32 are under way.  k of a matrix instruction: element i of the four lane groups' pieces of four.
+// Every 64 elements four sums of 16 are added to the wave's total, then the waves' totals in wave order, so that no chain of
+// roundings is longer than the tiled kernel's (largest error of a weight, 2048 x 128 x 2048: 2.0e-7 both).
+// Bound by the matrix instructions (32 cycles per 2048 flops; nothing faster keeps 32 bits): 2048 tokens x 128 experts x 2048
+// 47 -> 18 us against the tiled kernel above, which fetches every row of X once per four experts.
+typedef float r_f32x4 __attribute__((ext_vector_type(4)));
+__global__ __launch_bounds__(256) void route_logits_mfma_kernel(const float* X, const float* router_w, uint32_t T, uint32_t hidden,
+                                                                uint32_t n_experts, float* logits_out)
+{
+    constexpr uint32_t PITCH = 36;   // floats between rows: nine 16-byte units, so rows start in different banks
+    __shared__ __align__(16) float st[4][2][80 * PITCH];
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t t0 = blockIdx.y * 16u, e0 = blockIdx.x * 64u, share = hidden / 4u, k0 = wave * share;
+    const uint32_t r8 = lane >> 3, c4 = 4u * (lane & 7u), g = lane >> 4, r16 = lane & 15u;
+    const float* src[10];
+#pragma unroll
+    for (uint32_t i = 0; i < 10u; ++i)
+        src[i] = (i < 2u ? X + (size_t)min(t0 + 8u * i + r8, T - 1u) * hidden
+                         : router_w + (size_t)min(e0 + 8u * (i - 2u) + r8, n_experts - 1u) * hidden) + k0 + c4;
+    r_f32x4 reg[10], tot[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) tot[n] = r_f32x4{0, 0, 0, 0};
+#pragma unroll
+    for (uint32_t i = 0; i < 10u; ++i) reg[i] = *(const r_f32x4*)src[i];
+    for (uint32_t k = 0; k < share; k += 64u) {
+        r_f32x4 acc[2][2][4];
+#pragma unroll
+        for (int a = 0; a < 16; ++a) acc[a >> 3][(a >> 2) & 1][a & 3] = r_f32x4{0, 0, 0, 0};
+#pragma unroll
+        for (uint32_t half = 0; half < 2u; ++half) {
+            if (k + 32u * half >= share) break;   // (uniform)
+            float* buf = st[wave][half];
+#pragma unroll
+            for (uint32_t i = 0; i < 10u; ++i) *(r_f32x4*)(buf + (8u * i + r8) * PITCH + c4) = reg[i];
+            const uint32_t kn = min(k + 32u * half + 32u, share - 32u);   // (the last pieces are requested again)
+#pragma unroll
+            for (uint32_t i = 0; i < 10u; ++i) reg[i] = *(const r_f32x4*)(src[i] + kn);
+            __builtin_amdgcn_wave_barrier();
+            r_f32x4 a[2], b[2][4];
+#pragma unroll
+            for (uint32_t h = 0; h < 2u; ++h) {
+                a[h] = *(const r_f32x4*)(buf + r16 * PITCH + 16u * h + 4u * g);
+#pragma unroll
+                for (uint32_t n = 0; n < 4u; ++n) b[h][n] = *(const r_f32x4*)(buf + (16u + 16u * n + r16) * PITCH + 16u * h + 4u * g);
+            }
+#pragma unroll
+            for (uint32_t h = 0; h < 2u; ++h)
+#pragma unroll
+                for (uint32_t i = 0; i < 4u; ++i)
+#pragma unroll
+                    for (uint32_t n = 0; n < 4u; ++n)
+                        acc[half][h][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[h][i], b[h][n][i], acc[half][h][n], 0, 0, 0);
+            __builtin_amdgcn_wave_barrier();
+        }
+#pragma unroll
+        for (int n = 0; n < 4; ++n) tot[n] += (acc[0][0][n] + acc[0][1][n]) + (acc[1][0][n] + acc[1][1][n]);
+    }
+    __syncthreads();
+    float* part = &st[0][0][0];   // [wave][token][expert]
+#pragma unroll
+    for (uint32_t n = 0; n < 4u; ++n)
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; ++i)
+            part[wave * 1024u + (4u * g + i) * 64u + 16u * n + r16] = tot[n][i];
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < 4u; ++i) {
+        const uint32_t at = threadIdx.x + 256u * i, t = t0 + (at >> 6), e = e0 + (at & 63u);
+        const float v = ((part[at] + part[1024u + at]) + part[2048u + at]) + part[3072u + at];
+        if (t < T && e < n_experts) logits_out[(size_t)t * n_experts + e] = v;
+    }
+}
+
 hipError_t launch_topk_softmax(const float* logits, uint32_t T, uint32_t n_experts, uint32_t k, int normalize,
                                uint32_t* idx, float* wt, hipStream_t s)
 {
@@ -242,6 +317,18 @@ hipError_t launch_route(const float* X, const float* router_w, uint32_t T, uint3
     // many tokens: logits by 8-token tiles, then the selection, as long as the logits have a place to go
     if (T >= ROUTE_SPREAD_TOKENS && (logits_out || (logits_scratch && (uint64_t)T * n_experts <= ROUTE_SCRATCH_FLOATS))) {
         float* lg = logits_out ? logits_out : logits_scratch;
+        // Prices in us: the matrix kernel 4 + 6.4 per 1000 of hidden and round of its workgroups over the CUs, the tiled one 4.5 + 8
+        // per 10^8 products + 1.5 per 10^6 of X.  Measured with the selection, us, tiled / matrix: 2048 x 128 x 2048 44 / 21,
+        // 1024 x 128 x 2048 27 / 20, 2048 x 64 x 1024 21 / 13, 2048 x 32 x 2048 26 / 20; 512 x 128 x 2048 17 / 19, 2048 x 8 x 2048 13 / 18 and
+        // 256 x 128 x 2048 13 / 18 stay.
+        const uint64_t wgs = (uint64_t)((n_experts + 63u) / 64u) * ((T + 15u) / 16u), cus = device_cu_count();
+        const double matrix_us = 4.0 + 6.4e-3 * hidden * (double)((wgs + cus - 1u) / cus);
+        const double tiled_us = 4.5 + (8e-8 * n_experts + 1.5e-6) * (double)T * hidden;
+        if (hidden % 128u == 0 && !(((uintptr_t)X | (uintptr_t)router_w) & 15u) && T <= 1000000u && matrix_us <= tiled_us) {
+            hipLaunchKernelGGL(route_logits_mfma_kernel, dim3((n_experts + 63u) / 64u, (T + 15u) / 16u), dim3(256), 0, s, X, router_w, T,
+                               hidden, n_experts, lg);
+            return launch_topk_softmax(lg, T, n_experts, k, normalize, idx, wt, s);
+        }
         hipLaunchKernelGGL(route_logits_tiled_kernel<8>, dim3((n_experts + 3u) / 4u, (T + 7u) / 8u), dim3(256), 0, s, X,
                            router_w, T, hidden, n_experts, lg);
         return launch_topk_softmax(lg, T, n_experts, k, normalize, idx, wt, s);

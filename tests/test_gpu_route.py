@@ -85,6 +85,24 @@ def test_route_matvec_and_selection(gpu, kqo, T, H, E, k):
     assert np.array_equal(idx2.cpu().numpy(), idx.cpu().numpy()) and np.array_equal(wt2.cpu().numpy(), wt.cpu().numpy())
 
 
+@pytest.mark.parametrize("T,H,E,k", [(2053, 256, 70, 4), (1100, 384, 128, 8), (3000, 128, 100, 3), (2048, 2048, 128, 8), (4100, 640, 33, 2)])
+def test_route_many_tokens_on_the_matrix_instructions(gpu, T, H, E, k):
+    """Ragged tokens and experts, one to five runs of hidden per wave.  Error bound: products and sums in fp32, no chain longer
+    than 64 roundings: 64 * 2^-24 of the sum of |products|; the selection must be the one of the logits returned."""
+    from backpack_amd import kquant
+    print("route matrix", T, H, E, k, flush=True)
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, H)).astype(np.float32)
+    w = (rng.standard_normal((E, H)) / np.sqrt(H)).astype(np.float32)
+    idx, wt, logits = kquant.moe_route(gpu.dev(x), gpu.dev(w), k, True, want_logits=True)
+    lg = logits.cpu().numpy()
+    exact = x.astype(np.float64) @ w.astype(np.float64).T
+    bound = 64 * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T)
+    assert np.all(np.abs(lg - exact) <= bound)
+    order = np.argsort(-lg, axis=1, kind="stable")[:, :k]
+    assert np.array_equal(idx.cpu().numpy(), order)
+
+
 def test_route_feeds_the_expert_ffn(gpu, kqo):
     """router -> top-k -> expert FFN, all on the device, against the oracle chain on the GPU's logits."""
     from backpack_amd import kquant
