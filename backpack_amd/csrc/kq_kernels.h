@@ -157,6 +157,8 @@ size_t wide_x_rest_bytes(uint32_t rows, uint32_t n_blocks);
 // x.xa may be X (no prologue): every superblock is read before it is written
 hipError_t launch_wide_x(int type, const float* X, int pro, const float* norm_w, float eps, uint32_t rows,
                          uint32_t n_blocks, const WideX& x, hipStream_t s);
+// launch_wide's price in us at up to 16 tokens, K in one piece
+double wide_price_16(int type, uint32_t N, uint32_t n_blocks);
 // grouped by expert: records of up to cap (16, 32, 48, 64) pairs, as launch_moe_group writes them with sets = cap / 2;
 // with a.W2, Y = silu(W x) * (W2 x).  records_expected: how many there will be (the launch's work split is chosen by it)
 hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32_t* records, const uint32_t* n_records,

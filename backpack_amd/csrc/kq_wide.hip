@@ -797,25 +797,37 @@ bool wide_supported(const MatmulArgs& a)
     return !(((uintptr_t)a.W | (uintptr_t)a.W2) & 15u) && !(a.row_stride_bytes & 15u);
 }
 
-// Groups of rows that a workgroup walks one after the other: what leaves the fewest us over the CUs, at `step` us per
-// superblock and `start` beside a workgroup's walks.  At 16 tokens two workgroups share a CU (a step of one takes half the
-// two's, and its start goes under the other's walk); alone on it a workgroup is little faster than as one of two.
+// Groups of rows that a workgroup walks one after the other, and the launch's price in us by which they are chosen: the
+// busiest CU's workgroups, at `step` us per superblock and `start` beside a workgroup's walks.  At 16 tokens two workgroups
+// share a CU: a step of one takes half the two's, and its start goes under the other's walk; alone on it a workgroup is
+// a sixth slower than that (too few bytes under way).  others: how many workgroups walk each group; spread: how far that
+// number, as a share of a round, may be off (records).
 // Measured, us, with one group / with those chosen: 128 experts x 8, 2048 / 768, gate and up, then down: 256 tokens (3, 4) 77 / 73
 // and 80 / 68, 2048 tokens (2, 2) 295 / 285 and 255 / 233, 24 tokens (1, 2) 52 / 52 (two groups 61, three 56) and 51.5 / 49.
-static uint32_t groups_per_wg(uint32_t row_groups, double others, int type, uint32_t tt, uint32_t blocks)
+static uint32_t groups_per_wg(uint32_t row_groups, double others, double spread, int type, uint32_t tt, uint32_t blocks, double* price)
 {
-    const bool q6 = type == KQ_TYPE_Q6_K, two = tt == 1u;
+    const bool q5 = type == KQ_TYPE_Q5_K, q6 = type == KQ_TYPE_Q6_K;
     const double cus = (double)device_cu_count();
-    const double step = two ? (q6 ? 3.0 : type == KQ_TYPE_Q5_K ? 2.1 : 1.75) : q6 ? 2.4 + 0.9 * tt : 0.8 + 0.8 * tt;
     uint32_t best = 1;
     double best_us = 1e30;
     for (uint32_t c = 1; c <= row_groups && c <= 64u; ++c) {
-        const double per_cu = (double)((row_groups + c - 1u) / c) * others / cus;
-        const bool shared = two && per_cu > 1.0;
-        const double us = std::fmax(1.0, std::ceil(per_cu - 0.05)) * (c * (blocks * step) * (two && !shared ? 1.15 : 1.0) + (shared ? 4.0 : 9.0));
+        const double n = std::fmax(1.0, std::ceil((double)((row_groups + c - 1u) / c) * others / cus - spread));
+        double step, start = 9.0;
+        if (tt > 1u) step = q6 ? 2.4 + 0.9 * tt : 0.8 + 0.8 * tt;
+        else if (n < 2.0) step = q6 ? 3.6 : q5 ? 2.5 : 2.1;
+        else { step = q6 ? 3.4 : q5 ? 2.1 : 1.75; start = 4.0; }
+        const double us = n * (c * (blocks * step) + start);
         if (us < best_us) { best_us = us; best = c; }
     }
+    if (price) *price = best_us;
     return best;
+}
+
+double wide_price_16(int type, uint32_t N, uint32_t n_blocks)
+{
+    double us;
+    groups_per_wg((N + 255u) / 256u, 1.0, 0.0, type, 1, n_blocks, &us);
+    return us + 3.0;   // (the split of X in front)
 }
 
 hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scratch, size_t x_bytes, int splits, hipStream_t s)
@@ -858,7 +870,7 @@ hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scra
         p.n_splits = (a.n_blocks + p.blocks_per_split - 1u) / p.blocks_per_split;
         p.partial = sc.partial;
         p.row_groups = gx;
-        p.per_wg = p.n_splits > 1u ? 1u : groups_per_wg(gx, (double)gy2, a.type, tt, a.n_blocks);
+        p.per_wg = p.n_splits > 1u ? 1u : groups_per_wg(gx, (double)gy2, 0.0, a.type, tt, a.n_blocks, nullptr);
         p.wgs = (gx + p.per_wg - 1u) / p.per_wg;
         if (hipError_t e = launch_wide_any(a.type, p, tt, dim3(p.wgs, gy2, p.n_splits), s); e != hipSuccess) return e;
         if (p.n_splits > 1u) {
@@ -883,7 +895,7 @@ hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32
     const uint32_t per_wg = a.W2 ? WIDE_WAVES * 16u : WIDE_WAVES * 32u;
     p.row_groups = (a.N + per_wg - 1u) / per_wg;
     const uint32_t tt = cap / 16u;
-    p.per_wg = groups_per_wg(p.row_groups, records_expected, a.type, tt, a.n_blocks);
+    p.per_wg = groups_per_wg(p.row_groups, records_expected, tt == 1u ? 0.02 : 0.05, a.type, tt, a.n_blocks, nullptr);
     p.wgs = (p.row_groups + p.per_wg - 1u) / p.per_wg;
     return launch_wide_any(a.type, p, tt, dim3((p.wgs * bound + 7u) / 8u * 8u), s);
 }

@@ -502,3 +502,19 @@ def test_dispatch_of_expert_layers_with_few_workgroups(gpu, kqo, tgu, tdn, E, k,
     want = kqo.moe_ffn(tgu, tdn, X, gp, up, dp, eidx, ew, H, I)
     rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
     assert np.all(np.abs(got - want) <= 1e-3 * rms + 1e-3 * np.abs(want))
+
+
+@pytest.mark.parametrize("type_,M,N,K,form", [(Q6_K, 3, 128256, 256, "many_token"), (Q6_K, 8, 61500, 1024, "many_token"), (Q4_K, 5, 128257, 512, "many_token"),
+                                              (Q5_K, 8, 131072, 256, "many_token"), (Q4_K, 8, 61500, 1024, ""), (Q5_K, 4, 80000, 512, "")])
+def test_few_tokens_on_many_rows(gpu, kqo, type_, M, N, K, form):  # noqa: F811
+    """3 to 8 tokens on matrices whose rows fill the CUs: the many-token kernel where its rounds come out, else the tiles.
+    Windows of rows against the oracle."""
+    from backpack_amd import capi, kquant, synth
+    print("few tokens", type_, M, N, K, flush=True)
+    raw, packed, w = gpu.make_weight(type_, N, K, seed=M)
+    X = np.random.default_rng(N).standard_normal((M, K)).astype(np.float32)
+    got = kquant.matmul(gpu.dev(X), w).cpu().numpy()
+    assert (capi.last_kernel(), capi.last_form()) == ("mtile", form)
+    words = synth.row_stride_words(type_, K)
+    for a, b in ((0, 270), (N // 2, N // 2 + 300), (N - 270, N)):
+        gpu.check_matmul(kqo, type_, np.ascontiguousarray(got[:, a:b]), X, packed[a * words:b * words], b - a, K, label="few tokens", slack=1e-5)
