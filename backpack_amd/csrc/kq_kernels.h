@@ -160,9 +160,9 @@ hipError_t launch_wide_x(int type, const float* X, int pro, const float* norm_w,
 // launch_wide's price in us at up to 16 tokens, K in one piece
 double wide_price_16(int type, uint32_t N, uint32_t n_blocks);
 // grouped by expert: records of up to cap (16, 32, 48, 64) pairs, as launch_moe_group writes them with sets = cap / 2;
-// with a.W2, Y = silu(W x) * (W2 x).  records_expected: how many there will be (the launch's work split is chosen by it)
+// with a.W2, Y = silu(W x) * (W2 x)
 hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32_t* records, const uint32_t* n_records,
-                               uint32_t bound, uint32_t cap, double records_expected, hipStream_t s);
+                               uint32_t bound, uint32_t cap, hipStream_t s);
 
 // bf16 X of a short prompt (kq_wide.hip): groups of up to 128 tokens, K cut over workgroups.  Takes what
 // gemm_bf16_supported accepts.

@@ -57,6 +57,7 @@ typedef uint32_t w_u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t w_u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int WIDE_WAVES = 8;
+constexpr int WIDE_MAX_GROUPS = 8;   // of rows, that a workgroup walks for a record
 constexpr uint32_t WIDE_XA = 1024, WIDE_XV = 32, WIDE_XI = 4;   // bytes per (token, superblock)
 
 WideX wide_x_layout(void* xa, void* rest, uint32_t rows, uint32_t n_blocks)
@@ -178,12 +179,18 @@ struct WideParams {
     uint32_t n_blocks, row_stride_bytes, y_offset, ldy;
     uint32_t n_splits, blocks_per_split;
     float* partial;          // [split][token group][row group][token][256 columns]
-    uint32_t row_groups, per_wg, wgs;   // groups of 256 rows (act: 128 gate and their up rows); how many a workgroup walks; workgroups
+    uint32_t row_groups, per_wg;        // groups of 256 rows (act: 128 gate and their up rows); how many a workgroup walks (dense)
     int act;                 // 0, or 2 / 3: Y = silu / gelu_tanh (W x) * (W2 x)
-    // grouped (records != nullptr): `wgs` workgroups to a record {expert, count, pair ids ...}; W and W2 advance by N rows per expert, a pair's X row is itself (x_per_slot) or pair / k_slots, its Y row the pair
+    // grouped (records != nullptr): workgroups walk records {expert, count, pair ids ...}; W and W2 advance by N rows per expert, a
+    // pair's X row is itself (x_per_slot) or pair / k_slots, its Y row the pair.  How many groups of rows a workgroup walks is chosen
+    // here, when the number of records is known (a round more than the choice counted on costs as much as all of them: 129
+    // records of which 128 were expected, three groups each, 334 us instead of 206): wgs_of[c - 1] workgroups to a record at c
+    // groups, `walk` us per group, `start` beside them, each for one workgroup per CU and for more
     const uint32_t* records;
     const uint32_t* n_records;
     uint32_t record_words, k_slots;
+    uint32_t wgs_of[WIDE_MAX_GROUPS];
+    float cus, walk[2], start[2];
     int x_per_slot;
 };
 
@@ -307,13 +314,24 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
 
     const uint32_t* rec = nullptr;
-    uint32_t count, t0 = 0, bx = blockIdx.x;
+    uint32_t count, t0 = 0, bx = blockIdx.x, per_wg = p.per_wg;
     const uint8_t *W = p.W, *W2 = p.W2;
     if (p.records) {
-        const uint32_t all = *p.n_records * p.wgs, share = (all + 7u) >> 3, at = (bx & 7u) * share + (bx >> 3);
+        const uint32_t records = *p.n_records;
+        uint32_t wgs = p.wgs_of[0];
+        float best = 3e38f;
+#pragma unroll
+        for (int c = 1; c <= WIDE_MAX_GROUPS; ++c) {
+            const float n = ceilf((float)(p.wgs_of[c - 1] * records) / p.cus);
+            const float us = fmaxf(n, 1.0f) * ((float)c * (n > 1.0f ? p.walk[1] : p.walk[0]) + (n > 1.0f ? p.start[1] : p.start[0]));
+            if (us < best) { best = us; per_wg = (uint32_t)c; wgs = p.wgs_of[c - 1]; }
+        }
+        per_wg = (uint32_t)__builtin_amdgcn_readfirstlane((int)per_wg);
+        wgs = (uint32_t)__builtin_amdgcn_readfirstlane((int)wgs);
+        const uint32_t all = records * wgs, share = (all + 7u) >> 3, at = (bx & 7u) * share + (bx >> 3);
         if ((bx >> 3) >= share || at >= all) return;   // whole workgroup
-        const uint32_t record = at / p.wgs;
-        bx = at - record * p.wgs;
+        const uint32_t record = at / wgs;
+        bx = at - record * wgs;
         rec = p.records + (size_t)record * p.record_words;
         count = rec[1];
         const size_t skip = (size_t)rec[0] * p.N * p.row_stride_bytes;
@@ -351,7 +369,7 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
         for (int r = 0; r < 2; ++r)
             wbase[r] = (r && p.act ? W2 : W) + (size_t)min(tile_row(group, r), p.N - rows) * p.row_stride_bytes + (size_t)((b0 + sb) * BB);
     };
-    const uint32_t group0 = bx * p.per_wg, n_groups = min(p.per_wg, p.row_groups - group0);
+    const uint32_t group0 = bx * per_wg, n_groups = min(per_wg, p.row_groups - group0);
     set_w(group0, 0);
     const uint32_t w_lds = lds0 + L::W_AT + wave * L::W_WAVE;
     // piece k of a superblock's weights: whole loads first, then each tile's last lanes (and d)
@@ -797,26 +815,30 @@ bool wide_supported(const MatmulArgs& a)
     return !(((uintptr_t)a.W | (uintptr_t)a.W2) & 15u) && !(a.row_stride_bytes & 15u);
 }
 
-// Groups of rows that a workgroup walks one after the other, and the launch's price in us by which they are chosen: the
-// busiest CU's workgroups, at `step` us per superblock and `start` beside a workgroup's walks.  At 16 tokens two workgroups
-// share a CU: a step of one takes half the two's, and its start goes under the other's walk; alone on it a workgroup is
-// a sixth slower than that (too few bytes under way).  others: how many workgroups walk each group; spread: how far that
-// number, as a share of a round, may be off (records).
+// Groups of rows that a workgroup walks one after the other are chosen by a launch's price in us: the busiest CU's workgroups,
+// at `walk` per group and `start` beside them, [0] for one workgroup per CU, [1] for more.  At 16 tokens two workgroups share a
+// CU: a step of one takes half the two's, and its start goes under the other's walk; alone on it a workgroup is a sixth
+// slower than that (too few bytes under way).
 // Measured, us, with one group / with those chosen: 128 experts x 8, 2048 / 768, gate and up, then down: 256 tokens (3, 4) 77 / 73
 // and 80 / 68, 2048 tokens (2, 2) 295 / 285 and 255 / 233, 24 tokens (1, 2) 52 / 52 (two groups 61, three 56) and 51.5 / 49.
-static uint32_t groups_per_wg(uint32_t row_groups, double others, double spread, int type, uint32_t tt, uint32_t blocks, double* price)
+struct WideWalk { double walk[2], start[2]; };
+static WideWalk wide_walk(int type, uint32_t tt, uint32_t blocks)
 {
     const bool q5 = type == KQ_TYPE_Q5_K, q6 = type == KQ_TYPE_Q6_K;
-    const double cus = (double)device_cu_count();
+    if (tt == 1u) return {{blocks * (q6 ? 3.6 : q5 ? 2.5 : 2.1), blocks * (q6 ? 3.4 : q5 ? 2.1 : 1.75)}, {9.0, 4.0}};
+    const double step = q6 ? 2.4 + 0.9 * tt : 0.8 + 0.8 * tt;
+    return {{blocks * step, blocks * step}, {9.0, 9.0}};
+}
+
+static uint32_t groups_per_wg(uint32_t row_groups, uint32_t others, int type, uint32_t tt, uint32_t blocks, double* price)
+{
+    const WideWalk w = wide_walk(type, tt, blocks);
+    const uint64_t cus = device_cu_count();
     uint32_t best = 1;
     double best_us = 1e30;
     for (uint32_t c = 1; c <= row_groups && c <= 64u; ++c) {
-        const double n = std::fmax(1.0, std::ceil((double)((row_groups + c - 1u) / c) * others / cus - spread));
-        double step, start = 9.0;
-        if (tt > 1u) step = q6 ? 2.4 + 0.9 * tt : 0.8 + 0.8 * tt;
-        else if (n < 2.0) step = q6 ? 3.6 : q5 ? 2.5 : 2.1;
-        else { step = q6 ? 3.4 : q5 ? 2.1 : 1.75; start = 4.0; }
-        const double us = n * (c * (blocks * step) + start);
+        const uint64_t n = ((uint64_t)((row_groups + c - 1u) / c) * others + cus - 1u) / cus;
+        const double us = (double)n * (c * w.walk[n > 1u] + w.start[n > 1u]);
         if (us < best_us) { best_us = us; best = c; }
     }
     if (price) *price = best_us;
@@ -826,7 +848,7 @@ static uint32_t groups_per_wg(uint32_t row_groups, double others, double spread,
 double wide_price_16(int type, uint32_t N, uint32_t n_blocks)
 {
     double us;
-    groups_per_wg((N + 255u) / 256u, 1.0, 0.0, type, 1, n_blocks, &us);
+    groups_per_wg((N + 255u) / 256u, 1, type, 1, n_blocks, &us);
     return us + 3.0;   // (the split of X in front)
 }
 
@@ -870,9 +892,8 @@ hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scra
         p.n_splits = (a.n_blocks + p.blocks_per_split - 1u) / p.blocks_per_split;
         p.partial = sc.partial;
         p.row_groups = gx;
-        p.per_wg = p.n_splits > 1u ? 1u : groups_per_wg(gx, (double)gy2, 0.0, a.type, tt, a.n_blocks, nullptr);
-        p.wgs = (gx + p.per_wg - 1u) / p.per_wg;
-        if (hipError_t e = launch_wide_any(a.type, p, tt, dim3(p.wgs, gy2, p.n_splits), s); e != hipSuccess) return e;
+        p.per_wg = p.n_splits > 1u ? 1u : groups_per_wg(gx, gy2, a.type, tt, a.n_blocks, nullptr);
+        if (hipError_t e = launch_wide_any(a.type, p, tt, dim3((gx + p.per_wg - 1u) / p.per_wg, gy2, p.n_splits), s); e != hipSuccess) return e;
         if (p.n_splits > 1u) {
             hipLaunchKernelGGL(wide_sum_kernel, dim3(gx, (M + 3u) / 4u), dim3(256), 0, s, p, tt * 16u, gy2);
             if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
@@ -882,7 +903,7 @@ hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scra
 }
 
 hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32_t* records, const uint32_t* n_records,
-                               uint32_t bound, uint32_t cap, double records_expected, hipStream_t s)
+                               uint32_t bound, uint32_t cap, hipStream_t s)
 {
     WideParams p{};
     p.x = x;
@@ -895,9 +916,11 @@ hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32
     const uint32_t per_wg = a.W2 ? WIDE_WAVES * 16u : WIDE_WAVES * 32u;
     p.row_groups = (a.N + per_wg - 1u) / per_wg;
     const uint32_t tt = cap / 16u;
-    p.per_wg = groups_per_wg(p.row_groups, records_expected, tt == 1u ? 0.02 : 0.05, a.type, tt, a.n_blocks, nullptr);
-    p.wgs = (p.row_groups + p.per_wg - 1u) / p.per_wg;
-    return launch_wide_any(a.type, p, tt, dim3((p.wgs * bound + 7u) / 8u * 8u), s);
+    const WideWalk w = wide_walk(a.type, tt, a.n_blocks);
+    p.cus = (float)device_cu_count();
+    for (int i = 0; i < 2; ++i) { p.walk[i] = (float)w.walk[i]; p.start[i] = (float)w.start[i]; }
+    for (uint32_t c = 1; c <= WIDE_MAX_GROUPS; ++c) p.wgs_of[c - 1u] = (p.row_groups + c - 1u) / c;
+    return launch_wide_any(a.type, p, tt, dim3((p.row_groups * bound + 7u) / 8u * 8u), s);
 }
 
 // ------------------------------------------------------------------------------------------------------------------

@@ -504,6 +504,34 @@ def test_dispatch_of_expert_layers_with_few_workgroups(gpu, kqo, tgu, tdn, E, k,
     assert np.all(np.abs(got - want) <= 1e-3 * rms + 1e-3 * np.abs(want))
 
 
+@pytest.mark.parametrize("extra", [0, 1, 40])
+def test_moe_records_around_a_round(gpu, kqo, extra):  # noqa: F811
+    """64 records, or a few more: the number of row groups that a workgroup walks is chosen on the device from the records'
+    number (64 x 4 workgroups are a round of 256 CUs).  All tokens against the 16-token tile kernel."""
+    from backpack_amd import capi, kquant
+    E, k, H, I = 64, 2, 512, 1536
+    _, gp, gw = gpu.make_weight(Q4_K, E * I, H, seed=41)
+    _, up, uw = gpu.make_weight(Q4_K, E * I, H, seed=42)
+    _, dp, dw = gpu.make_weight(Q6_K, E * H, I, seed=43)
+    rng = np.random.default_rng(extra)
+    eidx = np.tile(np.arange(E, dtype=np.uint32).repeat(16), 1)          # 16 pairs per expert
+    eidx = np.concatenate([eidx, np.arange(extra, dtype=np.uint32) % E, np.arange(extra, dtype=np.uint32) % E])
+    T = len(eidx) // k
+    eidx = eidx[: T * k].reshape(k, T).T.copy()
+    ew = rng.random((T, k)).astype(np.float32)
+    X = (rng.standard_normal((T, H)) * 0.1).astype(np.float32)
+    args = (gpu.dev(X), gw, uw, dw, gpu.dev(eidx.view(np.int32)), gpu.dev(ew), E)
+    capi.force_kernel(8)
+    try:
+        got = kquant.moe_ffn(*args).cpu().numpy()
+        capi.force_kernel(6)
+        tile = kquant.moe_ffn(*args).cpu().numpy()
+    finally:
+        capi.force_kernel(0)
+    rms = float(np.sqrt(np.mean(tile.astype(np.float64) ** 2)))
+    assert np.abs(got - tile).max() <= 1e-4 * rms + 1e-4 * np.abs(tile).max()
+
+
 @pytest.mark.parametrize("type_,M,N,K,form", [(Q6_K, 3, 128256, 256, "many_token"), (Q6_K, 8, 61500, 1024, "many_token"), (Q4_K, 5, 128257, 512, "many_token"),
                                               (Q5_K, 8, 131072, 256, "many_token"), (Q4_K, 8, 61500, 1024, ""), (Q5_K, 4, 80000, 512, "")])
 def test_few_tokens_on_many_rows(gpu, kqo, type_, M, N, K, form):  # noqa: F811
