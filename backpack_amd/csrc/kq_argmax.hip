@@ -2,8 +2,8 @@
 //
 // Replaces the two dispatches argmax + argmax_reduce (runtime/kernels/.../argmax.wgsl: per-workgroup
 // scan of a chunk with `v > best` from best = -1e30, index 0; argmax_reduce.wgsl: the same over the
-// partials; wired in runtime/model_runner.cpp:2441-2453) by one launch: ARGMAX_PARTS workgroups per row
-// leave a partial each, the last of them to arrive (a ticket per row) reduces the partials and re-arms
+// partials; wired in runtime/model_runner.cpp:2441-2453) by one launch: up to ARGMAX_PARTS workgroups per
+// row leave a partial each, the last of them to arrive (a ticket per row) reduces the partials and re-arms
 // the ticket.  Among equal maxima the lowest index is returned (the reference's butterfly leaves that
 // to the lane order); a row with nothing above -1e30 yields index 0.
 #include <hip/hip_runtime.h>
@@ -109,11 +109,17 @@ hipError_t argmax_static_scratch(uint32_t** out)
 hipError_t launch_argmax_rows(const float* logits, uint32_t M, uint32_t N, uint32_t ld, int32_t* out_idx,
                               float* out_val, float* part_val, uint32_t* part_idx, uint32_t* tickets, hipStream_t s)
 {
-    // a part is worth at least a few thousand logits
-    uint32_t parts = (N + 4095u) / 4096u;
-    parts = parts < 1u ? 1u : parts > ARGMAX_PARTS ? ARGMAX_PARTS : parts;
+    const uint32_t at_most = 2u * device_cu_count();
     for (uint32_t m0 = 0; m0 < M; m0 += ARGMAX_MAX_ROWS) {
         const uint32_t rows = M - m0 < ARGMAX_MAX_ROWS ? M - m0 : ARGMAX_MAX_ROWS;
+        // a part is worth at least a few thousand logits, and a launch at most two workgroups per CU: the partials and tickets
+        // of more, past the non-coherent cache levels, cost more than their loads in flight give.  Calls in a row, without
+        // this bound, with four per CU and with two: 48 rows of 128256 15.5, 11.0, 10.6 us (10.4 is the host's share),
+        // 128 rows 27.8, 13.9, 13.5, 256 rows 39.0, 21.8, 22.3; 48 rows of 262144 32.5, 15.5, 12.7, 256 rows 81, 42, 40.
+        uint32_t parts = (N + 4095u) / 4096u;
+        parts = parts < ARGMAX_PARTS ? parts : ARGMAX_PARTS;
+        parts = parts * rows <= at_most ? parts : at_most / rows;
+        parts = parts < 1u ? 1u : parts;
         hipLaunchKernelGGL(argmax_rows_kernel, dim3(parts, rows), dim3(256), 0, s, logits + (size_t)m0 * ld, N, ld,
                            out_idx + m0, out_val ? out_val + m0 : nullptr, part_val, part_idx, tickets);
     }

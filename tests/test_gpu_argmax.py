@@ -29,6 +29,24 @@ def test_argmax_rows_vs_oracle(gpu, kqo, M, N):
         assert np.array_equal(val.cpu().numpy(), lg.max(axis=1))
 
 
+@pytest.mark.parametrize("M,N", [(16, 131072), (17, 131071), (48, 40001), (256, 8191), (257, 12289)])
+def test_argmax_parts_of_many_rows(gpu, kqo, M, N):
+    """Row counts at which a row gets fewer parts than its length asks for: exact, with the maximum at every
+    part's edge in turn, also twice in a row (the lower index) and in the last, ragged launch of rows."""
+    from backpack_amd import kquant
+    print("argmax parts", M, N, flush=True)
+    lg = np.random.default_rng(M + N).standard_normal((M, N)).astype(np.float32)
+    for r in range(M):
+        at = min(r * 4096 - r % 3, N - 1) if r * 4096 < N else N - 1 - r % 5
+        lg[r, max(at, 0)] = 50.0
+        if r % 2:
+            lg[r, N - 1] = 50.0
+    for _ in range(2):      # twice: the tickets must have been re-armed
+        idx, val = kquant.argmax_rows(gpu.dev(lg))
+        assert np.array_equal(idx.cpu().numpy(), kqo.argmax_rows(lg))
+        assert np.array_equal(val.cpu().numpy(), lg.max(axis=1))
+
+
 def test_argmax_ties_and_degenerate_rows(gpu, kqo):
     from backpack_amd import kquant
     N = 20000
