@@ -16,12 +16,13 @@
  *
  * One host thread per stream, as in the reference (runtime/model_runner.h:27-30).
  * Beside what the caller brings, calls use scratch memory that the library keeps
- * per device: matmuls that cut K over workgroups and fp32 ones of more than eight
- * tokens, bpk_kq_moe_matmul, an expert FFN on its row kernel, bpk_moe_route
- * without a logits buffer, bpk_argmax_rows, bpk_argmax_rows_static and
- * bpk_kq_matmul_argmax.  Which matmuls cut K is the library's choice, so: on one
- * device calls go to one stream, or are ordered by the caller, so that no two of
- * them overlap; a captured graph's replay counts as its calls.
+ * per device: matmuls that cut K over workgroups and those on the many-token
+ * kernel (fp32 X; any of three tokens and more may be one), bpk_kq_moe_matmul, an
+ * expert FFN on its row kernel, bpk_moe_route without a logits buffer,
+ * bpk_argmax_rows, bpk_argmax_rows_static and bpk_kq_matmul_argmax.  Which matmuls
+ * those are is the library's choice, so: on one device calls go to one stream, or
+ * are ordered by the caller, so that no two of them overlap; a captured graph's
+ * replay counts as its calls.
  */
 #ifndef BPK_KQUANT_H
 #define BPK_KQUANT_H
@@ -521,8 +522,8 @@ BPK_API const char *bpk_last_form(void);
  * (bf16 X only), 5 = lanes-along-K GEMV (M = 1), 6 = 16-row x 16-token
  * matrix-core tiles (groups of 16 tokens), 7 = one token on the matrix cores
  * (Q4_K rows of up to 16 superblocks), 8 = matrix-core tiles of up to 64 tokens
- * (taken by itself from 17 tokens on, from 9 on matrices whose rows fill the
- * part; bpk_last_kernel says "mtile" for 6 and 8), 9 = the short-prompt kernel
+ * (taken by itself from 17 tokens on, on matrices whose rows fill the part from
+ * 9 on, and from 3 where it is priced lower; bpk_last_kernel says "mtile" for 6 and 8), 9 = the short-prompt kernel
  * (bf16 X of up to 512 tokens; bpk_last_kernel says "gemm_bf16" for 4 and 9).
  * A forced fp32 family that cannot serve the call's shape fails with
  * BPK_ERR_SHAPE instead of falling back, and so do 8 and 9 where the call has no

@@ -546,3 +546,17 @@ def test_few_tokens_on_many_rows(gpu, kqo, type_, M, N, K, form):  # noqa: F811
     words = synth.row_stride_words(type_, K)
     for a, b in ((0, 270), (N // 2, N // 2 + 300), (N - 270, N)):
         gpu.check_matmul(kqo, type_, np.ascontiguousarray(got[:, a:b]), X, packed[a * words:b * words], b - a, K, label="few tokens", slack=1e-5)
+
+
+def test_header_names_the_smallest_call_that_uses_the_shared_scratch(gpu):  # noqa: F811
+    """The many-token kernel's split X lies in scratch that calls share: from the number of tokens that the header's list gives,
+    on the matrices it takes first (many rows), and from no smaller one."""
+    import os
+    from backpack_amd import capi, kquant
+    header = open(os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "include", "bpk_kquant.h")).read()
+    assert "any of three tokens and more" in " ".join(header.replace("\n *", " ").split())
+    N, K = 128256, 256
+    raw, packed, w = gpu.make_weight(Q6_K, N, K, seed=1)
+    for M, form in ((1, ""), (2, ""), (3, "many_token")):
+        kquant.matmul(gpu.dev(np.ones((M, K), np.float32)), w)
+        assert capi.last_form() == form, M
