@@ -35,13 +35,16 @@ __global__ __launch_bounds__(256) void argmax_rows_kernel(const float* logits, u
     __shared__ bool last;
     const uint32_t row = blockIdx.y, parts = gridDim.x;
     const float* x = logits + (size_t)row * ld;
-    const uint32_t chunk = ((N + parts - 1u) / parts + 3u) & ~3u;
-    const uint32_t begin = min(blockIdx.x * chunk, N), end = min(begin + chunk, N);
+    // (places beyond 32 bits where N is near 2^32: 64-bit ones, and a walk that counts from the part's start)
+    const uint64_t chunk = (((uint64_t)N + parts - 1u) / parts + 3u) & ~3ull;
+    const uint64_t at = blockIdx.x * chunk;
+    const uint32_t begin = at < N ? (uint32_t)at : N, len = chunk < N - begin ? (uint32_t)chunk : N - begin;
     float v = -1e30f;
     uint32_t i = 0xFFFFFFFFu;   // "none yet": any real index is lower
     // four logits per lane and load (a row may start at any float), four loads in flight
-    const uint32_t whole = begin + ((end - begin) & ~3u);
-    for (uint32_t k0 = begin + 4u * threadIdx.x; k0 < whole; k0 += 4096u) {
+    const uint32_t whole = len & ~3u;
+    x += begin;
+    for (uint32_t k0 = 4u * threadIdx.x; k0 < whole; k0 += 4096u) {
         float t[4][4];
 #pragma unroll
         for (uint32_t u = 0; u < 4u; ++u) __builtin_memcpy(t[u], x + min(k0 + 1024u * u, whole - 4u), 16);
@@ -51,11 +54,11 @@ __global__ __launch_bounds__(256) void argmax_rows_kernel(const float* logits, u
             for (uint32_t e = 0; e < 4u; ++e)
                 // ascending k per lane: the first of equals stays (a piece past the end is the last one again, seen by the lane
                 // that owns it or lost to it: equal values, and best_of takes the lower index)
-                if (t[u][e] > v) { v = t[u][e]; i = min(k0 + 1024u * u, whole - 4u) + e; }
+                if (t[u][e] > v) { v = t[u][e]; i = begin + min(k0 + 1024u * u, whole - 4u) + e; }
     }
-    if (threadIdx.x < end - whole) {
+    if (threadIdx.x < len - whole) {
         const float t = x[whole + threadIdx.x];
-        if (t > v) { v = t; i = whole + threadIdx.x; }
+        if (t > v) { v = t; i = begin + whole + threadIdx.x; }
     }
     argmax_block(v, i, sv, si);
     if (threadIdx.x == 0) {
@@ -116,7 +119,7 @@ hipError_t launch_argmax_rows(const float* logits, uint32_t M, uint32_t N, uint3
         // of more, past the non-coherent cache levels, cost more than their loads in flight give.  Calls in a row, without
         // this bound, with four per CU and with two: 48 rows of 128256 15.5, 11.0, 10.6 us (10.4 is the host's share),
         // 128 rows 27.8, 13.9, 13.5, 256 rows 39.0, 21.8, 22.3; 48 rows of 262144 32.5, 15.5, 12.7, 256 rows 81, 42, 40.
-        uint32_t parts = (N + 4095u) / 4096u;
+        uint32_t parts = (uint32_t)(((uint64_t)N + 4095u) / 4096u);
         parts = parts < ARGMAX_PARTS ? parts : ARGMAX_PARTS;
         parts = parts * rows <= at_most ? parts : at_most / rows;
         parts = parts < 1u ? 1u : parts;

@@ -147,3 +147,18 @@ def test_argmax_pieces_of_four(gpu, kqo, M, N, ld):
     got, val = kquant.argmax_rows(torch.from_numpy(buf).cuda()[:, :N])
     assert np.array_equal(got.cpu().numpy(), kqo.argmax_rows(np.ascontiguousarray(buf[:, :N])))
     assert np.array_equal(val.cpu().numpy(), np.nanmax(buf[:, :N], axis=1))
+
+
+@pytest.mark.parametrize("N", [2 ** 32 - 1001, 2 ** 32 - 1])
+def test_argmax_of_a_row_of_nearly_2_to_the_32_logits(gpu, N):
+    """The walk ends and every logit is seen where a place plus a stride leaves 32 bits (the index returns as 32 bits)."""
+    import torch
+    from backpack_amd import kquant
+    print("argmax", N, flush=True)
+    x = torch.full((1, N), -1.0, dtype=torch.float32, device="cuda")
+    for at in (N - 1, N - 4096, N // 2 + 1, 2):     # each below the one before: the lowest of equals
+        x[0, at] = 5.0
+        idx, val = kquant.argmax_rows(x)
+        assert (int(idx[0]) & 0xFFFFFFFF, float(val[0])) == (at, 5.0)
+    del x
+    torch.cuda.empty_cache()
