@@ -46,7 +46,7 @@ __device__ __forceinline__ void put_four(uint16_t* out, size_t at, float4 v)
     *(bf16x4*)(out + at) = bf16x4{(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
 }
 
-// Up to 8192 elements, 512 lanes.  2048 rows of 4096 17 -> 10 us, 100 rows 10 -> 6 (bf16 out; one dependent pass less, and 16
+// Up to 8192 elements, 512 lanes (fewer than 2^23 rows: a grid holds fewer than 2^32 threads).  2048 rows of 4096 17 -> 10 us, 100 rows 10 -> 6 (bf16 out; one dependent pass less, and 16
 // bytes a load).
 template <typename OUT>
 __global__ __launch_bounds__(512) void rms_norm_rows4_kernel(const float* X, const float* w, float eps, uint32_t K, OUT* out)
@@ -155,7 +155,7 @@ static hipError_t launch_prologue_rows_as(int pro, const float* X, const float* 
         const dim3 grid((K / 4u + 511u) / 512u, M);
         if (pro == 2) hipLaunchKernelGGL((act_mul_rows4_kernel<false, OUT>), grid, dim3(256), 0, s, X, K, out);
         else hipLaunchKernelGGL((act_mul_rows4_kernel<true, OUT>), grid, dim3(256), 0, s, X, K, out);
-    } else if (fours && K <= 8192u) hipLaunchKernelGGL(rms_norm_rows4_kernel<OUT>, dim3(M), dim3(512), 0, s, X, norm_w, eps, K, out);
+    } else if (fours && K <= 8192u && M < (1u << 23)) hipLaunchKernelGGL(rms_norm_rows4_kernel<OUT>, dim3(M), dim3(512), 0, s, X, norm_w, eps, K, out);
     else if (pro == 1) hipLaunchKernelGGL(rms_norm_rows_kernel<OUT>, dim3(M), dim3(256), 0, s, X, norm_w, eps, K, out);
     else if (pro == 2) hipLaunchKernelGGL((act_mul_rows_kernel<false, OUT>), dim3((K + 255u) / 256u, M), dim3(256), 0, s, X, K, out);
     else hipLaunchKernelGGL((act_mul_rows_kernel<true, OUT>), dim3((K + 255u) / 256u, M), dim3(256), 0, s, X, K, out);

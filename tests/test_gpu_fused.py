@@ -342,3 +342,21 @@ def test_prefill_rows_in_pieces_of_four(gpu, M, K, offset):
             v = u * (torch.nn.functional.silu(g) if pro == capi.PRO_SILU_MUL else torch.nn.functional.gelu(g, approximate="tanh"))
         outside = int(((got - v).abs() > (2.0 ** -8 + 1e-5) * v.abs() + 1e-6).sum())
         assert outside == 0, (pro, offset)
+
+
+def test_prefill_norm_of_more_rows_than_a_grid_of_512_lanes_holds(gpu):
+    """2^23 rows and a few: a launch of one workgroup of 512 lanes per row would have more than 2^32 - 1 threads."""
+    import torch
+    from backpack_amd import capi, kquant
+    M, K = (1 << 23) + 3, 4
+    print("norm rows", M, K, flush=True)
+    x = torch.randn(M, K, device="cuda")
+    w = torch.rand(K, device="cuda") + 0.5
+    got = kquant.prefill_rows_bf16(x, K, prologue=capi.PRO_RMS_NORM, norm_w=w, eps=1e-5)
+    for a, b in ((0, 1000), (M // 2, M // 2 + 1000), (M - 1000, M)):
+        v = x[a:b].double()
+        want = v * torch.rsqrt((v * v).mean(1, keepdim=True) + 1e-5) * w.double()
+        # one rounding to bf16, 2^-8 of the value at most, plus fp32 noise
+        assert bool(((got[a:b].double() - want).abs() <= (2.0 ** -8 + 1e-5) * want.abs() + 1e-6).all())
+    del x, got
+    torch.cuda.empty_cache()
