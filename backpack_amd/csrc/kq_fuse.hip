@@ -46,8 +46,9 @@ __device__ __forceinline__ void put_four(uint16_t* out, size_t at, float4 v)
     *(bf16x4*)(out + at) = bf16x4{(__bf16)v.x, (__bf16)v.y, (__bf16)v.z, (__bf16)v.w};
 }
 
-// Up to 8192 elements, 512 lanes (fewer than 2^23 rows: a grid holds fewer than 2^32 threads).  2048 rows of 4096 17 -> 10 us, 100 rows 10 -> 6 (bf16 out; one dependent pass less, and 16
-// bytes a load).
+// 1280 to 8192 elements, 512 lanes (fewer than 2^23 rows: a grid holds fewer than 2^32 threads).  2048 rows of 4096 17 -> 10 us, 100
+// rows 10 -> 6 (bf16 out; one dependent pass less, and 16 bytes a load).  Shorter rows leave most lanes idle and stay on the scalar
+// form: 8008 rows of 256 9.9 us here, 5.6 there, 2048 rows of 1024 4.2 and 4.0, of 1280 4.3 and 4.5.
 template <typename OUT>
 __global__ __launch_bounds__(512) void rms_norm_rows4_kernel(const float* X, const float* w, float eps, uint32_t K, OUT* out)
 {
@@ -104,23 +105,23 @@ __device__ __forceinline__ float act_of(float gv)
     return gv / (expf(-gv) + 1.0f);
 }
 
-// GU rows are gate | up (2K floats); out rows are K floats.  Two pieces of four per lane, all four loads in flight: 2048 rows of
-// 14336 (294 MB) 75 -> 55 us.
-template <bool GELU, typename OUT>
+// GU rows are gate | up (2K floats); out rows are K floats.  P pieces of four per lane, all their loads in flight: with two, 2048 rows
+// of 14336 (294 MB) 75 -> 55 us.
+template <int P, bool GELU, typename OUT>
 __global__ __launch_bounds__(256) void act_mul_rows4_kernel(const float* GU, uint32_t K, OUT* out)
 {
     const float* row = GU + (size_t)blockIdx.y * 2u * K;
-    float4 g[2], u[2];
-    uint32_t k[2];
+    float4 g[P], u[P];
+    uint32_t k[P];
 #pragma unroll
-    for (uint32_t i = 0; i < 2u; ++i) {
-        k[i] = 4u * (blockIdx.x * 512u + i * 256u + threadIdx.x);
-        const uint32_t at = min(k[i], K - 4u);
-        g[i] = *(const float4*)(row + at);
-        u[i] = *(const float4*)(row + K + at);
+    for (uint32_t i = 0; i < (uint32_t)P; ++i) {
+        k[i] = 4u * (blockIdx.x * (256u * P) + i * 256u + threadIdx.x);
+        if (k[i] >= K) continue;
+        g[i] = *(const float4*)(row + k[i]);
+        u[i] = *(const float4*)(row + K + k[i]);
     }
 #pragma unroll
-    for (uint32_t i = 0; i < 2u; ++i)
+    for (uint32_t i = 0; i < (uint32_t)P; ++i)
         if (k[i] < K)
             put_four(out, (size_t)blockIdx.y * K + k[i], float4{act_of<GELU>(g[i].x) * u[i].x, act_of<GELU>(g[i].y) * u[i].y,
                                                                act_of<GELU>(g[i].z) * u[i].z, act_of<GELU>(g[i].w) * u[i].w});
@@ -152,10 +153,17 @@ static hipError_t launch_prologue_rows_as(int pro, const float* X, const float* 
 {
     const bool fours = K >= 4u && K % 4u == 0 && !(((uintptr_t)X | (uintptr_t)out | (pro == 1 ? (uintptr_t)norm_w : 0u)) & 15u);
     if (fours && pro != 1) {
-        const dim3 grid((K / 4u + 511u) / 512u, M);
-        if (pro == 2) hipLaunchKernelGGL((act_mul_rows4_kernel<false, OUT>), grid, dim3(256), 0, s, X, K, out);
-        else hipLaunchKernelGGL((act_mul_rows4_kernel<true, OUT>), grid, dim3(256), 0, s, X, K, out);
-    } else if (fours && K <= 8192u && M < (1u << 23)) hipLaunchKernelGGL(rms_norm_rows4_kernel<OUT>, dim3(M), dim3(512), 0, s, X, norm_w, eps, K, out);
+        // Two pieces per lane from 2^22 outputs on, unless workgroups of 2048 outputs would leave more than a quarter of theirs beyond
+        // the row; other calls need the workgroups more than the loads in flight.  us, scalar / two pieces / one: GELU 521 x 2560 3.4 /
+        // 4.3 / 3.3, 1292 x 2560 6.5 / 8.0 / 5.0, SILU 2048 x 2560 10.0 / 10.4 / 8.7; with two SILU 2048 x 14336 66 / 43.
+        const bool fits = (uint64_t)(K + 2047u) / 2048u * 2048u * 4u <= 5ull * K;
+        const uint32_t P = fits && (uint64_t)M * K >= (1u << 22) ? 2u : 1u;
+        const dim3 grid((K / 4u + 256u * P - 1u) / (256u * P), M);
+        if (pro == 2 && P == 2u) hipLaunchKernelGGL((act_mul_rows4_kernel<2, false, OUT>), grid, dim3(256), 0, s, X, K, out);
+        else if (pro == 2) hipLaunchKernelGGL((act_mul_rows4_kernel<1, false, OUT>), grid, dim3(256), 0, s, X, K, out);
+        else if (P == 2u) hipLaunchKernelGGL((act_mul_rows4_kernel<2, true, OUT>), grid, dim3(256), 0, s, X, K, out);
+        else hipLaunchKernelGGL((act_mul_rows4_kernel<1, true, OUT>), grid, dim3(256), 0, s, X, K, out);
+    } else if (fours && K >= 1280u && K <= 8192u && M < (1u << 23)) hipLaunchKernelGGL(rms_norm_rows4_kernel<OUT>, dim3(M), dim3(512), 0, s, X, norm_w, eps, K, out);
     else if (pro == 1) hipLaunchKernelGGL(rms_norm_rows_kernel<OUT>, dim3(M), dim3(256), 0, s, X, norm_w, eps, K, out);
     else if (pro == 2) hipLaunchKernelGGL((act_mul_rows_kernel<false, OUT>), dim3((K + 255u) / 256u, M), dim3(256), 0, s, X, K, out);
     else hipLaunchKernelGGL((act_mul_rows_kernel<true, OUT>), dim3((K + 255u) / 256u, M), dim3(256), 0, s, X, K, out);

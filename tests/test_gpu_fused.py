@@ -360,3 +360,22 @@ def test_prefill_norm_of_more_rows_than_a_grid_of_512_lanes_holds(gpu):
         assert bool(((got[a:b].double() - want).abs() <= (2.0 ** -8 + 1e-5) * want.abs() + 1e-6).all())
     del x, got
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("pro,M,K", [(NORM, 3, 1276), (NORM, 3, 1280), (NORM, 70, 2052), (SILU, 2048, 2048), (SILU, 2049, 2044), (GELU, 2048, 2052),
+                                     (GELU, 1641, 2560), (SILU, 1025, 4096), (GELU, 3, 1024), (SILU, 5, 1028)])
+def test_prefill_rows_around_their_rules(gpu, pro, M, K):
+    """Norm rows on both sides of the length from which a row has a workgroup of 512 lanes; activations on both sides of 2^22 outputs
+    (two pieces of four per lane from there on) and of rows that would leave a quarter of those pieces empty.  Bound as above."""
+    import torch
+    from backpack_amd import kquant
+    x = gpu.dev(np.random.default_rng(M + K).standard_normal((M, K if pro == NORM else 2 * K)).astype(np.float32))
+    w = gpu.dev((1 + 0.1 * np.random.default_rng(K).standard_normal(K)).astype(np.float32))
+    got = kquant.prefill_rows_bf16(x, K, prologue=pro, norm_w=w if pro == NORM else None, eps=1e-5).double()
+    v = x.double()
+    if pro == NORM:
+        v = v * torch.rsqrt((v * v).mean(1, keepdim=True) + 1e-5) * w.double()
+    else:
+        g, u = v[:, :K], v[:, K:]
+        v = u * (torch.nn.functional.silu(g) if pro == SILU else torch.nn.functional.gelu(g, approximate="tanh"))
+    assert int(((got - v).abs() > (2.0 ** -8 + 1e-5) * v.abs() + 1e-6).sum()) == 0
