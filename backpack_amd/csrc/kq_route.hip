@@ -317,14 +317,18 @@ hipError_t launch_route(const float* X, const float* router_w, uint32_t T, uint3
     // many tokens: logits by 8-token tiles, then the selection, as long as the logits have a place to go
     if (T >= ROUTE_SPREAD_TOKENS && (logits_out || (logits_scratch && (uint64_t)T * n_experts <= ROUTE_SCRATCH_FLOATS))) {
         float* lg = logits_out ? logits_out : logits_scratch;
-        // Prices in us: the matrix kernel 4 + 6.4 per 1000 of hidden and round of its workgroups over the CUs, the tiled one 4.5 + 8
-        // per 10^8 products + 1.5 per 10^6 of X.  Measured with the selection, us, tiled / matrix: 2048 x 128 x 2048 44 / 21,
-        // 1024 x 128 x 2048 27 / 20, 2048 x 64 x 1024 21 / 13, 2048 x 32 x 2048 26 / 20; 512 x 128 x 2048 17 / 19, 2048 x 8 x 2048 13 / 18 and
-        // 256 x 128 x 2048 13 / 18 stay.
+        // Prices in us, with the selection, fitted to 4767 calls of 64 to 8192 tokens: the matrix kernel 6 + 1.8 and 6.7 per 1000 of
+        // hidden for each round of its workgroups over the CUs; the tiled one 7.8, 2.8 per 10^8 products, 1 per 10^6 of X, 7 per 10^5
+        // logits and 0.5 per 1000 of hidden for each 1024 of its workgroups.  A matrix workgroup always computes 64 experts: of few it
+        // wastes most (6184 x 8 x 4608 42 tiled, 74 matrix; 4268 x 16 x 4096 48, 64; 2048 x 8 x 2048 12, 22).  tiled / matrix: 2048 x
+        // 128 x 2048 46 / 22, 1024 x 128 x 2048 29 / 22, 2048 x 64 x 1024 26 / 17, 2048 x 32 x 2048 30 / 22; 512 x 128 x 1920 19 / 20 and
+        // 256 x 128 x 1792 16 / 21 stay.  Of those calls the choice is more than 3 % behind the tiled kernel on 4.
         const uint64_t wgs = (uint64_t)((n_experts + 63u) / 64u) * ((T + 15u) / 16u), cus = device_cu_count();
-        const double matrix_us = 4.0 + 6.4e-3 * hidden * (double)((wgs + cus - 1u) / cus);
-        const double tiled_us = 4.5 + (8e-8 * n_experts + 1.5e-6) * (double)T * hidden;
-        if (hidden % 128u == 0 && !(((uintptr_t)X | (uintptr_t)router_w) & 15u) && T <= 1000000u && matrix_us <= tiled_us) {
+        const uint64_t tiled_wgs = (uint64_t)((n_experts + 3u) / 4u) * ((T + 7u) / 8u);
+        const double matrix_us = 6.0 + (double)((wgs + cus - 1u) / cus) * (1.8 + 6.7e-3 * hidden);
+        const double tiled_us = 7.8 + (2.8e-8 * n_experts + 1e-6) * (double)T * hidden + 7e-5 * (double)T * n_experts +
+                                5e-4 * hidden * (double)((tiled_wgs + 1023u) / 1024u);
+        if (hidden % 128u == 0 && !(((uintptr_t)X | (uintptr_t)router_w) & 15u) && T <= 1000000u && matrix_us <= 0.97 * tiled_us) {
             hipLaunchKernelGGL(route_logits_mfma_kernel, dim3((n_experts + 63u) / 64u, (T + 15u) / 16u), dim3(256), 0, s, X, router_w, T,
                                hidden, n_experts, lg);
             return launch_topk_softmax(lg, T, n_experts, k, normalize, idx, wt, s);

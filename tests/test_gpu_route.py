@@ -103,6 +103,22 @@ def test_route_many_tokens_on_the_matrix_instructions(gpu, T, H, E, k):
     assert np.array_equal(idx.cpu().numpy(), order)
 
 
+@pytest.mark.parametrize("T,H,E,k", [(2048, 512, 8, 2), (4113, 256, 6, 3), (4500, 512, 16, 4)])
+def test_route_many_tokens_of_few_experts(gpu, T, H, E, k):
+    """Few experts stay on the 8-token tiles, however many tokens there are: the same bound and selection as above."""
+    from backpack_amd import kquant
+    print("route few experts", T, H, E, k, flush=True)
+    rng = np.random.default_rng(T)
+    x = rng.standard_normal((T, H)).astype(np.float32)
+    w = (rng.standard_normal((E, H)) / np.sqrt(H)).astype(np.float32)
+    idx, wt, logits = kquant.moe_route(gpu.dev(x), gpu.dev(w), k, True, want_logits=True)
+    lg = logits.cpu().numpy()
+    exact = x.astype(np.float64) @ w.astype(np.float64).T
+    bound = 64 * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).astype(np.float64).T)
+    assert np.all(np.abs(lg - exact) <= bound)
+    assert np.array_equal(idx.cpu().numpy(), np.argsort(-lg, axis=1, kind="stable")[:, :k])
+
+
 def test_route_feeds_the_expert_ffn(gpu, kqo):
     """router -> top-k -> expert FFN, all on the device, against the oracle chain on the GPU's logits."""
     from backpack_amd import kquant
