@@ -1223,6 +1223,7 @@ bool mtile_supported(const MatmulArgs& a)
     // tokens on small Q6_K matrices and for rows too long for the many-token kernel's scratch (and when forced)
     if (!a.expert_idx && (a.M < 1 || a.M > 65536u)) return false;   // grouped calls bring their tokens in records
     if (((uintptr_t)a.X & 15u)) return false;
+    if ((uint64_t)16u * a.row_stride_bytes > 0xFFFFFFFFull) return false;   // a tile's rows lie at 32-bit offsets
     if (a.type == KQ_TYPE_Q4_K || a.type == KQ_TYPE_Q5_K) return !(((uintptr_t)a.W & 15u) || (a.row_stride_bytes & 15u));
     if (a.type == KQ_TYPE_Q6_K) return !(((uintptr_t)a.W & 1u) || (a.row_stride_bytes & 1u));
     return false;

@@ -812,6 +812,7 @@ bool wide_supported(const MatmulArgs& a)
     // X in 16-byte loads; Q4_K and Q5_K blocks too (their 144 and 176 bytes keep a 16-byte aligned row aligned)
     if (((uintptr_t)a.X | (uintptr_t)a.norm_w) & 15u) return false;
     if (a.n_blocks * KQ_QK != a.K || a.N == 0) return false;
+    if ((uint64_t)16u * a.row_stride_bytes > 0xFFFFFFFFull) return false;   // a tile's rows lie at 32-bit offsets
     if (a.type == KQ_TYPE_Q6_K) return !((uintptr_t)a.W & 1u) && !((uintptr_t)a.W2 & 1u);
     return !(((uintptr_t)a.W | (uintptr_t)a.W2) & 15u) && !(a.row_stride_bytes & 15u);
 }

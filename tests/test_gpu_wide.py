@@ -560,3 +560,33 @@ def test_header_names_the_smallest_call_that_uses_the_shared_scratch(gpu):  # no
     for M, form in ((1, ""), (2, ""), (3, "many_token")):
         kquant.matmul(gpu.dev(np.ones((M, K), np.float32)), w)
         assert capi.last_form() == form, M
+
+
+@pytest.mark.parametrize("type_,M", [(Q4_K, 17), (Q6_K, 17), (Q4_K, 5)])
+def test_rows_farther_apart_than_32_bit_offsets_reach(gpu, kqo, type_, M):  # noqa: F811
+    """Rows 302 MB apart: a tile of sixteen spans more than 2^32 bytes.  The kernels that hold a row's place in 32 bits leave such a
+    call to one that does not."""
+    import torch
+    from backpack_amd import capi, kquant, synth
+    N, K, stride = 17, 256, 0x12000000
+    print("far rows", type_, M, flush=True)
+    raw, packed, w = gpu.make_weight(type_, N, K, seed=9)
+    row = synth.row_stride_words(type_, K) * 4
+    data = torch.zeros(N * stride + 16, dtype=torch.uint8, device="cuda")
+    body = torch.from_numpy(packed.view(np.uint8).reshape(N, row)).cuda()
+    for n in range(N):
+        data[n * stride:n * stride + row] = body[n]
+    far = kquant.KQuantPacked(data, type_, N, K, stride // 4, 1)
+    X = np.random.default_rng(M).standard_normal((M, K)).astype(np.float32)
+    got = kquant.matmul(gpu.dev(X), far).cpu().numpy()
+    gpu.check_matmul(kqo, type_, got, X, packed, N, K, label="far rows", slack=1e-5)
+    for family in (6, 8):
+        capi.force_kernel(family)
+        try:
+            with pytest.raises(capi.BpkError) as e:
+                kquant.matmul(gpu.dev(X), far)
+            assert e.value.code == -2
+        finally:
+            capi.force_kernel(0)
+    del data, far
+    torch.cuda.empty_cache()
