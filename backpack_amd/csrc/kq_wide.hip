@@ -259,35 +259,57 @@ __device__ __forceinline__ void wide_barrier() { asm volatile("s_waitcnt lgkmcnt
 // kernel's own (wide_meet).  No register is written, so none can be reused while a load is in flight.  The compiler does not
 // see into these statements, so the wait states between a vector instruction that writes a scalar register (a spill read
 // back, a readfirstlane) and a load that uses it (5), and ahead of a load that uses m0 (1), stand in them.
-__device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* src)
+// SKIP: not at all where go is 0 (the branch lies inside the statement, so the steps of the walk stay one basic block).
+#define WIDE_SKIP "s_cmp_eq_u32 %2, 0\n\ts_mov_b32 m0, %0\n\ts_cbranch_scc1 .Lwide_skip%=\n\t"
+template <bool SKIP> __device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* src, int go)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+    if constexpr (SKIP) asm volatile(WIDE_SKIP "global_load_lds_dwordx4 %1, off\n.Lwide_skip%=:" ::"s"(lds), "v"(src), "s"(go) : "scc", "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
 }
-__device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* base, uint32_t off)
+template <bool SKIP> __device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* base, uint32_t off, int go)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
+    if constexpr (SKIP)
+        asm volatile(WIDE_SKIP "s_nop 1\n\tglobal_load_lds_dwordx4 %1, %3\n.Lwide_skip%=:" ::"s"(lds), "v"(off), "s"(go), "s"(base) : "scc", "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base) : "memory");
 }
-// ... with the lanes of `lanes` only (none: it moves nothing, but keeps its place in the count of loads in flight).  Called
-// with every lane active; no branch, so the steps of the walk stay one basic block.
-__device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* src, int lanes)
+// ... with the lanes of `lanes` only (none: it moves nothing).  Called with every lane active.
+template <bool SKIP> __device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* base, uint32_t off, uint64_t lanes, int go)
+{
+    if constexpr (SKIP)
+        asm volatile(WIDE_SKIP "s_mov_b64 exec, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %3\n\ts_mov_b64 exec, -1\n.Lwide_skip%=:" ::"s"(lds), "v"(off), "s"(go), "s"(base), "s"(lanes) : "scc", "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\ts_nop 2\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(off), "s"(base), "s"(lanes) : "memory");
+}
+template <bool SKIP> __device__ __forceinline__ void lds_dma4(uint32_t lds, const uint8_t* base, uint32_t off, uint64_t lanes, int go)
+{
+    if constexpr (SKIP)
+        asm volatile(WIDE_SKIP "s_mov_b64 exec, %4\n\ts_nop 0\n\tglobal_load_lds_dword %1, %3\n\ts_mov_b64 exec, -1\n.Lwide_skip%=:" ::"s"(lds), "v"(off), "s"(go), "s"(base), "s"(lanes) : "scc", "memory");
+    else asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\ts_nop 2\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(off), "s"(base), "s"(lanes) : "memory");
+}
+template <bool SKIP> __device__ __forceinline__ void lds_dma4(uint32_t lds, const void* src, int go)
+{
+    static_assert(SKIP, "");
+    asm volatile(WIDE_SKIP "global_load_lds_dword %1, off\n.Lwide_skip%=:" ::"s"(lds), "v"(src), "s"(go) : "scc", "memory");
+}
+#undef WIDE_SKIP
+// (an int: all lanes or none)
+__device__ __forceinline__ void lds_dma16_or_none(uint32_t lds, const uint8_t* src, int lanes)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(src), "s"(lanes) : "memory");
 }
-__device__ __forceinline__ void lds_dma16(uint32_t lds, const uint8_t* base, uint32_t off, uint64_t lanes)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\ts_nop 2\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(off), "s"(base), "s"(lanes) : "memory");
-}
-__device__ __forceinline__ void lds_dma4(uint32_t lds, const uint8_t* base, uint32_t off, uint64_t lanes)
-{
-    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %3\n\ts_nop 2\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(off), "s"(base), "s"(lanes) : "memory");
-}
-__device__ __forceinline__ void lds_dma4(uint32_t lds, const void* src, int lanes)
+__device__ __forceinline__ void lds_dma4_or_none(uint32_t lds, const void* src, int lanes)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\tglobal_load_lds_dword %1, off\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(src), "s"(lanes) : "memory");
 }
 // At most N of this wave's loads are still in flight, its LDS reads have returned, and so have the other waves'.
 template <int N>
 __device__ __forceinline__ void wide_meet() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory"); }
+
+// None of this wave's loads is still in flight, if go is 0.  (wide_meet's counts take all of the walk's loads to have been sent;
+// the branch lies inside the statement.)
+__device__ __forceinline__ void wide_drain_unless(int go)
+{
+    asm volatile("s_cmp_lg_u32 %0, 0\n\ts_cbranch_scc1 .Lwide_go%=\n\ts_waitcnt vmcnt(0)\n.Lwide_go%=:" ::"s"(go) : "scc", "memory");
+}
 
 // The kernel's LDS, in bytes.  X: a ring of three halves of a superblock, [token][hi, lo][16 pieces of 16 bytes], a piece's
 // place exchanged by its token (^ token % 16) so that the 16 tokens that a wave reads a piece of lie in different banks.
@@ -351,7 +373,7 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     uint32_t* const out_rows = (uint32_t*)(lds + L::R_AT + wave * (TT * 128u));
     uint32_t* const x_rows = out_rows + TT * 16u;
     const uint32_t slot0 = min(lane, min(count, TT * 16u) - 1u);
-    if (rec) lds_dma4(lds0 + L::R_AT + wave * (TT * 128u), (const uint8_t*)rec, slot0 * 4u, TT == 4 ? ~0ull : (1ull << (TT * 16u % 64u)) - 1ull);
+    if (rec) lds_dma4<false>(lds0 + L::R_AT + wave * (TT * 128u), (const uint8_t*)rec, slot0 * 4u, TT == 4 ? ~0ull : (1ull << (TT * 16u % 64u)) - 1ull, -1);
 
     // W: the wave's two tiles of 16 rows, unit after unit.  The last rows of a matrix that does not fill its tiles are read from
     // N - 16 on (what a tile has of an earlier one is not stored), so a lane's offsets are the same for every tile.
@@ -374,37 +396,49 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     set_w(group0, 0);
     const uint32_t w_lds = lds0 + L::W_AT + wave * L::W_WAVE;
     // piece k of a superblock's weights: whole loads first, then each tile's last lanes (and d)
-    auto request_w = [&](int k) {
+    constexpr bool SKIP = TT == 1;
+    auto request_w = [&](int k, int go) {
         constexpr int WHOLE = 2 * ((int)L::W_INSTR - 1);
         if (k < WHOLE) {
             const uint32_t r = (uint32_t)k & 1u, i = (uint32_t)k >> 1;
-            lds_dma16(w_lds + r * L::W_TILE + i * 1024u, wbase[r], woff[i]);
+            lds_dma16<SKIP>(w_lds + r * L::W_TILE + i * 1024u, wbase[r], woff[i], go);
         } else if (k < WHOLE + 2) {
             const uint32_t r = (uint32_t)k & 1u;
-            lds_dma16(w_lds + r * L::W_TILE + (L::W_INSTR - 1u) * 1024u, wbase[r], woff[L::W_INSTR - 1u], (1ull << L::W_LAST) - 1ull);
+            lds_dma16<SKIP>(w_lds + r * L::W_TILE + (L::W_INSTR - 1u) * 1024u, wbase[r], woff[L::W_INSTR - 1u], (1ull << L::W_LAST) - 1ull, go);
         } else {
             const uint32_t r = (uint32_t)k & 1u;
-            lds_dma4(w_lds + 2u * L::W_TILE + r * 64u, wbase[r], doff, 0xFFFFull);
+            lds_dma4<SKIP>(w_lds + 2u * L::W_TILE + r * 64u, wbase[r], doff, 0xFFFFull, go);
         }
     };
     // The walk: n_groups groups of rows against the same tokens, n_sb superblocks each, as one sequence of `all` superblocks:
     // W and X of the next group are under way while a group's outputs leave.  Half h of it is superblock h / 2.  Requested
-    // ahead: X by two halves, W by one superblock (into the place it was read from), S half a superblock less; past the
-    // end the last is requested again.
+    // ahead: X by two halves, W by one superblock (into the place it was read from), S half a superblock less.  Past the
+    // end the last is requested again — or, at 16 tokens (SKIP), nothing is: there a walk of few superblocks waits for those loads a
+    // second time before its last meeting and at its end (64 tokens, 128 experts x 8, 2048 / 768 Q4_K / Q6_K: 121.8 us without, 120.3 with it; 195998 x 768 Q4_K at 9 tokens 28.5 and 27.3).  At more
+    // tokens the walk is bound by issue, and the test for it costs as much or more (28672 x 4096 at 48 tokens 37.0 us, 38.1 with it).
     constexpr int WAS = (TT + L::N_W + 3) / 4, XBS = (TT + 3) / 4;   // requests per step
     const uint32_t n_sb = b1 - b0, all = n_groups * n_sb;
     auto wrap = [&](uint32_t sb) { return sb + 1u == n_sb ? 0u : sb + 1u; };
     uint32_t w_group = group0;   // the group whose W is requested
     auto next_w = [&](uint32_t at, uint32_t sb) {   // from superblock `at`, number sb of its group, to the one behind it
-        const uint32_t go = at + 1u < all ? 1u : 0u, to = wrap(sb);
+        const uint32_t go = SKIP || at + 1u < all ? 1u : 0u, to = wrap(sb);
         w_group += to == 0u ? go : 0u;
         set_w(w_group, go ? to : sb);
     };
     // the way of X from the second half of superblock `at`, number sb of its group; of S from the superblock
-    auto x_step = [&](uint32_t at, uint32_t sb) -> int { return at + 1u >= all ? -256 : wrap(sb) ? 768 : -(int)(sb * WIDE_XA) - 256; };
-    auto s_step = [&](uint32_t at, uint32_t sb) -> int { return at + 1u >= all ? 0 : wrap(sb) ? 1 : -(int)sb; };
+    auto x_step = [&](uint32_t at, uint32_t sb) -> int { return !SKIP && at + 1u >= all ? -256 : wrap(sb) ? 768 : -(int)(sb * WIDE_XA) - 256; };
+    auto s_step = [&](uint32_t at, uint32_t sb) -> int { return !SKIP && at + 1u >= all ? 0 : wrap(sb) ? 1 : -(int)sb; };
+    // is superblock `at` there (a scalar register, as below)
+    auto there = [&](uint32_t at) -> int {
+        int go = -1;
+        if constexpr (SKIP) {
+            const int in = at < all ? -1 : 0;
+            asm("s_nop 1\n\tv_readfirstlane_b32 %0, %1" : "=s"(go) : "v"(in));
+        }
+        return go;
+    };
 #pragma unroll
-    for (int k = 0; k < L::N_W; ++k) request_w(k);
+    for (int k = 0; k < L::N_W; ++k) request_w(k, -1);
     next_w(0, 0);
 
     if (rec) {
@@ -428,13 +462,18 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     // (a scalar register each: the compiler would keep such a choice in a vector register)
     asm("s_nop 1\n\tv_readfirstlane_b32 %0, %1" : "=s"(s_lanes) : "v"(s_lanes));
     asm("s_nop 1\n\tv_readfirstlane_b32 %0, %1" : "=s"(i_lanes) : "v"(i_lanes));
-    auto request_x = [&](uint32_t ring, int i, int step) {   // piece i, which moves on by `step` bytes
-        lds_dma16(lds0 + ring * L::X_HALF + (wave * TT + i) * 1024u, xp[i]);
+    auto request_x = [&](uint32_t ring, int i, int step, int go) {   // piece i, which moves on by `step` bytes
+        lds_dma16<SKIP>(lds0 + ring * L::X_HALF + (wave * TT + i) * 1024u, xp[i], go);
         xp[i] += step;
     };
-    auto request_s = [&](uint32_t buf, int step) {   // step: superblocks
-        if constexpr (!Q6) lds_dma16(lds0 + L::V_AT + buf * L::V_BUF + (wave & 1u) * 1024u, vp, s_lanes);
-        lds_dma4(lds0 + L::I_AT + buf * L::I_BUF, (const void*)ip, i_lanes);
+    auto request_s = [&](uint32_t buf, int step, int go) {   // step: superblocks
+        if constexpr (SKIP) {
+            if constexpr (!Q6) lds_dma16<true>(lds0 + L::V_AT + buf * L::V_BUF + (wave & 1u) * 1024u, vp, s_lanes & go);
+            lds_dma4<true>(lds0 + L::I_AT + buf * L::I_BUF, (const void*)ip, i_lanes & go);
+        } else {
+            if constexpr (!Q6) lds_dma16_or_none(lds0 + L::V_AT + buf * L::V_BUF + (wave & 1u) * 1024u, vp, s_lanes);
+            lds_dma4_or_none(lds0 + L::I_AT + buf * L::I_BUF, (const void*)ip, i_lanes);
+        }
         vp += step * (int)WIDE_XV;
         ip += step;
     };
@@ -606,16 +645,17 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    request_s(0, s_step(0, 0));
+    request_s(0, s_step(0, 0), -1);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int i = 0; i < TT; ++i) request_x(h, i, h == 0 ? 256 : x_step(0, 0));
+        for (int i = 0; i < TT; ++i) request_x(h, i, h == 0 ? 256 : x_step(0, 0), -1);
     wide_meet<TT>();
     read_w();
     w[0].arrived(); w[1].arrived();
+    int go = there(1);   // is there a superblock behind the one under way
 #pragma unroll
-    for (int k = 0; k < WAS; ++k) request_w(k);
+    for (int k = 0; k < WAS; ++k) request_w(k, go);
     headers();
     read_a(0, 0);
     expand(0);
@@ -677,14 +717,16 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     for (uint32_t at = 0; at < all; ++at) {
         const uint32_t ring1 = ring + 1u == 3u ? 0u : ring + 1u, ring2 = ring == 0u ? 2u : ring - 1u;
         const uint32_t sb1 = wrap(sb);   // number of the superblock behind this one in its group
+        const int go2 = there(at + 2u);
         add_up(at == 0u ? 0u : (at - 1u) & 1u);   // of the superblock before (a group's last is done: nothing)
         headers2();
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
             if (j == 3) {
                 // every wave has read the first half; the second has arrived
+                if constexpr (SKIP) wide_drain_unless(go);
                 wide_meet<TT + L::N_W>();
-                request_s((at + 1u) & 1u, s_step(at + 1u, sb1));
+                request_s((at + 1u) & 1u, s_step(at + 1u, sb1), go);
                 read_a(ring1, 4);
                 expand(4);
             } else if (j == 7) {
@@ -693,7 +735,7 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
                 read_a(ring2, 0);
                 w[0].arrived(); w[1].arrived();
 #pragma unroll
-                for (int k = 0; k < WAS; ++k) request_w(k);
+                for (int k = 0; k < WAS; ++k) request_w(k, go2);
                 headers();
                 expand(0);
             } else {
@@ -702,14 +744,14 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
                 if (j < 3) {
 #pragma unroll
                     for (int k = (j + 1) * WAS; k < (j + 2) * WAS && k < TT + L::N_W; ++k) {
-                        if (k < L::N_W) request_w(k);
-                        else request_x(ring2, k - L::N_W, 256);
+                        if (k < L::N_W) request_w(k, go);
+                        else request_x(ring2, k - L::N_W, 256, go);
                     }
                 }
             }
             if (j >= 3 && j < 7) {
 #pragma unroll
-                for (int i = (j - 3) * XBS; i < (j - 2) * XBS && i < TT; ++i) request_x(ring, i, x_step(at + 1u, sb1));
+                for (int i = (j - 3) * XBS; i < (j - 2) * XBS && i < TT; ++i) request_x(ring, i, x_step(at + 1u, sb1), go);
             }
             multiply(j);
             if (j == 0) __builtin_amdgcn_sched_barrier(0);   // (with the scaling of the superblock before: the compiler's own order)
@@ -731,6 +773,7 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
         }
         sb = sb1;
         ring = ring2;
+        go = go2;
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in LDS that is no longer this workgroup's
     if (p.n_splits == 1u) return;

@@ -590,3 +590,24 @@ def test_rows_farther_apart_than_32_bit_offsets_reach(gpu, kqo, type_, M):  # no
             capi.force_kernel(0)
     del data, far
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("type_", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("M,blocks", [(1, 1), (16, 1), (9, 2), (16, 3), (16, 4), (16, 6)])
+def test_walks_of_few_superblocks_at_16_tokens(gpu, kqo, type_, M, blocks):  # noqa: F811
+    """Nothing is requested past the end of the walk: every place in the ring as the last one, K in one piece and cut into walks of
+    one superblock."""
+    from backpack_amd import capi, kquant
+    N, K = 270, 256 * blocks
+    raw, packed, w = gpu.make_weight(type_, N, K, seed=blocks)
+    X = np.random.default_rng(M).standard_normal((M, K)).astype(np.float32)
+    capi.force_kernel(8)
+    try:
+        for splits in (1, blocks):
+            capi.set_option("gemv_splits", splits)
+            got = kquant.matmul(gpu.dev(X), w).cpu().numpy()
+            assert capi.last_form() == "many_token"
+            gpu.check_matmul(kqo, type_, got, X, packed, N, K, label="walk", slack=1e-5)
+    finally:
+        capi.force_kernel(0)
+        capi.set_option("gemv_splits", 0)
