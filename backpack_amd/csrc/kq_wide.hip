@@ -185,12 +185,14 @@ struct WideParams {
     // pair's X row is itself (x_per_slot) or pair / k_slots, its Y row the pair.  How many groups of rows a workgroup walks is chosen
     // here, when the number of records is known (a round more than the choice counted on costs as much as all of them: 129
     // records of which 128 were expected, three groups each, 334 us instead of 206): wgs_of[c - 1] workgroups to a record at c
-    // groups, `walk` us per group, `start` beside them, each for one workgroup per CU and for more
+    // groups, `walk` us per group, `start` beside them.  Records of 16 pairs: one group, always.  Over 2069 such layers that was
+    // 2 % ahead of the choice, which was the better one by 3 % on 2 % of them, and the choice itself takes 0.8 us at a workgroup's
+    // start (3 tokens, 4 experts x 2, 256 / 512: 23.4 us for the layer with it, 22.5 without).
     const uint32_t* records;
     const uint32_t* n_records;
     uint32_t record_words, k_slots;
     uint32_t wgs_of[WIDE_MAX_GROUPS];
-    float cus, walk[2], start[2];
+    float per_cu, walk, start;
     int x_per_slot;
 };
 
@@ -342,15 +344,17 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
         const uint32_t records = *p.n_records;
         bx += gridDim.x * blockIdx.y;
         uint32_t wgs = p.wgs_of[0];
-        float best = 3e38f;
+        if constexpr (TT > 1) {   // (of 16 pairs: one group each)
+            float best = 3e38f;
 #pragma unroll
-        for (int c = 1; c <= WIDE_MAX_GROUPS; ++c) {
-            const float n = ceilf((float)(p.wgs_of[c - 1] * records) / p.cus);
-            const float us = fmaxf(n, 1.0f) * ((float)c * (n > 1.0f ? p.walk[1] : p.walk[0]) + (n > 1.0f ? p.start[1] : p.start[0]));
-            if (us < best) { best = us; per_wg = (uint32_t)c; wgs = p.wgs_of[c - 1]; }
+            for (int c = 1; c <= WIDE_MAX_GROUPS; ++c) {
+                const float n = fmaxf(ceilf(((float)(p.wgs_of[c - 1] * records) - 0.5f) * p.per_cu), 1.0f);
+                const float us = n * ((float)c * p.walk + p.start);
+                if (us < best) { best = us; per_wg = (uint32_t)c; wgs = p.wgs_of[c - 1]; }
+            }
+            per_wg = (uint32_t)__builtin_amdgcn_readfirstlane((int)per_wg);
+            wgs = (uint32_t)__builtin_amdgcn_readfirstlane((int)wgs);
         }
-        per_wg = (uint32_t)__builtin_amdgcn_readfirstlane((int)per_wg);
-        wgs = (uint32_t)__builtin_amdgcn_readfirstlane((int)wgs);
         const uint32_t all = records * wgs, share = (all + 7u) >> 3, at = (bx & 7u) * share + (bx >> 3);
         if ((bx >> 3) >= share || at >= all) return;   // whole workgroup
         const uint32_t record = at / wgs;
@@ -367,13 +371,13 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     }
     constexpr uint32_t BB = TYPE == KQ_TYPE_Q4_K ? KQ_Q4K_BYTES : TYPE == KQ_TYPE_Q5_K ? KQ_Q5K_BYTES : KQ_Q6K_BYTES;
     const uint32_t b0 = blockIdx.z * p.blocks_per_split, b1 = min(b0 + p.blocks_per_split, p.n_blocks);
-    // The slots' rows of Y and X, a copy per wave (no meeting).  A record's go straight into LDS: the first weights are requested
-    // behind them and are under way while the rows are turned into addresses.  Slots beyond the count repeat the last: their
-    // outputs are dropped.
+    // The slots' rows of Y and X, a copy per wave (no meeting).  A record's go straight into LDS, all its words (those beyond the
+    // count have no meaning: no wait for the count); the first weights are requested behind them and are under way while the
+    // rows are turned into addresses.  Slots beyond the count repeat the last slot's X: their outputs are dropped.
     uint32_t* const out_rows = (uint32_t*)(lds + L::R_AT + wave * (TT * 128u));
     uint32_t* const x_rows = out_rows + TT * 16u;
-    const uint32_t slot0 = min(lane, min(count, TT * 16u) - 1u);
-    if (rec) lds_dma4<false>(lds0 + L::R_AT + wave * (TT * 128u), (const uint8_t*)rec, slot0 * 4u, TT == 4 ? ~0ull : (1ull << (TT * 16u % 64u)) - 1ull, -1);
+    const uint32_t last = min(count, TT * 16u) - 1u;
+    if (rec) lds_dma4<false>(lds0 + L::R_AT + wave * (TT * 128u), (const uint8_t*)rec, lane * 4u, TT == 4 ? ~0ull : (1ull << (TT * 16u % 64u)) - 1ull, -1);
 
     // W: the wave's two tiles of 16 rows, unit after unit.  The last rows of a matrix that does not fill its tiles are read from
     // N - 16 on (what a tile has of an earlier one is not stored), so a lane's offsets are the same for every tile.
@@ -443,9 +447,10 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
 
     if (rec) {
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"(L::N_W) : "memory");   // the record's words
-        if (lane < TT * 16u) x_rows[lane] = p.x_per_slot ? out_rows[lane] : out_rows[lane] / p.k_slots;
+        const uint32_t pair = out_rows[min(lane, last)];
+        if (lane < TT * 16u) x_rows[lane] = p.x_per_slot ? pair : pair / p.k_slots;
     } else if (lane < TT * 16u) {
-        out_rows[lane] = x_rows[lane] = t0 + slot0;
+        out_rows[lane] = x_rows[lane] = t0 + min(lane, last);
     }
     // X: load i of the wave takes half a superblock of two tokens
     const uint8_t* xp[TT];
@@ -874,7 +879,7 @@ bool wide_supported(const MatmulArgs& a)
 // CU: a step of one takes half the two's, and its start goes under the other's walk; alone on it a workgroup is a sixth
 // slower than that (too few bytes under way).
 // Measured, us, with one group / with those chosen: 128 experts x 8, 2048 / 768, gate and up, then down: 256 tokens (3, 4) 77 / 73
-// and 80 / 68, 2048 tokens (2, 2) 295 / 285 and 255 / 233, 24 tokens (1, 2) 52 / 52 (two groups 61, three 56) and 51.5 / 49.
+// and 80 / 68, 2048 tokens (2, 2) 295 / 285 and 255 / 233.
 struct WideWalk { double walk[2], start[2]; };
 static WideWalk wide_walk(int type, uint32_t tt, uint32_t blocks)
 {
@@ -965,15 +970,15 @@ hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32
     p.W = a.W; p.W2 = a.W2 ? a.W2 : a.W;
     p.Y = a.Y;
     p.M = a.M; p.N = a.N; p.n_blocks = a.n_blocks; p.row_stride_bytes = a.row_stride_bytes; p.ldy = a.ldy;
-    p.n_splits = 1; p.blocks_per_split = a.n_blocks;
+    p.n_splits = 1; p.blocks_per_split = a.n_blocks; p.per_wg = 1;
     p.act = a.W2 ? 2 : 0;
     p.records = records; p.n_records = n_records; p.record_words = 2u + cap; p.k_slots = a.k_slots; p.x_per_slot = a.x_per_slot;
     const uint32_t per_wg = a.W2 ? WIDE_WAVES * 16u : WIDE_WAVES * 32u;
     p.row_groups = (a.N + per_wg - 1u) / per_wg;
     const uint32_t tt = cap / 16u;
     const WideWalk w = wide_walk(a.type, tt, a.n_blocks);
-    p.cus = (float)device_cu_count();
-    for (int i = 0; i < 2; ++i) { p.walk[i] = (float)w.walk[i]; p.start[i] = (float)w.start[i]; }
+    p.per_cu = 1.0f / (float)device_cu_count();
+    p.walk = (float)w.walk[0]; p.start = (float)w.start[0];
     for (uint32_t c = 1; c <= WIDE_MAX_GROUPS; ++c) p.wgs_of[c - 1u] = (p.row_groups + c - 1u) / c;
     // (a dimension of the grid holds fewer than 2^32 threads; its first one a multiple of the XCDs)
     const uint64_t wgs = ((uint64_t)p.row_groups * bound + 7u) / 8u * 8u, gx = wgs < (1u << 22) ? wgs : (1u << 22);

@@ -507,29 +507,42 @@ def test_dispatch_of_expert_layers_with_few_workgroups(gpu, kqo, tgu, tdn, E, k,
 @pytest.mark.parametrize("extra", [0, 1, 40])
 def test_moe_records_around_a_round(gpu, kqo, extra):  # noqa: F811
     """64 records, or a few more: the number of row groups that a workgroup walks is chosen on the device from the records'
-    number (64 x 4 workgroups are a round of 256 CUs).  All tokens against the 16-token tile kernel."""
+    number.  Gate and up have 14 groups: four each at 64 records (64 x 4 workgroups are a round of 256 CUs, the last of a
+    record's walks two), five from 65 on, seven at 104.  Some tokens in 64 bits, all against the 16-token tile kernel."""
     from backpack_amd import capi, kquant
-    E, k, H, I = 64, 2, 512, 1536
-    _, gp, gw = gpu.make_weight(Q4_K, E * I, H, seed=41)
-    _, up, uw = gpu.make_weight(Q4_K, E * I, H, seed=42)
-    _, dp, dw = gpu.make_weight(Q6_K, E * H, I, seed=43)
+    E, k, H, I, cap = 64, 2, 512, 1792, 32
+    raw_g, _, gw = gpu.make_weight(Q4_K, E * I, H, seed=41)
+    raw_u, _, uw = gpu.make_weight(Q4_K, E * I, H, seed=42)
+    raw_d, _, dw = gpu.make_weight(Q6_K, E * H, I, seed=43)
     rng = np.random.default_rng(extra)
-    eidx = np.tile(np.arange(E, dtype=np.uint32).repeat(16), 1)          # 16 pairs per expert
-    eidx = np.concatenate([eidx, np.arange(extra, dtype=np.uint32) % E, np.arange(extra, dtype=np.uint32) % E])
+    counts = np.array([33] * extra + [24] * (E - extra))            # 33 pairs take two records
+    counts[-1] += counts.sum() % k
+    eidx = np.repeat(np.arange(E, dtype=np.uint32), counts)
     T = len(eidx) // k
-    eidx = eidx[: T * k].reshape(k, T).T.copy()
+    eidx = eidx.reshape(k, T).T.copy()
+    records = int(sum((c + cap - 1) // cap for c in np.bincount(eidx.reshape(-1), minlength=E)))
+    assert records == 64 + extra
     ew = rng.random((T, k)).astype(np.float32)
     X = (rng.standard_normal((T, H)) * 0.1).astype(np.float32)
     args = (gpu.dev(X), gw, uw, dw, gpu.dev(eidx.view(np.int32)), gpu.dev(ew), E)
-    capi.force_kernel(8)
+    got = kquant.moe_ffn(*args).cpu().numpy()
+    assert capi.last_form() == f"records_{cap}"
+    capi.force_kernel(6)
     try:
-        got = kquant.moe_ffn(*args).cpu().numpy()
-        capi.force_kernel(6)
         tile = kquant.moe_ffn(*args).cpu().numpy()
     finally:
         capi.force_kernel(0)
     rms = float(np.sqrt(np.mean(tile.astype(np.float64) ** 2)))
     assert np.abs(got - tile).max() <= 1e-4 * rms + 1e-4 * np.abs(tile).max()
+    for t in rng.choice(T, 12, replace=False):
+        want = np.zeros(H)
+        for s in range(k):
+            e = int(eidx[t, s])
+            g = kqo.dequant(Q4_K, raw_g[e * I:(e + 1) * I], I, H).astype(np.float64) @ X[t]
+            u = kqo.dequant(Q4_K, raw_u[e * I:(e + 1) * I], I, H).astype(np.float64) @ X[t]
+            want += float(ew[t, s]) * (kqo.dequant(Q6_K, raw_d[e * H:(e + 1) * H], H, I).astype(np.float64) @ (g / (1 + np.exp(-g)) * u))
+        # two products of 22-bit splits one after the other, fp32 sums, an expf
+        assert np.abs(got[t] - want).max() <= 2.0 ** -15 * rms, float(np.abs(got[t] - want).max()) / rms
 
 
 @pytest.mark.parametrize("type_,M,N,K,form", [(Q6_K, 3, 128256, 256, "many_token"), (Q6_K, 8, 61500, 1024, "many_token"), (Q4_K, 5, 128257, 512, "many_token"),
