@@ -875,16 +875,18 @@ bool wide_supported(const MatmulArgs& a)
 }
 
 // Groups of rows that a workgroup walks one after the other are chosen by a launch's price in us: the busiest CU's workgroups,
-// at `walk` per group and `start` beside them, [0] for one workgroup per CU, [1] for more.  At 16 tokens two workgroups share a
-// CU: a step of one takes half the two's, and its start goes under the other's walk; alone on it a workgroup is a sixth
-// slower than that (too few bytes under way).
+// at `walk` per group and `start` beside them, [0] for one alone on its CU, [1] for two that share it.  At 16 tokens two
+// workgroups do: a step of one takes half the two's, and its start goes under the other's walk; alone on it — all of one round,
+// the odd one of several — a workgroup is a sixth slower than that (too few bytes under way).  Of 3730 dense calls of 9 to
+// 16 tokens on 61441 to 262144 rows this choice is 0.3 % behind the best of one to four groups (priced without the odd one
+// apart 0.9 %, by up to 16 %: Q5_K 160000 x 256 at 10 tokens 16.1 us against 14.5 with three groups).
 // Measured, us, with one group / with those chosen: 128 experts x 8, 2048 / 768, gate and up, then down: 256 tokens (3, 4) 77 / 73
 // and 80 / 68, 2048 tokens (2, 2) 295 / 285 and 255 / 233.
 struct WideWalk { double walk[2], start[2]; };
 static WideWalk wide_walk(int type, uint32_t tt, uint32_t blocks)
 {
     const bool q5 = type == KQ_TYPE_Q5_K, q6 = type == KQ_TYPE_Q6_K;
-    if (tt == 1u) return {{blocks * (q6 ? 3.6 : q5 ? 2.5 : 2.1), blocks * (q6 ? 3.4 : q5 ? 2.1 : 1.75)}, {9.0, 4.0}};
+    if (tt == 1u) return {{blocks * (q6 ? 3.6 : q5 ? 2.5 : 2.1), blocks * (q6 ? 3.4 : q5 ? 2.1 : 1.75)}, {6.0, 3.0}};
     const double step = q6 ? 2.4 + 0.9 * tt : 0.8 + 0.8 * tt;
     return {{blocks * step, blocks * step}, {9.0, 9.0}};
 }
@@ -897,7 +899,7 @@ static uint32_t groups_per_wg(uint32_t row_groups, uint32_t others, int type, ui
     double best_us = 1e30;
     for (uint32_t c = 1; c <= row_groups && c <= 64u; ++c) {
         const uint64_t n = ((uint64_t)((row_groups + c - 1u) / c) * others + cus - 1u) / cus;
-        const double us = (double)n * (c * w.walk[n > 1u] + w.start[n > 1u]);
+        const double us = (double)(n / 2u * 2u) * (c * w.walk[1] + w.start[1]) + (double)(n % 2u) * (c * w.walk[0] + w.start[0]);
         if (us < best_us) { best_us = us; best = c; }
     }
     if (price) *price = best_us;
@@ -908,7 +910,7 @@ double wide_price_16(int type, uint32_t N, uint32_t n_blocks)
 {
     double us;
     groups_per_wg((N + 255u) / 256u, 1, type, 1, n_blocks, &us);
-    return us + 3.0;   // (the split of X in front)
+    return us + 4.0;   // (the split of X in front)
 }
 
 hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scratch, size_t x_bytes, int splits, hipStream_t s)

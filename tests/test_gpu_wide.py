@@ -624,3 +624,18 @@ def test_walks_of_few_superblocks_at_16_tokens(gpu, kqo, type_, M, blocks):  # n
     finally:
         capi.force_kernel(0)
         capi.set_option("gemv_splits", 0)
+
+
+@pytest.mark.parametrize("type_,M,N,K", [(Q4_K, 9, 256 * 601 + 3, 256), (Q5_K, 16, 256 * 513 + 1, 512), (Q6_K, 12, 256 * 767, 256)])
+def test_three_row_groups_per_workgroup_at_16_tokens(gpu, kqo, type_, M, N, K):  # noqa: F811
+    """Between two and three rounds of 256 rows per CU: workgroups of three groups, the last one ragged.  Windows of rows around the
+    workgroups' borders against the oracle."""
+    from backpack_amd import capi, kquant, synth
+    print("three groups", type_, M, N, K, flush=True)
+    raw, packed, w = gpu.make_weight(type_, N, K, seed=M)
+    X = np.random.default_rng(N).standard_normal((M, K)).astype(np.float32)
+    got = kquant.matmul(gpu.dev(X), w).cpu().numpy()
+    assert (capi.last_kernel(), capi.last_form()) == ("mtile", "many_token")
+    words = synth.row_stride_words(type_, K)
+    for a, b in ((0, 300), (768 * 100 - 20, 768 * 100 + 300), (N - 900, N)):
+        gpu.check_matmul(kqo, type_, np.ascontiguousarray(got[:, a:b]), X, packed[a * words:b * words], b - a, K, label="three groups", slack=1e-5)
