@@ -21,9 +21,9 @@ namespace kq {
 // first pairs of a thread stay in registers until the records' places are known; the first record of
 // every expert comes from a scan over the workgroup (eight experts per thread, a wave scan, the waves'
 // totals through LDS) instead of one thread walking all experts.
-// KEEP: pairs per thread kept in registers (more are read again, one dependent load after the other: 16384 pairs took 17.5 us
-// with 4 kept, 14 with all of them; up to 4096 pairs the short form is 0.7 us ahead).
-template <int KEEP>
+// KEEP: pairs per thread kept in registers; MORE: there may be others, which are read again, one dependent load after the other
+// (16384 pairs took 17.5 us with 4 kept, 14 with all of them; up to 4096 pairs the short form is 0.7 us ahead).
+template <int KEEP, bool MORE>
 __global__ __launch_bounds__(1024) void moe_group_kernel(const uint32_t* __restrict__ expert_idx, uint32_t n_pairs,
                                                          uint32_t n_experts, uint32_t cap, uint32_t* __restrict__ tiles,
                                                          uint32_t* __restrict__ n_tiles)
@@ -51,7 +51,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const uint32_t* __restr
         if (my_e[i] < n_experts) my_pos[i] = atomicAdd(&count[my_e[i]], 1u);   // out-of-range ids are dropped
     }
     __syncthreads();
-    const bool more = n_pairs > KEEP * 1024u;   // (uniform)
+    const bool more = MORE && n_pairs > KEEP * 1024u;   // (uniform)
     if (more) {
         // pairs beyond the kept ones: counted now, placed behind the kept ones by a second read below
         for (uint32_t e = tid; e < n_experts; e += 1024u) fill[e] = count[e];
@@ -213,10 +213,10 @@ hipError_t launch_moe_group(const uint32_t* expert_idx, uint32_t n_pairs, uint32
 {
     if (n_experts > 8192u) return hipErrorInvalidValue;   // three LDS arrays of n_experts words, eight experts per thread
     if (n_pairs <= 4096u)
-        hipLaunchKernelGGL(moe_group_kernel<4>, dim3(1), dim3(1024), 3 * n_experts * sizeof(uint32_t), s, expert_idx, n_pairs,
+        hipLaunchKernelGGL((moe_group_kernel<4, false>), dim3(1), dim3(1024), 3 * n_experts * sizeof(uint32_t), s, expert_idx, n_pairs,
                            n_experts, 2u * (uint32_t)sets, tiles, n_tiles);
     else
-        hipLaunchKernelGGL(moe_group_kernel<16>, dim3(1), dim3(1024), 3 * n_experts * sizeof(uint32_t), s, expert_idx, n_pairs,
+        hipLaunchKernelGGL((moe_group_kernel<16, true>), dim3(1), dim3(1024), 3 * n_experts * sizeof(uint32_t), s, expert_idx, n_pairs,
                            n_experts, 2u * (uint32_t)sets, tiles, n_tiles);
     return hipGetLastError();
 }

@@ -810,12 +810,13 @@ def test_moe_matmul_grouped_ragged(gpu, kqo, type_, N, K, per_slot, family, kern
     assert np.all(np.abs(got - want) <= 1e-3 * rms + 1e-3 * np.abs(want))
 
 
-def test_moe_matmul_grouped_many_pairs(gpu, kqo):
-    """More pairs than the grouping pass keeps in registers (4 per thread of its one workgroup): the rest are
-    counted first and placed behind the kept ones by a second read."""
+@pytest.mark.parametrize("T", [1100, 4203])
+def test_moe_matmul_grouped_many_pairs(gpu, kqo, T):
+    """More pairs than the grouping pass's short form keeps in registers (4 per thread of its one workgroup), and more than the
+    long one does (16): the rest are counted first and placed behind the kept ones by a second read."""
     from backpack_amd import capi, kquant
     type_, N, K = Q4_K, 128, 256
-    E, T, k = 20, 1100, 4
+    E, k = 20, 4
     raw, packed, w = gpu.make_weight(type_, E * N, K, seed=71)
     rng = np.random.default_rng(72)
     eidx = rng.integers(0, E, size=(T, k)).astype(np.uint32)

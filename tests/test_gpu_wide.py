@@ -639,3 +639,24 @@ def test_three_row_groups_per_workgroup_at_16_tokens(gpu, kqo, type_, M, N, K): 
     words = synth.row_stride_words(type_, K)
     for a, b in ((0, 300), (768 * 100 - 20, 768 * 100 + 300), (N - 900, N)):
         gpu.check_matmul(kqo, type_, np.ascontiguousarray(got[:, a:b]), X, packed[a * words:b * words], b - a, K, label="three groups", slack=1e-5)
+
+
+@pytest.mark.parametrize("k", [8, 9, 11])
+def test_moe_ffn_of_more_than_eight_slots(gpu, kqo, k):  # noqa: F811
+    """The sum over a token's slots takes them eight at a time: exactly eight, one and three more."""
+    from backpack_amd import capi, kquant
+    T, E, H, I = 30, 16, 768, 256
+    print("slots", k, flush=True)
+    _, gp, gw = gpu.make_weight(Q4_K, E * I, H, seed=61)
+    _, up, uw = gpu.make_weight(Q4_K, E * I, H, seed=62)
+    _, dp, dw = gpu.make_weight(Q5_K, E * H, I, seed=63)
+    rng = np.random.default_rng(k)
+    eidx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32)
+    ew = rng.random((T, k)).astype(np.float32)
+    X = (rng.standard_normal((T, H)) * 0.1).astype(np.float32)
+    got = kquant.moe_ffn(gpu.dev(X), gw, uw, dw, gpu.dev(eidx.view(np.int32)), gpu.dev(ew), E).cpu().numpy()
+    assert capi.last_form().startswith("records_")
+    want = kqo.moe_ffn(Q4_K, Q5_K, X, gp, up, dp, eidx, ew, H, I)
+    rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
+    # (a slot left out or counted twice is off by a third of the rms)
+    assert np.all(np.abs(got - want) <= 1e-3 * rms + 1e-3 * np.abs(want))
