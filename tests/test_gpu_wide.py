@@ -660,3 +660,79 @@ def test_moe_ffn_of_more_than_eight_slots(gpu, kqo, k):  # noqa: F811
     rms = float(np.sqrt(np.mean(want.astype(np.float64) ** 2)))
     # (a slot left out or counted twice is off by a third of the rms)
     assert np.all(np.abs(got - want) <= 1e-3 * rms + 1e-3 * np.abs(want))
+
+
+def _q6_of_the_whole_range(gpu, N, K, seed):
+    """A Q6_K matrix with scales over the whole of int8 and quants over all 64 values: (packed, w, exact weights, weights with
+    scale * (q - 32) rounded to fp16, as a kernel without the third product would multiply them)."""
+    from backpack_amd import kquant, synth
+    rng = np.random.default_rng(seed)
+    d, _, q = synth.q6k_fields(rng, N, K // 256)
+    sc = rng.integers(-128, 128, size=(N, K // 256, 16), dtype=np.int8)
+    sc[:, :, 0], sc[:, :, 5] = -128, 127                      # (products of up to 13 bits: 128 * 32)
+    q.reshape(-1)[::97] = 0
+    packed = synth.pack_rows(synth.Q6_K, synth.q6k_encode(d, sc, q).reshape(N, -1), N, K)
+    exact = synth.q6k_decode_f64(d, sc, q)
+    dd = np.repeat(d.astype(np.float64).reshape(N, -1), 256, axis=1)
+    dd[dd == 0.0] = 1.0
+    coarse = (exact / dd).astype(np.float16).astype(np.float64) * dd
+    return packed, kquant.upload(synth.Q6_K, packed, N, K), exact, coarse
+
+
+# tiles of 16 tokens one to four; few tokens on many rows (by itself); K cut into walks of a superblock and in one piece
+@pytest.mark.parametrize("M,N,K,splits", [(16, 257, 1280, 0), (17, 300, 512, 1), (33, 270, 1024, 0), (64, 256, 768, 1), (100, 130, 2816, 0), (5, 61500, 512, 0)])
+def test_q6_scales_of_the_whole_range(gpu, kqo, M, N, K, splits):  # noqa: F811
+    """Beyond 2048 scale * (q - 32) needs the third product: against 64 bits, with a limit that weights rounded to fp16 exceed."""
+    from backpack_amd import capi, kquant
+    print("q6 range", M, N, K, splits, flush=True)
+    packed, w, exact, coarse = _q6_of_the_whole_range(gpu, N, K, seed=M)
+    X = np.random.default_rng(K).standard_normal((M, K)).astype(np.float32)
+    if M > 8:
+        capi.force_kernel(8)
+    capi.set_option("gemv_splits", splits)
+    try:
+        got = kquant.matmul(gpu.dev(X), w).cpu().numpy()
+    finally:
+        capi.force_kernel(0)
+        capi.set_option("gemv_splits", 0)
+    assert capi.last_form() == "many_token"
+    want, bad = X.astype(np.float64) @ exact.T, X.astype(np.float64) @ coarse.T
+    rms = float(np.sqrt(np.mean(want ** 2)))
+    # x keeps 22 bits of its superblock's largest, lo * Wl (2^-22 of a product) is dropped, sums in fp32 over chains of up to 8 + K / 256
+    # instructions: 2^-17 of the rms is above all of them together
+    limit = 2.0 ** -17 * rms
+    assert float(np.abs(got - want).max()) <= limit, float(np.abs(got - want).max()) / rms
+    assert float(np.abs(bad - want).max()) > 20 * limit
+
+
+@pytest.mark.parametrize("T,cap", [(30, 16), (300, 48)])
+def test_moe_ffn_q6_scales_of_the_whole_range(gpu, T, cap):  # noqa: F811
+    """The same in both launches of an expert layer, on records of 16 and of more pairs, against 64 bits."""
+    from backpack_amd import capi, kquant
+    E, k, H, I = 4, 2, 512, 512
+    print("moe q6 range", T, flush=True)
+    _, gw, g64, g16 = _q6_of_the_whole_range(gpu, E * I, H, 1)
+    _, uw, u64, u16 = _q6_of_the_whole_range(gpu, E * I, H, 2)
+    _, dw, d64, d16 = _q6_of_the_whole_range(gpu, E * H, I, 3)
+    rng = np.random.default_rng(T)
+    eidx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32)
+    ew = rng.random((T, k)).astype(np.float32)
+    X = (rng.standard_normal((T, H)) * 0.01).astype(np.float32)
+    got = kquant.moe_ffn(gpu.dev(X), gw, uw, dw, gpu.dev(eidx.view(np.int32)), gpu.dev(ew), E).cpu().numpy()
+    assert capi.last_form() == f"records_{cap}"
+
+    def layer(g, u, d):
+        out = np.zeros((T, H))
+        for e in range(E):
+            t, s = np.nonzero(eidx == e)
+            x = X[t].astype(np.float64)
+            gate, up = x @ g[e * I:(e + 1) * I].T, x @ u[e * I:(e + 1) * I].T
+            np.add.at(out, t, ew[t, s].astype(np.float64)[:, None] * ((gate / (1 + np.exp(-gate)) * up) @ d[e * H:(e + 1) * H].T))
+        return out
+    want = layer(g64, u64, d64)
+    rms = float(np.sqrt(np.mean(want ** 2)))
+    # two products as above one after the other, gate's error through silu (slope up to 1.1, beside |gate| of the rms's size) and expf's
+    limit = 2.0 ** -16 * rms
+    assert float(np.abs(got - want).max()) <= limit, float(np.abs(got - want).max()) / rms
+    for planted in (layer(g16, u16, d64), layer(g64, u64, d16)):
+        assert float(np.abs(planted - want).max()) > 5 * limit
