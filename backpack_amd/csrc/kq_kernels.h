@@ -27,6 +27,7 @@ struct MatmulArgs {
     const uint8_t* W2;
     float* Y2;
     const float* X2;
+    uint32_t grid_x;       // many-token kernel over records: workgroups in the grid's first dimension (0: up to 2^22)
     uint32_t tile_iters;   // grouped tile launch of one chunk of K: tiles a wave walks with X staged once (0: chosen by the launcher)
     // fused forms of the dense decode matvec, honoured by the lanes-along-K launch only (other launches
     // must be given pro == 0 and residual == nullptr): pro 1 = RMSNorm of the X row with weight norm_w,

@@ -983,8 +983,10 @@ hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32
     p.walk = (float)w.walk[0]; p.start = (float)w.start[0];
     for (uint32_t c = 1; c <= WIDE_MAX_GROUPS; ++c) p.wgs_of[c - 1u] = (p.row_groups + c - 1u) / c;
     // (a dimension of the grid holds fewer than 2^32 threads; its first one a multiple of the XCDs)
-    const uint64_t wgs = ((uint64_t)p.row_groups * bound + 7u) / 8u * 8u, gx = wgs < (1u << 22) ? wgs : (1u << 22);
-    return launch_wide_any(a.type, p, tt, dim3((uint32_t)gx, (uint32_t)((wgs + gx - 1u) / gx)), s);
+    const uint64_t wgs = ((uint64_t)p.row_groups * bound + 7u) / 8u * 8u, most = a.grid_x ? a.grid_x : 1u << 22;
+    const uint64_t gx = wgs < most ? wgs : most, gy = (wgs + gx - 1u) / gx;
+    if (gy > 65535u) return hipErrorInvalidValue;
+    return launch_wide_any(a.type, p, tt, dim3((uint32_t)gx, (uint32_t)gy), s);
 }
 
 // ------------------------------------------------------------------------------------------------------------------

@@ -556,6 +556,9 @@ BPK_API int bpk_force_kernel(int family);
  * of that path walks with a record's activations staged once, where
  * K is at most four superblocks (1, 2, 4 or 8; 0 = chosen per call from the
  * expected number of records, so that the workgroups fill whole rounds);
+ * "moe_grid": workgroups in the first dimension of the many-token kernel's grid over
+ * records of pairs, a multiple of 8 (0 = up to 2^22; a hook for tests of calls that
+ * have more);
  * "chain_spin_us": bound of a wait between the ops of a chain in microseconds
  * (at most ten seconds);
  * "chain_hold" (test hook, refused unless chain_spin_us is 1..100000): 1 keeps

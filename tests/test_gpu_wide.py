@@ -736,3 +736,28 @@ def test_moe_ffn_q6_scales_of_the_whole_range(gpu, T, cap):  # noqa: F811
     assert float(np.abs(got - want).max()) <= limit, float(np.abs(got - want).max()) / rms
     for planted in (layer(g16, u16, d64), layer(g64, u64, d16)):
         assert float(np.abs(planted - want).max()) > 5 * limit
+
+
+@pytest.mark.parametrize("grid", [8, 24, 4096])
+def test_moe_records_in_a_second_dimension_of_the_grid(gpu, grid):  # noqa: F811
+    """What a launch of more than 2^22 workgroups over records does, at a size that a test can afford: the same outputs, bit for
+    bit, with the first dimension held to a few workgroups."""
+    from backpack_amd import capi, kquant
+    E, k, H, I = 6, 2, 512, 768
+    _, gp, gw = gpu.make_weight(Q4_K, E * I, H, seed=51)
+    _, up, uw = gpu.make_weight(Q4_K, E * I, H, seed=52)
+    _, dp, dw = gpu.make_weight(Q6_K, E * H, I, seed=53)
+    for T in (37, 400):
+        rng = np.random.default_rng(T)
+        eidx = np.stack([rng.permutation(E)[:k] for _ in range(T)]).astype(np.uint32)
+        args = (gpu.dev((rng.standard_normal((T, H)) * 0.1).astype(np.float32)), gw, uw, dw, gpu.dev(eidx.view(np.int32)), gpu.dev(rng.random((T, k)).astype(np.float32)), E)
+        want = kquant.moe_ffn(*args).cpu().numpy()
+        assert capi.last_form().startswith("records_")
+        capi.set_option("moe_grid", grid)
+        try:
+            got = kquant.moe_ffn(*args).cpu().numpy()
+        finally:
+            capi.set_option("moe_grid", 0)
+        assert np.array_equal(got, want)
+    with pytest.raises(capi.BpkError):
+        capi.set_option("moe_grid", 12)      # not a multiple of the XCDs
