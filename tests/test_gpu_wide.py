@@ -705,7 +705,7 @@ def test_q6_scales_of_the_whole_range(gpu, kqo, M, N, K, splits):  # noqa: F811
     assert float(np.abs(bad - want).max()) > 20 * limit
 
 
-@pytest.mark.parametrize("T,cap", [(30, 16), (300, 48)])
+@pytest.mark.parametrize("T,cap", [(30, 16), (700, 32), (1300, 48)])
 def test_moe_ffn_q6_scales_of_the_whole_range(gpu, T, cap):  # noqa: F811
     """The same in both launches of an expert layer, on records of 16 and of more pairs, against 64 bits."""
     from backpack_amd import capi, kquant
