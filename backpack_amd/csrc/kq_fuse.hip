@@ -134,7 +134,8 @@ __global__ __launch_bounds__(256) void act_mul_rows_kernel(const float* GU, uint
     const float* g = GU + (size_t)blockIdx.y * 2u * K;
     const uint32_t k = blockIdx.x * 256u + threadIdx.x;
     if (k >= K) return;
-    put_out(out, (size_t)blockIdx.y * K + k, act_of<GELU>(g[k]) * g[K + k]);
+    const float gv = g[k], uv = g[K + k];   // (both requested ahead of tanhf's branches)
+    put_out(out, (size_t)blockIdx.y * K + k, act_of<GELU>(gv) * uv);
 }
 
 // Y[m, y_offset + n] = T[m, n] + R[m, y_offset + n]   (R may be Y)
