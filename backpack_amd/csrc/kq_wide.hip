@@ -400,7 +400,7 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     set_w(group0, 0);
     const uint32_t w_lds = lds0 + L::W_AT + wave * L::W_WAVE;
     // piece k of a superblock's weights: whole loads first, then each tile's last lanes (and d)
-    constexpr bool SKIP = TT == 1;
+    constexpr bool SKIP = TT == 1 && Q6;
     auto request_w = [&](int k, int go) {
         constexpr int WHOLE = 2 * ((int)L::W_INSTR - 1);
         if (k < WHOLE) {
@@ -417,9 +417,9 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     // The walk: n_groups groups of rows against the same tokens, n_sb superblocks each, as one sequence of `all` superblocks:
     // W and X of the next group are under way while a group's outputs leave.  Half h of it is superblock h / 2.  Requested
     // ahead: X by two halves, W by one superblock (into the place it was read from), S half a superblock less.  Past the
-    // end the last is requested again — or, at 16 tokens (SKIP), nothing is: there a walk of few superblocks waits for those loads a
-    // second time before its last meeting and at its end (64 tokens, 128 experts x 8, 2048 / 768 Q4_K / Q6_K: 121.8 us without, 120.3 with it; 195998 x 768 Q4_K at 9 tokens 28.5 and 27.3).  At more
-    // tokens the walk is bound by issue, and the test for it costs as much or more (28672 x 4096 at 48 tokens 37.0 us, 38.1 with it).
+    // end the last is requested again, and waited for at the end — or, for Q6_K at 16 tokens (SKIP), nothing is.  Elsewhere the test
+    // for it costs more than the loads (means as at `schedule` below, us, without / with it: Q4_K 1.0 / 1.7 and -1.4 / -1.4, Q5_K
+    // -0.5 / 0.5 and -3.7 / -3.3, Q6_K -8.7 / -9.1 on the dense calls; 28672 x 4096 at 48 tokens 37.0 and 38.1 us).
     constexpr int WAS = (TT + L::N_W + 3) / 4, XBS = (TT + 3) / 4;   // requests per step
     const uint32_t n_sb = b1 - b0, all = n_groups * n_sb;
     auto wrap = [&](uint32_t sb) { return sb + 1u == n_sb ? 0u : sb + 1u; };
@@ -473,7 +473,6 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     };
     auto request_s = [&](uint32_t buf, int step, int go) {   // step: superblocks
         if constexpr (SKIP) {
-            if constexpr (!Q6) lds_dma16<true>(lds0 + L::V_AT + buf * L::V_BUF + (wave & 1u) * 1024u, vp, s_lanes & go);
             lds_dma4<true>(lds0 + L::I_AT + buf * L::I_BUF, (const void*)ip, i_lanes & go);
         } else {
             if constexpr (!Q6) lds_dma16_or_none(lds0 + L::V_AT + buf * L::V_BUF + (wave & 1u) * 1024u, vp, s_lanes);
@@ -640,6 +639,15 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
 
     // A step's matrix instructions with the next step's LDS reads and vector work between them
     auto schedule = [&]() {
+        // One tile: four matrix instructions a step are too few to hide the next step's LDS reads, so in the fixed order every step
+        // waits for its operands; there the compiler's own order is better (Q5_K: within a step).  Mean difference to the walk
+        // through registers that came before, us, in the fixed order / the compiler's, over layers of 1.25 .. 4 pairs per expert and
+        // over dense calls of 9 .. 16 tokens on 61441 rows and more: Q4_K 1.0 / 0.4 and -1.4 / -1.9, Q5_K -0.5 / -0.7 and -3.7 / -4.0
+        // (1.5 slower where steps may mix).
+        if constexpr (TT == 1 && !Q6) {
+            if constexpr (Q5) __builtin_amdgcn_sched_barrier(0);
+            return;
+        }
         constexpr int NM = (Q6 ? 6 : 4) * TT, NV = Q6 ? 4 : Q5 ? 4 : 2;
 #pragma unroll
         for (int i = 0; i < NM; ++i) {
@@ -780,7 +788,8 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
         ring = ring2;
         go = go2;
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in LDS that is no longer this workgroup's
+    // no load may land in LDS that is no longer this workgroup's (SKIP: none is under way since the last superblock's first meeting)
+    if constexpr (!SKIP) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (p.n_splits == 1u) return;
     // A share of K (dense calls, one group): wide_sum_kernel adds the shares' tiles.  They change hands through LDS and leave in
     // whole rows (from the accumulators, in 64-byte pieces, a 28672 x 4096 call of 48 tokens took 1.5 us more).
@@ -879,7 +888,7 @@ bool wide_supported(const MatmulArgs& a)
 // workgroups do: a step of one takes half the two's, and its start goes under the other's walk; alone on it — all of one round,
 // the odd one of several — a workgroup is a sixth slower than that (too few bytes under way).  Of 3730 dense calls of 9 to
 // 16 tokens on 61441 to 262144 rows this choice is 0.3 % behind the best of one to four groups (priced without the odd one
-// apart 0.9 %, by up to 16 %: Q5_K 160000 x 256 at 10 tokens 16.1 us against 14.5 with three groups).
+// apart 0.9 %, by up to 16 %: Q5_K 160000 x 256 at 10 tokens 16.1 us against 14.5 with three groups; 13.9 with the compiler's order).
 // Measured, us, with one group / with those chosen: 128 experts x 8, 2048 / 768, gate and up, then down: 256 tokens (3, 4) 77 / 73
 // and 80 / 68, 2048 tokens (2, 2) 295 / 285 and 255 / 233.
 struct WideWalk { double walk[2], start[2]; };
