@@ -32,8 +32,10 @@
 // stand between the matrix instructions of the step before (sched_group_barrier), and the two meetings per superblock lie
 // ahead of a step whose operands are already in registers.  What that replaced: every lane fetched its 16-byte pieces
 // of W and X itself (52 cache accesses per load instruction, 20 now) and the compiler read operands right ahead of their
-// use.  A workgroup's walk still takes 1.4 times its matrix instructions' time: a matrix instruction holds the issue for 8
-// cycles and a vector one for 4, so beside two vector instructions each they no longer overlap.
+// use.  A matrix instruction holds a SIMD's issue for 8 cycles and a vector one for 4, so beside two vector instructions each they
+// no longer overlap: in the launches of 2048 tokens (128 experts x 8, 2048 / 768, 64 pairs per record) issue takes 60 % of the
+// clocks (Q4_K; Q6_K 59 %), the matrix cores are busy 45 % (37 %); the rest are waits (0.28 and 0.31 of the waves' cycles),
+// workgroups' starts and the last round.  With one tile of 16 tokens a step is too short for the fixed order (`schedule`).
 //
 // A workgroup may walk several groups of 256 rows against the same tokens as one sequence of superblocks (groups_per_wg): its
 // start (records, addresses, the first loads' way: 8 us of 25 .. 40) is paid once and a group's stores go under the next
@@ -41,8 +43,8 @@
 //
 // Mixture layers (records of pairs of one expert): consecutive workgroups go to the same XCD, so a record's row groups
 // and an expert's records meet their X and W in that L2 (128 experts x 8 slots, 2048 / 768, 2048 tokens: 750 -> 703 us).
-// us with the router, now / with the walk before / on the 16-token tiles: 2048 tokens 592 / 734 / 1264, 256 tokens
-// 164 / 191 / 267, 24 tokens 125 / 128 / 153.
+// us with the router, now / with the walk before / on the 16-token tiles: 2048 tokens 561 / 739 / 1264, 256 tokens
+// 168 / 191 / 267, 24 tokens 123 / 128 / 153.
 #include "kq_format.h"
 #include "kq_kernels.h"
 #include "kq_wave.h"
@@ -184,7 +186,7 @@ struct WideParams {
     // grouped (records != nullptr): workgroups walk records {expert, count, pair ids ...}; W and W2 advance by N rows per expert, a
     // pair's X row is itself (x_per_slot) or pair / k_slots, its Y row the pair.  How many groups of rows a workgroup walks is chosen
     // here, when the number of records is known (a round more than the choice counted on costs as much as all of them: 129
-    // records of which 128 were expected, three groups each, 334 us instead of 206): wgs_of[c - 1] workgroups to a record at c
+    // records of which 128 were expected, three groups each, 334 us instead of 206; chosen here 201 and 203): wgs_of[c - 1] workgroups to a record at c
     // groups, `walk` us per group, `start` beside them.  Records of 16 pairs: one group, always.  Over 2069 such layers that was
     // 2 % ahead of the choice, which was the better one by 3 % on 2 % of them, and the choice itself takes 0.8 us at a workgroup's
     // start (3 tokens, 4 experts x 2, 256 / 512: 23.4 us for the layer with it, 22.5 without).
