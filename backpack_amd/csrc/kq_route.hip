@@ -322,13 +322,15 @@ hipError_t launch_route(const float* X, const float* router_w, uint32_t T, uint3
         // logits and 0.5 per 1000 of hidden for each 1024 of its workgroups.  A matrix workgroup always computes 64 experts: of few it
         // wastes most (6184 x 8 x 4608 42 tiled, 74 matrix; 4268 x 16 x 4096 48, 64; 2048 x 8 x 2048 12, 22).  tiled / matrix: 2048 x
         // 128 x 2048 46 / 22, 1024 x 128 x 2048 29 / 22, 2048 x 64 x 1024 26 / 17, 2048 x 32 x 2048 30 / 22; 512 x 128 x 1920 19 / 20 and
-        // 256 x 128 x 1792 16 / 21 stay.  Of those calls the choice is more than 3 % behind the tiled kernel on 4.
+        // 256 x 128 x 1792 16 / 21 stay.  Of those calls the choice is more than 3 % behind the tiled kernel on 4.  Up to 8 experts the
+        // prices have to be 5 % apart: of 25 such calls with less between them the matrix kernel was ahead of the other by 2 % at most
+        // and behind by up to 18 (3888 x 8 x 1024, all 8 chosen: 15.0 / 17.8).
         const uint64_t wgs = (uint64_t)((n_experts + 63u) / 64u) * ((T + 15u) / 16u), cus = device_cu_count();
         const uint64_t tiled_wgs = (uint64_t)((n_experts + 3u) / 4u) * ((T + 7u) / 8u);
         const double matrix_us = 6.0 + (double)((wgs + cus - 1u) / cus) * (1.8 + 6.7e-3 * hidden);
         const double tiled_us = 7.8 + (2.8e-8 * n_experts + 1e-6) * (double)T * hidden + 7e-5 * (double)T * n_experts +
                                 5e-4 * hidden * (double)((tiled_wgs + 1023u) / 1024u);
-        if (hidden % 128u == 0 && !(((uintptr_t)X | (uintptr_t)router_w) & 15u) && T <= 1000000u && matrix_us <= 0.97 * tiled_us) {
+        if (hidden % 128u == 0 && !(((uintptr_t)X | (uintptr_t)router_w) & 15u) && T <= 1000000u && matrix_us <= (n_experts > 8u ? 0.97 : 0.95) * tiled_us) {
             hipLaunchKernelGGL(route_logits_mfma_kernel, dim3((n_experts + 63u) / 64u, (T + 15u) / 16u), dim3(256), 0, s, X, router_w, T,
                                hidden, n_experts, lg);
             return launch_topk_softmax(lg, T, n_experts, k, normalize, idx, wt, s);

@@ -103,7 +103,7 @@ def test_route_many_tokens_on_the_matrix_instructions(gpu, T, H, E, k):
     assert np.array_equal(idx.cpu().numpy(), order)
 
 
-@pytest.mark.parametrize("T,H,E,k", [(2048, 512, 8, 2), (4113, 256, 6, 3), (4500, 512, 16, 4)])
+@pytest.mark.parametrize("T,H,E,k", [(2048, 512, 8, 2), (4113, 256, 6, 3), (4500, 512, 16, 4), (3888, 1024, 8, 8)])
 def test_route_many_tokens_of_few_experts(gpu, T, H, E, k):
     """Few experts stay on the 8-token tiles, however many tokens there are: the same bound and selection as above."""
     from backpack_amd import kquant
