@@ -329,48 +329,17 @@ template <int TYPE, int TT> struct WideLds {
     static constexpr int N_W = 2 * (int)W_INSTR + (Q6 ? 2 : 0);   // a wave's loads for its weights of a superblock
 };
 
+// A workgroup's walk: its groups of rows from group0 on against up to TT tiles of 16 tokens, t0 .. t0 + count - 1 or a record's
+// `count` pairs.
 template <int TYPE, int TT>
-__global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WideParams p)
+__device__ __forceinline__ void wide_walk(const WideParams& p, uint8_t* lds, uint32_t bx, uint32_t per_wg, const uint32_t* rec,
+                                          uint32_t t0, uint32_t count, const uint8_t* W, const uint8_t* W2)
 {
     using L = WideLds<TYPE, TT>;
     constexpr bool Q6 = TYPE == KQ_TYPE_Q6_K, Q5 = TYPE == KQ_TYPE_Q5_K;
-    __shared__ __align__(16) uint8_t lds[L::BYTES];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, kq = lane >> 4, r16 = lane & 15u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
-
-    const uint32_t* rec = nullptr;
-    uint32_t count, t0 = 0, bx = blockIdx.x, per_wg = p.per_wg;
-    const uint8_t *W = p.W, *W2 = p.W2;
-    if (p.records) {
-        const uint32_t records = *p.n_records;
-        bx += gridDim.x * blockIdx.y;
-        uint32_t wgs = p.wgs_of[0];
-        if constexpr (TT > 1) {   // (of 16 pairs: one group each)
-            float best = 3e38f;
-#pragma unroll
-            for (int c = 1; c <= WIDE_MAX_GROUPS; ++c) {
-                const float n = fmaxf(ceilf(((float)(p.wgs_of[c - 1] * records) - 0.5f) * p.per_cu), 1.0f);
-                const float us = n * ((float)c * p.walk + p.start);
-                if (us < best) { best = us; per_wg = (uint32_t)c; wgs = p.wgs_of[c - 1]; }
-            }
-            per_wg = (uint32_t)__builtin_amdgcn_readfirstlane((int)per_wg);
-            wgs = (uint32_t)__builtin_amdgcn_readfirstlane((int)wgs);
-        }
-        const uint32_t all = records * wgs, share = (all + 7u) >> 3, at = (bx & 7u) * share + (bx >> 3);
-        if ((bx >> 3) >= share || at >= all) return;   // whole workgroup
-        const uint32_t record = at / wgs;
-        bx = at - record * wgs;
-        rec = p.records + (size_t)record * p.record_words;
-        count = rec[1];
-        const size_t skip = (size_t)rec[0] * p.N * p.row_stride_bytes;
-        W += skip;
-        W2 += skip;
-        rec += 2;
-    } else {
-        t0 = blockIdx.y * (TT * 16u);
-        count = min(p.M - t0, TT * 16u);
-    }
     constexpr uint32_t BB = TYPE == KQ_TYPE_Q4_K ? KQ_Q4K_BYTES : TYPE == KQ_TYPE_Q5_K ? KQ_Q5K_BYTES : KQ_Q6K_BYTES;
     const uint32_t b0 = blockIdx.z * p.blocks_per_split, b1 = min(b0 + p.blocks_per_split, p.n_blocks);
     // The slots' rows of Y and X, a copy per wave (no meeting).  A record's go straight into LDS, all its words (those beyond the
@@ -395,8 +364,11 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     const uint8_t* wbase[2];
     auto set_w = [&](uint32_t group, uint32_t sb) {   // (no branch: the steps of the walk stay one basic block)
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
-            wbase[r] = (r && p.act ? W2 : W) + (size_t)min(tile_row(group, r), p.N - rows) * p.row_stride_bytes + (size_t)((b0 + sb) * BB);
+        for (int r = 0; r < 2; ++r) {
+            const uint64_t at = (uint64_t)((r && p.act ? W2 : W) + (size_t)min(tile_row(group, r), p.N - rows) * p.row_stride_bytes + (size_t)((b0 + sb) * BB));
+            // (scalar registers: the compiler would keep the choice of a superblock in vector registers)
+            wbase[r] = (const uint8_t*)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)at));
+        }
     };
     const uint32_t group0 = bx * per_wg, n_groups = min(per_wg, p.row_groups - group0);
     set_w(group0, 0);
@@ -735,7 +707,7 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
     uint32_t ring = 0;   // where the superblock's first half lies
     uint32_t sb = 0, group = group0;
     for (uint32_t at = 0; at < all; ++at) {
-        const uint32_t ring1 = ring + 1u == 3u ? 0u : ring + 1u, ring2 = ring == 0u ? 2u : ring - 1u;
+        const uint32_t ring1 = ring + 1u == 3u ? 0u : ring + 1u, ring2 = 3u - ring - ring1;
         const uint32_t sb1 = wrap(sb);   // number of the superblock behind this one in its group
         const int go2 = there(at + 2u);
         add_up(at == 0u ? 0u : (at - 1u) & 1u);   // of the superblock before (a group's last is done: nothing)
@@ -820,6 +792,52 @@ __global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WidePa
         *(float4*)(tile + 4u * n) = *(const float4*)(ot + (n >> 6) * OP + 4u * (n & 63u));
 }
 
+template <int TYPE, int TT>
+__global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_kernel(const WideParams p)
+{
+    __shared__ __align__(16) uint8_t lds[WideLds<TYPE, TT>::BYTES];
+    const uint32_t t0 = blockIdx.y * (TT * 16u);
+    wide_walk<TYPE, TT>(p, lds, blockIdx.x, p.per_wg, nullptr, t0, min(p.M - t0, TT * 16u), p.W, p.W2);
+}
+
+// Records of up to TT * 16 pairs: a workgroup walks the tiles that its record fills, each number of tiles with a walk of its own
+// (a branch per tile inside one would cut its steps into pieces).  An expert's last record is half empty in the mean: with all tiles
+// walked 128 experts x 8, 2048 / 768, took 555.8 / 194.1 / 154.2 us at 2048 / 512 / 256 tokens (64 / 48 / 32 pairs per record), now
+// 538.9 / 183.3 / 147.3.  Records of 48 and 64 pairs walk two tiles where one is filled: a walk for it, too, gave 0.3 % more.
+template <int TYPE, int TT>
+__global__ __launch_bounds__(512, TT == 1 ? 4 : 2) void wide_records_kernel(const WideParams p)
+{
+    __shared__ __align__(16) uint8_t lds[WideLds<TYPE, TT>::BYTES];
+    const uint32_t records = *p.n_records, bx = blockIdx.x + gridDim.x * blockIdx.y;
+    uint32_t per_wg = p.per_wg, wgs = p.wgs_of[0];
+    if constexpr (TT > 1) {   // (of 16 pairs: one group each)
+        float best = 3e38f;
+#pragma unroll
+        for (int c = 1; c <= WIDE_MAX_GROUPS; ++c) {
+            const float n = fmaxf(ceilf(((float)(p.wgs_of[c - 1] * records) - 0.5f) * p.per_cu), 1.0f);
+            const float us = n * ((float)c * p.walk + p.start);
+            if (us < best) { best = us; per_wg = (uint32_t)c; wgs = p.wgs_of[c - 1]; }
+        }
+        per_wg = (uint32_t)__builtin_amdgcn_readfirstlane((int)per_wg);
+        wgs = (uint32_t)__builtin_amdgcn_readfirstlane((int)wgs);
+    }
+    const uint32_t all = records * wgs, share = (all + 7u) >> 3, at = (bx & 7u) * share + (bx >> 3);
+    if ((bx >> 3) >= share || at >= all) return;   // whole workgroup
+    const uint32_t record = (uint32_t)__builtin_amdgcn_readfirstlane((int)(at / wgs)), group = at - record * wgs;
+    const uint32_t* rec = p.records + (size_t)record * p.record_words;
+    const uint32_t expert = (uint32_t)__builtin_amdgcn_readfirstlane((int)rec[0]), count = (uint32_t)__builtin_amdgcn_readfirstlane((int)rec[1]);
+    const size_t skip = (size_t)expert * p.N * p.row_stride_bytes;
+    const uint8_t *W = p.W + skip, *W2 = p.W2 + skip;
+    rec += 2;
+    if constexpr (TT > 2)
+        if (count <= 32u) return wide_walk<TYPE, 2>(p, lds, group, per_wg, rec, 0, count, W, W2);
+    if constexpr (TT > 3)
+        if (count <= 48u) return wide_walk<TYPE, 3>(p, lds, group, per_wg, rec, 0, count, W, W2);
+    if constexpr (TT == 2)
+        if (count <= 16u) return wide_walk<TYPE, 1>(p, lds, group, per_wg, rec, 0, count, W, W2);
+    wide_walk<TYPE, TT>(p, lds, group, per_wg, rec, 0, count, W, W2);
+}
+
 // Adds the splits' partial tiles in split order, with the call's epilogue.  Workgroup (x, y): 256 columns of four
 // tokens.  A launch of its own: added by the last workgroup of a tile to arrive, the splits were read one round
 // trip after the other by that one workgroup (19 us of a 64-token call with eight splits).
@@ -866,10 +884,14 @@ __global__ __launch_bounds__(256) void wide_sum_kernel(const WideParams p, uint3
 template <int TYPE>
 static void launch_wide_type(const WideParams& p, uint32_t tt, dim3 grid, hipStream_t s)
 {
-    if (tt == 1u) hipLaunchKernelGGL((wide_kernel<TYPE, 1>), grid, dim3(512), 0, s, p);
-    else if (tt == 2u) hipLaunchKernelGGL((wide_kernel<TYPE, 2>), grid, dim3(512), 0, s, p);
-    else if (tt == 3u) hipLaunchKernelGGL((wide_kernel<TYPE, 3>), grid, dim3(512), 0, s, p);
-    else hipLaunchKernelGGL((wide_kernel<TYPE, 4>), grid, dim3(512), 0, s, p);
+    const auto go = [&](auto dense, auto grouped) {
+        if (p.records) hipLaunchKernelGGL(grouped, grid, dim3(512), 0, s, p);
+        else hipLaunchKernelGGL(dense, grid, dim3(512), 0, s, p);
+    };
+    if (tt == 1u) go(wide_kernel<TYPE, 1>, wide_records_kernel<TYPE, 1>);
+    else if (tt == 2u) go(wide_kernel<TYPE, 2>, wide_records_kernel<TYPE, 2>);
+    else if (tt == 3u) go(wide_kernel<TYPE, 3>, wide_records_kernel<TYPE, 3>);
+    else go(wide_kernel<TYPE, 4>, wide_records_kernel<TYPE, 4>);
 }
 
 static hipError_t launch_wide_any(int type, const WideParams& p, uint32_t tt, dim3 grid, hipStream_t s)

@@ -308,6 +308,42 @@ def test_moe_ffn_records_of_32_to_64_pairs(gpu, kqo, tgu, tdn, T, H, I, cap):  #
     assert np.abs(got - tile).max() <= 1e-4 * rms + 1e-4 * np.abs(tile).max()
 
 
+@pytest.mark.parametrize("inter,cap", [(512, 32), (1024, 48), (768, 64)])
+@pytest.mark.parametrize("tgu,tdn", [(Q4_K, Q6_K), (Q5_K, Q4_K), (Q6_K, Q5_K)])
+def test_moe_ffn_records_of_every_fill(gpu, kqo, tgu, tdn, inter, cap):  # noqa: F811
+    """A workgroup walks the tiles of 16 pairs that its record fills: last records of one pair, of a tile less one, a tile, a tile
+    and one more, up to the whole record.  Every token against its expert's matvec in 64 bits."""
+    from backpack_amd import capi, kquant
+    H = 512
+    left = [n for t in range(0, cap, 16) for n in (t + 1, t + 15, t + 16)]
+    whole = {32: 8, 48: 2, 64: 2}[cap]          # full records beside each: enough pairs that records of this size are chosen
+    counts = np.array([whole * cap + n for n in left])
+    E, k = len(counts), 2
+    counts[0] += counts.sum() % k
+    print("records of every fill", tgu, tdn, inter, cap, counts.sum(), flush=True)
+    raw_g, _, gw = gpu.make_weight(tgu, E * inter, H, seed=51)
+    raw_u, _, uw = gpu.make_weight(tgu, E * inter, H, seed=52)
+    raw_d, _, dw = gpu.make_weight(tdn, E * H, inter, seed=53)
+    rng = np.random.default_rng(cap)
+    T = int(counts.sum()) // k
+    eidx = np.repeat(np.arange(E, dtype=np.uint32), counts).reshape(k, T).T.copy()
+    ew = rng.random((T, k)).astype(np.float32)
+    X = (rng.standard_normal((T, H)) * 0.1).astype(np.float32)
+    got = kquant.moe_ffn(gpu.dev(X), gw, uw, dw, gpu.dev(eidx.view(np.int32)), gpu.dev(ew), E).cpu().numpy()
+    assert capi.last_form() == f"records_{cap}"
+    want = np.zeros((T, H))
+    for e in range(E):
+        t, s = np.nonzero(eidx == e)
+        x = X[t].astype(np.float64)
+        g = x @ kqo.dequant(tgu, raw_g[e * inter:(e + 1) * inter], inter, H).astype(np.float64).T
+        u = x @ kqo.dequant(tgu, raw_u[e * inter:(e + 1) * inter], inter, H).astype(np.float64).T
+        y = (g / (1 + np.exp(-g)) * u) @ kqo.dequant(tdn, raw_d[e * H:(e + 1) * H], H, inter).astype(np.float64).T
+        np.add.at(want, t, ew[t, s, None] * y)
+    rms = float(np.sqrt(np.mean(want ** 2)))
+    # two products of 22-bit splits one after the other, fp32 sums, an expf
+    assert np.abs(got - want).max() <= 2.0 ** -15 * rms, float(np.abs(got - want).max()) / rms
+
+
 @pytest.mark.parametrize("family", [0, 6])
 def test_moe_ffn_pair_without_an_expert_adds_nothing(gpu, kqo, family):  # noqa: F811
     """Where pairs are grouped, one whose id is no expert's is dropped: its token gets the sum over its other slots,
