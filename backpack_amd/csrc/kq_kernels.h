@@ -155,6 +155,9 @@ hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scra
 WideX wide_x_layout(void* xa, void* rest, uint32_t rows, uint32_t n_blocks);
 size_t wide_x_bytes(uint32_t rows, uint32_t n_blocks);
 size_t wide_x_rest_bytes(uint32_t rows, uint32_t n_blocks);
+// launch_wide_x (no prologue) and launch_moe_group (cap pairs per record) in one launch
+hipError_t launch_wide_prepare(const uint32_t* expert_idx, uint32_t n_pairs, uint32_t n_experts, uint32_t cap, uint32_t* records,
+                               uint32_t* n_records, int type, const float* X, uint32_t rows, uint32_t n_blocks, const WideX& x, hipStream_t s);
 // x.xa may be X (no prologue): every superblock is read before it is written
 hipError_t launch_wide_x(int type, const float* X, int pro, const float* norm_w, float eps, uint32_t rows,
                          uint32_t n_blocks, const WideX& x, hipStream_t s);

@@ -46,6 +46,7 @@
 // us with the router, now / with the walk before / on the 16-token tiles: 2048 tokens 561 / 739 / 1264, 256 tokens
 // 168 / 191 / 267, 24 tokens 123 / 128 / 153.
 #include "kq_format.h"
+#include "kq_group.h"
 #include "kq_kernels.h"
 #include "kq_wave.h"
 #include <cmath>
@@ -79,6 +80,45 @@ size_t wide_x_rest_bytes(uint32_t rows, uint32_t n_blocks) { return (size_t)rows
 __device__ __forceinline__ float wide_act(int act, float g)
 {
     return act == 2 ? g / (expf(-g) + 1.0f) : 0.5f * g * (1.0f + tanhf(0.7978845608f * (g + 0.044715f * g * g * g)));
+}
+
+// Eight elements of superblock `cell` (a token's), run `sub` of its 32, split and put in operand order by the half wave that has them.
+__device__ __forceinline__ void wide_split(const float (&v)[8], uint32_t sub, size_t cell, int q6, uint8_t* xa, uint8_t* xv, float* xi)
+{
+    uint32_t amax = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = max(amax, __builtin_bit_cast(uint32_t, v[i]) & 0x7FFFFFFFu);
+#pragma unroll
+    for (int o = 1; o < 32; o <<= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, o, 32));
+    uint32_t e = amax >> 23;
+    e = e < 15u ? 15u : (e > 253u ? 253u : e);
+    const float s = __builtin_bit_cast(float, (268u - e) << 23);     // 2^(141-e): amax * s in [2^14, 2^15)
+    if (sub == 0) xi[cell] = __builtin_bit_cast(float, (e - 14u) << 23);
+    _Float16 h[8], l[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const float a = v[i] * s;
+        h[i] = (_Float16)a;
+        l[i] = (_Float16)(a - (float)h[i]);
+    }
+    // the step and lane group that take this run of eight
+    const uint32_t j = q6 ? 2u * ((sub >> 2) & 3u) + (sub & 1u) : 2u * (sub & 3u) + ((sub >> 2) & 1u);
+    const uint32_t kq = q6 ? 2u * (sub >> 4) + ((sub >> 1) & 1u) : sub >> 3;
+    uint8_t* dst = xa + cell * WIDE_XA + j * 64u + kq * 16u;
+    *(w_half8*)dst = w_half8{h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
+    *(w_half8*)(dst + 512) = w_half8{l[0], l[2], l[1], l[3], l[4], l[6], l[5], l[7]};
+    if (!q6) {
+        float t = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
+        t += group_partner<1>(t);
+        t += group_partner<2>(t);
+        if ((sub & 3u) == 0) {
+            const float a = t * (s * 0.03125f);   // 32 elements of at most 2^15 fit an fp16
+            const _Float16 th = (_Float16)a;
+            _Float16* o = (_Float16*)(xv + cell * WIDE_XV) + (sub >> 2);
+            o[0] = th;
+            o[8] = (_Float16)(a - (float)th);
+        }
+    }
 }
 
 // One workgroup: 16 superblocks of a row at a time, 32 threads each, 8 consecutive elements per thread.  pro as in
@@ -123,41 +163,7 @@ __global__ __launch_bounds__(512) void wide_x_kernel(const float* X, const float
                 v[i] = wide_act(pro, g) * u[i];
             }
         }
-        uint32_t amax = 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) amax = max(amax, __builtin_bit_cast(uint32_t, v[i]) & 0x7FFFFFFFu);
-#pragma unroll
-        for (int o = 1; o < 32; o <<= 1) amax = max(amax, (uint32_t)__shfl_xor((int)amax, o, 32));
-        uint32_t e = amax >> 23;
-        e = e < 15u ? 15u : (e > 253u ? 253u : e);
-        const float s = __builtin_bit_cast(float, (268u - e) << 23);     // 2^(141-e): amax * s in [2^14, 2^15)
-        const size_t cell = (size_t)tok * n_blocks + b;
-        if (sub == 0) xi[cell] = __builtin_bit_cast(float, (e - 14u) << 23);
-        _Float16 h[8], l[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const float a = v[i] * s;
-            h[i] = (_Float16)a;
-            l[i] = (_Float16)(a - (float)h[i]);
-        }
-        // the step and lane group that take this run of eight
-        const uint32_t j = q6 ? 2u * ((sub >> 2) & 3u) + (sub & 1u) : 2u * (sub & 3u) + ((sub >> 2) & 1u);
-        const uint32_t kq = q6 ? 2u * (sub >> 4) + ((sub >> 1) & 1u) : sub >> 3;
-        uint8_t* dst = xa + cell * WIDE_XA + j * 64u + kq * 16u;
-        *(w_half8*)dst = w_half8{h[0], h[2], h[1], h[3], h[4], h[6], h[5], h[7]};
-        *(w_half8*)(dst + 512) = w_half8{l[0], l[2], l[1], l[3], l[4], l[6], l[5], l[7]};
-        if (!q6) {
-            float t = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-            t += group_partner<1>(t);
-            t += group_partner<2>(t);
-            if ((sub & 3u) == 0) {
-                const float a = t * (s * 0.03125f);   // 32 elements of at most 2^15 fit an fp16
-                const _Float16 th = (_Float16)a;
-                _Float16* o = (_Float16*)(xv + cell * WIDE_XV) + (sub >> 2);
-                o[0] = th;
-                o[8] = (_Float16)(a - (float)th);
-            }
-        }
+        wide_split(v, sub, (size_t)tok * n_blocks + b, q6, xa, xv, xi);
     }
 }
 
@@ -166,6 +172,45 @@ hipError_t launch_wide_x(int type, const float* X, int pro, const float* norm_w,
 {
     hipLaunchKernelGGL(wide_x_kernel, dim3(rows, pro == 1 ? 1u : (n_blocks + 15u) / 16u), dim3(512), 0, s, X, norm_w, eps,
                        n_blocks, pro, type == KQ_TYPE_Q6_K ? 1 : 0, x.xa, x.xv, x.xi);
+    return hipGetLastError();
+}
+
+// A mixture layer's start in one launch: the first workgroup buckets the pairs, the others split X, a half wave per superblock.  The two
+// need nothing from each other, and as launches of their own they cost 2.7 us more: 128 experts x 8, 2048 / 768, with the router, 24 /
+// 256 / 2048 tokens 116.5 / 159.8 / 534.5 -> 113.9 / 156.9 / 529.5, 8 experts x 2, 1024 / 512, 8 tokens 29.9 -> 27.8.
+template <int KEEP, bool MORE>
+__global__ __launch_bounds__(1024) void wide_prepare_kernel(const uint32_t* __restrict__ expert_idx, uint32_t n_pairs, uint32_t n_experts,
+                                                            uint32_t cap, uint32_t* __restrict__ records, uint32_t* __restrict__ n_records,
+                                                            const float* X, uint64_t cells, int q6, uint8_t* xa, uint8_t* xv, float* xi)
+{
+    extern __shared__ uint32_t sm[];
+    if (blockIdx.x == 0) {
+        group_pairs<KEEP, MORE>(expert_idx, n_pairs, n_experts, cap, records, n_records, sm);
+        return;
+    }
+    const uint32_t sub = threadIdx.x & 31u;
+    for (uint64_t cell = (uint64_t)(blockIdx.x - 1u) * 32u + (threadIdx.x >> 5); cell < cells; cell += (uint64_t)(gridDim.x - 1u) * 32u) {
+        const float* x = X + (size_t)cell * KQ_QK + sub * 8u;
+        float v[8];
+        *(float4*)v = *(const float4*)x;
+        *(float4*)(v + 4) = *(const float4*)(x + 4);
+        wide_split(v, sub, (size_t)cell, q6, xa, xv, xi);
+    }
+}
+
+hipError_t launch_wide_prepare(const uint32_t* expert_idx, uint32_t n_pairs, uint32_t n_experts, uint32_t cap, uint32_t* records,
+                               uint32_t* n_records, int type, const float* X, uint32_t rows, uint32_t n_blocks, const WideX& x, hipStream_t s)
+{
+    if (n_experts > 8192u) return hipErrorInvalidValue;   // three LDS arrays of n_experts words, eight experts per thread
+    const uint64_t cells = (uint64_t)rows * n_blocks, wgs = (cells + 31u) / 32u;
+    const dim3 grid(1u + (uint32_t)(wgs < 65536u ? wgs : 65536u));
+    const int q6 = type == KQ_TYPE_Q6_K ? 1 : 0;
+    const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(1024), 3 * n_experts * sizeof(uint32_t), s, expert_idx, n_pairs, n_experts, cap, records,
+                           n_records, X, cells, q6, x.xa, x.xv, x.xi);
+    };
+    if (n_pairs <= 4096u) go(wide_prepare_kernel<4, false>);
+    else go(wide_prepare_kernel<16, true>);
     return hipGetLastError();
 }
 
