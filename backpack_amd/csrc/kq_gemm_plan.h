@@ -86,4 +86,35 @@ inline GemmPlan plan_gemm_bf16(int type, uint32_t M, uint32_t N, uint32_t K, uin
     return GemmPlan{GEMM_FORM_SMALL, 0u, 0u};
 }
 
+// What the form chosen above takes, us.  Fitted to 31400 timed calls of 17 to 512 tokens (512 to 60000 rows, 256 to 14336 of K, the
+// three types, one part of 256 CUs): 5 to 9 % rms per form.  `ragged`: rows beyond the last whole 64 tokens are stored one by one.
+inline double gemm_price_us(int type, uint32_t M, uint32_t N, uint32_t K, uint32_t cus)
+{
+    const int t = type == KQ_TYPE_Q4_K ? 0 : type == KQ_TYPE_Q5_K ? 1 : 2;
+    const GemmPlan plan = plan_gemm_bf16(type, M, N, K, cus, 0, 0);
+    const uint32_t nk = K / 64u, m256 = (M + 255u) / 256u;
+    const uint64_t big = (uint64_t)m256 * ((N + 255u) / 256u);
+    const auto rounds = [&](uint64_t tiles, uint32_t at_once) { return (double)((tiles + at_once - 1u) / at_once); };
+    const double out = 1e-6 * (double)M * N, ragged = (M % 64u) / 64.0, any = M % 64u ? 1.0 : 0.0;
+    if (plan.form == GEMM_FORM_SHARES) {
+        const uint64_t one = (big * nk + cus - 1u) / cus, runs = (big * nk + one - 1u) / one;
+        const double step[3] = {2.02, 2.5, 2.45};
+        return 14.0 + step[t] * one + 0.063 * runs + 3.0 * out - 36.0 * one / nk;
+    }
+    if (plan.form == GEMM_FORM_HALF) {
+        const double step[3] = {0.764, 0.803, 0.83}, r = rounds((uint64_t)m256 * ((N + 127u) / 128u), cus);
+        return step[t] * r * nk + 3.8 * r + (1.3 + 0.2 * any) * out + 5.6 * ragged - 0.5;
+    }
+    if (plan.form == GEMM_FORM_SMALL) {
+        const double step[3] = {1.19, 1.2, 1.8}, r = rounds((uint64_t)((M + 127u) / 128u) * ((N + 127u) / 128u), 2u * cus);
+        return 2.5 + step[t] * r * nk + 0.5 * r + (0.8 + 0.2 * any) * out + 4.3 * ragged;
+    }
+    if (plan.form == GEMM_FORM_192) {
+        const double step[3] = {1.35, 1.49, 1.52};
+        return 0.3 + step[t] * nk + 1.3 * out + 9.0 * ragged;
+    }
+    const double step[3] = {1.585, 1.82, 1.835}, r = rounds(big, cus);
+    return 6.5 + step[t] * r * nk - 3.0 * r + (1.25 + 0.14 * any + 0.3 * ragged) * out;
+}
+
 }  // namespace kq

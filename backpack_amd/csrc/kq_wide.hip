@@ -46,6 +46,7 @@
 // us with the router, now / with the walk before / on the 16-token tiles: 2048 tokens 561 / 739 / 1264, 256 tokens
 // 168 / 191 / 267, 24 tokens 123 / 128 / 153.
 #include "kq_format.h"
+#include "kq_gemm_plan.h"
 #include "kq_group.h"
 #include "kq_kernels.h"
 #include "kq_wave.h"
@@ -348,6 +349,15 @@ __device__ __forceinline__ void lds_dma16_or_none(uint32_t lds, const uint8_t* s
 __device__ __forceinline__ void lds_dma4_or_none(uint32_t lds, const void* src, int lanes)
 {
     asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %2\n\ts_mov_b32 exec_hi, %2\n\tglobal_load_lds_dword %1, off\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(src), "s"(lanes) : "memory");
+}
+// ... from 64-bit addresses
+__device__ __forceinline__ void lds_dma16_lanes(uint32_t lds, const uint8_t* src, uint64_t lanes)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dwordx4 %1, off\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(src), "s"(lanes) : "memory");
+}
+__device__ __forceinline__ void lds_dma4_lanes(uint32_t lds, const uint8_t* src, uint64_t lanes)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b64 exec, %2\n\tglobal_load_lds_dword %1, off\n\ts_mov_b64 exec, -1" ::"s"(lds), "v"(src), "s"(lanes) : "memory");
 }
 // At most N of this wave's loads are still in flight, its LDS reads have returned, and so have the other waves'.
 template <int N>
@@ -1076,14 +1086,14 @@ hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32
 // bf16 rows of a short prompt (one launch serves up to 128 tokens per workgroup, K cut over workgroups).
 //
 // The GEMM's tiles of 128 and 256 tokens walk K in steps of 64 with one barrier each and mostly find one workgroup per
-// CU here: 1.4 us per step and CU, whatever the tokens.  This kernel walks whole superblocks: the X of TT tiles of 16
-// tokens is staged in LDS (two buffers), a wave turns its 32 rows' weights into bf16 in registers (the GEMM's formula and
-// its one rounding, so both compute the same products) and meets every token with them: no weight passes through LDS,
-// and a step is bounded by the matrix cores and the LDS reads about equally at 128 tokens.  Accumulation is in fp32
-// over the workgroup's whole range of K.
-//
-// LDS order of X: [tile][step][lane group kq][token] of 16 bytes; the token's place is turned by 2 * step + kq % 2, so that
-// the 16-byte pieces that a wave has read along K (whole lines) go to different banks.
+// CU here: 1.4 us per step and CU, whatever the tokens.  This kernel walks whole superblocks as wide_walk does: X (halves of a
+// superblock, a ring of three) and W go from memory to LDS without registers, a step's LDS reads and the expansion of its weights
+// stand between the matrix instructions of the step before.  A wave turns its 32 rows' weights into bf16 in registers (the GEMM's
+// formula and its one rounding, so both compute the same products; the quants enter v_fma_mix_f32 as fp16 subnormals where their
+// bits lie) and meets every token with them: no weight passes through LDS as bf16.  Accumulation is in fp32 over the workgroup's
+// whole range of K.  Read through registers, X and W ahead of a superblock and the operands right ahead of their use: 28672 x 4096
+// Q4_K at 100 tokens 52.0 -> 43.4 us, 4096 x 14336 Q6_K 37.9 -> 32.6, 28672 x 4096 at 32 tokens 28.9 -> 24.5, a layer at 100 tokens
+// 148 -> 131.
 typedef __bf16 w_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 w_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float w_f32x2 __attribute__((ext_vector_type(2)));
@@ -1093,133 +1103,251 @@ __device__ __forceinline__ uint32_t w_pack_bf16(float lo, float hi)
     return __builtin_bit_cast(uint32_t, __builtin_convertvector((w_f32x2{lo, hi}), w_bf16x2));
 }
 
+// Its LDS.  X: a ring of three halves of a superblock, [token][16 pieces of 16 bytes], a piece's place exchanged by its token
+// (^ token % 16).  W: as in WideLds.
+template <int TYPE, int TT> struct ShortLds {
+    using L = WideLds<TYPE, 1>;
+    static constexpr uint32_t X_HALF = TT * 4096u, W_AT = 3u * X_HALF, END = W_AT + 8u * L::W_WAVE, O_BYTES = TT * 16u * 260u * 4u;
+    static constexpr uint32_t BYTES = END > O_BYTES ? END : O_BYTES;
+    static constexpr int N_X = (TT + 1) / 2;   // a wave's loads for half a superblock of X
+};
+
 template <int TYPE, int TT>
 __global__ __launch_bounds__(512, 2) void short_kernel(const WideParams p)
 {
+    using L = WideLds<TYPE, 1>;
+    using S = ShortLds<TYPE, TT>;
     constexpr bool Q6 = TYPE == KQ_TYPE_Q6_K, Q5 = TYPE == KQ_TYPE_Q5_K;
     constexpr uint32_t OP = 260;   // floats between tokens of the output tile, as in wide_kernel
-    constexpr uint32_t X_BYTES = TT * 8192u, O_BYTES = TT * 16u * OP * 4u;
-    __shared__ __align__(16) uint8_t xs[2u * X_BYTES > O_BYTES ? 2u * X_BYTES : O_BYTES];
-    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, kq = lane >> 4, r16 = lane & 15u;
+    __shared__ __align__(16) uint8_t lds[S::BYTES];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, kq = lane >> 4, r16 = lane & 15u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)lds;
     const uint32_t t0 = blockIdx.y * (TT * 16u), count = min(p.M - t0, TT * 16u);
-
-    // X: 32 threads copy a token's 512 bytes of a superblock; piece c (eight k) goes to step cj of lane group ck
-    const uint32_t c = tid & 31u, tok = tid >> 5;
-    const uint32_t cj = Q6 ? 2u * ((c >> 2) & 3u) + (c & 1u) : 2u * (c & 3u) + ((c >> 2) & 1u);
-    const uint32_t ck = Q6 ? 2u * (c >> 4) + ((c >> 1) & 1u) : c >> 3;
-    const uint32_t xdst = cj * 1024u + ck * 256u + ((tok + 2u * cj + (ck & 1u)) & 15u) * 16u;
-    const size_t x_row = (size_t)p.n_blocks * 512u;
-    const uint8_t* xsrc[TT];   // tokens beyond the count repeat the last: their outputs are dropped
-#pragma unroll
-    for (int t = 0; t < TT; ++t) xsrc[t] = p.x.xa + (size_t)(t0 + min(16u * t + tok, count - 1u)) * x_row + c * 16u;
-
-    const uint32_t out0 = (blockIdx.x * WIDE_WAVES + wave) * 32u;
-    const uint8_t* wrow[2];
-#pragma unroll
-    for (int r = 0; r < 2; ++r) wrow[r] = p.W + (size_t)min(out0 + 16u * r + r16, p.N - 1u) * p.row_stride_bytes;
     constexpr uint32_t BB = TYPE == KQ_TYPE_Q4_K ? KQ_Q4K_BYTES : TYPE == KQ_TYPE_Q5_K ? KQ_Q5K_BYTES : KQ_Q6K_BYTES;
-    const uint32_t b0 = blockIdx.z * p.blocks_per_split, b1 = min(b0 + p.blocks_per_split, p.n_blocks);
+    const uint32_t b0 = blockIdx.z * p.blocks_per_split, all = min(b0 + p.blocks_per_split, p.n_blocks) - b0;
 
-    w_u32x4 xreg[TT];
-    auto fetch_x = [&](uint32_t b) {
+    // W: lane offsets (64 bits: any row stride) from the wave's two tiles' bases.  A matrix's last tile is read from its last 16
+    // rows on, what it has of an earlier one is not stored.
+    const uint32_t rows = min(p.N, 16u);
+    uint64_t woff[L::W_INSTR];
 #pragma unroll
-        for (int t = 0; t < TT; ++t) xreg[t] = *(const w_u32x4*)(xsrc[t] + (size_t)b * 512u);
+    for (uint32_t i = 0; i < L::W_INSTR; ++i) {
+        const uint32_t n = i * 64u + lane, row = n / L::UNITS, u = n % L::UNITS;
+        woff[i] = (uint64_t)min(row, rows - 1u) * p.row_stride_bytes + u * 16u;
+    }
+    const uint64_t doff = (uint64_t)min(r16, rows - 1u) * p.row_stride_bytes + 206u;
+    const uint32_t from0 = (blockIdx.x * WIDE_WAVES + wave) * 32u;
+    const uint8_t* wsrc[2];
+#pragma unroll
+    for (int r = 0; r < 2; ++r) wsrc[r] = p.W + (size_t)min(from0 + 16u * r, p.N - rows) * p.row_stride_bytes + (size_t)b0 * BB;
+    const uint32_t w_lds = lds0 + S::W_AT + wave * L::W_WAVE;
+    auto request_w = [&](int k) {   // piece k of a superblock's weights: whole loads, then each tile's last lanes (and d)
+        constexpr int WHOLE = 2 * ((int)L::W_INSTR - 1);
+        const int r = k & 1, i = k >> 1;
+        if (k < WHOLE) lds_dma16<false>(w_lds + r * L::W_TILE + i * 1024u, wsrc[r] + woff[i], -1);
+        else if (k < WHOLE + 2) lds_dma16_lanes(w_lds + r * L::W_TILE + (L::W_INSTR - 1u) * 1024u, wsrc[r] + woff[L::W_INSTR - 1u], (1ull << L::W_LAST) - 1ull);
+        else lds_dma4_lanes(w_lds + 2u * L::W_TILE + r * 64u, wsrc[r] + doff, 0xFFFFull);
     };
-    auto park_x = [&](uint32_t buf) {
+    // X: load i of the wave takes half a superblock of four tokens (beyond the count the last again: outputs that are dropped).  The
+    // halves are chosen so that a half's pieces lie together: Q4_K, Q5_K the low nibbles' elements, then the high ones' (64 bytes of each
+    // 128), Q6_K elements 0 .. 63 of each 128, then 64 .. 127.
+    const uint8_t* xp[S::N_X];
 #pragma unroll
-        for (int t = 0; t < TT; ++t) *(w_u32x4*)(&xs[buf * X_BYTES + t * 8192u + xdst]) = xreg[t];
+    for (int i = 0; i < S::N_X; ++i) {
+        const uint32_t n = i * WIDE_WAVES + wave, tok = 4u * n + (lane >> 4), piece = (lane ^ tok) & 15u, jj = piece >> 2, g = piece & 3u;
+        const uint32_t c = Q6 ? 16u * (g >> 1) + 4u * (jj >> 1) + 2u * (g & 1u) + (jj & 1u) : 8u * g + jj;
+        xp[i] = p.x.xa + ((size_t)(t0 + min(tok, count - 1u)) * p.n_blocks + b0) * 512u + c * 16u;
+    }
+    int x_last = (S::N_X - 1) * WIDE_WAVES + wave < TT * 4u ? -1 : 0;   // is the last of these there: all lanes or none
+    asm("s_nop 1\n\tv_readfirstlane_b32 %0, %1" : "=s"(x_last) : "v"(x_last));
+    constexpr int HALF = Q6 ? 128 : 64;   // bytes from a piece to the second half's
+    auto request_x = [&](uint32_t ring, int i, int step) {
+        const uint32_t to = lds0 + ring * S::X_HALF + (i * WIDE_WAVES + wave) * 1024u;
+        if (TT % 2 && i == S::N_X - 1) lds_dma16_or_none(to, xp[i], x_last);
+        else lds_dma16<false>(to, xp[i], -1);
+        xp[i] += step;
+    };
+
+    uint32_t a_lane[4];   // operands of X for step j: four places of the exchanged pieces
+#pragma unroll
+    for (int jj = 0; jj < 4; ++jj) a_lane[jj] = r16 * 256u + (((4u * jj + kq) ^ r16) & 15u) * 16u;
+    w_bf16x8 A[2][TT];
+    auto read_a = [&](uint32_t ring, int j) {
+        const uint8_t* x = lds + ring * S::X_HALF + a_lane[j & 3];
+#pragma unroll
+        for (int t = 0; t < TT; ++t) A[j & 1][t] = *(const w_bf16x8*)(x + t * 4096);
+    };
+    WideW<TYPE> w[2];
+    auto read_w = [&]() {
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+            w[r].load_lds(lds + S::W_AT + wave * L::W_WAVE + r * L::W_TILE + r16 * (L::UNITS * 16u),
+                          lds + S::W_AT + wave * L::W_WAVE + 2u * L::W_TILE + r * 64u + r16 * 4u, kq);
+    };
+    // a weight is q * sa + sb, q read as an fp16 subnormal where its bits lie (q * 2^-24; Q4_K's high nibbles q * 2^-20: the scale
+    // carries the power of two, which is exact, so the sum rounds the same value)
+    float sa[2][Q6 ? 4 : 2], sb[2][Q6 ? 4 : 2];
+    auto headers = [&]() {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            if constexpr (Q6) {
+                const float d = half_bits_to_float(w[r].d);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const uint32_t word = t < 2 ? w[r].sc.x : w[r].sc.y;
+                    const float s = d * (float)(int)(int8_t)(word >> (16 * (t & 1) + 8 * (kq & 1u)));
+                    sa[r][t] = s * 16777216.0f;
+                    sb[r][t] = -32.0f * s;   // exact: the sum rounds once, as s * (q - 32) does
+                }
+            } else {
+                const w_u32x4 h = w[r].hdr;
+                const float d = half_bits_to_float(h.x & 0xFFFFu), dmin = half_bits_to_float(h.x >> 16);
+                // (arithmetic, no choice between the two: the compiler would branch)
+                const uint32_t sc = ((kq < 2u ? h.y : h.w) & 0x0F0F0F0Fu) | ((h.y >> (kq & 2u)) & 0x30303030u);
+                const uint32_t mn = (((kq < 2u ? h.z : h.w) >> (2u * (kq & 2u))) & 0x0F0F0F0Fu) | ((h.z >> (kq & 2u)) & 0x30303030u);
+                const uint32_t s2 = sc >> (16u * (kq & 1u)), m2 = mn >> (16u * (kq & 1u));
+                sa[r][0] = d * (float)(s2 & 255u) * 16777216.0f;
+                sa[r][1] = d * (float)((s2 >> 8) & 255u) * 1048576.0f;
+                sb[r][0] = -(dmin * (float)(m2 & 255u));
+                sb[r][1] = -(dmin * (float)((m2 >> 8) & 255u));
+            }
+        }
+    };
+    w_bf16x8 B[2][2];   // [step % 2][tile]
+    auto expand = [&](int j) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            w_u32x4 o;
+            const int n = Q6 ? j >> 1 : j >> 2;   // which scale
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                w_half2 a, b;   // elements 0 and 2, 1 and 3
+                if constexpr (Q6) {
+                    const int t = j >> 1, u = j & 1;
+                    const uint32_t l = w[r].ql[t & 1][2 * u + i], h = w[r].qh[2 * u + i];
+                    const uint32_t c = ((l >> (4 * (t >> 1))) & 0x0F0F0F0Fu) | ((t < 2 ? h << (4 - 2 * t) : h >> (2 * t - 4)) & 0x30303030u);
+                    a = __builtin_bit_cast(w_half2, __builtin_amdgcn_perm(0u, c, 0x0c020c00u));
+                    b = __builtin_bit_cast(w_half2, __builtin_amdgcn_perm(0u, c, 0x0c030c01u));
+                } else {
+                    const int i8 = j & 3;
+                    const uint32_t d = w[r].q[i8 >> 1][2 * (i8 & 1) + i], m = n ? 0x00F000F0u : 0x000F000Fu;
+                    uint32_t e = d & m, f = (d >> 8) & m;
+                    if constexpr (Q5) {
+                        // bit 2kq + n of a byte of fifth bits: bit 4 beside a low nibble, bit 8 beside a high one
+                        const uint32_t g = w[r].f[i8 >> 1][2 * (i8 & 1) + i] >> (2u * kq);
+                        e |= n ? (g << 7) & 0x01000100u : (g << 4) & 0x00100010u;
+                        f |= n ? (g >> 1) & 0x01000100u : (g >> 4) & 0x00100010u;
+                    }
+                    a = __builtin_bit_cast(w_half2, e);
+                    b = __builtin_bit_cast(w_half2, f);
+                }
+                const _Float16 a0 = a.x, a1 = a.y, c0 = b.x, c1 = b.y;
+                o[2 * i] = w_pack_bf16(fmaf((float)a0, sa[r][n], sb[r][n]), fmaf((float)c0, sa[r][n], sb[r][n]));
+                o[2 * i + 1] = w_pack_bf16(fmaf((float)a1, sa[r][n], sb[r][n]), fmaf((float)c1, sa[r][n], sb[r][n]));
+            }
+            B[j & 1][r] = __builtin_bit_cast(w_bf16x8, o);
+        }
     };
     w_f32x4 acc[2][TT];
 #pragma unroll
     for (int r = 0; r < 2; ++r)
 #pragma unroll
         for (int t = 0; t < TT; ++t) acc[r][t] = w_f32x4{0, 0, 0, 0};
-
-    WideW<TYPE> w[2], wn[2];
-    fetch_x(b0);
-#pragma unroll
-    for (int r = 0; r < 2; ++r) wn[r].load(wrow[r] + (size_t)b0 * BB, kq);
-    park_x(0);
-    wide_barrier();
-    for (uint32_t b = b0; b < b1; ++b) {
-        const uint32_t buf = (b - b0) & 1u;
-        const uint32_t bn = min(b + 1u, b1 - 1u);   // (the last step requests its own superblock again)
-        fetch_x(bn);
-        float sa[2][Q6 ? 4 : 2], sb[2][Q6 ? 4 : 2];   // a weight is q * sa + sb
-#pragma unroll
-        for (int r = 0; r < 2; ++r) {
-            w[r] = wn[r];
-            wn[r].load(wrow[r] + (size_t)bn * BB, kq);
-            if constexpr (Q6) {
-                const float d = half_bits_to_float(w[r].d);
-#pragma unroll
-                for (int t = 0; t < 4; ++t) {
-                    const uint32_t word = t < 2 ? w[r].sc.x : w[r].sc.y;
-                    sa[r][t] = d * (float)(int)(int8_t)(word >> (16 * (t & 1) + 8 * (kq & 1u)));
-                    sb[r][t] = -32.0f * sa[r][t];   // exact: the sum rounds once, as s * (q - 32) does
-                }
-            } else {
-                const w_u32x4 h = w[r].hdr;
-                const float d = half_bits_to_float(h.x & 0xFFFFu), dmin = half_bits_to_float(h.x >> 16);
-                const uint32_t sc = kq < 2u ? h.y & 0x3F3F3F3Fu : (h.w & 0x0F0F0F0Fu) | ((h.y >> 2) & 0x30303030u);
-                const uint32_t mn = kq < 2u ? h.z & 0x3F3F3F3Fu : ((h.w >> 4) & 0x0F0F0F0Fu) | ((h.z >> 2) & 0x30303030u);
-                const uint32_t s2 = sc >> (16u * (kq & 1u)), m2 = mn >> (16u * (kq & 1u));
-                sa[r][0] = d * (float)(s2 & 255u);
-                sa[r][1] = d * (float)((s2 >> 8) & 255u);
-                sb[r][0] = -(dmin * (float)(m2 & 255u));
-                sb[r][1] = -(dmin * (float)((m2 >> 8) & 255u));
-            }
-        }
-        const uint8_t* xb = xs + buf * X_BYTES + kq * 256u;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            w_bf16x8 B[2];
-#pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                uint32_t q[2];
-                if constexpr (Q6) {
-                    const int t = j >> 1, u = j & 1;
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-                        q[i] = ((w[r].ql[t & 1][2 * u + i] >> (4 * (t >> 1))) & 0x0F0F0F0Fu) |
-                               (((w[r].qh[2 * u + i] >> (2 * t)) & 0x03030303u) << 4);
-                } else {
-                    const int i8 = j >> 1;
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        q[i] = (w[r].q[i8 >> 1][2 * (i8 & 1) + i] >> (4 * (j & 1))) & 0x0F0F0F0Fu;
-                        if constexpr (Q5) q[i] |= ((w[r].f[i8 >> 1][2 * (i8 & 1) + i] >> (2u * kq + (j & 1))) & 0x01010101u) << 4;
-                    }
-                }
-                const float a = sa[r][Q6 ? j >> 1 : j & 1], nb = sb[r][Q6 ? j >> 1 : j & 1];
-                w_u32x4 o;
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    o[2 * i] = w_pack_bf16(fmaf(a, (float)(q[i] & 255u), nb), fmaf(a, (float)((q[i] >> 8) & 255u), nb));
-                    o[2 * i + 1] = w_pack_bf16(fmaf(a, (float)((q[i] >> 16) & 255u), nb), fmaf(a, (float)(q[i] >> 24), nb));
-                }
-                B[r] = __builtin_bit_cast(w_bf16x8, o);
-            }
-            const uint8_t* xj = xb + j * 1024 + ((r16 + 2u * j + (kq & 1u)) & 15u) * 16u;
-#pragma unroll
-            for (int t = 0; t < TT; ++t) {
-                const w_bf16x8 A = *(const w_bf16x8*)(xj + t * 8192);
-#pragma unroll
-                for (int r = 0; r < 2; ++r) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[r], acc[r][t], 0, 0, 0);
-            }
-        }
-        park_x(buf ^ 1u);
-        wide_barrier();
-    }
-
-    // outputs through LDS, as in wide_kernel
-    float* ot = (float*)xs;
-#pragma unroll
-    for (int r = 0; r < 2; ++r)
+    auto multiply = [&](int j) {
 #pragma unroll
         for (int t = 0; t < TT; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) ot[(16 * t + 4u * kq + i) * OP + wave * 32u + 16u * r + r16] = acc[r][t][i];
+            for (int r = 0; r < 2; ++r) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[j & 1][t], B[j & 1][r], acc[r][t], 0, 0, 0);
+    };
+    auto schedule = [&]() {
+        constexpr int NV = ((Q6 ? 50 : Q5 ? 54 : 38) + 2 * TT - 1) / (2 * TT);
+#pragma unroll
+        for (int i = 0; i < 2 * TT; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            if (i < TT) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, NV, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // The walk, as wide_walk's: W a superblock ahead, X two halves; past the end the last is requested again.
+    constexpr int N_X = S::N_X, N_W = L::N_W, WAS = (N_X + N_W + 3) / 4, XBS = (N_X + 3) / 4;
+    auto next_w = [&](uint32_t at) {
+        const uint32_t step = at + 1u < all ? BB : 0u;
+        wsrc[0] += step;
+        wsrc[1] += step;
+    };
+    auto x_step = [&](uint32_t at) -> int { return at + 1u >= all ? -HALF : 512 - HALF; };
+#pragma unroll
+    for (int k = 0; k < N_W; ++k) request_w(k);
+    next_w(0);
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < N_X; ++i) request_x(h, i, h == 0 ? HALF : x_step(0));
+    wide_meet<N_X>();
+    read_w();
+    w[0].arrived(); w[1].arrived();
+#pragma unroll
+    for (int k = 0; k < WAS; ++k) request_w(k);
+    headers();
+    read_a(0, 0);
+    expand(0);
+    uint32_t ring = 0;   // where the superblock's first half lies
+    for (uint32_t at = 0; at < all; ++at) {
+        const uint32_t ring1 = ring + 1u == 3u ? 0u : ring + 1u, ring2 = 3u - ring - ring1;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (j == 3) {
+                // every wave has read the first half; the second has arrived
+                wide_meet<N_X + N_W>();
+                read_a(ring1, 4);
+                expand(4);
+            } else if (j == 7) {
+                wide_meet<N_X>();
+                read_w();
+                read_a(ring2, 0);
+                w[0].arrived(); w[1].arrived();
+#pragma unroll
+                for (int k = 0; k < WAS; ++k) request_w(k);
+                headers();
+                expand(0);
+            } else {
+                read_a(j < 3 ? ring : ring1, j + 1);
+                expand(j + 1);
+                if (j < 3) {
+#pragma unroll
+                    for (int k = (j + 1) * WAS; k < (j + 2) * WAS && k < N_X + N_W; ++k) {
+                        if (k < N_W) request_w(k);
+                        else request_x(ring2, k - N_W, HALF);
+                    }
+                }
+            }
+            if (j >= 3 && j < 7) {
+#pragma unroll
+                for (int i = (j - 3) * XBS; i < (j - 2) * XBS && i < N_X; ++i) request_x(ring, i, x_step(at + 1u));
+            }
+            multiply(j);
+            schedule();
+            if (j == 2) next_w(at + 1u);
+        }
+        ring = ring2;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // no load may land in the output tile
+    __syncthreads();
+
+    // outputs through LDS, as in wide_kernel
+    float* ot = (float*)lds;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+        const uint32_t from = from0 + 16u * r, first = wave * 32u + 16u * r, col = first + min(from, p.N - rows) + r16 - from;
+#pragma unroll
+        for (int t = 0; t < TT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (col >= first && col < first + 16u) ot[(16 * t + 4u * kq + i) * OP + col] = acc[r][t][i];
+    }
     __syncthreads();
     if (p.n_splits > 1) {   // wide_sum_kernel adds the splits' tiles
         float* tile = p.partial + (((size_t)blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * (TT * 16u * 256u);
@@ -1249,11 +1377,13 @@ static void launch_short_type(const WideParams& p, uint32_t tt, dim3 grid, hipSt
 }
 
 // How a call of M bf16 tokens is cut, its price in us and what the GEMM takes.  A superblock of a workgroup's walk costs
-// 1.35 + 0.41 per tile of tokens (Q5_K 1.6 + 0.41, Q6_K 3.5 + 0.27), a round over the CUs 5, the launch that adds the splits
-// 3 and 1.2 per 10^6 floats.  Measured against the GEMM, us, at 100 / 128 / 256 tokens: Q4_K 4096x4096 20 / 22 / 28 against
-// 37 / 37 / 39, 6144x4096 23 / 25 / 36 against 38, 28672x4096 55 / 62 / 89 against 65 / 62 / 66 (32 tokens 30 against 61),
-// Q6_K 4096x14336 40 / 43 / 61 against 61 / 61 / 63, 7168x1024 21 / 21 / 27 against 22 / 20 / 20; at 384 tokens 4096x4096 36
-// against 51, 28672x4096 163 against 108.
+// 1.1 + 0.27 per tile of tokens (Q5_K 1.7 + 0.25, Q6_K 2.15 + 0.24), a round over the CUs 2.7 + 0.15 per tile and 2.5 behind the
+// first, the launch that adds the splits 3.5 and 1.4 per 10^6 floats, 10^6 outputs 0.9: fitted to 31400 timed calls of 17 to 512
+// tokens to 6 % rms.  Over these calls the choice is 0.5 % slower than the faster of the two kernels in the mean and more than 5 %
+// slower on 1107; with the prices of the walk through registers that came before it was 6 % and 6145.  The GEMM has to be 5 %
+// dearer: close calls stay where they were.  us at 100 / 128 / 256 tokens, with the walk before / this one / the GEMM: Q4_K
+// 28672x4096 51.7 / 41.9 / 62.6, 57.5 / 46.6 / 60.0, 88.8 / 63.9 / 63.6; Q6_K 4096x14336 37.8 / 32.5 / 57.9, 40.4 / 35.2 / 58.3,
+// 56.4 / 46.1 / 59.5.
 ShortPlan plan_short(int type, uint32_t M, uint32_t N, uint32_t K, size_t capacity_floats, uint32_t cus)
 {
     ShortPlan best{0, 0, 0, 0, 1e30, 0.0};
@@ -1261,33 +1391,18 @@ ShortPlan plan_short(int type, uint32_t M, uint32_t N, uint32_t K, size_t capaci
     uint32_t tt = (tiles + gy0 - 1u) / gy0;
     if (tt < 2u) tt = 2u;
     const uint32_t gy = (tiles + tt - 1u) / tt, gx = (N + 255u) / 256u;
-    const double step_us = type == KQ_TYPE_Q4_K ? 1.35 + 0.41 * tt : type == KQ_TYPE_Q5_K ? 1.6 + 0.41 * tt : 3.5 + 0.27 * tt;
+    const double step_us = type == KQ_TYPE_Q4_K ? 1.1 + 0.27 * tt : type == KQ_TYPE_Q5_K ? 1.7 + 0.25 * tt : 2.15 + 0.24 * tt;
     const size_t tile_floats = (size_t)gy * tt * 16u * gx * 256u;
+    const double out = 1e-6 * (double)M * N;
     for (uint32_t c = 1; c <= n_blocks && c <= 16u; ++c) {
         const uint32_t per = (n_blocks + c - 1u) / c, z = (n_blocks + per - 1u) / per;
         if (z > 1u && z * tile_floats > capacity_floats) break;
         const double rounds = (double)(((uint64_t)gx * gy * z + cus - 1u) / cus);
-        const double us = 2.0 + rounds * (per * step_us + 5.0) + (z > 1u ? 3.0 + 1.2e-6 * (double)z * (double)tile_floats : 0.0);
+        const double us = 1.6 + 2.5 * (rounds - 1.0) + rounds * (per * step_us + 2.7 + 0.15 * tt) +
+                          (z > 1u ? 3.5 + 1.4e-6 * (double)z * (double)tile_floats + 0.9 * out : 0.95 * out);
         if (us < best.us) best = ShortPlan{tt, gy, z, per, us, 0.0};
     }
-    // The GEMM up to 256 tokens: 14 + 5.7 per 1024 of K while its tiles leave CUs idle (60 at most: it cuts K too), from
-    // there on 16 + 1.5 per 1000 rows of 4096; up to 512 tokens 1.4 times the former, measured at K from 4096 on only (rows
-    // shorter than that stay on the GEMM, and so do matrices of many rows, whose longer GEMM this price leaves out)
-    const double few = std::fmin(60.0, 14.0 + 5.7 * K / 1024.0), many = 16.0 + 1.5e-3 * N * (K / 4096.0);
-    if (M <= 256u) best.gemm_us = std::fmax(few, many);
-    else if (K >= 4096u) best.gemm_us = 1.4 * few;
-    // Rows of at most five superblocks, up to 256 tokens: those figures are up to twice too high and the ones above 2 too
-    // high without a cut of K, where the stores of many rows then count.  The GEMM takes 5.5 + 11 per 1024 of K, or per 1000 rows
-    // 0.06 (0.16 beyond 128 tokens) + 1.5 per 4096 of K, and 0.08 for each token beyond the last whole 64.  Measured, us, this
-    // kernel / the GEMM: Q4_K 4096x512 at 100 / 128 / 256 tokens 12.9 / 13.8, 13.5 / 10.8, 15.5 / 10.7, 28672x1024 24.9 / 24.0,
-    // 26.9 / 21.6, 29.3 / 23.7, 4096x1024 at 128 14.2 / 16.6, Q6_K 4096x512 at 64 / 100 / 128 15.0 / 11.4, 16.3 / 14.6, 17.0 / 11.6.
-    if (M <= 256u && n_blocks < 6u) {
-        const double ragged = 0.08 * (M % 64u);
-        const double few_s = std::fmin(14.0 + 5.7 * K / 1024.0, 5.5 + 11.0 * K / 1024.0);
-        const double many_s = 5.5 + N * ((M > 128u ? 1.6e-4 : 6e-5) + 1.5e-3 * (K / 4096.0));
-        best.gemm_us = std::fmin(best.gemm_us, std::fmax(few_s, many_s) + ragged);
-        best.us += 4e-7 * (double)M * N - 2.0;
-    }
+    best.gemm_us = 0.95 * gemm_price_us(type, M, N, K, cus);
     return best;
 }
 

@@ -413,6 +413,32 @@ def test_short_prompt_vs_oracle(gpu, kqo, type_, M, N, K):  # noqa: F811
     assert np.abs(got - gemm).max() <= 2.0 ** -23 * K ** 0.5 * 8 * max(rms, float(np.abs(want).max()))
 
 
+@pytest.mark.parametrize("type_", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("M", [32, 48, 63, 80, 81, 112, 113])
+@pytest.mark.parametrize("N,blocks", [(271, 1), (40, 2), (9, 3), (257, 18)])
+def test_short_prompt_tiles_and_walks(gpu, kqo, type_, M, N, blocks):  # noqa: F811
+    """Every number of token tiles (odd ones, where half the waves have a load less), walks of one superblock, of two and three (K is
+    cut into single ones on rows this short, so 18 blocks walk two), fewer rows than a tile; against 64-bit sums of the bf16 weights."""
+    import torch
+    from backpack_amd import capi, kquant
+    K = 256 * blocks
+    raw, _, w = gpu.make_weight(type_, N, K, seed=M + N)
+    rng = np.random.default_rng(K + M)
+    X = gpu.dev(rng.standard_normal((M, K)).astype(np.float32)).bfloat16()
+    capi.force_kernel(9)
+    try:
+        got = kquant.matmul(X, w).cpu().numpy()
+        again = kquant.matmul(X, w).cpu().numpy()
+    finally:
+        capi.force_kernel(0)
+    assert capi.last_form() == "short_prompt" and np.array_equal(got, again)
+    wb = torch.from_numpy(kqo.dequant(type_, raw, N, K)).bfloat16().double().numpy()
+    want = X.double().cpu().numpy() @ wb.T
+    rms = float(np.sqrt(np.mean(want ** 2)))
+    # fp32 sums of K products
+    assert np.abs(got - want).max() <= 2.0 ** -23 * K ** 0.5 * 8 * max(rms, float(np.abs(want).max()))
+
+
 def test_forced_families_run_what_they_name(gpu):  # noqa: F811
     """Family 4 on bf16 X is the tiled GEMM and 9 the short-prompt kernel, whatever the price says; families that have
     no form of a call refuse it instead of answering from another kernel."""
