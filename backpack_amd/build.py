@@ -14,6 +14,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OBJ = os.path.join(CSRC, "build")
 LIB = os.path.join(HERE, "libbpk_kquant.so")
+CALLS = os.path.join(HERE, "_torch_calls.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = [
@@ -208,5 +209,28 @@ def build_library(jobs: int = 8) -> str:
     return LIB
 
 
+def build_calls() -> str:
+    """backpack_amd/_torch_calls.so: the per-call part of kquant.py (csrc/host/torch_calls.cpp), host code only."""
+    import sysconfig
+
+    from torch.utils import cpp_extension
+    inc = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"], "/opt/rocm/include"]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-w", "-D__HIP_PLATFORM_AMD__",
+           *[f"-I{i}" for i in inc], os.path.join(CSRC, "host", "torch_calls.cpp"), "-o", CALLS,
+           *[f"-L{d}" for d in cpp_extension.library_paths()], "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode:
+        raise RuntimeError(f"building {CALLS} failed:\n{r.stderr[-4000:]}")
+    return CALLS
+
+
+def build_all() -> str:
+    with cf.ThreadPoolExecutor(max_workers=2) as ex:
+        calls = ex.submit(build_calls)
+        lib = build_library()
+        calls.result()
+    return lib
+
+
 if __name__ == "__main__":
-    print(build_library())
+    print(build_all())

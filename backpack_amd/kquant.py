@@ -17,8 +17,28 @@ from . import capi
 from .capi import Q4_K, Q5_K, Q6_K  # noqa: F401
 
 
+_bound = None     # the library whose functions the native calls go to
+_calls = None
+
+
+def _native():
+    """The native form of the calls below (csrc/host/torch_calls.cpp), on the library that capi has loaded.  It returns NotImplemented
+    for what is not a plain call, ahead of any effect: the Python form then takes or refuses it."""
+    global _bound, _calls
+    lib = capi.lib()
+    if lib is not _bound:
+        import ctypes as C
+
+        from . import _torch_calls     # built with the library; missing, this raises
+        names = ("bpk_kq_matmul", "bpk_kq_matmul_bf16", "bpk_kq_matmul_fused", "bpk_kq_matmul_fused_workspace_bytes", "bpk_kq_matmul_argmax",
+                 "bpk_prefill_rows_bf16", "bpk_kq_dequant_rows", "bpk_moe_route", "bpk_kq_moe_ffn", "bpk_kq_moe_ffn_scratch_bytes")
+        _torch_calls.bind([C.cast(getattr(lib, n), C.c_void_p).value for n in names], capi.check)
+        _bound, _calls = lib, _torch_calls
+    return _calls
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return _native().stream()
 
 
 def _ptr(t) -> int:
@@ -108,6 +128,9 @@ def fuse(parts: list[KQuantPacked]) -> KQuantPacked:
 def matmul(x: torch.Tensor, w: KQuantPacked, bias: torch.Tensor | None = None,
            out: torch.Tensor | None = None, y_offset: int = 0) -> torch.Tensor:
     """Y[m, y_offset+n] = bias[n] + sum_k X[m,k] * dequant(W)[n,k]; fp32 or bf16 X."""
+    y = _native().matmul(x, w, bias, out, y_offset)
+    if y is not NotImplemented:
+        return y
     assert x.is_cuda and x.is_contiguous() and x.shape[-1] == w.K
     M = x.numel() // w.K
     if out is None:
@@ -132,6 +155,9 @@ def prefill_rows_bf16(x: torch.Tensor, K: int, prologue: int = capi.PRO_NONE, no
                       eps: float = 0.0) -> torch.Tensor:
     """fp32 rows -> the bf16 activation rows of the prefill GEMM, [M, K]: x as it is, its RMSNorm, or
     act(gate) * up of gate|up rows of 2K floats, evaluated in fp32 and rounded to nearest even."""
+    y = _native().prefill_rows_bf16(x, K, prologue, norm_w, eps)
+    if y is not NotImplemented:
+        return y
     assert x.is_cuda and x.is_contiguous() and x.dtype == torch.float32
     row = 2 * K if prologue in (capi.PRO_SILU_MUL, capi.PRO_GELU_MUL) else K
     assert x.shape[-1] == row
@@ -148,6 +174,9 @@ def matmul_fused(x: torch.Tensor, w: KQuantPacked, prologue: int = capi.PRO_NONE
     """The decode matvec with what surrounds it folded in: RMSNorm of x, or act(gate)*up of a gate|up
     row (x is then [M, 2K]), and a residual added to the output (residual may be `out`).  With an
     epilogue, w is the stacked gate|up matrix and the result is act(gate.x) * (up.x), [M, w.N / 2]."""
+    y = _native().matmul_fused(x, w, prologue, norm_w, eps, residual, bias, out, workspace, allow_workspace, epilogue)
+    if y is not NotImplemented:
+        return y
     assert x.is_cuda and x.is_contiguous() and x.dtype == torch.float32
     xk = w.K * (2 if prologue in (capi.PRO_SILU_MUL, capi.PRO_GELU_MUL) else 1)
     assert x.shape[-1] == xk
@@ -229,6 +258,9 @@ def argmax_rows(logits: torch.Tensor):
 
 def matmul_argmax(x: torch.Tensor, w: KQuantPacked, bias: torch.Tensor | None = None):
     """lm_head and greedy pick in one call: (logits [M,N], index int32 [M], value f32 [M])."""
+    y = _native().matmul_argmax(x, w, bias)
+    if y is not NotImplemented:
+        return y
     assert x.is_cuda and x.is_contiguous() and x.dtype == torch.float32 and x.shape[-1] == w.K
     M = x.numel() // w.K
     logits = torch.empty((M, w.N), dtype=torch.float32, device=x.device)
@@ -241,6 +273,10 @@ def matmul_argmax(x: torch.Tensor, w: KQuantPacked, bias: torch.Tensor | None = 
 
 def dequant_rows(w: KQuantPacked, rows: torch.Tensor | None = None, M: int | None = None) -> torch.Tensor:
     """fp32 rows of the matrix (the q6k_gather contract); rows: int32 device tensor."""
+    if rows is not None:
+        y = _native().dequant_rows(w, rows)
+        if y is not NotImplemented:
+            return y
     if rows is not None:
         assert rows.dtype == torch.int32 and rows.is_cuda
         M = rows.numel()
@@ -278,6 +314,10 @@ def moe_topk_softmax(logits: torch.Tensor, k: int, normalize: bool = True):
 
 def moe_route(x: torch.Tensor, router_w: torch.Tensor, k: int, normalize: bool = True, want_logits: bool = False):
     """Router matvec (fp32 [n_experts, hidden]) and selection in one launch."""
+    if not want_logits:
+        y = _native().moe_route(x, router_w, k, normalize)
+        if y is not NotImplemented:
+            return y
     assert x.is_contiguous() and router_w.is_contiguous() and x.dtype == router_w.dtype == torch.float32
     T, H = x.shape
     E = router_w.shape[0]
@@ -292,6 +332,9 @@ def moe_route(x: torch.Tensor, router_w: torch.Tensor, k: int, normalize: bool =
 def moe_ffn(x: torch.Tensor, gate: KQuantPacked, up: KQuantPacked, down: KQuantPacked,
             expert_idx: torch.Tensor, expert_wt: torch.Tensor, n_experts: int) -> torch.Tensor:
     """Routed-expert FFN: sum_s wt[t,s] * down_e(silu(gate_e x) * up_e x)."""
+    y = _native().moe_ffn(x, gate, up, down, expert_idx, expert_wt, n_experts)
+    if y is not NotImplemented:
+        return y
     T, k = expert_idx.shape
     hidden, inter = gate.K, down.K
     L = capi.lib()
