@@ -163,6 +163,9 @@ hipError_t launch_wide_x(int type, const float* X, int pro, const float* norm_w,
                          uint32_t n_blocks, const WideX& x, hipStream_t s);
 // launch_wide's price in us at up to 16 tokens, K in one piece
 double wide_price_16(int type, uint32_t N, uint32_t n_blocks);
+// us that a call of 5 to 16 tokens takes on the many-token and on the tile kernel (no prologue or a norm; residual, epilogue)
+double wide_price_5_to_16(const MatmulArgs& a, const SplitScratch& sc);
+double mtile_price_5_to_16(const MatmulArgs& a, const SplitScratch& sc);
 // grouped by expert: records of up to cap (16, 32, 48, 64) pairs, as launch_moe_group writes them with sets = cap / 2;
 // with a.W2, Y = silu(W x) * (W2 x)
 hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32_t* records, const uint32_t* n_records,

@@ -41,6 +41,7 @@
 // owns a tile and walks all of K; with R = 1 (matrices of few rows) the waves of
 // the workgroup take different superblocks of the chunk and fold their partial
 // tiles through LDS at the end.  There is no fold across workgroups.
+#include <algorithm>
 #include <cmath>
 
 #include "kq_format.h"
@@ -1334,6 +1335,50 @@ hipError_t launch_mtile_grouped(const MatmulArgs& a, const uint32_t* tiles, cons
     return launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, false>(p, wgs, tiles_bound, s, slices);
 }
 
+// Work split.  A wave per tile, `per_wg` tiles per workgroup (they share the conversion of X; pairs of gate and up take an even
+// number), and K cut into `splits` runs of whole chunks when the rows alone give too few workgroups.  Candidates are priced as
+// rounds x (chunks walked + 1.5 for launch, prologue and fold), a partly idle last round costing half its idle share extra; one
+// tile per workgroup with the waves taking different superblocks is the fallback for matrices of a few rows.  extra: floats per 16
+// rows of a workgroup's partial tile beside its sums (the sums of squares of a norm prologue).
+struct MtileSplit {
+    uint32_t per_wg, splits, chunks, rounds;
+    float cost;
+};
+static MtileSplit mtile_split(uint32_t tiles, uint32_t n_blocks, bool pairs, uint32_t extra, const SplitScratch& sc)
+{
+    const uint32_t n_chunks = (n_blocks + MT_KC - 1) / MT_KC, cus = device_cu_count();
+    MtileSplit best{8u, 1u, n_chunks, 1u, 1e30f};
+    for (uint32_t tpw = 8; tpw >= 4; tpw -= pairs ? 2u : 1u) {
+        const uint32_t groups = pairs ? (tiles / 2u + tpw / 2u - 1u) / (tpw / 2u) : (tiles + tpw - 1u) / tpw;
+        for (uint32_t splits = 1; splits <= n_chunks && splits <= 16u; ++splits) {
+            const uint32_t cps = (n_chunks + splits - 1u) / splits;
+            if ((splits - 1u) * cps >= n_chunks) continue;   // a split would be empty
+            if (splits > 1u && ((size_t)splits * 16u * groups * (tpw * 16u + extra) > sc.capacity_floats || groups > sc.n_counters)) continue;
+            const uint32_t wgs = groups * splits, rounds = (wgs + cus - 1u) / cus;
+            const float idle = 1.0f - (float)wgs / (float)(rounds * cus);
+            const float cost = (float)rounds * ((float)cps + 1.5f) * (1.0f + 0.5f * idle);
+            if (cost < best.cost) best = MtileSplit{tpw, splits, cps, rounds, cost};
+        }
+    }
+    return best;
+}
+
+double mtile_price_5_to_16(const MatmulArgs& a, const SplitScratch& sc)
+{
+    const MtileSplit b = mtile_split((a.N + 15u) / 16u, a.n_blocks, a.epi != 0, 1u, sc);
+    const double rounds = b.rounds, M = a.M, walk = rounds * std::min(b.chunks * (uint32_t)MT_KC, a.n_blocks), out = 1e-6 * M * (a.epi ? a.N / 2u : a.N);
+    // The launch, a superblock of a workgroup's walk (beside that per token and per tile), a round, the fold and its splits, a norm per chunk
+    // of the walk and beside it, 10^6 outputs: fitted to 40000 timed calls of 5 to 16 tokens (as for the many-token kernel), 8 to 10 % rms.
+    // Q4_K, Q5_K, Q6_K up to 8 tokens, then beyond.
+    const double c[6][10] = {{1.239, 0.109, 0.026, 0.092, 2.632, 1.382, 0.241, 0.557, 0.698, 5.602}, {1.242, 0.253, 0.017, 0.114, 2.174, 1.627, 0.281, 0.575, 0.772, 12.128},
+                             {1.141, 0.252, 0.008, 0.221, 1.754, 2.511, 0.280, 0.866, 1.196, 20.591}, {1.227, 0.118, 0.031, 0.128, 2.670, 1.434, 0.314, 0.762, 0.660, 4.926},
+                             {0.995, 0.216, 0.032, 0.136, 2.583, 1.718, 0.332, 0.839, 0.704, 7.462}, {1.059, 0.369, 0.025, 0.238, 1.953, 2.546, 0.341, 0.907, 1.137, 13.148}};
+    const double* k = c[(a.M > 8u ? 3 : 0) + (a.type == KQ_TYPE_Q4_K ? 0 : a.type == KQ_TYPE_Q5_K ? 1 : 2)];
+    const double norm = a.pro == 1 ? 1.0 : 0.0;
+    return k[0] + walk * (k[1] + k[2] * M + k[3] * b.per_wg) + k[4] * rounds + (b.splits > 1u ? k[5] : 0.0) + k[6] * b.splits +
+           norm * (k[7] * rounds * b.chunks + k[8]) + k[9] * out;
+}
+
 hipError_t launch_mtile(const MatmulArgs& a, const SplitScratch& sc, hipStream_t s)
 {
     const bool q6 = a.type == KQ_TYPE_Q6_K;
@@ -1343,29 +1388,10 @@ hipError_t launch_mtile(const MatmulArgs& a, const SplitScratch& sc, hipStream_t
     const uint32_t tiles = (a.N + 15u) / 16u;
     const uint32_t n_chunks = (a.n_blocks + MT_KC - 1) / MT_KC;
     const uint32_t cus = device_cu_count();
-
-    // Work split.  A wave per tile, tpw tiles per workgroup (they share the conversion of X), and K cut into
-    // n_splits runs of whole chunks when the rows alone give too few workgroups.  Candidates are priced as
-    // rounds x (chunks walked + 1.5 for launch, prologue and fold), a partly idle last round costing half its
-    // idle share extra; one tile per workgroup with the waves taking different superblocks is the fallback
-    // for matrices of a few rows.
-    uint32_t best_tpw = 0, best_splits = 1, best_cps = n_chunks;
-    float best_cost = 1e30f;
-    for (uint32_t tpw = 8; tpw >= 4; --tpw) {
-        const uint32_t groups = (tiles + tpw - 1u) / tpw;
-        for (uint32_t splits = 1; splits <= n_chunks && splits <= 16u; ++splits) {
-            const uint32_t cps = (n_chunks + splits - 1u) / splits;
-            if ((splits - 1u) * cps >= n_chunks) continue;   // a split would be empty
-            if (splits > 1u && ((size_t)splits * 16u * groups * tpw * 16u > sc.capacity_floats || groups > sc.n_counters)) continue;
-            const uint32_t wgs = groups * splits, rounds = (wgs + cus - 1u) / cus;
-            const float idle = 1.0f - (float)wgs / (float)(rounds * cus);
-            const float cost = (float)rounds * ((float)cps + 1.5f) * (1.0f + 0.5f * idle);
-            if (cost < best_cost) { best_cost = cost; best_tpw = tpw; best_splits = splits; best_cps = cps; }
-        }
-    }
+    const MtileSplit best = mtile_split(tiles, a.n_blocks, false, 0u, sc);
     // one tile per workgroup of 4 waves, two workgroups per CU: every workgroup converts all of X itself
     const float shared_rounds = (float)((tiles + 2u * cus - 1u) / (2u * cus));
-    const bool shared_tile = shared_rounds * ((float)n_chunks * 1.25f + 1.5f) < best_cost;
+    const bool shared_tile = shared_rounds * ((float)n_chunks * 1.25f + 1.5f) < best.cost;
 
     for (uint32_t m0 = 0; m0 < a.M; m0 += group) {
         MtileParams p;
@@ -1391,25 +1417,25 @@ hipError_t launch_mtile(const MatmulArgs& a, const SplitScratch& sc, hipStream_t
                 : q6 ? launch_mtile_one<KQ_TYPE_Q6_K, 4, 1>(p, tiles, 1, s)
                 : q5 ? launch_mtile_one<KQ_TYPE_Q5_K, 4, 1>(p, tiles, 1, s) : launch_mtile_one<KQ_TYPE_Q4_K, 4, 1>(p, tiles, 1, s);
         } else {
-            p.tiles_per_wg = best_tpw;
-            p.n_splits = best_splits;
-            p.chunks_per_split = best_cps;
-            const uint32_t wgs = (tiles + best_tpw - 1u) / best_tpw;
+            p.tiles_per_wg = best.per_wg;
+            p.n_splits = best.splits;
+            p.chunks_per_split = best.chunks;
+            const uint32_t wgs = (tiles + best.per_wg - 1u) / best.per_wg;
             // 5..8 tokens: the conversion of X is spread over twice the threads per (token, superblock), so
             // that all waves take part (measured +2-3 %; with 4 tokens or fewer the wider exchange costs more)
             // Q4_K / Q5_K with at most 8 tokens: hi and lo parts as token slots of one matrix instruction
             if (p.M > 4u && p.M <= 8u)
-                e = q6 ? launch_mtile_one<KQ_TYPE_Q6_K, 8, 8, true, 8>(p, wgs, 1, s, best_splits)
-                    : q5 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 8, false, 0, true>(p, wgs, 1, s, best_splits)
-                         : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 8, false, 0, true>(p, wgs, 1, s, best_splits);
+                e = q6 ? launch_mtile_one<KQ_TYPE_Q6_K, 8, 8, true, 8>(p, wgs, 1, s, best.splits)
+                    : q5 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 8, false, 0, true>(p, wgs, 1, s, best.splits)
+                         : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 8, false, 0, true>(p, wgs, 1, s, best.splits);
             else if (p.M <= 4u && !q6)
-                e = q5 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, false, 0, true>(p, wgs, 1, s, best_splits)
-                       : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, false, 0, true>(p, wgs, 1, s, best_splits);
+                e = q5 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, false, 0, true>(p, wgs, 1, s, best.splits)
+                       : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, false, 0, true>(p, wgs, 1, s, best.splits);
             else
-                e = q6_wide ? launch_mtile_one<MT_TYPE_Q6K_WIDE, 8, 8, true, 16>(p, wgs, 1, s, best_splits)
-                    : q6 ? launch_mtile_one<KQ_TYPE_Q6_K, 8, 8, true, 16>(p, wgs, 1, s, best_splits)
-                    : q5 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16>(p, wgs, 1, s, best_splits)
-                         : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16>(p, wgs, 1, s, best_splits);
+                e = q6_wide ? launch_mtile_one<MT_TYPE_Q6K_WIDE, 8, 8, true, 16>(p, wgs, 1, s, best.splits)
+                    : q6 ? launch_mtile_one<KQ_TYPE_Q6_K, 8, 8, true, 16>(p, wgs, 1, s, best.splits)
+                    : q5 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16>(p, wgs, 1, s, best.splits)
+                         : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16>(p, wgs, 1, s, best.splits);
         }
         if (e != hipSuccess) return e;
     }
@@ -1432,24 +1458,7 @@ hipError_t launch_mtile_fused(const MatmulArgs& a, const SplitScratch& sc, hipSt
 {
     const bool q6 = a.type == KQ_TYPE_Q6_K, q5 = a.type == KQ_TYPE_Q5_K, q6_wide = q6 && a.M > 8u;
     const uint32_t tiles = (a.N + 15u) / 16u;
-    const uint32_t n_chunks = (a.n_blocks + MT_KC - 1) / MT_KC;
-    const uint32_t cus = device_cu_count();
-    // the work split of launch_mtile; pairs take an even number of tiles per workgroup
-    uint32_t best_tpw = 8, best_splits = 1, best_cps = n_chunks;
-    float best_cost = 1e30f;
-    for (uint32_t tpw = 8; tpw >= 4; tpw -= a.epi ? 2u : 1u) {
-        const uint32_t groups = a.epi ? (tiles / 2u + tpw / 2u - 1u) / (tpw / 2u) : (tiles + tpw - 1u) / tpw;
-        for (uint32_t splits = 1; splits <= n_chunks && splits <= 16u; ++splits) {
-            const uint32_t cps = (n_chunks + splits - 1u) / splits;
-            if ((splits - 1u) * cps >= n_chunks) continue;   // a split would be empty
-            // (partial tiles, then 16 sums of squares per workgroup for the norm prologue)
-            if (splits > 1u && ((size_t)splits * 16u * groups * (tpw * 16u + 1u) > sc.capacity_floats || groups > sc.n_counters)) continue;
-            const uint32_t wgs = groups * splits, rounds = (wgs + cus - 1u) / cus;
-            const float idle = 1.0f - (float)wgs / (float)(rounds * cus);
-            const float cost = (float)rounds * ((float)cps + 1.5f) * (1.0f + 0.5f * idle);
-            if (cost < best_cost) { best_cost = cost; best_tpw = tpw; best_splits = splits; best_cps = cps; }
-        }
-    }
+    const MtileSplit best = mtile_split(tiles, a.n_blocks, a.epi != 0, 1u, sc);   // (16 sums of squares per workgroup for the norm prologue)
     MtileParams p;
     p.W2 = nullptr;
     p.X = (const float*)a.X;
@@ -1461,36 +1470,36 @@ hipError_t launch_mtile_fused(const MatmulArgs& a, const SplitScratch& sc, hipSt
     p.row_stride_bytes = a.row_stride_bytes;
     p.y_offset = a.y_offset;
     p.ldy = a.ldy;
-    p.tiles_per_wg = best_tpw;
+    p.tiles_per_wg = best.per_wg;
     p.tiles = nullptr; p.n_tiles = nullptr; p.tile_stride = 0; p.tile_iters = 1; p.k_slots = 1; p.x_per_slot = 0;
-    p.n_splits = best_splits; p.chunks_per_split = best_cps; p.partial = sc.partial; p.counters = sc.counters;
+    p.n_splits = best.splits; p.chunks_per_split = best.chunks; p.partial = sc.partial; p.counters = sc.counters;
     p.pro = a.pro; p.epi = a.epi; p.eps = a.eps; p.norm_w = a.norm_w; p.residual = a.residual;
     p.x_stride = a.pro >= 2 ? 2u * a.K : a.K;
     p.pair_tile0 = tiles / 2u;
-    const uint32_t wgs = a.epi ? (tiles / 2u + best_tpw / 2u - 1u) / (best_tpw / 2u) : (tiles + best_tpw - 1u) / best_tpw;
+    const uint32_t wgs = a.epi ? (tiles / 2u + best.per_wg / 2u - 1u) / (best.per_wg / 2u) : (tiles + best.per_wg - 1u) / best.per_wg;
     const bool hl8 = !q6 && a.M <= 8u;   // hi and lo parts as token slots of one matrix instruction
     if (a.pro == 1) {
-        if (q6_wide) return launch_mtile_one<MT_TYPE_Q6K_WIDE, 8, 8, true, 16, true, 1>(p, wgs, 1, s, best_splits);
-        if (q6) return launch_mtile_one<KQ_TYPE_Q6_K, 8, 8, true, 16, true, 1>(p, wgs, 1, s, best_splits);
-        if (q5) return hl8 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true, 1, true>(p, wgs, 1, s, best_splits)
-                           : launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true, 1>(p, wgs, 1, s, best_splits);
-        return hl8 ? launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true, 1, true>(p, wgs, 1, s, best_splits)
-                   : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true, 1>(p, wgs, 1, s, best_splits);
+        if (q6_wide) return launch_mtile_one<MT_TYPE_Q6K_WIDE, 8, 8, true, 16, true, 1>(p, wgs, 1, s, best.splits);
+        if (q6) return launch_mtile_one<KQ_TYPE_Q6_K, 8, 8, true, 16, true, 1>(p, wgs, 1, s, best.splits);
+        if (q5) return hl8 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true, 1, true>(p, wgs, 1, s, best.splits)
+                           : launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true, 1>(p, wgs, 1, s, best.splits);
+        return hl8 ? launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true, 1, true>(p, wgs, 1, s, best.splits)
+                   : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true, 1>(p, wgs, 1, s, best.splits);
     }
     if (a.pro != 0) {
         // (the 16-slot Q6_K kernel has no registers for a second operand: mtile_fused_supported declines)
-        if (q6) return launch_mtile_one<KQ_TYPE_Q6_K, 8, 8, true, 16, true, 2>(p, wgs, 1, s, best_splits);
-        if (q5) return hl8 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true, 2, true>(p, wgs, 1, s, best_splits)
-                           : launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true, 2>(p, wgs, 1, s, best_splits);
-        return hl8 ? launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true, 2, true>(p, wgs, 1, s, best_splits)
-                   : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true, 2>(p, wgs, 1, s, best_splits);
+        if (q6) return launch_mtile_one<KQ_TYPE_Q6_K, 8, 8, true, 16, true, 2>(p, wgs, 1, s, best.splits);
+        if (q5) return hl8 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true, 2, true>(p, wgs, 1, s, best.splits)
+                           : launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true, 2>(p, wgs, 1, s, best.splits);
+        return hl8 ? launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true, 2, true>(p, wgs, 1, s, best.splits)
+                   : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true, 2>(p, wgs, 1, s, best.splits);
     }
-    if (q6_wide) return launch_mtile_one<MT_TYPE_Q6K_WIDE, 8, 8, true, 16, true>(p, wgs, 1, s, best_splits);
-    if (q6) return launch_mtile_one<KQ_TYPE_Q6_K, 8, 8, true, 16, true>(p, wgs, 1, s, best_splits);
-    if (q5) return hl8 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true, 0, true>(p, wgs, 1, s, best_splits)
-                       : launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true>(p, wgs, 1, s, best_splits);
-    return hl8 ? launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true, 0, true>(p, wgs, 1, s, best_splits)
-               : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true>(p, wgs, 1, s, best_splits);
+    if (q6_wide) return launch_mtile_one<MT_TYPE_Q6K_WIDE, 8, 8, true, 16, true>(p, wgs, 1, s, best.splits);
+    if (q6) return launch_mtile_one<KQ_TYPE_Q6_K, 8, 8, true, 16, true>(p, wgs, 1, s, best.splits);
+    if (q5) return hl8 ? launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true, 0, true>(p, wgs, 1, s, best.splits)
+                       : launch_mtile_one<KQ_TYPE_Q5_K, 8, 8, true, 16, true>(p, wgs, 1, s, best.splits);
+    return hl8 ? launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true, 0, true>(p, wgs, 1, s, best.splits)
+               : launch_mtile_one<KQ_TYPE_Q4_K, 8, 8, true, 16, true>(p, wgs, 1, s, best.splits);
 }
 
 }  // namespace kq

@@ -999,11 +999,49 @@ static uint32_t groups_per_wg(uint32_t row_groups, uint32_t others, int type, ui
     return best;
 }
 
+// K is cut where the rows alone leave CUs idle (one workgroup per CU).  Prices in us, measured: a superblock of a
+// workgroup's walk 0.8 + 0.7 per tile of tokens (Q6_K 3 + 0.9), the launch that adds the splits 5, and its
+// traffic, written and read once, at 4 TB/s.  (Of the walk before this one; the choice is still within 4 % of the best of
+// eight forced ones on 80 calls, 20 to 128 tokens, Q4_K and Q6_K.)  splits: at most so many, 0 = the cheapest.
+static uint32_t wide_cut(int type, uint32_t tt, uint32_t row_groups, uint32_t token_groups, uint32_t n_blocks, size_t capacity_floats, int splits)
+{
+    const double step_us = type == KQ_TYPE_Q6_K ? 3.0 + 0.9 * tt : 0.8 + 0.7 * tt;
+    const size_t tile_floats = (size_t)token_groups * tt * 16u * row_groups * (WIDE_WAVES * 32u);
+    uint32_t z = 1;
+    double best = 1e30;
+    for (uint32_t c = 1; c <= n_blocks && c <= 16u; ++c) {
+        if (c > 1u && c * tile_floats > capacity_floats) break;
+        const uint32_t cus = device_cu_count(), rounds = (row_groups * token_groups * c + cus - 1u) / cus;
+        const double t = (double)rounds * ((n_blocks + c - 1u) / c) * step_us + (c > 1u ? 5.0 + 2e-6 * c * tile_floats : 0.0);
+        if (splits ? (uint32_t)splits >= c : t < best) { best = t; z = c; }
+    }
+    return z;
+}
+
 double wide_price_16(int type, uint32_t N, uint32_t n_blocks)
 {
     double us;
     groups_per_wg((N + 255u) / 256u, 1, type, 1, n_blocks, &us);
     return us + 4.0;   // (the split of X in front)
+}
+
+double wide_price_5_to_16(const MatmulArgs& a, const SplitScratch& sc)
+{
+    const uint32_t outs = a.epi ? a.N / 2u : a.N, per_wg = a.epi ? WIDE_WAVES * 16u : WIDE_WAVES * 32u, gx = (outs + per_wg - 1u) / per_wg;
+    const uint32_t cut = wide_cut(a.type, 1, gx, 1, a.n_blocks, sc.capacity_floats, 0), per = (a.n_blocks + cut - 1u) / cut, z = (a.n_blocks + per - 1u) / per;
+    double walk;
+    if (z > 1u) {
+        const WideWalk w = wide_walk(a.type, 1, per);
+        const uint32_t n = (gx * z + device_cu_count() - 1u) / device_cu_count();
+        walk = (double)(n / 2u * 2u) * (w.walk[1] + w.start[1]) + (double)(n % 2u) * (w.walk[0] + w.start[0]);
+    } else {
+        groups_per_wg(gx, 1, a.type, 1, a.n_blocks, &walk);
+    }
+    // The launches' sum, walk, the one that adds the splits and its floats, 10^6 outputs, a norm: fitted to 27000 timed calls of 5 to 16
+    // tokens (512 to 64000 rows, plain, with a norm, a residual, a norm and act * up), 5 to 6 % rms
+    const double c[3][6] = {{0.59, 0.78, 4.13, 2.96, 2.35, 0.68}, {0.78, 0.82, 3.96, 3.32, 2.77, 0.76}, {0.47, 0.81, 4.71, 2.21, 2.30, 0.73}};
+    const double* k = c[a.type == KQ_TYPE_Q4_K ? 0 : a.type == KQ_TYPE_Q5_K ? 1 : 2];
+    return k[0] + k[1] * walk + (z > 1u ? k[2] + k[3] * 1e-6 * z * 16.0 * gx * 256.0 : 0.0) + k[4] * 1e-6 * (double)a.M * outs + (a.pro == 1 ? k[5] : 0.0);
 }
 
 hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scratch, size_t x_bytes, int splits, hipStream_t s)
@@ -1029,20 +1067,7 @@ hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scra
         const uint32_t gy = (M + 63u) / 64u, tiles = (M + 15u) / 16u, tt = (tiles + gy - 1u) / gy;
         const uint32_t gy2 = (tiles + tt - 1u) / tt;
         const uint32_t per_wg = a.epi ? WIDE_WAVES * 16u : WIDE_WAVES * 32u, gx = (outs + per_wg - 1u) / per_wg;
-        // K is cut where the rows alone leave CUs idle (one workgroup per CU).  Prices in us, measured: a superblock of a
-        // workgroup's walk 0.8 + 0.7 per tile of tokens (Q6_K 3 + 0.9), the launch that adds the splits 5, and its
-        // traffic, written and read once, at 4 TB/s.  (Of the walk before this one; the choice is still within 4 % of the best of
-        // eight forced ones on 80 calls, 20 to 128 tokens, Q4_K and Q6_K.)
-        const double step_us = a.type == KQ_TYPE_Q6_K ? 3.0 + 0.9 * tt : 0.8 + 0.7 * tt;
-        const size_t tile_floats = (size_t)gy2 * tt * 16u * gx * (WIDE_WAVES * 32u);
-        uint32_t z = 1;
-        double best = 1e30;
-        for (uint32_t c = 1; c <= a.n_blocks && c <= 16u; ++c) {
-            if (c > 1u && c * tile_floats > sc.capacity_floats) break;
-            const uint32_t cus = device_cu_count(), rounds = (gx * gy2 * c + cus - 1u) / cus;
-            const double t = (double)rounds * ((a.n_blocks + c - 1u) / c) * step_us + (c > 1u ? 5.0 + 2e-6 * c * tile_floats : 0.0);
-            if (splits ? (uint32_t)splits >= c : t < best) { best = t; z = c; }
-        }
+        const uint32_t z = wide_cut(a.type, tt, gx, gy2, a.n_blocks, sc.capacity_floats, splits);
         p.blocks_per_split = (a.n_blocks + z - 1u) / z;
         p.n_splits = (a.n_blocks + p.blocks_per_split - 1u) / p.blocks_per_split;
         p.partial = sc.partial;

@@ -268,7 +268,8 @@ BPK_API int bpk_kq_matmul(int type, const float *X, const void *W,
  * (K <= 28672 for one token, K <= 14336 for two; N <= 32768) is one launch
  * and needs no workspace; so are verify batches, M <= 16, on the tile kernel
  * (X, W and norm_w 16-byte aligned; not Q6_K with M > 8 under an act * up
- * prologue).  Other shapes need `workspace` (device memory, 16-byte aligned, at
+ * prologue), but for calls of 5 to 16 tokens that are given the workspace and
+ * priced lower on the many-token kernel.  Other shapes need `workspace` (device memory, 16-byte aligned, at
  * least bpk_kq_matmul_fused_workspace_bytes(M, N, K) bytes) and fail with
  * BPK_ERR_WORKSPACE without it: they run the same function as prologue, matmul
  * and add launches through it, or, where the many-token kernel takes the call

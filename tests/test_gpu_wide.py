@@ -823,3 +823,41 @@ def test_moe_records_in_a_second_dimension_of_the_grid(gpu, grid):  # noqa: F811
         assert np.array_equal(got, want)
     with pytest.raises(capi.BpkError):
         capi.set_option("moe_grid", 12)      # not a multiple of the XCDs
+
+
+@pytest.mark.parametrize("type_,M,N,K,pro,epi,res,form", [
+    (Q4_K, 16, 28672, 4096, 1, 2, False, "many_token"), (Q6_K, 16, 4096, 14336, 0, 0, True, "many_token"), (Q6_K, 9, 4096, 14336, 0, 0, True, "many_token"),
+    (Q4_K, 16, 4096, 4096, 0, 0, True, None), (Q4_K, 8, 6144, 4096, 1, 0, False, None), (Q5_K, 12, 36896, 1024, 1, 3, False, "many_token"),
+    (Q6_K, 13, 35999, 1024, 0, 0, False, "many_token"), (Q5_K, 13, 20817, 4608, 0, 0, False, "many_token"), (Q4_K, 5, 700, 512, 1, 0, True, None)])
+def test_dispatch_of_5_to_16_tokens(gpu, type_, M, N, K, pro, epi, res, form):  # noqa: F811
+    """The many-token kernel where it is priced below the tiles, both ways the same function: against the tile kernel, which splits x
+    into the same 22 bits; without a workspace a fused call stays one launch."""
+    import torch
+    from backpack_amd import capi, kquant
+    print("5 to 16 tokens", type_, M, N, K, pro, epi, res, flush=True)
+    _, _, w = gpu.make_weight(type_, N, K, seed=M)
+    rng = np.random.default_rng(N)
+    X = gpu.dev(rng.standard_normal((M, K)).astype(np.float32))
+    nw = gpu.dev((1 + 0.1 * rng.standard_normal(K)).astype(np.float32)) if pro == 1 else None
+    R = gpu.dev(rng.standard_normal((M, N)).astype(np.float32)) if res else None
+    fused = pro or epi or res
+
+    def call(**k):
+        return kquant.matmul_fused(X, w, pro, norm_w=nw, eps=1e-5, residual=R, epilogue=epi, **k) if fused else kquant.matmul(X, w)
+    got = call()
+    assert (capi.last_kernel(), capi.last_form()) == (("mtile", form) if form or not fused else ("mtile_fused", ""))
+    capi.force_kernel(6)
+    try:
+        tile = call()
+    finally:
+        capi.force_kernel(0)
+    if fused:
+        one = call(allow_workspace=False)
+        assert capi.last_kernel() == "mtile_fused" and torch.equal(one, tile)
+    if res:      # in place
+        y = R.clone()
+        kquant.matmul_fused(X, w, pro, norm_w=nw, eps=1e-5, residual=y, out=y)
+        assert torch.equal(y, got)
+    rms = float(tile.double().pow(2).mean().sqrt())
+    # two 22-bit splits of x, fp32 sums in another order; an activation multiplies two such
+    assert float((got - tile).abs().max()) <= 4e-5 * (rms + float(tile.abs().max()))
