@@ -1389,8 +1389,12 @@ hipError_t launch_mtile(const MatmulArgs& a, const SplitScratch& sc, hipStream_t
     const uint32_t n_chunks = (a.n_blocks + MT_KC - 1) / MT_KC;
     const uint32_t cus = device_cu_count();
     const MtileSplit best = mtile_split(tiles, a.n_blocks, false, 0u, sc);
-    // one tile per workgroup of 4 waves, two workgroups per CU: every workgroup converts all of X itself
-    const float shared_rounds = (float)((tiles + 2u * cus - 1u) / (2u * cus));
+    // One tile per workgroup of 4 waves: every workgroup converts all of X itself, and a CU takes one of them at a time.  Up to a tile per CU
+    // that beats the split (up to 1024 columns, 12 tokens: Q4_K 1.08 to 1.21 times as long on the split, Q5_K 1.15 to 1.32, Q6_K 1.4 to 1.7);
+    // with more tiles than CUs it loses (4097..8192 rows, 256..1024 columns, 3..24 tokens: Q4_K 1.4 to 1.9 times the split's time, Q5_K 1.3 to
+    // 1.8, Q6_K 1.03 to 1.5; Q4_K, 8192x768, 8 tokens: 10.0 us, 6.0 on the split;
+    // Q6_K 11.0 and 9.2).
+    const float shared_rounds = (float)((tiles + cus - 1u) / cus);
     const bool shared_tile = shared_rounds * ((float)n_chunks * 1.25f + 1.5f) < best.cost;
 
     for (uint32_t m0 = 0; m0 < a.M; m0 += group) {

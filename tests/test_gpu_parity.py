@@ -114,6 +114,22 @@ def test_four_token_stream_kernels(gpu, kqo, type_, M, N, K):
     gpu.check_matmul(kqo, type_, got[:M], X, packed, N, K, bias=bias, label=f"four {type_} {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("type_", [Q4_K, Q5_K, Q6_K])
+@pytest.mark.parametrize("M,N,K", [(3, 4096, 256), (5, 4097, 256), (8, 4112, 1024), (16, 4096, 1024), (12, 8191, 512), (24, 4200, 768)])
+def test_tiles_around_one_per_cu(gpu, kqo, type_, M, N, K):
+    """The tile kernel on either side of a tile per compute unit (256 of 16 rows), where its form changes."""
+    from backpack_amd import capi, kquant
+    _say("tiles around one per CU", type_, M, N, K)
+    raw, packed, w = gpu.make_weight(type_, N, K, seed=M + N)
+    X = np.random.default_rng(K).standard_normal((M, K)).astype(np.float32)
+    capi.force_kernel(6)
+    try:
+        got = kquant.matmul(gpu.dev(X), w).cpu().numpy()
+    finally:
+        capi.force_kernel(0)
+    gpu.check_matmul(kqo, type_, got, X, packed, N, K, label=f"{type_} {M}x{N}x{K}", slack=2e-5)
+
+
 # ---- Q5_K: the fp32 matmul's automatic choice (lanes-along-K kernel, tile kernel, generic) ---------
 @pytest.mark.parametrize("M,N,K,kernel", [(1, 300, 4096, "gemv_stream"), (2, 64, 768, "gemv_stream"),
                                           (1, 4096, 4096, "gemv_stream"), (2, 6144, 4096, "gemv_stream"),
