@@ -37,7 +37,7 @@ struct StreamDense {          // 64 bytes = the 16 dwords that kernel-argument p
     const float* bias;
     float* Y;
     uint32_t N, K, n_blocks, row_stride_bytes, y_offset, ldy;
-    uint32_t M;   // tokens; read only by the four-token kernels (three tokens run as four, the last one masked)
+    uint32_t M;   // tokens; a kernel's are its MT, only the combining launch reads this (its slots per token)
     uint32_t grid_x;   // workgroups of the launch along x (as an argument: the hidden one would be a fetch of its own)
     static constexpr bool kGrouped = false, kFused = false, kCombine = false;
 };
@@ -208,7 +208,8 @@ template <int P, int NW, int D, int MT, typename PT, bool Q5 = false, int KW = 1
 __device__ __forceinline__ void q4k_stream_body(PT p)
 {
     stream_select_pair(p);
-    __shared__ float part[KW > 1 ? KW * NW : 1][MT][64];
+    constexpr bool QUAD = MT > 2;   // three or four tokens: each row's sums wait in LDS for the end of the chunk
+    __shared__ float part[KW > 1 || QUAD ? KW * NW : 1][QUAD ? 64 : MT][QUAD ? 4 : 64];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // NW > 1 and KW > 1 together: the workgroup is KW K slices x NW walkers; the walkers of a slice share its
@@ -267,8 +268,7 @@ __device__ __forceinline__ void q4k_stream_body(PT p)
             hoff[pass] = b * BLOCK;
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                const uint32_t xt = MT > 2 ? min((uint32_t)t, p.M - 1u) : (uint32_t)t;   // a masked token re-reads the last one
-                const float4* xp = (const float4*)(p.X + (size_t)xt * ldx + (size_t)b * KQ_QK + 64u * g + 16u * h);
+                const float4* xp = (const float4*)(p.X + (size_t)t * ldx + (size_t)b * KQ_QK + 64u * g + 16u * h);
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     float4 lo = stream_x4<PRO, PT::kFused>(xp + i, x2_off), hi = stream_x4<PRO, PT::kFused>(xp + 8 + i, x2_off);
@@ -342,8 +342,7 @@ __device__ __forceinline__ void q4k_stream_body(PT p)
             const size_t at = (size_t)b * KQ_QK + 64u * g + 16u * h + 32u * (q >> 2) + 4u * (q & 3u);
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
-                const uint32_t xt = MT > 2 ? min((uint32_t)t, p.M - 1u) : (uint32_t)t;   // a masked token re-reads the last one
-                const float* xp = p.X + (size_t)xt * ldx + at;
+                const float* xp = p.X + (size_t)t * ldx + at;
                 ring_load16(xr[t][k], (const uint8_t*)xp);
                 if constexpr (EXTRA) {
                     const float* ep = pro_rt == STREAM_PRO_NORM ? stream_norm_w(p) + at
@@ -459,6 +458,7 @@ __device__ __forceinline__ void q4k_stream_body(PT p)
 #pragma unroll
             for (int d = 0; d < D; ++d) {
                 const uint32_t i = i0 + d;
+                if (QUAD && d && i >= cnt) break;   // (nothing waits on the ring any more but its drain)
                 ring[d].template wait<(D - 1) * SLOT_LOADS>();
                 float acc[MT];
 #pragma unroll
@@ -469,9 +469,13 @@ __device__ __forceinline__ void q4k_stream_body(PT p)
                                           xs_hi[pass], sel_hi, sh, acc, ring[d].qh[Q5 ? pass : 0], 2u * g);
                 ring[d].fill(p.W + row_of(c0 + i + D) * p.row_stride_bytes, hoff, j);
 #pragma unroll
-                for (int t = 0; t < MT; ++t) {
+                for (int t = 0; t < (QUAD ? 0 : MT); ++t) {
                     const float tot = wave_sum(acc[t]);
                     res[t] = (lane == i && i < cnt) ? tot : res[t];
+                }
+                if constexpr (QUAD) {
+                    const float tot = quad_sum(acc);
+                    if (!(lane & 15u)) part[slice * NW + walker][i][lane >> 4] = tot;
                 }
             }
         }
@@ -479,8 +483,10 @@ __device__ __forceinline__ void q4k_stream_body(PT p)
         // differ by a chunk; a wave that has ended no longer counts at a barrier.)
         if (KW > 1) {
 #pragma unroll
-            for (int t = 0; t < MT; ++t) part[slice * NW + walker][t][lane] = res[t];
+            for (int t = 0; t < (QUAD ? 0 : MT); ++t) part[slice * NW + walker][t][lane] = res[t];
             lds_barrier();
+        } else if (QUAD) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the lanes' writes of this wave
         }
         // (the lane guard stays outside: with it inside, the gate|up launch measured 3 us slower.  In pair
         // mode cnt is even, so a lane inside the guard finds its partner there too.)
@@ -490,10 +496,10 @@ __device__ __forceinline__ void q4k_stream_body(PT p)
 #pragma unroll
             for (int t = 0; t < MT; ++t) {
                 float y = res[t];
-                if (KW > 1) {
-                    y = part[walker][t][lane];
+                if (KW > 1 || QUAD) {
+                    y = QUAD ? part[walker][lane][t] : part[walker][t][lane];
 #pragma unroll
-                    for (int w = 1; w < KW; ++w) y += part[w * NW + walker][t][lane];
+                    for (int w = 1; w < KW; ++w) y += QUAD ? part[w * NW + walker][lane][t] : part[w * NW + walker][t][lane];
                 }
                 if constexpr (PT::kFused) y *= t == 0 ? rstd0 : rstd1;
                 y += bias;
@@ -505,7 +511,6 @@ __device__ __forceinline__ void q4k_stream_body(PT p)
                     if (!(lane & 1u)) p.Y[(size_t)t * p.ldy + p.y_offset + r] = y;
                     continue;
                 }
-                if (MT > 2 && (uint32_t)t >= p.M) continue;
                 const size_t at = (size_t)t * p.ldy + p.y_offset + r;
                 if constexpr (PT::kFused) y += stream_residual(p) ? stream_residual(p)[at] : 0.0f;
                 p.Y[at] = y;
@@ -538,7 +543,8 @@ __device__ __forceinline__ void q6k_stream_body(PT p)
     constexpr bool COMBINE = PT::kCombine;   // the waves are a token's slots, not K slices
     static_assert(RW == 1 || (RW == 2 && (COMBINE || (PT::kGrouped && KW == 1)) && P == 1 && MT == 1),
                   "two rows per step: the combining launch, or a grouped one whose rows one wave walks");
-    __shared__ float part[KW > 1 ? KW : 1][MT][64];
+    constexpr bool QUAD = MT > 2;
+    __shared__ float part[KW][QUAD ? 64 : MT][QUAD ? 4 : 64];
     const uint32_t lane = threadIdx.x & 63u;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t slots = COMBINE ? min(p.M, (uint32_t)KW) : (uint32_t)KW;   // (a combining launch passes its slots per token in M)
@@ -578,8 +584,7 @@ __device__ __forceinline__ void q6k_stream_body(PT p)
             boff[pass] = b * KQ_Q6K_BYTES;
 #pragma unroll
             for (int tk = 0; tk < MT; ++tk) {
-                const uint32_t xt = MT > 2 ? min((uint32_t)tk, p.M - 1u) : (uint32_t)tk;
-                const float4* xp = (const float4*)(p.X + (size_t)xt * ldx + (size_t)b * KQ_QK + 128u * n + 8u * lg);
+                const float4* xp = (const float4*)(p.X + (size_t)tk * ldx + (size_t)b * KQ_QK + 128u * n + 8u * lg);
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     float4 lo = stream_x4<PRO, PT::kFused>(xp + 8 * k, x2_off), hi = stream_x4<PRO, PT::kFused>(xp + 8 * k + 1, x2_off);
@@ -652,6 +657,7 @@ __device__ __forceinline__ void q6k_stream_body(PT p)
 #pragma unroll
             for (int d = 0; d < D; ++d) {
                 const uint32_t i = i0 + d;   // step of the chunk: row i, or (RW = 2) rows 2i and 2i + 1
+                if (QUAD && d && i >= cnt) break;
                 ring[d].template wait<(D - 1) * SLOT_LOADS>();
                 float acc[MT];
 #pragma unroll
@@ -670,17 +676,23 @@ __device__ __forceinline__ void q6k_stream_body(PT p)
                     res[0] = lane == 2u * i ? q0 + q1 : lane == 2u * i + 1u ? q2 + q3 : res[0];   // (rows past cnt are not stored)
                 } else {
 #pragma unroll
-                    for (int tk = 0; tk < MT; ++tk) {
+                    for (int tk = 0; tk < (QUAD ? 0 : MT); ++tk) {
                         const float tot = wave_sum(acc[tk]);
                         res[tk] = (lane == i && i < cnt) ? tot : res[tk];
+                    }
+                    if constexpr (QUAD) {
+                        const float tot = quad_sum(acc);
+                        if (!(lane & 15u)) part[wave][i][lane >> 4] = tot;
                     }
                 }
             }
         }
         if (KW > 1) {
 #pragma unroll
-            for (int tk = 0; tk < MT; ++tk) part[wave][tk][lane] = COMBINE ? slot_wt * res[tk] : res[tk];
+            for (int tk = 0; tk < (QUAD ? 0 : MT); ++tk) part[wave][tk][lane] = COMBINE ? slot_wt * res[tk] : res[tk];
             __syncthreads();
+        } else if (QUAD) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         }
         if (wave == 0 && lane < cnt) {
             const uint32_t r = g + (c0 + lane) * stride;
@@ -688,13 +700,12 @@ __device__ __forceinline__ void q6k_stream_body(PT p)
 #pragma unroll
             for (int tk = 0; tk < MT; ++tk) {
                 float y = res[tk];
-                if (KW > 1) {
-                    y = part[0][tk][lane];
+                if (KW > 1 || QUAD) {
+                    y = QUAD ? part[0][lane][tk] : part[0][tk][lane];
 #pragma unroll
                     for (int w = 1; w < KW; ++w)
-                        if (!COMBINE || (uint32_t)w < slots) y += part[w][tk][lane];
+                        if (!COMBINE || (uint32_t)w < slots) y += QUAD ? part[w][lane][tk] : part[w][tk][lane];
                 }
-                if (!COMBINE && MT > 2 && (uint32_t)tk >= p.M) continue;
                 const size_t at = (size_t)tk * p.ldy + p.y_offset + r;
                 if constexpr (PT::kFused) y *= tk == 0 ? rstd0 : rstd1;
                 y += bias;
@@ -864,8 +875,12 @@ static void launch_q4k_sliced(dim3 grid, hipStream_t s, const PT& p)
 
 // Three or four tokens (dense calls): every wave holds a K slice of eight superblocks for four tokens (128
 // activations per lane), so rows of any length up to 56 superblocks are cut over 1, 2, 4 or 7 waves; two
-// rows in flight.  Three tokens run as four with the last one masked.
-template <typename PT>
+// rows in flight.  At this many tokens the vector units bound the loop, not the weights: three tokens have a
+// form of their own, a walker's last step is not run for a row that is not there, and quad_sum adds up all
+// tokens of a row at once.  Q5_K 5003 x 2816, 3 tokens: 10.1 us as four masked tokens, 8.6 as three, 7.9
+// without the absent row, 7.5 with the sums; Q4_K 4096 x 8192 12.6 -> 9.6, Q6_K 4096 x 14336 20.4 -> 17.4;
+// four tokens: Q4_K 4096 x 4096 7.6 -> 7.1, 5003 x 4096 9.5 -> 8.0, Q5_K 2000 x 14336 13.3 -> 12.5.
+template <int T, typename PT>
 static hipError_t launch_stream_four(const MatmulArgs& a, hipStream_t s, const PT& p)
 {
     const uint32_t nb = a.n_blocks;
@@ -878,27 +893,27 @@ static hipError_t launch_stream_four(const MatmulArgs& a, hipStream_t s, const P
         const dim3 grid4(wgs4, 1, 1);
         const bool q5 = a.type == KQ_TYPE_Q5_K;
         if (kw == 1) {
-            if (q5) launch_q4k_entry<1, 4, 2, 4, true, 1>(grid4, dim3(256), s, p);
-            else launch_q4k_entry<1, 4, 2, 4, false, 1>(grid4, dim3(256), s, p);
+            if (q5) launch_q4k_entry<1, 4, 2, T, true, 1>(grid4, dim3(256), s, p);
+            else launch_q4k_entry<1, 4, 2, T, false, 1>(grid4, dim3(256), s, p);
         } else {
-            if (q5) launch_q4k_entry<1, 4, 2, 4, true, 2>(grid4, dim3(512), s, p);
-            else launch_q4k_entry<1, 4, 2, 4, false, 2>(grid4, dim3(512), s, p);
+            if (q5) launch_q4k_entry<1, 4, 2, T, true, 2>(grid4, dim3(512), s, p);
+            else launch_q4k_entry<1, 4, 2, T, false, 2>(grid4, dim3(512), s, p);
         }
         return hipGetLastError();
     }
     const uint32_t wgs = stream_workgroups(a.N, kw >= 7 ? 1u : 8u / (uint32_t)kw, 0);
     const dim3 grid(wgs, 1, 1);
     if (a.type == KQ_TYPE_Q6_K) {
-        if (kw == 1) launch_q6k_entry<1, 1, 2, 4>(grid, dim3(64), s, p);
-        else if (kw == 2) launch_q6k_entry<1, 2, 2, 4>(grid, dim3(128), s, p);
-        else if (kw == 4) launch_q6k_entry<1, 4, 2, 4>(grid, dim3(256), s, p);
-        else launch_q6k_entry<1, 7, 2, 4>(grid, dim3(448), s, p);
+        if (kw == 1) launch_q6k_entry<1, 1, 2, T>(grid, dim3(64), s, p);
+        else if (kw == 2) launch_q6k_entry<1, 2, 2, T>(grid, dim3(128), s, p);
+        else if (kw == 4) launch_q6k_entry<1, 4, 2, T>(grid, dim3(256), s, p);
+        else launch_q6k_entry<1, 7, 2, T>(grid, dim3(448), s, p);
     } else if (a.type == KQ_TYPE_Q5_K) {
-        if (kw == 4) launch_q4k_entry<1, 1, 2, 4, true, 4>(grid, dim3(256), s, p);
-        else launch_q4k_entry<1, 1, 2, 4, true, 7>(grid, dim3(448), s, p);
+        if (kw == 4) launch_q4k_entry<1, 1, 2, T, true, 4>(grid, dim3(256), s, p);
+        else launch_q4k_entry<1, 1, 2, T, true, 7>(grid, dim3(448), s, p);
     } else {
-        if (kw == 4) launch_q4k_entry<1, 1, 2, 4, false, 4>(grid, dim3(256), s, p);
-        else launch_q4k_entry<1, 1, 2, 4, false, 7>(grid, dim3(448), s, p);
+        if (kw == 4) launch_q4k_entry<1, 1, 2, T, false, 4>(grid, dim3(256), s, p);
+        else launch_q4k_entry<1, 1, 2, T, false, 7>(grid, dim3(448), s, p);
     }
     return hipGetLastError();
 }
@@ -909,7 +924,7 @@ static hipError_t launch_stream_with(const MatmulArgs& a, const GemvTuning& t, h
 {
     const bool two = !PT::kGrouped && a.M == 2;       // two tokens share every weight load
     if constexpr (!PT::kGrouped && !PT::kFused) {
-        if (a.M > 2) return launch_stream_four(a, s, p);
+        if (a.M > 2) return a.M == 3 ? launch_stream_four<3>(a, s, p) : launch_stream_four<4>(a, s, p);
     }
     // Measured on MI355X: these kernels run best with about 40 KB of weight loads
     // in flight per CU: 4 to 8 waves, two to four rows in flight each.  More waves
