@@ -114,6 +114,28 @@ def test_four_token_stream_kernels(gpu, kqo, type_, M, N, K):
     gpu.check_matmul(kqo, type_, got[:M], X, packed, N, K, bias=bias, label=f"four {type_} {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("type_,M,N,K", [
+    (Q4_K, 3, 67593, 256), (Q5_K, 4, 67593, 256), (Q6_K, 3, 133121, 256), (Q6_K, 4, 133121, 256),    # a chunk of 64 rows per walker and a last one
+    (Q4_K, 4, 5003, 2816), (Q5_K, 3, 5003, 2816), (Q6_K, 4, 5003, 2816), (Q4_K, 3, 1281, 8192), (Q6_K, 3, 769, 14336),   # K slices, odd rows
+    (Q4_K, 1, 5003, 2816), (Q5_K, 1, 5003, 2816), (Q6_K, 1, 5003, 2816), (Q4_K, 1, 3, 256), (Q6_K, 4, 1, 256)])
+def test_odd_rows_per_walker(gpu, kqo, type_, M, N, K):
+    """The lanes-along-K kernel where a walker's last step has one row, and past a chunk of 64 rows."""
+    from backpack_amd import capi, kquant
+    _say("odd rows per walker", type_, M, N, K)
+    raw, packed, w = gpu.make_weight(type_, N, K, seed=M + N)
+    X = np.random.default_rng(K).standard_normal((M, K)).astype(np.float32)
+    out = gpu.dev(np.full((M + 1, N), 7.5, np.float32))
+    capi.force_kernel(5)
+    try:
+        kquant.matmul(gpu.dev(X), w, out=out[:M])
+        assert capi.last_kernel() == "gemv_stream"
+    finally:
+        capi.force_kernel(0)
+    got = out.cpu().numpy()
+    assert np.all(got[M] == 7.5)
+    gpu.check_matmul(kqo, type_, got[:M], X, packed, N, K, label=f"{type_} {M}x{N}x{K}")
+
+
 @pytest.mark.parametrize("type_", [Q4_K, Q5_K, Q6_K])
 @pytest.mark.parametrize("M,N,K", [(3, 4096, 256), (5, 4097, 256), (8, 4112, 1024), (16, 4096, 1024), (12, 8191, 512), (24, 4200, 768)])
 def test_tiles_around_one_per_cu(gpu, kqo, type_, M, N, K):
