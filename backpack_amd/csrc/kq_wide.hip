@@ -32,10 +32,11 @@
 // stand between the matrix instructions of the step before (sched_group_barrier), and the two meetings per superblock lie
 // ahead of a step whose operands are already in registers.  What that replaced: every lane fetched its 16-byte pieces
 // of W and X itself (52 cache accesses per load instruction, 20 now) and the compiler read operands right ahead of their
-// use.  A matrix instruction holds a SIMD's issue for 8 cycles and a vector one for 4, so beside two vector instructions each they
-// no longer overlap: in the launches of 2048 tokens (128 experts x 8, 2048 / 768, 64 pairs per record) issue takes 60 % of the
-// clocks (Q4_K; Q6_K 59 %), the matrix cores are busy 45 % (37 %); the rest are waits (0.28 and 0.31 of the waves' cycles),
-// workgroups' starts and the last round.  With one tile of 16 tokens a step is too short for the fixed order (`schedule`).
+// use.  What is left at 32 tokens and more is the board's power: with all CUs in these kernels the clock falls to 1.55 .. 1.78 GHz of 2.4
+// (s_memtime against s_memrealtime), so taking stalls or cheap instructions out changes little (the same walk with W a step earlier in
+// registers: +1 %), fewer matrix instructions or less switching on the vector units does (v_perm for the Q6_K fields: 31 -> 24 vector
+// instructions per eight weights, 5 to 7 % of its launches).  At 16 tokens and fewer it is the memory: 144 and 210 B pieces of rows reach 83
+// to 92 % of a contiguous read.  With one tile of 16 tokens a step is too short for the fixed order (`schedule`).
 //
 // A workgroup may walk several groups of 256 rows against the same tokens as one sequence of superblocks (groups_per_wg): its
 // start (records, addresses, the first loads' way: 8 us of 25 .. 40) is paid once and a group's stores go under the next
@@ -43,8 +44,8 @@
 //
 // Mixture layers (records of pairs of one expert): consecutive workgroups go to the same XCD, so a record's row groups
 // and an expert's records meet their X and W in that L2 (128 experts x 8 slots, 2048 / 768, 2048 tokens: 750 -> 703 us).
-// us with the router, now / with the walk before / on the 16-token tiles: 2048 tokens 561 / 739 / 1264, 256 tokens
-// 168 / 191 / 267, 24 tokens 123 / 128 / 153.
+// us with the router, now / with the walk before / on the 16-token tiles: 2048 tokens 547 / 739 / 1264, 256 tokens
+// 158 / 191 / 267, 24 tokens 117 / 128 / 153.
 #include "kq_format.h"
 #include "kq_gemm_plan.h"
 #include "kq_group.h"
