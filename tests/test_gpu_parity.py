@@ -114,6 +114,20 @@ def test_four_token_stream_kernels(gpu, kqo, type_, M, N, K):
     gpu.check_matmul(kqo, type_, got[:M], X, packed, N, K, bias=bias, label=f"four {type_} {M}x{N}x{K}")
 
 
+@pytest.mark.parametrize("M,N,K,kernel", [(3, 40001, 1024, "gemv_stream"), (4, 40001, 1024, "mtile"), (3, 40001, 768, "mtile"),
+                                          (3, 32769, 2048, "gemv_stream"), (3, 40001, 4608, "mtile")])
+def test_q6k_three_tokens_beyond_four(gpu, kqo, M, N, K, kernel):
+    """Three tokens of Q6_K stay on the lanes-along-K kernel where four go to the tiles."""
+    from backpack_amd import capi, kquant
+    _say("q6k three tokens", M, N, K)
+    raw, packed, w = gpu.make_weight(Q6_K, N, K, seed=M + N)
+    X = np.random.default_rng(K).standard_normal((M, K)).astype(np.float32)
+    y = kquant.matmul(gpu.dev(X), w)
+    assert capi.last_kernel() == kernel
+    if N * K <= 80 << 20:      # (the oracle's time and memory)
+        gpu.check_matmul(kqo, Q6_K, y.cpu().numpy(), X, packed, N, K, label=f"{M}x{N}x{K}", slack=2e-5 if kernel == "mtile" else 1e-6)
+
+
 @pytest.mark.parametrize("type_,M,N,K", [
     (Q4_K, 3, 67593, 256), (Q5_K, 4, 67593, 256), (Q6_K, 3, 133121, 256), (Q6_K, 4, 133121, 256),    # a chunk of 64 rows per walker and a last one
     (Q4_K, 4, 5003, 2816), (Q5_K, 3, 5003, 2816), (Q6_K, 4, 5003, 2816), (Q4_K, 3, 1281, 8192), (Q6_K, 3, 769, 14336),   # K slices, odd rows
