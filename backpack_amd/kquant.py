@@ -17,24 +17,24 @@ from . import capi
 from .capi import Q4_K, Q5_K, Q6_K  # noqa: F401
 
 
-_bound = None     # the library whose functions the native calls go to
-_calls = None
+_bound = (None, None)     # the library whose functions the native calls go to, and their module: one name, so that no thread sees half
 
 
 def _native():
     """The native form of the calls below (csrc/host/torch_calls.cpp), on the library that capi has loaded.  It returns NotImplemented
     for what is not a plain call, ahead of any effect: the Python form then takes or refuses it."""
-    global _bound, _calls
+    global _bound
     lib = capi.lib()
-    if lib is not _bound:
+    bound, calls = _bound
+    if lib is not bound:
         import ctypes as C
 
-        from . import _torch_calls     # built with the library; missing, this raises
+        from . import _torch_calls as calls     # built with the library; missing, this raises
         names = ("bpk_kq_matmul", "bpk_kq_matmul_bf16", "bpk_kq_matmul_fused", "bpk_kq_matmul_fused_workspace_bytes", "bpk_kq_matmul_argmax",
                  "bpk_prefill_rows_bf16", "bpk_kq_dequant_rows", "bpk_moe_route", "bpk_kq_moe_ffn", "bpk_kq_moe_ffn_scratch_bytes")
-        _torch_calls.bind([C.cast(getattr(lib, n), C.c_void_p).value for n in names], capi.check)
-        _bound, _calls = lib, _torch_calls
-    return _calls
+        calls.bind([C.cast(getattr(lib, n), C.c_void_p).value for n in names], capi.check)
+        _bound = (lib, calls)
+    return calls
 
 
 def _stream() -> int:

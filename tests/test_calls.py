@@ -1,5 +1,9 @@
 """The native form of kquant's calls (csrc/host/torch_calls.cpp): it takes plain calls and gives what the Python form gives, and leaves
 everything else to the Python form, which accepts or refuses it as it did."""
+import importlib.util
+import sys
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -65,6 +69,39 @@ def test_calls_on_host_tensors_are_refused_as_before(both):
                  (kquant.prefill_rows_bf16, (torch.zeros(1, 256), 256)), (kquant.dequant_rows, (w, torch.zeros(3, dtype=torch.int32)))):
         n, g, took = both(f, *a)
         assert not took and n[0] == g[0] == "raised" and n[1] is g[1] is AssertionError
+
+
+def test_native_calls_are_there_for_every_thread_at_every_moment():
+    """Between any two instructions of a thread's first call another thread's call gets the native module."""
+    from backpack_amd import kquant as loaded
+    spec = importlib.util.spec_from_file_location("backpack_amd.kquant_once_more", loaded.__file__)
+    kquant = importlib.util.module_from_spec(spec)       # as it is ahead of its first call
+    sys.modules[spec.name] = kquant                      # (its dataclass looks its module up)
+    spec.loader.exec_module(kquant)
+    state, asked = vars(kquant), []
+
+    def another_thread():
+        got, before = [], dict(state)
+        t = threading.Thread(target=lambda: got.append(kquant._native()))
+        t.start()
+        t.join()
+        state.update(before)      # (the traced call goes on as if alone)
+        asked.append(got[0])
+
+    def trace(frame, event, arg):
+        if frame.f_code is not kquant._native.__code__:
+            return None
+        frame.f_trace_opcodes = True
+        if event == "opcode":
+            another_thread()
+        return trace
+    sys.settrace(trace)
+    try:
+        mine = kquant._native()
+    finally:
+        sys.settrace(None)
+        del sys.modules[spec.name]
+    assert mine is not None and len(asked) > 20 and all(a is mine for a in asked)
 
 
 @pytest.mark.gpu
