@@ -1,10 +1,12 @@
 """Builds backpack_amd/libbpk_kquant.so from backpack_amd/csrc/*.hip with hipcc
-for gfx950.  Run as `python -m backpack_amd.build`; hipcc cross-compiles, so no
-GPU is needed."""
+for gfx950 and, where torch is installed, backpack_amd/_torch_calls.so, which
+kquant.py needs.  Run as `python -m backpack_amd.build`; hipcc cross-compiles, so
+no GPU is needed."""
 from __future__ import annotations
 
 import concurrent.futures as cf
 import glob
+import importlib.util
 import os
 import re
 import subprocess
@@ -196,7 +198,8 @@ def _compile(src: str) -> str:
     return obj
 
 
-def build_library(jobs: int = 8) -> str:
+def build_kernels(jobs: int = 8) -> str:
+    """backpack_amd/libbpk_kquant.so"""
     os.makedirs(OBJ, exist_ok=True)
     check_compiler()
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
@@ -224,13 +227,16 @@ def build_calls() -> str:
     return CALLS
 
 
-def build_all() -> str:
+def build_library(jobs: int = 8) -> str:
+    """Everything that the package loads; a host of the C ABI without torch gets its library alone."""
+    if importlib.util.find_spec("torch") is None:
+        return build_kernels(jobs)
     with cf.ThreadPoolExecutor(max_workers=2) as ex:
         calls = ex.submit(build_calls)
-        lib = build_library()
+        lib = build_kernels(jobs)
         calls.result()
     return lib
 
 
 if __name__ == "__main__":
-    print(build_all())
+    print(build_library())

@@ -84,3 +84,21 @@ def test_generated_code_of_the_library_was_checked():
     if os.path.exists(path):
         assert "; ringld" in open(path).read()
         assert b.check_ring_registers(path) == [] and b.check_ring_order(path) == []
+
+
+def test_build_library_makes_what_the_package_loads(monkeypatch):
+    """build_library() alone gives a package whose calls work; without torch, which only the binding needs, the C library is built."""
+    made = []
+    monkeypatch.setattr(b, "_compile", lambda src: made.append("object") or "x.o")
+    monkeypatch.setattr(b, "check_compiler", lambda: None)
+
+    class Done:
+        returncode, stderr, stdout = 0, "", ""
+    monkeypatch.setattr(b.subprocess, "run", lambda cmd, **k: made.append(cmd[cmd.index("-o") + 1]) or Done())
+    assert b.build_library() == b.LIB
+    assert {b.LIB, b.CALLS} <= set(made) and "object" in made
+    made.clear()
+    find = b.importlib.util.find_spec
+    monkeypatch.setattr(b.importlib.util, "find_spec", lambda n, *a: None if n == "torch" else find(n, *a))
+    assert b.build_library() == b.LIB
+    assert b.LIB in made and b.CALLS not in made
