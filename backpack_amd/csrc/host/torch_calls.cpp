@@ -9,7 +9,8 @@
 // Every function takes plain tensors and whole numbers in their range and returns NotImplemented for anything else (a subclass, a
 // weight that the library owns, a layout that the checks refuse) before it has done anything: kquant.py then takes the general
 // path, which accepts or refuses the call.  Exceptions of the C++ side become Python's; a status of the library goes to the
-// checker that bind() was given.  The interpreter's lock is released around the library's call, as ctypes does.
+// checker that bind() was given.  The interpreter's lock is released around the allocation of outputs and the library's call, as torch.empty
+// and ctypes do: an allocation may free cached memory and wait for the device, where a host callback may want the lock.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -103,13 +104,19 @@ at::Tensor make(at::IntArrayRef size, at::ScalarType dtype, at::Device device)
 }
 void* stream() { return (void*)c10::hip::getCurrentHIPStream().stream(); }
 
-// false with Python's exception set
+struct Unlocked {   // of the interpreter's lock, also where something throws
+    PyThreadState* state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
+
+// Runs c without the interpreter's lock; false with Python's exception set
 template <class CALL> bool call(CALL&& c)
 {
     int rc;
-    Py_BEGIN_ALLOW_THREADS
-    rc = c();
-    Py_END_ALLOW_THREADS
+    {
+        const Unlocked unlocked;
+        rc = c();
+    }
     if (rc == 0) return true;
     PyObject* r = PyObject_CallFunction(g_check, "i", rc);
     if (r) {
@@ -135,15 +142,16 @@ PyObject* matmul(PyObject*, PyObject* const* a, Py_ssize_t nargs)
     const int64_t M = x->numel() / w.K;
     if (M > 0xFFFFFFFFll || (y_offset && (bf16 || a[3] == Py_None))) return not_implemented();
     at::Tensor y;
-    if (a[3] == Py_None) {
-        y = make({M, (int64_t)w.N}, at::kFloat, x->device());
-    } else {
+    if (a[3] != Py_None) {
         const at::Tensor* out = tensor(a[3]);
         if (!out || !out->is_contiguous() || out->scalar_type() != at::kFloat) return not_implemented();
         y = *out;
     }
-    void *px = x->data_ptr(), *py = y.data_ptr(), *s = stream();
+    void* px = x->data_ptr();
+    const at::Device device = x->device();
     if (!call([&] {
+            if (!y.defined()) y = make({M, (int64_t)w.N}, at::kFloat, device);
+            void *py = y.data_ptr(), *s = stream();
             return bf16 ? f_matmul_bf16(w.type, (const uint16_t*)px, w.data, (const float*)bias, (float*)py, (uint32_t)M, w.N, w.K, w.n_blocks,
                                         w.row_stride_words, s)
                         : f_matmul(w.type, (const float*)px, w.data, (const float*)bias, (float*)py, (uint32_t)M, w.N, w.K, w.n_blocks,
@@ -180,18 +188,23 @@ PyObject* matmul_fused(PyObject*, PyObject* const* a, Py_ssize_t nargs)
     size_t ws_bytes = 0;
     const at::Tensor *out = a[7] == Py_None ? nullptr : tensor(a[7]), *given = a[8] == Py_None ? nullptr : tensor(a[8]);
     if ((a[7] != Py_None && !out) || (a[8] != Py_None && !given)) return not_implemented();
-    y = out ? *out : make({M, n_out}, at::kFloat, x->device());
+    if (out) y = *out;
     if (given) {
         ws_bytes = (size_t)given->numel() * given->element_size();
         pws = given->data_ptr();
-    } else if (a[9] == Py_True) {
-        ws_bytes = f_workspace_bytes((uint32_t)M, (uint32_t)n_out, w.K);
-        ws = make({(int64_t)ws_bytes}, at::kByte, x->device());
-        pws = ws.data_ptr();
     }
+    const bool own_workspace = !given && a[9] == Py_True;
     const bpk_kq_fusion f{(int)pro, (const float*)norm_w, eps, (const float*)residual, (int)epi};
-    void *px = x->data_ptr(), *py = y.data_ptr(), *s = stream();
+    void* px = x->data_ptr();
+    const at::Device device = x->device();
     if (!call([&] {
+            if (!out) y = make({M, n_out}, at::kFloat, device);
+            if (own_workspace) {
+                ws_bytes = f_workspace_bytes((uint32_t)M, (uint32_t)n_out, w.K);
+                ws = make({(int64_t)ws_bytes}, at::kByte, device);
+                pws = ws.data_ptr();
+            }
+            void *py = y.data_ptr(), *s = stream();
             return f_matmul_fused(w.type, (const float*)px, w.data, (const float*)bias, (float*)py, (uint32_t)M, (uint32_t)n_out, w.K, w.n_blocks,
                                   w.row_stride_words, 0, &f, pws, ws_bytes, s);
         }))
@@ -215,9 +228,14 @@ PyObject* matmul_argmax(PyObject*, PyObject* const* a, Py_ssize_t nargs)
     if (!x || !w.from(a[1]) || x->size(-1) != (int64_t)w.K || !memory(a[2], bias)) return not_implemented();
     const int64_t M = x->numel() / w.K;
     if (M > 0xFFFFFFFFll) return not_implemented();
-    at::Tensor y = make({M, (int64_t)w.N}, at::kFloat, x->device()), index = make({M}, at::kInt, x->device()), value = make({M}, at::kFloat, x->device());
-    void *px = x->data_ptr(), *py = y.data_ptr(), *pi = index.data_ptr(), *pv = value.data_ptr(), *s = stream();
+    at::Tensor y, index, value;
+    void* px = x->data_ptr();
+    const at::Device device = x->device();
     if (!call([&] {
+            y = make({M, (int64_t)w.N}, at::kFloat, device);
+            index = make({M}, at::kInt, device);
+            value = make({M}, at::kFloat, device);
+            void *py = y.data_ptr(), *pi = index.data_ptr(), *pv = value.data_ptr(), *s = stream();
             return f_matmul_argmax(w.type, (const float*)px, w.data, (const float*)bias, (float*)py, (uint32_t)M, w.N, w.K, w.n_blocks,
                                    w.row_stride_words, (int32_t*)pi, (float*)pv, s);
         }))
@@ -240,9 +258,15 @@ PyObject* prefill_rows_bf16(PyObject*, PyObject* const* a, Py_ssize_t nargs)
     if (x->size(-1) != row) return not_implemented();
     const int64_t M = x->numel() / row;
     if (M > 0xFFFFFFFFll) return not_implemented();
-    at::Tensor y = make({M, (int64_t)K}, at::kBFloat16, x->device());
-    void *px = x->data_ptr(), *py = y.data_ptr(), *s = stream();
-    if (!call([&] { return f_prefill_rows((int)pro, (const float*)px, (const float*)norm_w, eps, (uint32_t)M, K, (uint16_t*)py, s); })) return nullptr;
+    at::Tensor y;
+    void* px = x->data_ptr();
+    const at::Device device = x->device();
+    if (!call([&] {
+            y = make({M, (int64_t)K}, at::kBFloat16, device);
+            void *py = y.data_ptr(), *s = stream();
+            return f_prefill_rows((int)pro, (const float*)px, (const float*)norm_w, eps, (uint32_t)M, K, (uint16_t*)py, s);
+        }))
+        return nullptr;
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -257,9 +281,14 @@ PyObject* dequant_rows(PyObject*, PyObject* const* a, Py_ssize_t nargs)
     if (!rows || !rows->is_cuda() || rows->scalar_type() != at::kInt || !w.from(a[0])) return not_implemented();
     const int64_t M = rows->numel();
     if (M > 0xFFFFFFFFll) return not_implemented();
-    at::Tensor y = make({M, (int64_t)w.K}, at::kFloat, w.device);
-    void *pr = rows->data_ptr(), *py = y.data_ptr(), *s = stream();
-    if (!call([&] { return f_dequant_rows(w.type, w.data, w.row_stride_words, (const int32_t*)pr, (uint32_t)M, w.K, (float*)py, s); })) return nullptr;
+    at::Tensor y;
+    void* pr = rows->data_ptr();
+    if (!call([&] {
+            y = make({M, (int64_t)w.K}, at::kFloat, w.device);
+            void *py = y.data_ptr(), *s = stream();
+            return f_dequant_rows(w.type, w.data, w.row_stride_words, (const int32_t*)pr, (uint32_t)M, w.K, (float*)py, s);
+        }))
+        return nullptr;
     return THPVariable_Wrap(std::move(y));
     END_HANDLE_TH_ERRORS
 }
@@ -276,10 +305,14 @@ PyObject* moe_route(PyObject*, PyObject* const* a, Py_ssize_t nargs)
         return not_implemented();
     const int64_t T = x->size(0), H = x->size(1), E = r->size(0);
     if ((T | H | E) > 0xFFFFFFFFll) return not_implemented();
-    at::Tensor index = make({T, (int64_t)k}, at::kInt, x->device()), weight = make({T, (int64_t)k}, at::kFloat, x->device());
-    void *px = x->data_ptr(), *pr = r->data_ptr(), *pi = index.data_ptr(), *pw = weight.data_ptr(), *s = stream();
+    at::Tensor index, weight;
+    void *px = x->data_ptr(), *pr = r->data_ptr();
+    const at::Device device = x->device();
     const int normalize = a[3] == Py_True;
     if (!call([&] {
+            index = make({T, (int64_t)k}, at::kInt, device);
+            weight = make({T, (int64_t)k}, at::kFloat, device);
+            void *pi = index.data_ptr(), *pw = weight.data_ptr(), *s = stream();
             return f_route((const float*)px, (const float*)pr, (uint32_t)T, (uint32_t)H, (uint32_t)E, k, normalize, nullptr, (uint32_t*)pi, (float*)pw, s);
         }))
         return nullptr;
@@ -298,10 +331,14 @@ PyObject* moe_ffn(PyObject*, PyObject* const* a, Py_ssize_t nargs)
     if (!x || !idx || !wt || idx->dim() != 2 || !gate.from(a[1]) || !up.from(a[2]) || !down.from(a[3]) || !whole(a[6], E)) return not_implemented();
     const int64_t T = idx->size(0), k = idx->size(1);
     if ((T | k) > 0xFFFFFFFFll) return not_implemented();
-    const size_t bytes = f_ffn_bytes((uint32_t)T, (uint32_t)k, gate.K, down.K);
-    at::Tensor scratch = make({(int64_t)bytes}, at::kByte, x->device()), y = make({T, (int64_t)gate.K}, at::kFloat, x->device());
-    void *px = x->data_ptr(), *pi = idx->data_ptr(), *pw = wt->data_ptr(), *py = y.data_ptr(), *ps = scratch.data_ptr(), *s = stream();
+    at::Tensor scratch, y;
+    void *px = x->data_ptr(), *pi = idx->data_ptr(), *pw = wt->data_ptr();
+    const at::Device device = x->device();
     if (!call([&] {
+            const size_t bytes = f_ffn_bytes((uint32_t)T, (uint32_t)k, gate.K, down.K);
+            scratch = make({(int64_t)bytes}, at::kByte, device);
+            y = make({T, (int64_t)gate.K}, at::kFloat, device);
+            void *py = y.data_ptr(), *ps = scratch.data_ptr(), *s = stream();
             return f_ffn(gate.type, down.type, (const float*)px, gate.data, up.data, down.data, (const uint32_t*)pi, (const float*)pw, (float*)py,
                          (uint32_t)T, (uint32_t)k, E, gate.K, down.K, ps, bytes, s);
         }))

@@ -1,6 +1,8 @@
 """The native form of kquant's calls (csrc/host/torch_calls.cpp): it takes plain calls and gives what the Python form gives, and leaves
 everything else to the Python form, which accepts or refuses it as it did."""
+import ctypes
 import importlib.util
+import subprocess
 import sys
 import threading
 
@@ -167,3 +169,53 @@ def test_calls_that_are_not_plain_are_answered_as_before(gpu, both):  # noqa: F8
         n, g, _ = both(f, *a, **k)
         assert (n[0] == "value") == fine, (f, n)
         _same(n, g)
+
+
+_ALLOCATOR = r"""
+#include <hip/hip_runtime_api.h>
+extern "C" int PyGILState_Check(void);
+extern "C" { int taken, locked; }
+extern "C" void* take(ssize_t n, int, hipStream_t) {
+    void* p = nullptr;
+    ++taken;
+    locked += PyGILState_Check();
+    return hipMalloc(&p, n) == hipSuccess ? p : nullptr;
+}
+extern "C" void give(void* p, ssize_t, int, hipStream_t) { (void)hipFree(p); }
+"""
+_kept = []     # the allocator outlives what it has given
+
+
+@pytest.mark.gpu
+def test_outputs_are_allocated_without_the_interpreter_lock(gpu, tmp_path):  # noqa: F811
+    """A device allocation may wait for the device; a host callback in a stream may wait for the lock.  Asked from an allocator that
+    the calls' outputs come from."""
+    from backpack_amd import capi, kquant
+    src, so = tmp_path / "a.cpp", tmp_path / "a.so"
+    src.write_text(_ALLOCATOR)
+    subprocess.run(["g++", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", str(src), "-o", str(so), "-L/opt/rocm/lib",
+                    "-lamdhip64"], check=True, timeout=60)
+    M, K, N, E = 2, 256, 64, 4
+    x, idx, wt = torch.randn(M, K, device="cuda"), torch.zeros(M, 2, dtype=torch.int32, device="cuda"), torch.rand(M, 2, device="cuda")
+    _, _, w = gpu.make_weight(Q4_K, N, K, seed=1)
+    _, _, experts = gpu.make_weight(Q4_K, E * 256, K, seed=2)
+    router, rows = torch.randn(E, K, device="cuda"), torch.zeros(3, dtype=torch.int32, device="cuda")
+    calls = [lambda: kquant.matmul(x, w), lambda: kquant.matmul_fused(x, w, capi.PRO_RMS_NORM, norm_w=x[0], eps=1e-5), lambda: kquant.matmul_argmax(x, w),
+             lambda: kquant.prefill_rows_bf16(x, K), lambda: kquant.dequant_rows(w, rows), lambda: kquant.moe_route(x, router, 2),
+             lambda: kquant.moe_ffn(x, experts, experts, experts, idx, wt, E)]
+    native = kquant._native()
+    for c in calls:
+        c()                    # (what the library allocates once is there)
+    torch.cuda.synchronize()
+    _kept.append(torch.cuda.memory.CUDAPluggableAllocator(str(so), "take", "give"))
+    seen = ctypes.CDLL(str(so))
+    taken, locked = (ctypes.c_int.in_dll(seen, n) for n in ("taken", "locked"))
+    assert native is kquant._native()
+    for i, c in enumerate(calls):
+        pool = torch.cuda.MemPool(_kept[-1].allocator())
+        before = taken.value
+        with torch.cuda.use_mem_pool(pool):
+            y = c()
+        torch.cuda.synchronize()
+        assert taken.value > before and locked.value == 0, (i, taken.value - before, locked.value)
+        del y, pool
