@@ -269,7 +269,10 @@ BPK_API int bpk_kq_matmul(int type, const float *X, const void *W,
  * and needs no workspace; so are verify batches, M <= 16, on the tile kernel
  * (X, W and norm_w 16-byte aligned; not Q6_K with M > 8 under an act * up
  * prologue), but for calls of 5 to 16 tokens that are given the workspace and
- * priced lower on the many-token kernel.  Other shapes need `workspace` (device memory, 16-byte aligned, at
+ * go to the many-token kernel: by price, and with an act * up prologue on some
+ * matrices of 61000 rows and more.  (Two kernels add in different orders:
+ * such a call's last bits differ with the workspace from those without.)
+ * Other shapes need `workspace` (device memory, 16-byte aligned, at
  * least bpk_kq_matmul_fused_workspace_bytes(M, N, K) bytes) and fail with
  * BPK_ERR_WORKSPACE without it: they run the same function as prologue, matmul
  * and add launches through it, or, where the many-token kernel takes the call

@@ -861,3 +861,48 @@ def test_dispatch_of_5_to_16_tokens(gpu, type_, M, N, K, pro, epi, res, form):  
     rms = float(tile.double().pow(2).mean().sqrt())
     # two 22-bit splits of x, fp32 sums in another order; an activation multiplies two such
     assert float((got - tile).abs().max()) <= 4e-5 * (rms + float(tile.abs().max()))
+
+
+# rows of W, us on one MI355X: the launches of prologue, product and epilogue, the many-token kernel with all of it inside
+@pytest.mark.parametrize("type_,M,rows,K,pro,epi,separate_us,wide_us", [
+    (Q6_K, 12, 32776, 256, 0, 2, 25.2, 9.5), (Q4_K, 15, 7182, 256, 1, 3, 17.5, 8.2), (Q6_K, 16, 1864, 11008, 1, 2, 44.6, 22.4),
+    (Q4_K, 8, 1954, 12032, 1, 3, 36.9, 18.0), (Q5_K, 16, 32770, 512, 1, 3, 21.6, 11.7),
+    (Q5_K, 5, 696, 1024, 0, 2, 7.8, 14.1), (Q6_K, 8, 2066, 768, 1, 3, 10.7, 13.9), (Q4_K, 5, 812, 3072, 0, 3, 10.2, 11.9),
+    # rows that fill the CUs
+    (Q4_K, 9, 61202, 256, 1, 2, None, None), (Q6_K, 16, 61202, 512, 0, 2, None, None)])
+def test_5_to_16_tokens_with_an_epilogue_over_any_rows(gpu, type_, M, rows, K, pro, epi, separate_us, wide_us):  # noqa: F811
+    """The tile kernel's gate and up tiles need a multiple of 32 rows; other calls weigh the many-token kernel against what would run."""
+    import torch
+    from backpack_amd import capi, kquant
+    print("epilogue, any rows", type_, M, rows, K, pro, epi, flush=True)
+    _, _, w = gpu.make_weight(type_, rows, K, seed=M)
+    rng = np.random.default_rng(rows)
+    X = gpu.dev(rng.standard_normal((M, K)).astype(np.float32))
+    nw = gpu.dev((1 + 0.1 * rng.standard_normal(K)).astype(np.float32)) if pro else None
+    got = kquant.matmul_fused(X, w, pro, norm_w=nw, eps=1e-5, epilogue=epi)
+    assert (capi.last_form() == "many_token") == (wide_us is None or wide_us < separate_us), (capi.last_kernel(), capi.last_form())
+    capi.set_option("fused_separate", 1)
+    try:
+        want = kquant.matmul_fused(X, w, pro, norm_w=nw, eps=1e-5, epilogue=epi)
+    finally:
+        capi.set_option("fused_separate", 0)
+    # splits of x into 22 bits and fp32 sums in two orders, in each of the two factors: 1e-5 apart at most over 150000 random calls
+    assert float((got - want).double().norm() / want.double().norm()) <= 2e-5
+
+
+@pytest.mark.parametrize("type_,M,N,wide", [(Q4_K, 9, 61185, True), (Q5_K, 16, 61185, True), (Q6_K, 7, 96678, True), (Q4_K, 5, 66000, False),
+                                            (Q4_K, 9, 60928, False)])
+def test_act_prologue_on_many_rows(gpu, type_, M, N, wide):  # noqa: F811
+    """Behind an act * up prologue 5 to 16 tokens go by the rows as plain calls do, given a workspace; without one the call is the tile
+    kernel's one launch."""
+    import torch
+    from backpack_amd import capi, kquant
+    K = 256
+    print("act prologue", type_, M, N, flush=True)
+    _, _, w = gpu.make_weight(type_, N, K, seed=M)
+    X = gpu.dev(np.random.default_rng(N).standard_normal((M, 2 * K)).astype(np.float32))
+    got = kquant.matmul_fused(X, w, capi.PRO_SILU_MUL)
+    assert (capi.last_form() == "many_token") == wide
+    want = kquant.matmul_fused(X, w, capi.PRO_SILU_MUL, allow_workspace=False)
+    assert capi.last_kernel() == "mtile_fused"
+    assert float((got - want).double().norm() / want.double().norm()) <= 2e-5     # (as above)
