@@ -1337,17 +1337,23 @@ hipError_t launch_mtile_grouped(const MatmulArgs& a, const uint32_t* tiles, cons
 
 // Work split.  A wave per tile, `per_wg` tiles per workgroup (they share the conversion of X; pairs of gate and up take an even
 // number), and K cut into `splits` runs of whole chunks when the rows alone give too few workgroups.  Candidates are priced as
-// rounds x (chunks walked + 1.5 for launch, prologue and fold), a partly idle last round costing half its idle share extra; one
-// tile per workgroup with the waves taking different superblocks is the fallback for matrices of a few rows.  extra: floats per 16
-// rows of a workgroup's partial tile beside its sums (the sums of squares of a norm prologue).
+// rounds x (chunks walked + 1.5 for launch, prologue and fold), a partly idle last round costing half its idle share extra.
+// `shared` (plain calls): one tile per workgroup of 4 waves that take different superblocks; every workgroup converts all of X itself,
+// and a CU takes one of them at a time.  Up to a tile per CU that beats the split (up to 1024 columns, 12 tokens: Q4_K 1.08 to 1.21
+// times as long on the split, Q5_K 1.15 to 1.32, Q6_K 1.4 to 1.7); with more tiles than CUs it loses (4097..8192 rows, 256..1024
+// columns, 3..24 tokens: Q4_K 1.4 to 1.9 times the split's time, Q5_K 1.3 to 1.8, Q6_K 1.03 to 1.5; Q4_K, 8192x768, 8 tokens: 10.0 us,
+// 6.0 on the split; Q6_K 11.0 and 9.2).
 struct MtileSplit {
-    uint32_t per_wg, splits, chunks, rounds;
-    float cost;
+    uint32_t per_wg, splits, chunks, rounds, groups;
+    bool shared;
 };
-static MtileSplit mtile_split(uint32_t tiles, uint32_t n_blocks, bool pairs, uint32_t extra, const SplitScratch& sc)
+static MtileSplit mtile_split(const MatmulArgs& a, const SplitScratch& sc)
 {
-    const uint32_t n_chunks = (n_blocks + MT_KC - 1) / MT_KC, cus = device_cu_count();
-    MtileSplit best{8u, 1u, n_chunks, 1u, 1e30f};
+    const uint32_t tiles = (a.N + 15u) / 16u, n_chunks = (a.n_blocks + MT_KC - 1) / MT_KC, cus = device_cu_count();
+    const bool pairs = a.epi != 0, fused = a.pro || a.residual || a.epi;
+    const uint32_t extra = fused ? 1u : 0u;   // 16 sums of squares per workgroup for the norm prologue
+    MtileSplit best{8u, 1u, n_chunks, 1u, 1u, false};
+    float best_cost = 1e30f;
     for (uint32_t tpw = 8; tpw >= 4; tpw -= pairs ? 2u : 1u) {
         const uint32_t groups = pairs ? (tiles / 2u + tpw / 2u - 1u) / (tpw / 2u) : (tiles + tpw - 1u) / tpw;
         for (uint32_t splits = 1; splits <= n_chunks && splits <= 16u; ++splits) {
@@ -1357,26 +1363,41 @@ static MtileSplit mtile_split(uint32_t tiles, uint32_t n_blocks, bool pairs, uin
             const uint32_t wgs = groups * splits, rounds = (wgs + cus - 1u) / cus;
             const float idle = 1.0f - (float)wgs / (float)(rounds * cus);
             const float cost = (float)rounds * ((float)cps + 1.5f) * (1.0f + 0.5f * idle);
-            if (cost < best.cost) best = MtileSplit{tpw, splits, cps, rounds, cost};
+            if (cost < best_cost) { best_cost = cost; best = MtileSplit{tpw, splits, cps, rounds, groups, false}; }
         }
     }
+    best.shared = !fused && (float)((tiles + cus - 1u) / cus) * ((float)n_chunks * 1.25f + 1.5f) < best_cost;
     return best;
 }
 
+// us.  Fitted to 128000 timed calls of 5 to 16 tokens (32 to 64000 rows, K 256 to 14336; plain, with a norm, a residual, an epilogue) of
+// the forms that the launch takes: 5 to 7 % rms on the split, 2 to 4 % on the shared form.
 double mtile_price_5_to_16(const MatmulArgs& a, const SplitScratch& sc)
 {
-    const MtileSplit b = mtile_split((a.N + 15u) / 16u, a.n_blocks, a.epi != 0, 1u, sc);
-    const double rounds = b.rounds, M = a.M, walk = rounds * std::min(b.chunks * (uint32_t)MT_KC, a.n_blocks), out = 1e-6 * M * (a.epi ? a.N / 2u : a.N);
-    // The launch, a superblock of a workgroup's walk (beside that per token and per tile), a round, the fold and its splits, a norm per chunk
-    // of the walk and beside it, 10^6 outputs: fitted to 40000 timed calls of 5 to 16 tokens (as for the many-token kernel), 8 to 10 % rms.
-    // Q4_K, Q5_K, Q6_K up to 8 tokens, then beyond.
-    const double c[6][10] = {{1.239, 0.109, 0.026, 0.092, 2.632, 1.382, 0.241, 0.557, 0.698, 5.602}, {1.242, 0.253, 0.017, 0.114, 2.174, 1.627, 0.281, 0.575, 0.772, 12.128},
-                             {1.141, 0.252, 0.008, 0.221, 1.754, 2.511, 0.280, 0.866, 1.196, 20.591}, {1.227, 0.118, 0.031, 0.128, 2.670, 1.434, 0.314, 0.762, 0.660, 4.926},
-                             {0.995, 0.216, 0.032, 0.136, 2.583, 1.718, 0.332, 0.839, 0.704, 7.462}, {1.059, 0.369, 0.025, 0.238, 1.953, 2.546, 0.341, 0.907, 1.137, 13.148}};
-    const double* k = c[(a.M > 8u ? 3 : 0) + (a.type == KQ_TYPE_Q4_K ? 0 : a.type == KQ_TYPE_Q5_K ? 1 : 2)];
-    const double norm = a.pro == 1 ? 1.0 : 0.0;
-    return k[0] + walk * (k[1] + k[2] * M + k[3] * b.per_wg) + k[4] * rounds + (b.splits > 1u ? k[5] : 0.0) + k[6] * b.splits +
-           norm * (k[7] * rounds * b.chunks + k[8]) + k[9] * out;
+    const MtileSplit b = mtile_split(a, sc);
+    const int t = (a.M > 8u ? 3 : 0) + (a.type == KQ_TYPE_Q4_K ? 0 : a.type == KQ_TYPE_Q5_K ? 1 : 2);   // (up to 8 tokens, beyond)
+    const double M = a.M, nb = a.n_blocks;
+    if (b.shared) {
+        // the launch, a superblock and one of a token, 10^6 outputs
+        const double c[6][4] = {{5.308, -0.036, 0.013, 11.356}, {5.4, -0.051, 0.013, 12.156}, {5.649, -0.083, 0.015, 12.589},
+                                {5.966, -0.658, 0.069, 8.802}, {5.958, -0.665, 0.069, 8.28}, {6.283, -0.693, 0.072, 8.277}};
+        return c[t][0] + nb * (c[t][1] + c[t][2] * M) + c[t][3] * 1e-6 * M * a.N;
+    }
+    // The launch; a superblock of a workgroup's walk, beside it per token, per tile of a workgroup, per wave of a SIMD that has a tile and
+    // that times the tokens (41 rows are 3 tiles and one wave: priced as the 8 tiles that a workgroup may have they went to the kernel that
+    // takes 1.8 times as long); two superblocks; a round; a chunk of one; a superblock of a chip that is full; the fold; a norm per chunk
+    const double c[6][12] = {{1.694, -0.359, 0.029, 0.022, 0.16, 0.007, 0.113, 3.319, 0.237, 0.364, 1.978, 1.279},
+                             {1.727, -0.493, 0.038, 0.038, 0.323, 0.001, 0.142, 3.804, -0.153, 0.404, 1.999, 1.334},
+                             {1.884, -2.51, 0.028, 0.126, 0.273, 0.006, 3.582, 3.145, 1.704, 0.463, 2.842, 1.459},
+                             {2.064, -0.778, 0.026, 0.057, 0.163, 0.009, 0.317, 3.312, 1.277, 0.408, 2.388, 1.41},
+                             {1.992, -0.87, 0.033, 0.059, 0.32, 0.005, 0.329, 3.747, 1.102, 0.413, 2.376, 1.394},
+                             {2.141, -3.371, 0.05, 0.144, 0.516, -0.007, 4.143, 3.267, 2.924, 0.461, 3.404, 1.341}};
+    const double* k = c[t];
+    const uint32_t blocks = std::min(b.chunks * (uint32_t)MT_KC, a.n_blocks), tiles = ((a.N + 15u) / 16u + b.groups - 1u) / b.groups;
+    const double rounds = b.rounds, waves = tiles > 4u ? 2.0 : 1.0;
+    return k[0] + rounds * blocks * (k[1] + k[2] * M + k[3] * b.per_wg + k[4] * waves + k[5] * waves * M) + rounds * ((blocks + 1u) / 2u) * k[6] +
+           rounds * (k[7] + k[8] * b.chunks) + k[9] * blocks * b.groups * b.splits / 256.0 + (b.splits > 1u ? k[10] : 0.0) +
+           (a.pro == 1 ? k[11] * rounds * b.chunks : 0.0);
 }
 
 hipError_t launch_mtile(const MatmulArgs& a, const SplitScratch& sc, hipStream_t s)
@@ -1387,15 +1408,7 @@ hipError_t launch_mtile(const MatmulArgs& a, const SplitScratch& sc, hipStream_t
     const uint32_t group = 16u;
     const uint32_t tiles = (a.N + 15u) / 16u;
     const uint32_t n_chunks = (a.n_blocks + MT_KC - 1) / MT_KC;
-    const uint32_t cus = device_cu_count();
-    const MtileSplit best = mtile_split(tiles, a.n_blocks, false, 0u, sc);
-    // One tile per workgroup of 4 waves: every workgroup converts all of X itself, and a CU takes one of them at a time.  Up to a tile per CU
-    // that beats the split (up to 1024 columns, 12 tokens: Q4_K 1.08 to 1.21 times as long on the split, Q5_K 1.15 to 1.32, Q6_K 1.4 to 1.7);
-    // with more tiles than CUs it loses (4097..8192 rows, 256..1024 columns, 3..24 tokens: Q4_K 1.4 to 1.9 times the split's time, Q5_K 1.3 to
-    // 1.8, Q6_K 1.03 to 1.5; Q4_K, 8192x768, 8 tokens: 10.0 us, 6.0 on the split;
-    // Q6_K 11.0 and 9.2).
-    const float shared_rounds = (float)((tiles + cus - 1u) / cus);
-    const bool shared_tile = shared_rounds * ((float)n_chunks * 1.25f + 1.5f) < best.cost;
+    const MtileSplit best = mtile_split(a, sc);
 
     for (uint32_t m0 = 0; m0 < a.M; m0 += group) {
         MtileParams p;
@@ -1416,7 +1429,7 @@ hipError_t launch_mtile(const MatmulArgs& a, const SplitScratch& sc, hipStream_t
         p.pro = 0; p.epi = 0; p.eps = 0.0f; p.norm_w = nullptr; p.residual = nullptr; p.x_stride = a.K; p.pair_tile0 = 0;
         hipError_t e;
         const bool q5 = a.type == KQ_TYPE_Q5_K;
-        if (shared_tile) {
+        if (best.shared) {
             e = q6_wide ? launch_mtile_one<MT_TYPE_Q6K_WIDE, 4, 1>(p, tiles, 1, s)
                 : q6 ? launch_mtile_one<KQ_TYPE_Q6_K, 4, 1>(p, tiles, 1, s)
                 : q5 ? launch_mtile_one<KQ_TYPE_Q5_K, 4, 1>(p, tiles, 1, s) : launch_mtile_one<KQ_TYPE_Q4_K, 4, 1>(p, tiles, 1, s);
@@ -1462,7 +1475,7 @@ hipError_t launch_mtile_fused(const MatmulArgs& a, const SplitScratch& sc, hipSt
 {
     const bool q6 = a.type == KQ_TYPE_Q6_K, q5 = a.type == KQ_TYPE_Q5_K, q6_wide = q6 && a.M > 8u;
     const uint32_t tiles = (a.N + 15u) / 16u;
-    const MtileSplit best = mtile_split(tiles, a.n_blocks, a.epi != 0, 1u, sc);   // (16 sums of squares per workgroup for the norm prologue)
+    const MtileSplit best = mtile_split(a, sc);
     MtileParams p;
     p.W2 = nullptr;
     p.X = (const float*)a.X;

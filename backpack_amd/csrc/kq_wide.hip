@@ -1038,11 +1038,12 @@ double wide_price_5_to_16(const MatmulArgs& a, const SplitScratch& sc)
     } else {
         groups_per_wg(gx, 1, a.type, 1, a.n_blocks, &walk);
     }
-    // The launches' sum, walk, the one that adds the splits and its floats, 10^6 outputs, a norm: fitted to 27000 timed calls of 5 to 16
-    // tokens (512 to 64000 rows, plain, with a norm, a residual, a norm and act * up), 5 to 6 % rms
-    const double c[3][6] = {{0.59, 0.78, 4.13, 2.96, 2.35, 0.68}, {0.78, 0.82, 3.96, 3.32, 2.77, 0.76}, {0.47, 0.81, 4.71, 2.21, 2.30, 0.73}};
+    // The launches' sum, walk, the one that adds the splits and its floats, 10^6 outputs, a norm (a workgroup walks its row first) and a
+    // superblock of it: fitted to 128000 timed calls of 5 to 16 tokens (32 to 64000 rows, plain, with a norm, a residual, an epilogue), 4 to 5 % rms
+    const double c[3][7] = {{1.364, 0.727, 3.638, 2.948, 2.733, 0.211, 0.07}, {1.165, 0.803, 3.669, 3.173, 3.368, 0.339, 0.063}, {0.953, 0.772, 4.486, 2.371, 3.407, 0.404, 0.057}};
     const double* k = c[a.type == KQ_TYPE_Q4_K ? 0 : a.type == KQ_TYPE_Q5_K ? 1 : 2];
-    return k[0] + k[1] * walk + (z > 1u ? k[2] + k[3] * 1e-6 * z * 16.0 * gx * 256.0 : 0.0) + k[4] * 1e-6 * (double)a.M * outs + (a.pro == 1 ? k[5] : 0.0);
+    return k[0] + k[1] * walk + (z > 1u ? k[2] + k[3] * 1e-6 * z * 16.0 * gx * 256.0 : 0.0) + k[4] * 1e-6 * (double)a.M * outs +
+           (a.pro == 1 ? k[5] + k[6] * a.n_blocks : 0.0);
 }
 
 hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scratch, size_t x_bytes, int splits, hipStream_t s)

@@ -906,3 +906,26 @@ def test_act_prologue_on_many_rows(gpu, type_, M, N, wide):  # noqa: F811
     want = kquant.matmul_fused(X, w, capi.PRO_SILU_MUL, allow_workspace=False)
     assert capi.last_kernel() == "mtile_fused"
     assert float((got - want).double().norm() / want.double().norm()) <= 2e-5     # (as above)
+
+
+# us on one MI355X, each kernel forced: the tile kernel, the many-token kernel
+@pytest.mark.parametrize("type_,M,N,K,pro,res,tile_us,wide_us", [
+    # few rows: a tile per workgroup; a workgroup whose tiles are not all there
+    (Q6_K, 13, 41, 1024, 0, False, 7.1, 12.8), (Q6_K, 14, 64, 1024, 0, False, 7.3, 12.8), (Q4_K, 14, 47, 5888, 0, False, 11.2, 15.4),
+    (Q5_K, 13, 43, 2048, 0, False, 11.3, 14.1), (Q4_K, 12, 64, 3584, 0, False, 10.5, 11.9), (Q6_K, 5, 44, 3840, 0, False, 12.2, 13.7),
+    # short rows, many of them, a few tokens
+    (Q6_K, 8, 31785, 512, 0, False, 9.4, 12.3), (Q6_K, 6, 29803, 512, 1, True, 10.4, 12.6),
+    # the other side
+    (Q6_K, 16, 33720, 256, 0, False, 24.4, 9.2), (Q6_K, 14, 34714, 256, 1, False, 25.3, 9.4), (Q6_K, 16, 47, 2048, 0, False, 15.4, 12.5),
+    (Q6_K, 16, 40009, 256, 0, True, 25.3, 9.6)])
+def test_5_to_16_tokens_take_the_faster_kernel(gpu, type_, M, N, K, pro, res, tile_us, wide_us):  # noqa: F811
+    import torch
+    from backpack_amd import capi, kquant
+    print("faster kernel", type_, M, N, K, pro, res, flush=True)
+    _, _, w = gpu.make_weight(type_, N, K, seed=M)
+    X, nw, R = torch.randn(M, K, device="cuda"), torch.rand(K, device="cuda"), torch.randn(M, N, device="cuda")
+    if pro or res:
+        kquant.matmul_fused(X, w, pro, norm_w=nw if pro else None, eps=1e-5, residual=R if res else None)
+    else:
+        kquant.matmul(X, w)
+    assert (capi.last_form() == "many_token") == (wide_us < tile_us), (capi.last_kernel(), capi.last_form())
