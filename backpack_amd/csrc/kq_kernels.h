@@ -48,6 +48,7 @@ struct SplitScratch {
     uint32_t* counters;    // n_counters words, zero between launches
     size_t capacity_floats;
     uint32_t n_counters;
+    uint32_t cus;          // the device's compute units (here, so that a call does not ask the runtime for each price)
 };
 
 hipError_t launch_dequant_rows(int type, const uint8_t* W, uint32_t row_stride_bytes,
@@ -162,7 +163,7 @@ hipError_t launch_wide_prepare(const uint32_t* expert_idx, uint32_t n_pairs, uin
 hipError_t launch_wide_x(int type, const float* X, int pro, const float* norm_w, float eps, uint32_t rows,
                          uint32_t n_blocks, const WideX& x, hipStream_t s);
 // launch_wide's price in us at up to 16 tokens, K in one piece
-double wide_price_16(int type, uint32_t N, uint32_t n_blocks);
+double wide_price_16(int type, uint32_t N, uint32_t n_blocks, uint32_t cus);
 // us that a call of 5 to 16 tokens takes on the many-token and on the tile kernel (no prologue or a norm; residual, epilogue)
 double wide_price_5_to_16(const MatmulArgs& a, const SplitScratch& sc);
 double mtile_price_5_to_16(const MatmulArgs& a, const SplitScratch& sc);

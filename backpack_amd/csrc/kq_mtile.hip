@@ -1349,7 +1349,7 @@ struct MtileSplit {
 };
 static MtileSplit mtile_split(const MatmulArgs& a, const SplitScratch& sc)
 {
-    const uint32_t tiles = (a.N + 15u) / 16u, n_chunks = (a.n_blocks + MT_KC - 1) / MT_KC, cus = device_cu_count();
+    const uint32_t tiles = (a.N + 15u) / 16u, n_chunks = (a.n_blocks + MT_KC - 1) / MT_KC, cus = sc.cus;
     const bool pairs = a.epi != 0, fused = a.pro || a.residual || a.epi;
     const uint32_t extra = fused ? 1u : 0u;   // 16 sums of squares per workgroup for the norm prologue
     MtileSplit best{8u, 1u, n_chunks, 1u, 1u, false};

@@ -985,10 +985,9 @@ static WideWalk wide_walk(int type, uint32_t tt, uint32_t blocks)
     return {{blocks * step, blocks * step}, {9.0, 9.0}};
 }
 
-static uint32_t groups_per_wg(uint32_t row_groups, uint32_t others, int type, uint32_t tt, uint32_t blocks, double* price)
+static uint32_t groups_per_wg(uint32_t row_groups, uint32_t others, int type, uint32_t tt, uint32_t blocks, uint32_t cus, double* price)
 {
     const WideWalk w = wide_walk(type, tt, blocks);
-    const uint64_t cus = device_cu_count();
     uint32_t best = 1;
     double best_us = 1e30;
     for (uint32_t c = 1; c <= row_groups && c <= 64u; ++c) {
@@ -1004,39 +1003,39 @@ static uint32_t groups_per_wg(uint32_t row_groups, uint32_t others, int type, ui
 // workgroup's walk 0.8 + 0.7 per tile of tokens (Q6_K 3 + 0.9), the launch that adds the splits 5, and its
 // traffic, written and read once, at 4 TB/s.  (Of the walk before this one; the choice is still within 4 % of the best of
 // eight forced ones on 80 calls, 20 to 128 tokens, Q4_K and Q6_K.)  splits: at most so many, 0 = the cheapest.
-static uint32_t wide_cut(int type, uint32_t tt, uint32_t row_groups, uint32_t token_groups, uint32_t n_blocks, size_t capacity_floats, int splits)
+static uint32_t wide_cut(int type, uint32_t tt, uint32_t row_groups, uint32_t token_groups, uint32_t n_blocks, const SplitScratch& sc, int splits)
 {
     const double step_us = type == KQ_TYPE_Q6_K ? 3.0 + 0.9 * tt : 0.8 + 0.7 * tt;
     const size_t tile_floats = (size_t)token_groups * tt * 16u * row_groups * (WIDE_WAVES * 32u);
     uint32_t z = 1;
     double best = 1e30;
     for (uint32_t c = 1; c <= n_blocks && c <= 16u; ++c) {
-        if (c > 1u && c * tile_floats > capacity_floats) break;
-        const uint32_t cus = device_cu_count(), rounds = (row_groups * token_groups * c + cus - 1u) / cus;
+        if (c > 1u && c * tile_floats > sc.capacity_floats) break;
+        const uint32_t rounds = (row_groups * token_groups * c + sc.cus - 1u) / sc.cus;
         const double t = (double)rounds * ((n_blocks + c - 1u) / c) * step_us + (c > 1u ? 5.0 + 2e-6 * c * tile_floats : 0.0);
         if (splits ? (uint32_t)splits >= c : t < best) { best = t; z = c; }
     }
     return z;
 }
 
-double wide_price_16(int type, uint32_t N, uint32_t n_blocks)
+double wide_price_16(int type, uint32_t N, uint32_t n_blocks, uint32_t cus)
 {
     double us;
-    groups_per_wg((N + 255u) / 256u, 1, type, 1, n_blocks, &us);
+    groups_per_wg((N + 255u) / 256u, 1, type, 1, n_blocks, cus, &us);
     return us + 4.0;   // (the split of X in front)
 }
 
 double wide_price_5_to_16(const MatmulArgs& a, const SplitScratch& sc)
 {
     const uint32_t outs = a.epi ? a.N / 2u : a.N, per_wg = a.epi ? WIDE_WAVES * 16u : WIDE_WAVES * 32u, gx = (outs + per_wg - 1u) / per_wg;
-    const uint32_t cut = wide_cut(a.type, 1, gx, 1, a.n_blocks, sc.capacity_floats, 0), per = (a.n_blocks + cut - 1u) / cut, z = (a.n_blocks + per - 1u) / per;
+    const uint32_t cut = wide_cut(a.type, 1, gx, 1, a.n_blocks, sc, 0), per = (a.n_blocks + cut - 1u) / cut, z = (a.n_blocks + per - 1u) / per;
     double walk;
     if (z > 1u) {
         const WideWalk w = wide_walk(a.type, 1, per);
-        const uint32_t n = (gx * z + device_cu_count() - 1u) / device_cu_count();
+        const uint32_t n = (gx * z + sc.cus - 1u) / sc.cus;
         walk = (double)(n / 2u * 2u) * (w.walk[1] + w.start[1]) + (double)(n % 2u) * (w.walk[0] + w.start[0]);
     } else {
-        groups_per_wg(gx, 1, a.type, 1, a.n_blocks, &walk);
+        groups_per_wg(gx, 1, a.type, 1, a.n_blocks, sc.cus, &walk);
     }
     // The launches' sum, walk, the one that adds the splits and its floats, 10^6 outputs, a norm (a workgroup walks its row first) and a
     // superblock of it: fitted to 128000 timed calls of 5 to 16 tokens (32 to 64000 rows, plain, with a norm, a residual, an epilogue), 4 to 5 % rms
@@ -1069,12 +1068,12 @@ hipError_t launch_wide(const MatmulArgs& a, const SplitScratch& sc, void* x_scra
         const uint32_t gy = (M + 63u) / 64u, tiles = (M + 15u) / 16u, tt = (tiles + gy - 1u) / gy;
         const uint32_t gy2 = (tiles + tt - 1u) / tt;
         const uint32_t per_wg = a.epi ? WIDE_WAVES * 16u : WIDE_WAVES * 32u, gx = (outs + per_wg - 1u) / per_wg;
-        const uint32_t z = wide_cut(a.type, tt, gx, gy2, a.n_blocks, sc.capacity_floats, splits);
+        const uint32_t z = wide_cut(a.type, tt, gx, gy2, a.n_blocks, sc, splits);
         p.blocks_per_split = (a.n_blocks + z - 1u) / z;
         p.n_splits = (a.n_blocks + p.blocks_per_split - 1u) / p.blocks_per_split;
         p.partial = sc.partial;
         p.row_groups = gx;
-        p.per_wg = p.n_splits > 1u ? 1u : groups_per_wg(gx, gy2, a.type, tt, a.n_blocks, nullptr);
+        p.per_wg = p.n_splits > 1u ? 1u : groups_per_wg(gx, gy2, a.type, tt, a.n_blocks, sc.cus, nullptr);
         if (hipError_t e = launch_wide_any(a.type, p, tt, dim3((gx + p.per_wg - 1u) / p.per_wg, gy2, p.n_splits), s); e != hipSuccess) return e;
         if (p.n_splits > 1u) {
             hipLaunchKernelGGL(wide_sum_kernel, dim3(gx, (M + 3u) / 4u), dim3(256), 0, s, p, tt * 16u, gy2);
