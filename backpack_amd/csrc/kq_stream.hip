@@ -454,21 +454,31 @@ __device__ __forceinline__ void q4k_stream_body(PT p)
         float res[MT];
 #pragma unroll
         for (int t = 0; t < MT; ++t) res[t] = 0.0f;
-        for (uint32_t i0 = 0; i0 < cnt; i0 += D) {
+        auto row = [&](int d, uint32_t i, float (&acc)[MT]) {
+            ring[d].template wait<(D - 1) * SLOT_LOADS>();
+#pragma unroll
+            for (int t = 0; t < MT; ++t) acc[t] = 0.0f;
+#pragma unroll
+            for (int pass = 0; pass < P; ++pass)
+                q4k_piece_dot<MT, Q5>(ring[d].hdr[pass], ring[d].q[pass], xlo[pass], xhi[pass], xs_lo[pass],
+                                      xs_hi[pass], sel_hi, sh, acc, ring[d].qh[Q5 ? pass : 0], 2u * g);
+            ring[d].fill(p.W + row_of(c0 + i + D) * p.row_stride_bytes, hoff, j);
+        };
+        // No step for a row that is not there (Q4_K 5003 x 2816, one token: 4.66 -> 4.46 us; two tokens: 2 % slower with the branch).
+        // Where the steps are short (four rows in flight of one pass) or many (plain K slices) the branches between them cost more than
+        // the absent rows do, and the last, partial round of steps stands behind the loop instead.  One token, us, all rows stepped /
+        // branches / this: Q4_K 49000 x 2048 13.1 / 14.1 / 12.9, 8300 x 1024 4.8 / 4.3 / 4.1, 53267 x 11264 84.8 / 91.9 / 85.3,
+        // 100000 x 5120 80.1 / 83.6 / 78.0, Q5_K 154712 x 4864 156 / 166 / 154; elsewhere the branches are up to 1.5 % ahead
+        // (6144 x 4096 with a norm 5.67 / 5.66 / 5.74, 4096 x 14336 with a residual 9.64 / 9.33 / 9.43).
+        constexpr bool TAIL = MT == 1 && (D == 4 ? P == 1 : KW > 1 && !PT::kFused);
+        const uint32_t steps = TAIL ? cnt / D * D : cnt;
+        for (uint32_t i0 = 0; i0 < steps; i0 += D) {
 #pragma unroll
             for (int d = 0; d < D; ++d) {
                 const uint32_t i = i0 + d;
-                // no step for a row that is not there (Q4_K 5003 x 2816, one token: 4.66 -> 4.46 us; two tokens: 2 % slower with the branch)
-                if (MT != 2 && d && i >= cnt) break;
-                ring[d].template wait<(D - 1) * SLOT_LOADS>();
+                if (MT != 2 && !TAIL && d && i >= cnt) break;
                 float acc[MT];
-#pragma unroll
-                for (int t = 0; t < MT; ++t) acc[t] = 0.0f;
-#pragma unroll
-                for (int pass = 0; pass < P; ++pass)
-                    q4k_piece_dot<MT, Q5>(ring[d].hdr[pass], ring[d].q[pass], xlo[pass], xhi[pass], xs_lo[pass],
-                                          xs_hi[pass], sel_hi, sh, acc, ring[d].qh[Q5 ? pass : 0], 2u * g);
-                ring[d].fill(p.W + row_of(c0 + i + D) * p.row_stride_bytes, hoff, j);
+                row(d, i, acc);
 #pragma unroll
                 for (int t = 0; t < (QUAD ? 0 : MT); ++t) {
                     const float tot = wave_sum(acc[t]);
@@ -478,6 +488,17 @@ __device__ __forceinline__ void q4k_stream_body(PT p)
                     const float tot = quad_sum(acc);
                     if (!(lane & 15u)) part[slice * NW + walker][i][lane >> 4] = tot;
                 }
+            }
+        }
+        if constexpr (TAIL) {
+#pragma unroll
+            for (int d = 0; d < D - 1; ++d) {
+                const uint32_t i = steps + d;
+                if (i >= cnt) break;
+                float acc[1];
+                row(d, i, acc);
+                const float tot = wave_sum(acc[0]);
+                res[0] = lane == i ? tot : res[0];
             }
         }
         // (the slices' barriers wait for LDS only: a full fence would drain the ring.  Walkers of a workgroup may

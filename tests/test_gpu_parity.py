@@ -99,8 +99,8 @@ def test_reference_recipe(gpu, kqo, name, family):
     (Q5_K, 3, 90, 1024), (Q5_K, 4, 300, 4096), (Q5_K, 4, 60, 8192), (Q5_K, 3, 50, 14336), (Q5_K, 4, 4096, 4096),
 ])
 def test_four_token_stream_kernels(gpu, kqo, type_, M, N, K):
-    """Every K-slice count (1, 2, 4, 7 waves), three tokens run as four with the last masked: the rows of Y
-    beyond M must stay untouched."""
+    """Every K-slice count (1, 2, 4, 7 waves) of the three- and the four-token form: the rows of Y beyond M must stay
+    untouched."""
     from backpack_amd import capi, kquant
     _say("four-token stream", type_, M, N, K)
     raw, packed, w = gpu.make_weight(type_, N, K, seed=M * 31 + N)
@@ -148,6 +148,27 @@ def test_odd_rows_per_walker(gpu, kqo, type_, M, N, K):
     got = out.cpu().numpy()
     assert np.all(got[M] == 7.5)
     gpu.check_matmul(kqo, type_, got[:M], X, packed, N, K, label=f"{type_} {M}x{N}x{K}")
+
+
+@pytest.mark.parametrize("type_,N,K", [
+    (Q4_K, 8193, 256), (Q4_K, 9216, 512), (Q4_K, 10240, 256), (Q4_K, 11264, 256), (Q4_K, 12288, 2048), (Q4_K, 66561, 256),   # four rows in flight
+    (Q4_K, 769, 8448), (Q4_K, 1537, 4352), (Q5_K, 769, 8448), (Q5_K, 1537, 4352), (Q4_K, 5, 8448), (Q5_K, 33281, 4352)])       # K slices
+def test_rows_behind_the_whole_rounds(gpu, kqo, type_, N, K):
+    """One token: a walker's rows are taken a round of its ring at a time, what is left of the last round behind the loop."""
+    from backpack_amd import capi, kquant
+    _say("rows behind the whole rounds", type_, N, K)
+    raw, packed, w = gpu.make_weight(type_, N, K, seed=N)
+    X = np.random.default_rng(K).standard_normal((1, K)).astype(np.float32)
+    out = gpu.dev(np.full((2, N), 7.5, np.float32))
+    capi.force_kernel(5)
+    try:
+        kquant.matmul(gpu.dev(X), w, out=out[:1])
+        assert capi.last_kernel() == "gemv_stream"
+    finally:
+        capi.force_kernel(0)
+    got = out.cpu().numpy()
+    assert np.all(got[1] == 7.5)
+    gpu.check_matmul(kqo, type_, got[:1], X, packed, N, K, label=f"{type_} {N}x{K}")
 
 
 @pytest.mark.parametrize("type_", [Q4_K, Q5_K, Q6_K])
