@@ -249,18 +249,17 @@ struct WideParams {
 template <int TYPE> struct WideW;
 template <> struct WideW<KQ_TYPE_Q4_K> {
     w_u32x4 hdr, q[2];
-    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t kq)
+    __device__ __forceinline__ void load_lds(const uint8_t* blk, const uint8_t*, uint32_t kq)
     {
         hdr = *(const w_u32x4*)blk;
         q[0] = *(const w_u32x4*)(blk + 16 + 32 * kq);
         q[1] = *(const w_u32x4*)(blk + 32 + 32 * kq);
     }
-    __device__ __forceinline__ void load_lds(const uint8_t* blk, const uint8_t*, uint32_t kq) { load(blk, kq); }
     __device__ __forceinline__ void arrived() const { asm volatile("" ::"v"(hdr), "v"(q[0]), "v"(q[1]) : "memory"); }
 };
 template <> struct WideW<KQ_TYPE_Q5_K> {
     w_u32x4 hdr, q[2], f[2];
-    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t kq)
+    __device__ __forceinline__ void load_lds(const uint8_t* blk, const uint8_t*, uint32_t kq)
     {
         hdr = *(const w_u32x4*)blk;
         f[0] = *(const w_u32x4*)(blk + 16);
@@ -268,22 +267,12 @@ template <> struct WideW<KQ_TYPE_Q5_K> {
         q[0] = *(const w_u32x4*)(blk + 48 + 32 * kq);
         q[1] = *(const w_u32x4*)(blk + 64 + 32 * kq);
     }
-    __device__ __forceinline__ void load_lds(const uint8_t* blk, const uint8_t*, uint32_t kq) { load(blk, kq); }
     __device__ __forceinline__ void arrived() const { asm volatile("" ::"v"(hdr), "v"(f[0]), "v"(f[1]), "v"(q[0]), "v"(q[1]) : "memory"); }
 };
 template <> struct WideW<KQ_TYPE_Q6_K> {
-    w_u32x4 ql[2], qh;   // (blocks are 210 bytes apart: 2-byte aligned loads)
+    w_u32x4 ql[2], qh;
     w_u32x2 sc;
     uint16_t d;
-    __device__ __forceinline__ void load(const uint8_t* blk, uint32_t kq)
-    {
-        const uint32_t h = kq >> 1, lh = kq & 1u;
-        __builtin_memcpy(&ql[0], blk + 64 * h + 16 * lh, 16);
-        __builtin_memcpy(&ql[1], blk + 64 * h + 32 + 16 * lh, 16);
-        __builtin_memcpy(&qh, blk + 128 + 32 * h + 16 * lh, 16);
-        __builtin_memcpy(&sc, blk + 192 + 8 * h, 8);
-        __builtin_memcpy(&d, blk + 208, 2);
-    }
     // the block's 208 bytes ahead of d on a 16-byte boundary, d in the upper half of a word of its own
     __device__ __forceinline__ void load_lds(const uint8_t* blk, const uint8_t* dw, uint32_t kq)
     {
@@ -301,9 +290,6 @@ __device__ __forceinline__ uint32_t w_mul2(uint32_t a, w_half2 s)
 {
     return __builtin_bit_cast(uint32_t, __builtin_bit_cast(w_half2, a) * s);
 }
-
-// LDS writes of the workgroup are visible behind it; loads in flight stay in flight.
-__device__ __forceinline__ void wide_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // Memory -> LDS without registers: lane l's 16 (4) bytes land at m0 + 16 l (4 l).  Inline asm, because the compiler
 // would wait for such a load ahead of every LDS read that it cannot tell apart from its target; the waits are the
