@@ -32,11 +32,12 @@
 // stand between the matrix instructions of the step before (sched_group_barrier), and the two meetings per superblock lie
 // ahead of a step whose operands are already in registers.  What that replaced: every lane fetched its 16-byte pieces
 // of W and X itself (52 cache accesses per load instruction, 20 now) and the compiler read operands right ahead of their
-// use.  What is left at 32 tokens and more is the board's power: with all CUs in these kernels the clock falls to 1.55 .. 1.78 GHz of 2.4
-// (s_memtime against s_memrealtime), so taking stalls or cheap instructions out changes little (the same walk with W a step earlier in
-// registers: +1 %), fewer matrix instructions or less switching on the vector units does (v_perm for the Q6_K fields: 31 -> 24 vector
-// instructions per eight weights, 5 to 7 % of its launches).  At 16 tokens and fewer it is the memory: 144 and 210 B pieces of rows reach 83
-// to 92 % of a contiguous read.  With one tile of 16 tokens a step is too short for the fixed order (`schedule`).
+// use.  What is left at 32 tokens and more: vector and matrix instructions on split operands (issue of both, and waits for 0.3 of the waves'
+// cycles), at a core clock of 1.8 .. 2.0 GHz of 2.43 while all CUs are in these kernels, in a launch alone as behind a thousand others
+// (s_memtime against s_memrealtime of each workgroup).  A walk with W a step earlier in registers gained 1 %, fewer vector
+// instructions more (v_perm for the Q6_K fields: 31 -> 24 per eight weights, 5 to 7 % of its launches).  At 16 tokens and fewer it is the
+// memory: 144 and 210 B pieces of rows reach 83 to 92 % of a contiguous read.  With one tile of 16 tokens a step is too short for the
+// fixed order (`schedule`).
 //
 // A workgroup may walk several groups of 256 rows against the same tokens as one sequence of superblocks (groups_per_wg): its
 // start (records, addresses, the first loads' way: 8 us of 25 .. 40) is paid once and a group's stores go under the next
@@ -564,9 +565,8 @@ __device__ __forceinline__ void wide_walk(const WideParams& p, uint8_t* lds, uin
     };
     w_half8 Bh[2][2], Bl[2][2];   // [step % 2][tile]
     // Q6_K: two of a word's bytes become 1024 + q in one byte permute against this constant, the shift that joins ql and qh is
-    // the one that takes the field to its place: 24 vector instructions per eight weights where masks and ors took 31.  These
-    // kernels run at the board's power limit (1.55 .. 1.78 GHz), so an instruction fewer counts although the matrix cores are no
-    // busier: 128256 x 4096 at 48 / 16 tokens 181.7 / 128.7 -> 174.7 / 123.3 us, 65536 x 4096 at 32 67.8 -> 64.4.
+    // the one that takes the field to its place: 24 vector instructions per eight weights where masks and ors took 31:
+    // 128256 x 4096 at 48 / 16 tokens 181.7 / 128.7 -> 174.7 / 123.3 us, 65536 x 4096 at 32 67.8 -> 64.4.
     uint32_t magic = 0x64646464u;
     asm("" : "+v"(magic));   // (in a vector register: v_perm_b32 takes one scalar)
     auto expand = [&](int j) {
@@ -1103,9 +1103,9 @@ hipError_t launch_wide_grouped(const MatmulArgs& a, const WideX& x, const uint32
 // stand between the matrix instructions of the step before.  A wave turns its 32 rows' weights into bf16 in registers (the GEMM's
 // formula and its one rounding, so both compute the same products; the quants enter v_fma_mix_f32 as fp16 subnormals where their
 // bits lie) and meets every token with them: no weight passes through LDS as bf16.  Accumulation is in fp32 over the workgroup's
-// whole range of K.  Read through registers, X and W ahead of a superblock and the operands right ahead of their use: 28672 x 4096
-// Q4_K at 100 tokens 52.0 -> 43.4 us, 4096 x 14336 Q6_K 37.9 -> 32.6, 28672 x 4096 at 32 tokens 28.9 -> 24.5, a layer at 100 tokens
-// 148 -> 131.
+// whole range of K.  Against X and W read through registers ahead of a superblock, and the operands right ahead of their use: 28672 x 4096
+// Q4_K at 100 tokens 51.7 -> 41.9 us, 4096 x 14336 Q6_K 37.8 -> 32.5, 28672 x 4096 at 32 tokens 28.9 -> 24.5, a layer with the launches
+// between its products at 100 tokens 158 -> 141.
 typedef __bf16 w_bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 w_bf16x2 __attribute__((ext_vector_type(2)));
 typedef float w_f32x2 __attribute__((ext_vector_type(2)));
